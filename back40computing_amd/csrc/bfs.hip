@@ -52,14 +52,21 @@ __global__ __launch_bounds__(256) void k_isolated(const int32_t* offs, int32_t n
 
 // Last node of a captured level loop: advances the phase base and publishes
 // the counters to the pinned host mirror, so the host's per-replay check
-// needs no separate device-to-host copy.
-__global__ void k_advance(BfsArgs a, int steps) {
+// needs no separate device-to-host copy.  The length published for the next
+// phase (`ph_rel` phases after the old base) includes the vertices that a
+// bottom-up step found, which are in no queue.
+__global__ void k_advance(BfsArgs a, int steps, int ph_rel) {
     constexpr int kWords = (int)(sizeof(DevCounters) / 4);
     constexpr int kPhWord = (int)(offsetof(DevCounters, ph_base) / 4);
     const uint32_t* src = reinterpret_cast<const uint32_t*>(a.ctr);
     uint32_t* dst = reinterpret_cast<uint32_t*>(a.hctr);
+    const int slot = (int)((src[kPhWord] + (uint32_t)ph_rel) & 3u);
+    unsigned long long sum = threadIdx.x < SPREAD ? *spread_at(a.spread, slot, threadIdx.x) : 0ull;
+    for (int d = SPREAD / 2; d >= 1; d >>= 1) sum += __shfl_xor(sum, d, kWave);
+    const uint32_t found = (uint32_t)__shfl(sum, 0, kWave);
     for (int i = threadIdx.x; i < kWords; i += blockDim.x) {
         uint32_t v = src[i];
+        if (i == slot) v += found;  // qlen[slot]
         if (i == kPhWord) {
             v += (uint32_t)steps;
             reinterpret_cast<uint32_t*>(a.ctr)[i] = v;
@@ -67,10 +74,11 @@ __global__ void k_advance(BfsArgs a, int steps) {
         dst[i] = v;
     }
 }
+static_assert(offsetof(DevCounters, qlen) == 0, "k_advance takes qlen[slot] for word `slot`");
 
 template <int KIND>
 __global__ __launch_bounds__(BFS_THREADS) void k_phase(BfsArgs a, int ph, int32_t depth, int slot) {
-    __shared__ LevelShared s;
+    __shared__ typename PhaseShared<KIND>::type s;
     phase_body<KIND>(a, ph, depth, slot, s);
 }
 
@@ -88,7 +96,7 @@ __global__ __launch_bounds__(BFS_THREADS) void k_heavy(BfsArgs a, int ph, int32_
 template <int KIND>
 __global__ __launch_bounds__(BFS_THREADS) void k_fused(BfsArgs a, int ph, int32_t depth, int max_levels,
                                                        uint32_t sat_limit) {
-    __shared__ LevelShared s;
+    __shared__ typename FusedShared<KIND>::type s;
     __shared__ typename FusedHeavy<KIND>::shared hs;
     fused_body<KIND>(a, ph, depth, max_levels, sat_limit, s, hs);
 }

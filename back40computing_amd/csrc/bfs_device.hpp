@@ -67,7 +67,23 @@ struct BfsArgs {
     int32_t coh_in;          // persistent: frontier inputs are read with coh_ld
     int32_t coh_out;         // persistent: outputs (queue, grid-tier entries) are written with coh_st
     long long edges;
+    int32_t by_label;        // small graphs: the depth labels mark visited vertices, not the bitmask (mark_claim)
+    unsigned long long* spread;  // direction-optimizing: per-level sums of what the steps found (spread_at)
 };
+
+// Same-address traffic is serialised at memory: every workgroup's atomic add
+// (or plain agent-scope store) to one 256-byte line costs 11.4 ns (33 ns), so
+// a counter that all 1,536 workgroups of a launch update costs 17.5 us per
+// launch, and 1.1 us when they update 16 counters 256 bytes apart.  Per-level
+// sums are therefore kept as SPREAD partial sums per level slot
+// (level & 3), one per 256-byte line; the next launch's readers add them up.
+// A partial sum is (edges << 32) | vertices (each fits: E < 2^31, V < 2^31).
+constexpr int SPREAD = 16;
+constexpr int SPREAD_STRIDE = 256 / (int)sizeof(unsigned long long);
+constexpr int SPREAD_WORDS = 4 * SPREAD * SPREAD_STRIDE;
+__device__ __forceinline__ unsigned long long* spread_at(unsigned long long* spread, int level, int i) {
+    return spread + ((level & 3) * SPREAD + i) * SPREAD_STRIDE;
+}
 
 // Frontier data that other workgroups of the same persistent launch read
 // after a grid barrier (queue entries, grid-tier entries and chunk maps).
@@ -99,8 +115,7 @@ __device__ __forceinline__ int2 coh_ld2(const int2* p, bool coh) {
     return make_int2((int32_t)(uint32_t)w, (int32_t)(uint32_t)(w >> 32));
 }
 
-constexpr int HEAVY_CHUNK = 256;     // grid-tier edges per work item (one per thread)
-constexpr int HEAVY_ROUND = 4;       // grid-tier work items a workgroup has in flight at once
+constexpr int HEAVY_CHUNK = 256;     // most grid-tier edges per work item
 
 // ---------------------------------------------------------------------------
 // LDS-buffered queue.  VCAP is the capacity of the value array: LQ_CAP for a
@@ -166,6 +181,52 @@ __device__ __forceinline__ void lq_append(LdsQueueT<VCAP>& q, const GlobalQueue&
     }
 }
 
+// lq_append of K entries per lane: one ballot per entry, but a single LDS
+// atomic for the wave.  Wave-uniform call.
+template <bool VALS, int K, int VCAP>
+__device__ __forceinline__ void lq_append_batch(LdsQueueT<VCAP>& q, const GlobalQueue& g, const bool (&want)[K],
+                                                const int32_t (&k)[K], const int32_t (&v)[K]) {
+    static_assert(!VALS || VCAP == LQ_CAP, "pair appends need a pair queue");
+    uint64_t m[K];
+    uint32_t cnt = 0;
+#pragma unroll
+    for (int r = 0; r < K; ++r) {
+        m[r] = __ballot(want[r]);
+        cnt += (uint32_t)__popcll(m[r]);
+    }
+    if (cnt == 0) return;
+    uint32_t base = 0;
+    if (lane_id() == 0) base = atomicAdd(&q.count, cnt);
+    base = (uint32_t)wave_bcast((int)base, 0);
+    // Entries past the LDS buffer go straight to the global queue.
+    const bool spills = base + cnt > (uint32_t)LQ_CAP;
+    const uint32_t spill_start = base > (uint32_t)LQ_CAP ? base : (uint32_t)LQ_CAP;
+    uint32_t gb = 0;
+    if (spills) {
+        if (lane_id() == 0) gb = atomic_add_u32(g.len, base + cnt - spill_start);
+        gb = (uint32_t)wave_bcast((int)gb, 0);
+    }
+    uint32_t at = base;
+#pragma unroll
+    for (int r = 0; r < K; ++r) {
+        const uint32_t pos = at + (uint32_t)lane_prefix(m[r]);
+        at += (uint32_t)__popcll(m[r]);
+        if (!want[r]) continue;
+        if (pos < (uint32_t)LQ_CAP) {
+            q.keys[pos] = k[r];
+            if (VALS) q.vals[pos] = v[r];
+        } else {
+            const uint32_t gp = gb + (pos - spill_start);
+            if (gp < g.cap) {
+                coh_st(&g.keys[gp], k[r], g.coh);
+                if (VALS) coh_st(&g.vals[gp], v[r], g.coh);
+            } else {
+                st_relaxed(g.overflow, 1u);
+            }
+        }
+    }
+}
+
 // Workgroup-uniform call.  Flushes when the buffer holds at least `min_fill`
 // entries (min_fill = 1: flush whatever is there).
 template <bool VALS, int VCAP>
@@ -205,6 +266,36 @@ __device__ __forceinline__ bool claim_exact(uint32_t* visited, int32_t v) {
     const uint32_t bit = 1u << (v & 31);
     if (*w & bit) return false;
     return (atomic_or_u32(w, bit) & bit) == 0;
+}
+
+// Marks of visited vertices.  Normally the bitmask: 32 times smaller than the
+// labels, so probes stay in L2.  But atomics on one 64-byte line are
+// serialised (11.4 ns each), a line of the bitmask holds 512 vertices, and a
+// graph of 4,096 vertices has only eight such lines: its widest top-down level
+// spent 23 us in claims.  Small graphs (by_label) therefore claim on the depth
+// label itself, 16 vertices to a line: an unsigned minimum, -1 being the
+// largest, which also labels the vertex.
+__device__ __forceinline__ uint32_t mark_load(const BfsArgs& a, int32_t v) {
+    return a.by_label ? (uint32_t)a.depth[v] : a.visited[v >> 5];
+}
+__device__ __forceinline__ bool mark_seen(const BfsArgs& a, int32_t v, uint32_t mark) {
+    return a.by_label ? mark != 0xFFFFFFFFu : ((mark >> (v & 31)) & 1u) != 0u;
+}
+// Returns the mark before the claim (mark_seen tells whether it was taken);
+// with by_label the winner's label is then already written.
+__device__ __forceinline__ uint32_t mark_claim(const BfsArgs& a, int32_t v, int32_t depth) {
+    if (a.by_label)
+        return __hip_atomic_fetch_min(reinterpret_cast<uint32_t*>(&a.depth[v]), (uint32_t)depth, __ATOMIC_RELAXED,
+                                      __HIP_MEMORY_SCOPE_AGENT);
+    return atomic_or_u32(&a.visited[v >> 5], 1u << (v & 31));
+}
+
+__device__ __forceinline__ bool visited_test(const BfsArgs& a, int32_t v) { return mark_seen(a, v, mark_load(a, v)); }
+
+// Exactly one caller per vertex returns true.
+__device__ __forceinline__ bool claim_exact(const BfsArgs& a, int32_t v, int32_t depth) {
+    if (visited_test(a, v)) return false;
+    return !mark_seen(a, v, mark_claim(a, v, depth));
 }
 
 struct HistoryHash {
@@ -314,6 +405,81 @@ __device__ __forceinline__ void tiered_gather(const int32_t* __restrict__ cols, 
         }
         __syncthreads();
     }
+}
+
+// ---------------------------------------------------------------------------
+// Positional gather: the lists of one tile (one per thread) laid end to end,
+// each thread taking K positions per step, BFS_THREADS apart.  A position is
+// mapped back to its list by binary search over the tile's ranks in LDS, so
+// work per step follows edges whatever the degrees, and the K edges' loads,
+// probes and claims (sink.step) are in flight together: a gather step is a
+// chain of dependent accesses and latency, not bandwidth, bounds it.
+// ---------------------------------------------------------------------------
+struct ListSmem {
+    int32_t rank[BFS_THREADS];  // first position of each list
+    int32_t base[BFS_THREADS];  // column index of position p of the list is base + p
+    int32_t src[BFS_THREADS];
+    int s_wave[BFS_WAVES];
+    uint32_t reserved;  // sinks that write in place: the tile's first output position
+};
+
+template <int K, typename Sink>
+__device__ __forceinline__ void gather_step(const int32_t* __restrict__ cols, const ListSmem& g, uint32_t p0,
+                                            uint32_t total, Sink& sink) {
+    int lo[K];
+    int32_t v[K], src[K];
+    bool valid[K];
+#pragma unroll
+    for (int r = 0; r < K; ++r) {
+        lo[r] = 0;
+        valid[r] = p0 + (uint32_t)(r * BFS_THREADS) + threadIdx.x < total;
+    }
+    // Last list with rank <= p; the K searches run side by side.
+#pragma unroll
+    for (int h = BFS_THREADS / 2; h >= 1; h >>= 1) {
+#pragma unroll
+        for (int r = 0; r < K; ++r) {
+            const int32_t p = (int32_t)(p0 + (uint32_t)(r * BFS_THREADS) + threadIdx.x);
+            if (g.rank[lo[r] + h] <= p) lo[r] += h;
+        }
+    }
+#pragma unroll
+    for (int r = 0; r < K; ++r) {
+        const int32_t p = (int32_t)(p0 + (uint32_t)(r * BFS_THREADS) + threadIdx.x);
+        src[r] = g.src[lo[r]];
+        v[r] = valid[r] ? cols[g.base[lo[r]] + p] : 0;
+    }
+    sink.template step<K>(p0, valid, v, src);
+}
+
+// Workgroup-uniform call.  sink.reserve(total, g) runs in thread 0 when the
+// tile has edges, sink.step wave-uniformly, sink.step_end() workgroup-
+// uniformly after every step.  With `parts` > 1 the
+// same tile is gathered by that many workgroups, each taking every parts-th
+// step (this one the part-th).
+constexpr int GATHER_K = 8;
+template <int KMAX, typename Sink>
+__device__ __forceinline__ void positional_gather(const int32_t* __restrict__ cols, int32_t src, int32_t start,
+                                                  int32_t deg, ListSmem& g, Sink& sink, uint32_t part = 0,
+                                                  uint32_t parts = 1) {
+    constexpr uint32_t STEP = (uint32_t)(KMAX * BFS_THREADS);
+    int sum;
+    const int rank = wg_exclusive_scan<BFS_THREADS>(deg, sum, g.s_wave);
+    const uint32_t total = (uint32_t)sum;
+    if ((uint64_t)part * STEP >= total) return;
+    g.rank[threadIdx.x] = rank;
+    g.base[threadIdx.x] = start - rank;
+    g.src[threadIdx.x] = src;
+    if (threadIdx.x == 0) sink.reserve(total, g);
+    __syncthreads();
+    for (uint64_t p0 = (uint64_t)part * STEP; p0 < total; p0 += (uint64_t)parts * STEP) {
+        if (total - (uint32_t)p0 <= 2u * BFS_THREADS)
+            gather_step<2>(cols, g, (uint32_t)p0, total, sink);
+        else
+            gather_step<KMAX>(cols, g, (uint32_t)p0, total, sink);
+        sink.step_end();
+    }
+    __syncthreads();
 }
 
 // ---------------------------------------------------------------------------

@@ -33,22 +33,43 @@ namespace b40c {
 // Level bodies (device).
 // ===========================================================================
 
-// LDS of a level step.  Keys-only steps (expand-contract, two-phase
-// contraction) and pair steps (contract-expand, two-phase filter) append to
-// the same pair-capable queue, so a persistent kernel that alternates them
-// keeps one valid count.
-struct LevelShared {
+constexpr int CONTRACT_K = 4;  // pairs per thread of a wide contraction
+
+// LDS of a level step.  Keys-only steps (two-phase contraction) and pair
+// steps (contract-expand, two-phase filter) append to the same pair-capable
+// queue, so a persistent kernel that alternates them keeps one valid count.
+struct PairLevelShared {
     LdsPairQueue q;
-    GatherSmem g;
+    ListSmem l;
     HistoryHash hist;
     unsigned long long red[BFS_WAVES];
     uint32_t ctl;  // persistent kernels: loop control, read by one thread per workgroup
 };
 
-__device__ __forceinline__ void shared_init(LevelShared& s) {
+// Contract-expand steps also hold the survivors of one wide tile.
+struct LevelShared : PairLevelShared {
+    int32_t kept_v[CONTRACT_K * BFS_THREADS];
+    int32_t kept_start[CONTRACT_K * BFS_THREADS];
+    int32_t kept_deg[CONTRACT_K * BFS_THREADS];
+};
+
+// Expand-contract and two-phase expand steps only ever append keys, if
+// anything, and keep no history: less than half the LDS, so more workgroups
+// stay resident.
+struct TdLevelShared {
+    LdsKeyQueue q;
+    ListSmem l;
+    unsigned long long red[BFS_WAVES];
+    uint32_t ctl;
+};
+
+__device__ __forceinline__ void shared_init(PairLevelShared& s) {
     if (threadIdx.x == 0) s.q.count = 0;
-    gather_init(s.g);
     history_init(s.hist);
+    __syncthreads();
+}
+__device__ __forceinline__ void shared_init(TdLevelShared& s) {
+    if (threadIdx.x == 0) s.q.count = 0;
     __syncthreads();
 }
 
@@ -75,28 +96,53 @@ __device__ __forceinline__ uint32_t input_len(const BfsArgs& a, int ph, uint32_t
     return n_in == kLenFromCounters ? phase_input_len(a, ph) : n_in;
 }
 
-__device__ __forceinline__ void phase_begin(const BfsArgs& a, int ph, uint32_t n_in) {
+// `frontier_depth` >= 0: the phase's input vertices carry that label, so a
+// nonempty input makes it the deepest one so far (one store by workgroup 0;
+// a maximum taken by every workgroup would be serialised at one address).
+__device__ __forceinline__ void phase_begin(const BfsArgs& a, int ph, uint32_t n_in, int32_t frontier_depth = -1) {
     if (blockIdx.x == 0 && threadIdx.x == 0) {
+        if (frontier_depth >= 0 && n_in) st_relaxed(a.max_depth, (uint32_t)frontier_depth);
         st_relaxed(&a.ctr->qlen[(ph + 2) & 3], 0u);
         __hip_atomic_store(&a.ctr->heavy_alloc[(ph + 1) & 1], 0ull, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-        a.ctr->level_edges[(ph + 2) & 3] = 0ull;
         if (n_in) atomic_add_u64(&a.ctr->queued, n_in);
     }
 }
 
-// Frontier entries per workgroup per step of a gathering phase.  Level
-// launches take full tiles of BFS_THREADS.  A persistent launch spreads a
-// frontier smaller than its grid's tiles evenly over all its workgroups: every level of a high-diameter graph is such a frontier, and
-// spread out each workgroup gathers its few lists' edges in one round of
-// the fine tier instead of a few workgroups gathering full tiles in several
-// rounds, each a dependent chain (column, visited word, claiming atomic).
-// Level launches run four times as many workgroups, and there the extra
-// workgroups' same-address queue and depth atomics cost more than the
-// rounds saved (200^3 lattice: 25 instead of 17 us per level).
-__device__ __forceinline__ uint32_t entries_per_wg(const BfsArgs& a, uint32_t n_in, uint32_t nblocks) {
-    if (!a.persistent || (uint64_t)n_in >= (uint64_t)nblocks * BFS_THREADS) return BFS_THREADS;
-    const uint32_t per = (n_in + nblocks - 1) / nblocks;
-    return per < 1u ? 1u : per;
+// How a gathering phase deals its input entries out to the `wgs` workgroups
+// taking part: in turns of 2^turn consecutive entries.  Neighbouring entries
+// thus go to different workgroups: discovery order puts an RMAT graph's hubs
+// (low ids, first in every sorted list) next to each other, and with
+// contiguous tiles the workgroup that got them was the level (RMAT-20's widest
+// level: 489 us for the slowest of 512 workgroups, 181 us on average).
+// Longer turns read the queue in fewer lines: single entries while a
+// workgroup gets fewer than 16 of them, 16 bytes (a line of an edge
+// frontier, which has more entries and culls most) up to a full tile (with
+// single entries there, a 100^3 lattice search is 5 % slower), then a line
+// of a vertex frontier; an edge frontier that wide is read in whole tiles
+// (with single entries RMAT-22 contract-expand took 5.9 instead of 4.4 ms),
+// since its culled tiles differ little.
+struct Deal {
+    uint32_t wgs, turn;
+    __device__ __forceinline__ uint32_t entry(uint32_t base, uint32_t wg) const {
+        const uint32_t t = threadIdx.x;
+        return base + ((((t >> turn) * wgs + wg) << turn) | (t & ((1u << turn) - 1u)));
+    }
+};
+__device__ __forceinline__ Deal deal_out(uint32_t n_in, uint32_t wgs, bool edges) {
+    const uint64_t w = wgs;
+    const uint32_t mid = edges ? 4u : 2u, wide = edges ? 8u : 4u;
+    return Deal{wgs, n_in < 16 * w ? 0u : n_in < BFS_THREADS * w ? mid : wide};
+}
+
+// Workgroups taking part.  Level launches use no more than there are full
+// tiles; a persistent launch uses all of its grid, so that on the narrow
+// levels of a high-diameter graph every workgroup gathers its few lists in one
+// step.  Level launches run four times as many workgroups, and there the extra
+// workgroups' same-address queue atomics cost more than the steps saved
+// (200^3 lattice: 25 instead of 17 us per level).
+__device__ __forceinline__ uint32_t sharing_wgs(const BfsArgs& a, uint32_t n_in, uint32_t nblocks) {
+    if (a.persistent) return nblocks;
+    return min(nblocks, (n_in + BFS_THREADS - 1) / BFS_THREADS);
 }
 
 __device__ __forceinline__ GlobalQueue out_queue(const BfsArgs& a, int ph) {
@@ -160,8 +206,34 @@ __device__ __forceinline__ void defer_heavy(const BfsArgs& a, int ph, int32_t v,
     }
 }
 
-// Top-down discovery sink: exact claim, labels, optional frontier bitmap bit
-// and degree accounting for the direction switch, then the LDS queue.
+// Top-down discovery: exact claims and labels of the K edges of a gather
+// step, each access for all of them together; `won` marks the edges that
+// discovered their neighbour.
+template <int K>
+__device__ __forceinline__ void td_claim(const BfsArgs& a, const bool (&valid)[K], const int32_t (&v)[K],
+                                         const int32_t (&src)[K], int32_t depth_next, bool (&won)[K]) {
+    uint32_t seen[K];
+#pragma unroll
+    for (int r = 0; r < K; ++r) {
+        seen[r] = 0u;
+        if (valid[r]) seen[r] = mark_load(a, v[r]);
+        won[r] = valid[r] && !mark_seen(a, v[r], seen[r]);
+    }
+#pragma unroll
+    for (int r = 0; r < K; ++r)
+        if (won[r]) seen[r] = mark_claim(a, v[r], depth_next);
+#pragma unroll
+    for (int r = 0; r < K; ++r) {
+        won[r] = won[r] && !mark_seen(a, v[r], seen[r]);
+        if (won[r]) {
+            if (!a.by_label) a.depth[v[r]] = depth_next;
+            a.pred[v[r]] = src[r];
+        }
+    }
+}
+
+// Top-down sink: optional frontier bitmap bit and degree accounting for the
+// direction switch, then the LDS queue.
 template <int VCAP>
 struct TdSink {
     const BfsArgs& a;
@@ -170,40 +242,78 @@ struct TdSink {
     uint32_t* next_bm;
     int32_t depth_next;
     bool count_edges;
-    bool found;
     unsigned long long eacc;
-    __device__ __forceinline__ void operator()(bool valid, int32_t v, int32_t src) {
-        const bool won = valid && claim_exact(a.visited, v);
-        if (won) {
-            a.depth[v] = depth_next;
-            a.pred[v] = src;
-            found = true;
-            if (next_bm) atomic_or_u32(&next_bm[v >> 5], 1u << (v & 31));
-            if (count_edges) eacc += (unsigned long long)(a.offs[v + 1] - a.offs[v]);
+    __device__ __forceinline__ void reserve(uint32_t, ListSmem&) {}
+    template <int K>
+    __device__ __forceinline__ void step(uint32_t, const bool (&valid)[K], const int32_t (&v)[K],
+                                         const int32_t (&src)[K]) {
+        bool won[K];
+        td_claim(a, valid, v, src, depth_next, won);
+        if (next_bm) {
+#pragma unroll
+            for (int r = 0; r < K; ++r)
+                if (won[r]) atomic_or_u32(&next_bm[v[r] >> 5], 1u << (v[r] & 31));
         }
-        lq_append<false>(q, out, won, v, 0);
+        if (count_edges) {
+#pragma unroll
+            for (int r = 0; r < K; ++r)
+                if (won[r]) eacc += (unsigned long long)(a.offs[v[r] + 1] - a.offs[v[r]]);
+        }
+        lq_append_batch<false>(q, out, won, v, v);
     }
+    __device__ __forceinline__ void step_end() { lq_flush<false>(q, out, LQ_CAP / 2); }
 };
 
+// Every edge as a (neighbour, source) pair through the LDS queue.
 struct PairSink {
-    LevelShared& s;
+    LdsPairQueue& q;
     const GlobalQueue& out;
-    __device__ __forceinline__ void operator()(bool valid, int32_t nbr, int32_t src) {
-        lq_append<true>(s.q, out, valid, nbr, src);
+    __device__ __forceinline__ void reserve(uint32_t, ListSmem&) {}
+    template <int K>
+    __device__ __forceinline__ void step(uint32_t, const bool (&valid)[K], const int32_t (&nbr)[K],
+                                         const int32_t (&src)[K]) {
+        lq_append_batch<true>(q, out, valid, nbr, src);
     }
+    __device__ __forceinline__ void step_end() { lq_flush<true>(q, out, LQ_CAP / 2); }
 };
 
-// The deepest label: one atomic per workgroup that found a vertex.  A
-// persistent launch leaves it to workgroup 0, which learns
-// after the level's barrier whether the next frontier is empty (every
-// vertex a top-down step claims is enqueued), so the grid's workgroups do
-// not all hit one counter at every level.
+// Every edge as a pair, written in place: all of a tile's edges are output,
+// so one atomic reserves them and position p goes to slot reserved + p.
+struct InPlaceSink {
+    const GlobalQueue& out;
+    ListSmem& g;
+    __device__ __forceinline__ void reserve(uint32_t total, ListSmem& l) {
+        const uint32_t base = atomic_add_u32(out.len, total);
+        if ((uint64_t)base + total > out.cap) st_relaxed(out.overflow, 1u);
+        l.reserved = base;
+    }
+    template <int K>
+    __device__ __forceinline__ void step(uint32_t p0, const bool (&valid)[K], const int32_t (&nbr)[K],
+                                         const int32_t (&src)[K]) {
+        const uint64_t base = (uint64_t)g.reserved + p0 + threadIdx.x;
+#pragma unroll
+        for (int r = 0; r < K; ++r) {
+            const uint64_t pos = base + (uint32_t)(r * BFS_THREADS);
+            if (valid[r] && pos < out.cap) {
+                coh_st(&out.keys[pos], nbr[r], out.coh);
+                coh_st(&out.vals[pos], src[r], out.coh);
+            }
+        }
+    }
+    __device__ __forceinline__ void step_end() {}
+};
+
+// Workgroup sum of a per-thread degree count, added to the level's partial
+// sums of the degrees of discovered vertices.
+__device__ __forceinline__ void add_level_edges(const BfsArgs& a, int ph, unsigned long long edges,
+                                                unsigned long long* red) {
+    wg_add_u64(edges << 32, spread_at(a.spread, ph + 1, blockIdx.x % SPREAD), red);
+}
+
 template <int VCAP>
 __device__ __forceinline__ void td_finish(const BfsArgs& a, int ph, TdSink<VCAP>& sink, unsigned long long* red) {
     lq_flush<false>(sink.q, sink.out, 1);
-    if (sink.count_edges) wg_add_u64(sink.eacc, &a.ctr->level_edges[(ph + 1) & 3], red);
-    if (a.persistent) return;
-    if (__syncthreads_or(sink.found) && threadIdx.x == 0) atomic_max_u32(a.max_depth, (uint32_t)sink.depth_next);
+    if (sink.count_edges) add_level_edges(a, ph, sink.eacc, red);
 }
 
 // Expand-contract (vertex frontier -> vertex frontier).  Neighbours are
@@ -211,30 +321,83 @@ __device__ __forceinline__ void td_finish(const BfsArgs& a, int ph, TdSink<VCAP>
 // expand_contract_atomic/cta.cuh:212-214, and compacted into the next vertex
 // frontier.
 // `nblocks` workgroups (the first ones of the launch) share the frontier;
-// lists of at least `grid_th` edges go to the grid tier (k_heavy).
-template <int VCAP>
+// lists of at least `grid_th` edges go to the grid tier (k_heavy), or, with
+// `split`, no list does: while the frontier has fewer tiles than half the
+// workgroups, several workgroups read the same tile and share its edges.
+// That replaces the grid tier's launch (4 us even when it finds nothing) on
+// the narrow levels where a hub would keep one workgroup busy.
+template <int KMAX, int VCAP>
 __device__ void td_phase(const BfsArgs& a, int ph, int32_t depth_next, uint32_t* next_bm, bool count_edges,
-                         LdsQueueT<VCAP>& q, GatherSmem& g, unsigned long long* red, uint32_t nblocks,
-                         int32_t grid_th, uint32_t n_in_arg = kLenFromCounters) {
+                         LdsQueueT<VCAP>& q, ListSmem& g, unsigned long long* red, uint32_t nblocks,
+                         int32_t grid_th, uint32_t n_in_arg = kLenFromCounters, bool split = false) {
     const uint32_t n_in = input_len(a, ph, n_in_arg);
-    phase_begin(a, ph, n_in);
+    phase_begin(a, ph, n_in, a.persistent ? -1 : depth_next - 1);
     const int32_t* qin = a.qk[ph & 1];
     const GlobalQueue out = out_queue(a, ph);
-    TdSink<VCAP> sink{a, q, out, next_bm, depth_next, count_edges, false, 0ull};
-    const uint32_t per = entries_per_wg(a, n_in, nblocks);
-    for (uint32_t base = blockIdx.x * per; base < n_in; base += nblocks * per) {
-        const uint32_t i = base + threadIdx.x;
+    TdSink<VCAP> sink{a, q, out, next_bm, depth_next, count_edges, 0ull};
+    uint32_t wgs = sharing_wgs(a, n_in, nblocks), wg = blockIdx.x, part = 0, parts = 1;
+    if (split && wgs && nblocks >= 2 * wgs) {
+        // The remainder of the division takes no part.
+        parts = nblocks / wgs;
+        part = blockIdx.x / wgs;
+        wg = part < parts ? blockIdx.x % wgs : wgs;
+    }
+    const Deal deal = deal_out(n_in, wgs, false);
+    for (uint32_t base = 0; wg < wgs && base < n_in; base += wgs * BFS_THREADS) {
+        const uint32_t i = deal.entry(base, wg);
         int32_t u = -1, start = 0, deg = 0;
-        if (threadIdx.x < per && i < n_in) {
+        if (i < n_in) {
             u = coh_ld(&qin[i], a.coh_in != 0);
             if (valid_vertex(a, u)) {
                 start = a.offs[u];
                 deg = a.offs[u + 1] - start;
             }
         }
-        defer_heavy(a, ph, u, deg, grid_th);
-        tiered_gather(a.cols, u, start, deg, a.cta_th, a.wave_th, g, sink);
-        lq_flush<false>(q, out, LQ_CAP / 2);
+        if (!split) defer_heavy(a, ph, u, deg, grid_th);
+        positional_gather<KMAX>(a.cols, u, start, deg, g, sink, part, parts);
+    }
+    td_finish(a, ph, sink, red);
+}
+
+// The same step over a frontier held as a bitmap (a bottom-up step leaves no
+// vertex queue): each workgroup takes 256-word pieces of the bitmap, lists
+// their vertices in LDS and gathers them 256 at a time.
+constexpr int BM_LIST = 1024;
+template <int KMAX, int VCAP>
+__device__ void td_bitmap_phase(const BfsArgs& a, int ph, int32_t depth_next, const uint32_t* cur, uint32_t* next_bm,
+                                LdsQueueT<VCAP>& q, ListSmem& g, int32_t* list, unsigned long long* red,
+                                uint32_t nblocks, int32_t grid_th, uint32_t n_in) {
+    phase_begin(a, ph, n_in, depth_next - 1);
+    const GlobalQueue out = out_queue(a, ph);
+    TdSink<VCAP> sink{a, q, out, next_bm, depth_next, true, 0ull};
+    for (int32_t w0 = (int32_t)blockIdx.x * BFS_THREADS; w0 < a.words; w0 += (int32_t)nblocks * BFS_THREADS) {
+        const int32_t w = w0 + (int32_t)threadIdx.x;
+        uint32_t bits = w < a.words ? cur[w] : 0u;
+        int total;
+        int at = wg_exclusive_scan<BFS_THREADS>(__popcll((unsigned long long)bits), total, g.s_wave);
+        for (int l0 = 0; l0 < total; l0 += BM_LIST) {
+            while (bits && at < l0 + BM_LIST) {
+                list[at - l0] = w * 32 + (__ffsll((unsigned long long)bits) - 1);
+                bits &= bits - 1;
+                ++at;
+            }
+            __syncthreads();
+            const int cnt = min(BM_LIST, total - l0);
+            for (int i0 = 0; i0 < cnt; i0 += BFS_THREADS) {
+                const int i = i0 + (int)threadIdx.x;
+                int32_t u = -1, start = 0, deg = 0;
+                if (i < cnt) {
+                    u = list[i];
+                    if (valid_vertex(a, u)) {
+                        start = a.offs[u];
+                        deg = a.offs[u + 1] - start;
+                    }
+                }
+                defer_heavy(a, ph, u, deg, grid_th);
+                positional_gather<KMAX>(a.cols, u, start, deg, g, sink);
+            }
+            __syncthreads();
+        }
     }
     td_finish(a, ph, sink, red);
 }
@@ -244,147 +407,162 @@ __device__ void td_phase(const BfsArgs& a, int ph, int32_t depth_next, uint32_t*
 // labelled at contraction (depth = depth_here), then the survivors'
 // neighbour lists are expanded into the outgoing edge frontier
 // (contract_expand_atomic/cta.cuh:573-709).
+//
+// Wide frontiers are contracted CONTRACT_K pairs per thread, each access of
+// the chain (pair, mark, claim, row offsets) for all of them together; the
+// few survivors are compacted in LDS and their lists gathered 256 at a time.
+
+// Contracts K pairs per thread; returns what each lane keeps.
+template <int K>
+__device__ __forceinline__ void contract_pairs(const BfsArgs& a, int ph, const uint32_t (&i)[K], uint32_t n_in,
+                                               int32_t depth_here, HistoryHash& hist, bool (&keep)[K],
+                                               int32_t (&v)[K]) {
+    const int32_t* qk = a.qk[ph & 1];
+    const int32_t* qv = a.qv[ph & 1];
+    int32_t p[K];
+    uint32_t mark[K];
+#pragma unroll
+    for (int r = 0; r < K; ++r) {
+        v[r] = i[r] < n_in ? coh_ld(&qk[i[r]], a.coh_in != 0) : -1;
+        p[r] = i[r] < n_in ? coh_ld(&qv[i[r]], a.coh_in != 0) : 0;
+    }
+#pragma unroll
+    for (int r = 0; r < K; ++r) {
+        keep[r] = i[r] < n_in && valid_vertex(a, v[r]);
+        mark[r] = keep[r] ? mark_load(a, v[r]) : 0u;
+    }
+#pragma unroll
+    for (int r = 0; r < K; ++r) keep[r] = keep[r] && !mark_seen(a, v[r], mark[r]) && !history_seen(hist, v[r]);
+#pragma unroll
+    for (int r = 0; r < K; ++r)
+        if (keep[r]) mark[r] = mark_claim(a, v[r], depth_here);
+#pragma unroll
+    for (int r = 0; r < K; ++r) {
+        keep[r] = keep[r] && !mark_seen(a, v[r], mark[r]);
+        if (keep[r]) {
+            if (!a.by_label) a.depth[v[r]] = depth_here;
+            a.pred[v[r]] = p[r];
+        }
+    }
+}
+
+// The deepest label: vertices that a contraction labels are the next phases'
+// frontier, or their edges are, so a later phase sees that there were some.
+// Only those without out-edges leave nothing behind (`sinks`).
+__device__ __forceinline__ void raise_max_depth(const BfsArgs& a, bool sinks, int32_t depth) {
+    if (__syncthreads_or(sinks) && threadIdx.x == 0) atomic_max_u32(a.max_depth, (uint32_t)depth);
+}
+
 __device__ void ce_phase(const BfsArgs& a, int ph, int32_t depth_here, LevelShared& s,
                          uint32_t n_in_arg = kLenFromCounters) {
     const uint32_t n_in = input_len(a, ph, n_in_arg);
-    phase_begin(a, ph, n_in);
-    const int32_t* qk = a.qk[ph & 1];
-    const int32_t* qv = a.qv[ph & 1];
+    phase_begin(a, ph, n_in, a.persistent ? -1 : depth_here - 1);
     const GlobalQueue out = out_queue(a, ph);
-    PairSink sink{s, out};
-    bool found = false;
-    const uint32_t per = entries_per_wg(a, n_in, gridDim.x);
-    for (uint32_t base = blockIdx.x * per; base < n_in; base += gridDim.x * per) {
-        const uint32_t i = base + threadIdx.x;
-        int32_t v = -1, start = 0, deg = 0;
-        if (threadIdx.x < per && i < n_in) {
-            v = coh_ld(&qk[i], a.coh_in != 0);
-            const int32_t p = coh_ld(&qv[i], a.coh_in != 0);
-            bool keep = valid_vertex(a, v);
-            if (keep) keep = !visited_test(a.visited, v);
-            if (keep) keep = !history_seen(s.hist, v);
-            if (keep) keep = claim_exact(a.visited, v);
-            if (keep) {
-                a.depth[v] = depth_here;
-                a.pred[v] = p;
-                found = true;
-                start = a.offs[v];
-                deg = a.offs[v + 1] - start;
+    PairSink sink{s.q, out};
+    bool sinks = false;
+    const uint32_t wgs = sharing_wgs(a, n_in, gridDim.x);
+    const Deal deal = deal_out(n_in, wgs, true);
+    uint32_t base = 0;
+    for (; blockIdx.x < wgs && n_in - base >= wgs * (uint32_t)(CONTRACT_K * BFS_THREADS);
+         base += wgs * (uint32_t)(CONTRACT_K * BFS_THREADS)) {
+        uint32_t i[CONTRACT_K];
+        bool keep[CONTRACT_K];
+        int32_t v[CONTRACT_K], start[CONTRACT_K], deg[CONTRACT_K];
+#pragma unroll
+        for (int r = 0; r < CONTRACT_K; ++r) i[r] = deal.entry(base + (uint32_t)r * wgs * BFS_THREADS, blockIdx.x);
+        contract_pairs<CONTRACT_K>(a, ph, i, n_in, depth_here, s.hist, keep, v);
+        int cnt = 0;
+#pragma unroll
+        for (int r = 0; r < CONTRACT_K; ++r) {
+            start[r] = deg[r] = 0;
+            if (keep[r]) {
+                start[r] = a.offs[v[r]];
+                deg[r] = a.offs[v[r] + 1];
             }
         }
-        defer_heavy(a, ph, v, deg, a.grid_th);
-        tiered_gather(a.cols, v, start, deg, a.cta_th, a.wave_th, s.g, sink);
-        lq_flush<true>(s.q, out, LQ_CAP / 2);
+#pragma unroll
+        for (int r = 0; r < CONTRACT_K; ++r) {
+            deg[r] -= start[r];
+            sinks |= keep[r] && deg[r] == 0;
+            cnt += deg[r] > 0 ? 1 : 0;
+        }
+        int kept;
+        int at = wg_exclusive_scan<BFS_THREADS>(cnt, kept, s.l.s_wave);
+#pragma unroll
+        for (int r = 0; r < CONTRACT_K; ++r)
+            if (deg[r] > 0) {
+                s.kept_v[at] = v[r];
+                s.kept_start[at] = start[r];
+                s.kept_deg[at] = deg[r];
+                ++at;
+            }
+        __syncthreads();
+        for (int k0 = 0; k0 < kept; k0 += BFS_THREADS) {
+            const int k = k0 + (int)threadIdx.x;
+            int32_t u = -1, us = 0, ud = 0;
+            if (k < kept) {
+                u = s.kept_v[k];
+                us = s.kept_start[k];
+                ud = s.kept_deg[k];
+            }
+            defer_heavy(a, ph, u, ud, a.grid_th);
+            positional_gather<GATHER_K>(a.cols, u, us, ud, s.l, sink);
+        }
+        __syncthreads();
+    }
+    for (; blockIdx.x < wgs && base < n_in; base += wgs * BFS_THREADS) {
+        const uint32_t i[1] = {deal.entry(base, blockIdx.x)};
+        bool keep[1];
+        int32_t v[1], start = 0, deg = 0;
+        contract_pairs<1>(a, ph, i, n_in, depth_here, s.hist, keep, v);
+        if (keep[0]) {
+            start = a.offs[v[0]];
+            deg = a.offs[v[0] + 1] - start;
+            sinks |= deg == 0;
+        }
+        defer_heavy(a, ph, v[0], deg, a.grid_th);
+        positional_gather<GATHER_K>(a.cols, v[0], start, deg, s.l, sink);
     }
     lq_flush<true>(s.q, out, 1);
-    if (__syncthreads_or(found) && threadIdx.x == 0) atomic_max_u32(a.max_depth, (uint32_t)depth_here);
+    raise_max_depth(a, sinks, depth_here);
 }
 
 // Two-phase contract (edge frontier -> vertex frontier + labels),
 // two_phase/contract_atomic/cta.cuh:494-572.
-__device__ void tp_contract_phase(const BfsArgs& a, int ph, int32_t depth_here, LevelShared& s,
+__device__ void tp_contract_phase(const BfsArgs& a, int ph, int32_t depth_here, PairLevelShared& s,
                                   uint32_t n_in_arg = kLenFromCounters) {
     const uint32_t n_in = input_len(a, ph, n_in_arg);
     phase_begin(a, ph, n_in);
-    const int32_t* qk = a.qk[ph & 1];
-    const int32_t* qv = a.qv[ph & 1];
     const GlobalQueue out = out_queue(a, ph);
-    bool found = false;
-    for (uint32_t base = blockIdx.x * BFS_THREADS; base < n_in; base += gridDim.x * BFS_THREADS) {
-        const uint32_t i = base + threadIdx.x;
-        bool keep = false;
-        int32_t v = -1;
-        if (i < n_in) {
-            v = coh_ld(&qk[i], a.coh_in != 0);
-            const int32_t p = coh_ld(&qv[i], a.coh_in != 0);
-            keep = valid_vertex(a, v);
-            if (keep) keep = !visited_test(a.visited, v);
-            if (keep) keep = !history_seen(s.hist, v);
-            if (keep) keep = claim_exact(a.visited, v);
-            if (keep) {
-                a.depth[v] = depth_here;
-                a.pred[v] = p;
-                found = true;
-            }
-        }
-        lq_append<false>(s.q, out, keep, v, 0);
+    for (uint64_t base = (uint64_t)blockIdx.x * BFS_THREADS; base < n_in;
+         base += (uint64_t)gridDim.x * BFS_THREADS * CONTRACT_K) {
+        uint32_t i[CONTRACT_K];
+        bool keep[CONTRACT_K];
+        int32_t v[CONTRACT_K];
+#pragma unroll
+        for (int r = 0; r < CONTRACT_K; ++r)
+            i[r] = (uint32_t)min<uint64_t>(base + (uint64_t)r * gridDim.x * BFS_THREADS + threadIdx.x, n_in);
+        contract_pairs<CONTRACT_K>(a, ph, i, n_in, depth_here, s.hist, keep, v);
+        lq_append_batch<false>(s.q, out, keep, v, v);
         lq_flush<false>(s.q, out, LQ_CAP / 2);
     }
     lq_flush<false>(s.q, out, 1);
-    if (__syncthreads_or(found) && threadIdx.x == 0) atomic_max_u32(a.max_depth, (uint32_t)depth_here);
-}
-
-// Positional expansion of one tile of lists (workgroup-uniform call): every
-// edge is output, so the tile's output size is the sum of its degrees.  One
-// atomic reserves it; each position is mapped back to its list by binary
-// search over the tile's ranks (staged in LDS) and written in place as
-// (neighbour, source), EXPAND_ITEMS positions per thread with their loads
-// issued together.  Work per workgroup follows edges, not lists.
-constexpr int EXPAND_ITEMS = 8;
-__device__ __forceinline__ void expand_tile_in_place(const BfsArgs& a, const GlobalQueue& out, int32_t u,
-                                                     int32_t start, int32_t deg, GatherSmem& g) {
-    const int tid = threadIdx.x;
-    int total;
-    const int rank = wg_exclusive_scan<BFS_THREADS>(deg, total, g.s_wave);
-    if (total == 0) return;
-    int32_t* s_rank = g.goff;
-    int32_t* s_start = g.goff + BFS_THREADS;
-    int32_t* s_src = g.gsrc;
-    s_rank[tid] = rank;
-    s_start[tid] = start;
-    s_src[tid] = u;
-    if (tid == 0) {
-        const uint32_t base = atomic_add_u32(out.len, (uint32_t)total);
-        if ((uint64_t)base + (uint64_t)total > out.cap) st_relaxed(out.overflow, 1u);
-        g.o_start = (int32_t)base;
-    }
-    __syncthreads();
-    const uint32_t base = (uint32_t)g.o_start;
-    int lo = 0;
-    for (int p0 = 0; p0 < total; p0 += BFS_THREADS * EXPAND_ITEMS) {
-        int32_t col[EXPAND_ITEMS], src[EXPAND_ITEMS];
-#pragma unroll
-        for (int r = 0; r < EXPAND_ITEMS; ++r) {
-            const int p = p0 + r * BFS_THREADS + tid;
-            col[r] = -1;
-            if (p < total) {
-                // Last list with rank <= p; positions rise with r and p0.
-                int hi = BFS_THREADS;
-                while (hi - lo > 1) {
-                    const int mid = (lo + hi) >> 1;
-                    if (s_rank[mid] <= p) lo = mid;
-                    else hi = mid;
-                }
-                col[r] = s_start[lo] + (p - s_rank[lo]);
-                src[r] = s_src[lo];
-            }
-        }
-        int32_t v[EXPAND_ITEMS];
-#pragma unroll
-        for (int r = 0; r < EXPAND_ITEMS; ++r) v[r] = col[r] >= 0 ? a.cols[col[r]] : 0;
-#pragma unroll
-        for (int r = 0; r < EXPAND_ITEMS; ++r) {
-            if (col[r] < 0) continue;
-            const uint64_t pos = (uint64_t)base + (uint32_t)(p0 + r * BFS_THREADS + tid);
-            if (pos < out.cap) {
-                coh_st(&out.keys[pos], v[r], out.coh);
-                coh_st(&out.vals[pos], src[r], out.coh);
-            }
-        }
-    }
-    __syncthreads();
 }
 
 // Two-phase expand (vertex frontier -> edge frontier of (neighbour, pred)),
 // two_phase/expand_atomic/cta.cuh:606-719.  No culling: lists below the
 // grid threshold are expanded in place per tile, longer ones by k_heavy.
-__device__ void tp_expand_phase(const BfsArgs& a, int ph, LevelShared& s, uint32_t n_in_arg = kLenFromCounters) {
+__device__ void tp_expand_phase(const BfsArgs& a, int ph, int32_t depth_here, ListSmem& l,
+                                uint32_t n_in_arg = kLenFromCounters) {
     const uint32_t n_in = input_len(a, ph, n_in_arg);
-    phase_begin(a, ph, n_in);
+    phase_begin(a, ph, n_in, depth_here);
     const int32_t* qin = a.qk[ph & 1];
     const GlobalQueue out = out_queue(a, ph);
-    for (uint32_t base = blockIdx.x * BFS_THREADS; base < n_in; base += gridDim.x * BFS_THREADS) {
-        const uint32_t i = base + threadIdx.x;
+    InPlaceSink sink{out, l};
+    const uint32_t wgs = sharing_wgs(a, n_in, gridDim.x);
+    const Deal deal = deal_out(n_in, wgs, false);
+    for (uint32_t base = 0; blockIdx.x < wgs && base < n_in; base += wgs * BFS_THREADS) {
+        const uint32_t i = deal.entry(base, blockIdx.x);
         int32_t u = -1, start = 0, deg = 0;
         if (i < n_in) {
             u = coh_ld(&qin[i], a.coh_in != 0);
@@ -394,30 +572,39 @@ __device__ void tp_expand_phase(const BfsArgs& a, int ph, LevelShared& s, uint32
             }
         }
         defer_heavy(a, ph, u, deg, a.grid_th);
-        expand_tile_in_place(a, out, u, start, deg, s.g);
+        positional_gather<GATHER_K>(a.cols, u, start, deg, l, sink);
     }
 }
 
 // Two-phase filter (edge frontier -> edge frontier), bitmask and history
 // culls only, no labelling (two_phase/filter_atomic/cta.cuh:308-388).
-__device__ void tp_filter_phase(const BfsArgs& a, int ph, LevelShared& s) {
+__device__ void tp_filter_phase(const BfsArgs& a, int ph, PairLevelShared& s) {
     const uint32_t n_in = phase_input_len(a, ph);
     phase_begin(a, ph, n_in);
     const int32_t* qk = a.qk[ph & 1];
     const int32_t* qv = a.qv[ph & 1];
     const GlobalQueue out = out_queue(a, ph);
-    for (uint32_t base = blockIdx.x * BFS_THREADS; base < n_in; base += gridDim.x * BFS_THREADS) {
-        const uint32_t i = base + threadIdx.x;
-        bool keep = false;
-        int32_t v = -1, p = 0;
-        if (i < n_in) {
-            v = coh_ld(&qk[i], a.coh_in != 0);
-            p = coh_ld(&qv[i], a.coh_in != 0);
-            keep = valid_vertex(a, v);
-            if (keep) keep = !visited_test(a.visited, v);
-            if (keep) keep = !history_seen(s.hist, v);
+    for (uint64_t base = (uint64_t)blockIdx.x * BFS_THREADS; base < n_in;
+         base += (uint64_t)gridDim.x * BFS_THREADS * CONTRACT_K) {
+        bool keep[CONTRACT_K];
+        int32_t v[CONTRACT_K], p[CONTRACT_K];
+        uint32_t mark[CONTRACT_K];
+#pragma unroll
+        for (int r = 0; r < CONTRACT_K; ++r) {
+            const uint64_t i = base + (uint64_t)r * gridDim.x * BFS_THREADS + threadIdx.x;
+            keep[r] = i < n_in;
+            v[r] = keep[r] ? coh_ld(&qk[i], a.coh_in != 0) : -1;
+            p[r] = keep[r] ? coh_ld(&qv[i], a.coh_in != 0) : 0;
         }
-        lq_append<true>(s.q, out, keep, v, p);
+#pragma unroll
+        for (int r = 0; r < CONTRACT_K; ++r) {
+            keep[r] = keep[r] && valid_vertex(a, v[r]);
+            mark[r] = keep[r] ? mark_load(a, v[r]) : 0u;
+        }
+#pragma unroll
+        for (int r = 0; r < CONTRACT_K; ++r)
+            keep[r] = keep[r] && !mark_seen(a, v[r], mark[r]) && !history_seen(s.hist, v[r]);
+        lq_append_batch<true>(s.q, out, keep, v, p);
         lq_flush<true>(s.q, out, LQ_CAP / 2);
     }
     lq_flush<true>(s.q, out, 1);
@@ -439,14 +626,17 @@ __device__ void tp_filter_phase(const BfsArgs& a, int ph, LevelShared& s) {
 //    BU_GROUP-lane groups of the wave, BU_GROUP neighbours per step, lowest
 //    lane wins (the first frontier neighbour in list order).
 // A wave owns the two bitmap words of its 64 vertices, so visited/next words
-// are written without atomics.  Discovered vertices go to the vertex queue
-// (one global atomic per wave tile) so that a top-down step can follow.
+// are written without atomics.  The next frontier is only its bitmap: a
+// top-down step that follows lists it itself (td_bitmap_phase), so a
+// bottom-up step reserves no queue space and its one atomic per workgroup is
+// the partial sum of what it found.
 // Measured on RMAT-22 (ms per search): BU_FIRST 1-3 within 1 % of each
 // other, 4 about 2 % slower, 6 and 8 4-10 % slower; BU_GROUP 4 and 16 no
 // better than 8.
 constexpr int BU_FIRST = 2;
 constexpr int BU_GROUP = 8;
 constexpr int BU_WAVE_GROUPS = kWave / BU_GROUP;
+constexpr int BU_LISTS = 4;  // lists each group scans side by side
 
 struct BuWave {
     int32_t start[kWave];  // pending entry: next edge to scan
@@ -454,31 +644,10 @@ struct BuWave {
     int32_t parent[kWave];
 };
 
-// Discovered vertices are buffered per wave and written to the global queue
-// with one atomic per workgroup at the end (or per wave when its buffer
-// fills), not one per tile: a single queue counter hit by every wave tile
-// serializes the whole step.
-constexpr int BU_QBUF = 512;
-
 struct BuShared {
     BuWave w[BFS_WAVES];
-    int32_t qbuf[BFS_WAVES][BU_QBUF];
-    uint32_t qn[BFS_WAVES];
-    uint32_t qbase[BFS_WAVES];
     unsigned long long red[BFS_WAVES];
 };
-
-// Copies `count` buffered vertices of this wave to the global queue at `base`.
-__device__ __forceinline__ void bu_copy_out(const int32_t* buf, uint32_t count, uint32_t base, int32_t* qout,
-                                            uint32_t qcap, uint32_t* overflow) {
-    for (uint32_t i = lane_id(); i < count; i += kWave) {
-        const uint32_t pos = base + i;
-        if (pos < qcap)
-            qout[pos] = buf[i];
-        else
-            st_relaxed(overflow, 1u);
-    }
-}
 
 // LDS written by some lanes of a wave and read by others after it: keep the
 // compiler from reordering across this point (a wave's LDS operations
@@ -490,16 +659,30 @@ __device__ __forceinline__ void wave_lds_sync() {
 }
 
 // LDS of a direction-optimizing level: the top-down step's queue and gather
-// staging or the bottom-up step's per-wave scratch (about 16.5 KB: eight
+// staging or the bottom-up step's per-wave scratch (about 15 KB: eight
 // workgroups of 256 threads can stay resident per CU).
+constexpr int DO_GATHER_K = 4;
 struct DoTdShared {
     LdsKeyQueue qv;
-    GatherSmem g;
+    ListSmem g;
+    int32_t list[BM_LIST];
     unsigned long long red[BFS_WAVES];
 };
-union DoShared {
-    DoTdShared td;
-    BuShared bu;
+// Start state of a level (do_level_in).
+struct DoLevelIn {
+    int32_t ph;
+    uint32_t queued;   // vertices a top-down step left in the queue
+    uint32_t n_f;      // frontier vertices: those and what a bottom-up step found
+    uint32_t prev_dir;
+    long long m_f;     // their degree sum
+    long long vis;     // degree sum of the vertices visited before them
+};
+struct DoShared {
+    union {
+        DoTdShared td;
+        BuShared bu;
+    };
+    DoLevelIn in;
 };
 
 __device__ __forceinline__ bool bm_test(const uint32_t* bm, int32_t u) { return (bm[u >> 5] >> (u & 31)) & 1u; }
@@ -511,39 +694,48 @@ __device__ void bu_waves(const BfsArgs& a, int ph, int32_t depth_next, const uin
     BuWave& W = s.w[wid];
     const int grp = lane / BU_GROUP, sub = lane % BU_GROUP;
     const int gbase = lane & ~(BU_GROUP - 1);
-    int32_t* qout = a.qk[(ph + 1) & 1];
-    uint32_t* qlen = &a.ctr->qlen[(ph + 1) & 3];
-    const uint32_t qcap = a.qcap[(ph + 1) & 1];
-    int32_t* qb = s.qbuf[wid];
-    uint32_t wq = 0;  // vertices in this wave's buffer (wave-uniform)
-    bool found_any = false;
-    unsigned long long eacc = 0;
-    const int64_t step = (int64_t)gridDim.x * BFS_WAVES * kWave;
+    unsigned long long acc = 0;  // (degree sum << 32) | vertices found by this lane
+    // The frontier by its labels in a small graph, else by its bitmap (which
+    // small graphs' top-down steps do not set).
+    auto in_frontier = [&](int32_t u) -> bool {
+        return a.by_label ? a.depth[u] == depth_next - 1 : bm_test(cur, u);
+    };
+    // Tiles go round by round over the launch's waves, each round rotated
+    // against the last: with equal residues every wave would get tiles of like
+    // ids, and in an RMAT graph ids with the same low bits zero are hubs
+    // together (the slowest wave of the first bottom-up level of RMAT-22 took
+    // 85 us, the average one 51).
+    const int64_t nw = (int64_t)gridDim.x * BFS_WAVES;
+    const int64_t turn = (nw * 5 / 13) | 1;
+    int64_t pos = (int64_t)blockIdx.x * BFS_WAVES + wid, round0 = 0;
     // The next tile's visited word and row offsets are loaded one iteration
     // ahead (whether or not the vertex turns out to be visited), so the
     // current tile's scan overlaps the next tile's first two round trips.
-    int64_t vb = ((int64_t)blockIdx.x * BFS_WAVES + wid) * kWave;
-    uint32_t nvw = 0xFFFFFFFFu;
+    int64_t vb = pos * kWave;
+    uint32_t nvw = 0u;
     int32_t noff0 = 0, noff1 = 0;
     if (vb + lane < a.n) {
         const int32_t v = (int32_t)(vb + lane);
-        nvw = a.visited[v >> 5];
+        nvw = mark_load(a, v);
         noff0 = a.offs[v];
         noff1 = a.offs[v + 1];
     }
-    for (; vb < a.n; vb += step) {
+    while (round0 * kWave < a.n) {
+        const int64_t vcur = vb;
         const int32_t v = (int32_t)(vb + lane);
         const uint32_t vw = nvw;
         const int32_t off0 = noff0, off1 = noff1;
-        if (vb + step + lane < a.n) {
-            const int32_t vn = (int32_t)(vb + step + lane);
-            nvw = a.visited[vn >> 5];
+        round0 += nw;
+        pos += turn;
+        if (pos >= nw) pos -= nw;
+        vb = (round0 + pos) * kWave;
+        if (vb + lane < a.n) {
+            const int32_t vn = (int32_t)(vb + lane);
+            nvw = mark_load(a, vn);
             noff0 = a.offs[vn];
             noff1 = a.offs[vn + 1];
-        } else {
-            nvw = 0xFFFFFFFFu;  // past the end: never active
         }
-        const bool active = (v < a.n) && !((vw >> (v & 31)) & 1u);
+        const bool active = (vcur + lane < a.n) && !mark_seen(a, v, vw);
         if (__ballot(active) == 0) continue;
         int32_t start = 0, deg = 0, parent = -1;
         if (active) {
@@ -557,7 +749,7 @@ __device__ void bu_waves(const BfsArgs& a, int ph, int32_t depth_next, const uin
             for (int k = 0; k < BU_FIRST; ++k) u[k] = (k < deg) ? a.cols[start + k] : -1;
 #pragma unroll
             for (int k = BU_FIRST - 1; k >= 0; --k)
-                if (u[k] >= 0 && bm_test(cur, u[k])) parent = u[k];
+                if (u[k] >= 0 && in_frontier(u[k])) parent = u[k];
         }
         // Stage 2: the wave's unresolved lists, one per BU_GROUP-lane group.
         const bool pend = parent < 0 && deg > BU_FIRST;
@@ -570,20 +762,42 @@ __device__ void bu_waves(const BfsArgs& a, int ph, int32_t depth_next, const uin
             }
             wave_lds_sync();
             const int np = __popcll(pm);
-            for (int i = grp; i < np; i += BU_WAVE_GROUPS) {
-                const int32_t e1 = W.end[i];
-                int32_t hit_u = -1;
-                for (int32_t e0 = W.start[i]; e0 < e1; e0 += BU_GROUP) {
-                    const int32_t e = e0 + sub;
-                    const int32_t u = (e < e1) ? a.cols[e] : -1;
-                    const bool hit = u >= 0 && bm_test(cur, u);
-                    const uint64_t hm = (__ballot(hit) >> gbase) & ((1ull << BU_GROUP) - 1);
-                    if (hm) {
-                        hit_u = __shfl(u, gbase + __ffsll((unsigned long long)hm) - 1, kWave);
-                        break;
-                    }
+            for (int i0 = grp; i0 - grp < np; i0 += BU_LISTS * BU_WAVE_GROUPS) {
+                int32_t e[BU_LISTS], e1[BU_LISTS], hit_u[BU_LISTS];
+#pragma unroll
+                for (int k = 0; k < BU_LISTS; ++k) {
+                    const int i = i0 + k * BU_WAVE_GROUPS;
+                    e[k] = i < np ? W.start[i] + sub : 0;
+                    e1[k] = i < np ? W.end[i] : 0;
+                    hit_u[k] = -1;
                 }
-                if (sub == 0) W.parent[i] = hit_u;
+                uint64_t live;
+                do {
+                    int32_t u[BU_LISTS];
+                    bool hit[BU_LISTS];
+                    bool more = false;
+#pragma unroll
+                    for (int k = 0; k < BU_LISTS; ++k) u[k] = e[k] < e1[k] ? a.cols[e[k]] : -1;
+#pragma unroll
+                    for (int k = 0; k < BU_LISTS; ++k) hit[k] = u[k] >= 0 && in_frontier(u[k]);
+#pragma unroll
+                    for (int k = 0; k < BU_LISTS; ++k) {
+                        const uint32_t hm = (uint32_t)(__ballot(hit[k]) >> gbase) & ((1u << BU_GROUP) - 1);
+                        const int32_t first = __shfl(u[k], gbase + (hm ? __ffsll((unsigned long long)hm) - 1 : 0), kWave);
+                        if (hm) {
+                            hit_u[k] = first;
+                            e1[k] = 0;  // resolved
+                        }
+                        e[k] += BU_GROUP;
+                        more |= e[k] < e1[k];
+                    }
+                    live = __ballot(more);
+                } while (live);
+#pragma unroll
+                for (int k = 0; k < BU_LISTS; ++k) {
+                    const int i = i0 + k * BU_WAVE_GROUPS;
+                    if (sub == 0 && i < np) W.parent[i] = hit_u[k];
+                }
             }
             wave_lds_sync();
             if (pend) parent = W.parent[slot];
@@ -593,8 +807,7 @@ __device__ void bu_waves(const BfsArgs& a, int ph, int32_t depth_next, const uin
         if (found) {
             a.depth[v] = depth_next;
             a.pred[v] = parent;
-            found_any = true;
-            eacc += (unsigned long long)deg;
+            acc += ((unsigned long long)deg << 32) | 1ull;
         }
         const uint64_t fm = __ballot(found);
         if ((lane & 31) == 0) {
@@ -602,39 +815,11 @@ __device__ void bu_waves(const BfsArgs& a, int ph, int32_t depth_next, const uin
             if (w < a.words) {
                 const uint32_t bits = (lane == 0) ? (uint32_t)fm : (uint32_t)(fm >> 32);
                 next[w] = bits;
-                if (bits) a.visited[w] = vw | bits;
+                if (bits && !a.by_label) a.visited[w] = vw | bits;
             }
         }
-        if (fm) {
-            const uint32_t nf = (uint32_t)__popcll(fm);
-            if (wq + nf > (uint32_t)BU_QBUF) {  // buffer full: flush this wave's part now
-                uint32_t base = 0;
-                if (lane == 0) base = atomic_add_u32(qlen, wq);
-                base = (uint32_t)wave_bcast((int)base, 0);
-                bu_copy_out(qb, wq, base, qout, qcap, &a.ctr->overflow);
-                wq = 0;
-                wave_lds_sync();
-            }
-            if (found) qb[wq + (uint32_t)lane_prefix(fm)] = v;
-            wq += nf;
-        }
     }
-    // One queue reservation for the whole workgroup's buffered vertices.
-    if (lane == 0) s.qn[wid] = wq;
-    __syncthreads();
-    if (threadIdx.x == 0) {
-        uint32_t total = 0;
-        for (int w = 0; w < BFS_WAVES; ++w) {
-            s.qbase[w] = total;
-            total += s.qn[w];
-        }
-        const uint32_t base = total ? atomic_add_u32(qlen, total) : 0u;
-        for (int w = 0; w < BFS_WAVES; ++w) s.qbase[w] += base;
-    }
-    __syncthreads();
-    bu_copy_out(qb, wq, s.qbase[wid], qout, qcap, &a.ctr->overflow);
-    wg_add_u64(eacc, &a.ctr->level_edges[(ph + 1) & 3], s.red);
-    if (__syncthreads_or(found_any) && threadIdx.x == 0) atomic_max_u32(a.max_depth, (uint32_t)depth_next);
+    wg_add_u64(acc, spread_at(a.spread, ph + 1, blockIdx.x % SPREAD), s.red);
 }
 
 // Direction for level ph of the direction-optimizing traversal (Beamer,
@@ -642,11 +827,9 @@ __device__ void bu_waves(const BfsArgs& a, int ph, int32_t depth_next, const uin
 // (finalized by the previous launch), so all agree without host involvement.
 // m_f = degree sum of the frontier, m_u = edges of unvisited vertices;
 // top-down -> bottom-up when m_f > m_u / alpha, back when n_f < n / beta.
-__device__ __forceinline__ uint32_t do_direction(const BfsArgs& a, int ph, uint32_t n_f) {
+__device__ __forceinline__ uint32_t do_direction(const BfsArgs& a, uint32_t n_f, long long m_f, long long vis,
+                                                 uint32_t prev) {
     if (!a.symmetric) return 0;
-    const long long m_f = (long long)a.ctr->level_edges[ph & 3];
-    const long long vis = (long long)a.ctr->vis_edges[ph & 3];
-    const uint32_t prev = a.ctr->dir[(ph + 3) & 3];
     long long m_u = a.edges - vis - m_f;
     if (m_u < 0) m_u = 0;
     if (prev == 0) return (m_f * (long long)a.do_alpha > m_u) ? 1u : 0u;
@@ -692,12 +875,16 @@ __device__ void reset_seed_body(const BfsArgs& a, int ph, int32_t src, int mode)
         fcur[w] = (mode == SEED_DO && w == sw) ? sbit : 0u;
         fnext[w] = 0u;
     }
-    if (threadIdx.x != 0 || blockIdx.x != 0) return;
+    if (blockIdx.x != 0) return;
+    if (mode == SEED_DO && threadIdx.x < 4 * SPREAD) {
+        const int level = (int)threadIdx.x / SPREAD, i = (int)threadIdx.x % SPREAD;
+        const bool first = level == (ph & 3) && i == 0;
+        *spread_at(a.spread, level, i) = first ? (unsigned long long)(a.offs[src + 1] - a.offs[src]) << 32 : 0ull;
+    }
+    if (threadIdx.x != 0) return;
     DevCounters* c = a.ctr;
     for (int i = 0; i < 4; ++i) {
         c->qlen[i] = 0;
-        c->level_edges[i] = 0;
-        c->level_verts[i] = 0;
         c->vis_edges[i] = 0;
         c->dir[i] = 0;
     }
@@ -709,16 +896,11 @@ __device__ void reset_seed_body(const BfsArgs& a, int ph, int32_t src, int mode)
     c->levels_run = 0;
     c->saturated = 0;
     c->queued = 0;
-    c->next_edges = 0;
-    c->next_edges_prev = 0;
     c->bar_abort = 0;
     c->corrupt = 0;
     *a.max_depth = 0;
     a.qk[ph & 1][0] = src;
-    if (mode == SEED_EDGE)
-        a.qv[ph & 1][0] = -2;
-    else
-        c->level_edges[ph & 3] = (unsigned long long)(a.offs[src + 1] - a.offs[src]);
+    if (mode == SEED_EDGE) a.qv[ph & 1][0] = -2;
     c->qlen[ph & 3] = 1;
 }
 
@@ -746,29 +928,84 @@ __device__ __forceinline__ void resolve_phase(const BfsArgs& a, int& ph, int32_t
 }
 
 enum PhaseKind { PK_TD = 0, PK_CE = 2, PK_TP_CONTRACT = 3, PK_TP_EXPAND = 4, PK_TP_FILTER = 5 };
-
 template <int KIND>
-__device__ void phase_body(BfsArgs a, int ph, int32_t depth, int slot, LevelShared& s) {
+struct PhaseShared {
+    typedef PairLevelShared type;
+};
+template <>
+struct PhaseShared<PK_TD> {
+    typedef TdLevelShared type;
+};
+template <>
+struct PhaseShared<PK_TP_EXPAND> {
+    typedef TdLevelShared type;
+};
+template <>
+struct PhaseShared<PK_CE> {
+    typedef LevelShared type;
+};
+
+template <int KIND, typename Shared>
+__device__ void phase_body(BfsArgs a, int ph, int32_t depth, int slot, Shared& s) {
     resolve_phase(a, ph, depth);
     unsigned long long t0 = 0;
     stats_begin(t0, a);
     shared_init(s);
-    if (KIND == PK_TD) td_phase(a, ph, depth, nullptr, false, s.q, s.g, s.red, gridDim.x, a.grid_th);
-    if (KIND == PK_CE) ce_phase(a, ph, depth, s);
-    if (KIND == PK_TP_CONTRACT) tp_contract_phase(a, ph, depth, s);
-    if (KIND == PK_TP_EXPAND) tp_expand_phase(a, ph, s);
-    if (KIND == PK_TP_FILTER) tp_filter_phase(a, ph, s);
+    if constexpr (KIND == PK_TD) td_phase<GATHER_K>(a, ph, depth, nullptr, false, s.q, s.l, s.red, gridDim.x, a.grid_th);
+    if constexpr (KIND == PK_CE) ce_phase(a, ph, depth, s);
+    if constexpr (KIND == PK_TP_CONTRACT) tp_contract_phase(a, ph, depth, s);
+    if constexpr (KIND == PK_TP_EXPAND) tp_expand_phase(a, ph, depth, s.l);
+    if constexpr (KIND == PK_TP_FILTER) tp_filter_phase(a, ph, s);
     stats_end(t0, a, slot);
+}
+
+// What a level kernel of the direction-optimizing traversal needs to know
+// before it can start, read in one round trip: one wave of the workgroup loads
+// every counter word and every partial sum of all four level slots together
+// (following the phase base to the level's slot would be three dependent round
+// trips, about 2.5 us of a 7 us level).
+constexpr int CTR_WORDS = (int)(sizeof(DevCounters) / 4);
+static_assert(CTR_WORDS == kWave && 4 * SPREAD == kWave, "one counter word and one partial sum per lane");
+
+__device__ __forceinline__ void do_level_in(const BfsArgs& a, int ph, DoLevelIn& in) {
+    if (threadIdx.x < kWave) {
+        const int lane = lane_id();
+        const uint32_t w = reinterpret_cast<const uint32_t*>(a.ctr)[lane];
+        unsigned long long part = *spread_at(a.spread, lane / SPREAD, lane % SPREAD);
+        constexpr int kPh = (int)(offsetof(DevCounters, ph_base) / 4), kDir = (int)(offsetof(DevCounters, dir) / 4),
+                      kVis = (int)(offsetof(DevCounters, vis_edges) / 4);
+        if (a.dev_base) ph += (int)__shfl(w, kPh, kWave);
+        if (lane / SPREAD != (ph & 3)) part = 0ull;
+#pragma unroll
+        for (int d = kWave / 2; d >= 1; d >>= 1) part += __shfl_xor(part, d, kWave);
+        uint32_t n_q = __shfl(w, ph & 3, kWave);
+        if (n_q > a.qcap[ph & 1]) n_q = 0;  // an overflowed queue counts as empty
+        const uint32_t dir = __shfl(w, kDir + ((ph + 3) & 3), kWave);
+        const uint32_t lo = __shfl(w, kVis + 2 * (ph & 3), kWave), hi = __shfl(w, kVis + 2 * (ph & 3) + 1, kWave);
+        if (lane == 0) {
+            in.ph = ph;
+            in.queued = n_q;
+            in.n_f = n_q + (uint32_t)part;
+            in.prev_dir = dir;
+            in.m_f = (long long)(part >> 32);
+            in.vis = (long long)(((unsigned long long)hi << 32) | lo);
+        }
+    }
+    __syncthreads();
 }
 
 // One level of the direction-optimizing traversal: the workgroups agree on
 // the direction from device counters, clear the bitmap two levels ahead and
 // run a top-down or bottom-up step.  An empty frontier makes it a no-op, so
 // the host can launch levels ahead of the termination check.
+// grid_tier: a k_heavy launch follows; without one, top-down steps split
+// their tiles over the workgroups instead.
 __device__ void do_level_body(BfsArgs a, int ph, int slot, int grid_tier, DoShared& s) {
-    int32_t unused_depth = 0;
-    resolve_phase(a, ph, unused_depth);
-    const uint32_t n_f = phase_input_len(a, ph);
+    do_level_in(a, ph, s.in);
+    ph = s.in.ph;
+    const uint32_t n_f = s.in.n_f, prev_dir = s.in.prev_dir;
+    const long long m_f = s.in.m_f, vis = s.in.vis;
+    if (blockIdx.x == 0 && threadIdx.x < SPREAD) *spread_at(a.spread, ph + 2, threadIdx.x) = 0ull;
     if (n_f == 0) {
         // Keep the slot rotation going so later no-op levels also read 0.
         phase_begin(a, ph, 0);
@@ -776,10 +1013,10 @@ __device__ void do_level_body(BfsArgs a, int ph, int slot, int grid_tier, DoShar
     }
     unsigned long long t0 = 0;
     stats_begin(t0, a);
-    const uint32_t dir = do_direction(a, ph, n_f);
+    const uint32_t dir = do_direction(a, n_f, m_f, vis, prev_dir);
     if (blockIdx.x == 0 && threadIdx.x == 0) {
         a.ctr->dir[ph & 3] = dir;
-        a.ctr->vis_edges[(ph + 1) & 3] = a.ctr->vis_edges[ph & 3] + a.ctr->level_edges[ph & 3];
+        a.ctr->vis_edges[(ph + 1) & 3] = (unsigned long long)(vis + m_f);
     }
     uint32_t* clear = a.fbm[(ph + 2) % 3];
     for (int32_t w = blockIdx.x * BFS_THREADS + threadIdx.x; w < a.words; w += gridDim.x * BFS_THREADS) clear[w] = 0;
@@ -789,13 +1026,18 @@ __device__ void do_level_body(BfsArgs a, int ph, int slot, int grid_tier, DoShar
         const uint32_t tdg = min(gridDim.x, (uint32_t)max(1, a.td_grid));
         if (blockIdx.x < tdg) {
             if (threadIdx.x == 0) s.td.qv.count = 0;
-            gather_init(s.td.g);
             __syncthreads();
-            td_phase(a, ph, ph + 1, a.fbm[(ph + 1) % 3], true, s.td.qv, s.td.g, s.td.red, tdg,
-                     grid_tier ? a.grid_th : INT_MAX);
+            const int32_t th = grid_tier ? a.grid_th : INT_MAX;
+            uint32_t* next_bm = a.by_label ? nullptr : a.fbm[(ph + 1) % 3];
+            if (prev_dir == 0)
+                td_phase<DO_GATHER_K>(a, ph, ph + 1, next_bm, true, s.td.qv, s.td.g, s.td.red, tdg, th, n_f, !grid_tier);
+            else
+                td_bitmap_phase<DO_GATHER_K>(a, ph, ph + 1, a.fbm[ph % 3], next_bm, s.td.qv, s.td.g, s.td.list, s.td.red, tdg, th,
+                                n_f);
         }
     } else {
         phase_begin(a, ph, 0);
+        if (blockIdx.x == 0 && threadIdx.x == 0) st_relaxed(a.max_depth, (uint32_t)ph);
         bu_waves(a, ph, ph + 1, a.fbm[ph % 3], a.fbm[(ph + 1) % 3], s.bu);
     }
     stats_end(t0, a, slot);
@@ -807,36 +1049,60 @@ __device__ void do_level_body(BfsArgs a, int ph, int slot, int grid_tier, DoShar
 // entry it names, so stale map words can never index outside a list.
 enum HeavyKind { HK_TD = 0, HK_TD_DO = 1, HK_PAIRS = 2 };
 
-// Top-down grid-tier launches need only a vertex queue; a small LDS block
-// keeps them at full residency.
+// Top-down grid-tier launches need a vertex queue, pair launches write in
+// place; small LDS blocks keep them at full residency.
 struct TdHeavyShared {
     LdsKeyQueue qv;
+    ListSmem l;
     unsigned long long red[BFS_WAVES];
+};
+struct PairsHeavyShared {
+    ListSmem l;
 };
 template <int KIND>
 struct HeavySharedOf {
     typedef TdHeavyShared type;
-};
-// Pair grid tier: a batch of the workgroup's chunks is measured first, then
-// reserved in the output queue with one atomic and written in place.
-constexpr int HEAVY_BATCH = 1024;  // chunks per reservation
-struct PairsHeavyShared {
-    int32_t u[HEAVY_BATCH];
-    int32_t start[HEAVY_BATCH];
-    uint32_t off[HEAVY_BATCH + 1];  // exclusive offsets of the chunks' lengths; [n] = total
-    int s_wave[BFS_WAVES];
-    uint32_t base;
 };
 template <>
 struct HeavySharedOf<HK_PAIRS> {
     typedef PairsHeavyShared type;
 };
 
+// The grid tier's chunks [0, C) of H entries: chunk base + t * gridDim.x + b
+// goes to thread t of workgroup b, which finds its piece of a list; the
+// workgroup then gathers its 256 pieces positionally, as the level steps do
+// with whole lists.
+template <typename Sink>
+__device__ __forceinline__ void gather_chunks(const BfsArgs& a, uint32_t H, uint32_t C, ListSmem& l, Sink& sink) {
+    auto piece = [&](uint32_t c, int32_t& u, int32_t& start, int32_t& len) {
+        const int32_t entry = coh_ld(&a.chunk_map[c], a.coh_out != 0);
+        if ((uint32_t)entry >= H) return;
+        const int2 eu = coh_ld2(&a.heavy[entry], a.coh_out != 0);
+        if (!valid_vertex(a, eu.x) || (uint32_t)eu.y > c) return;
+        const int32_t s0 = a.offs[eu.x], deg = a.offs[eu.x + 1] - s0;
+        const long long off = (long long)(c - (uint32_t)eu.y) * HEAVY_CHUNK;
+        if (off >= deg) return;
+        u = eu.x;
+        start = s0 + (int32_t)off;
+        len = min((int32_t)HEAVY_CHUNK, deg - (int32_t)off);
+    };
+    for (uint64_t base = 0; base + blockIdx.x < C; base += (uint64_t)gridDim.x * BFS_THREADS) {
+        int32_t u = -1, start = 0, len = 0;
+        const uint64_t c = base + (uint64_t)threadIdx.x * gridDim.x + blockIdx.x;
+        if (c < C) piece((uint32_t)c, u, start, len);
+        positional_gather<GATHER_K>(a.cols, u, start, len, l, sink);
+    }
+}
+
 template <int KIND>
 __device__ void heavy_body(BfsArgs a, int ph, int32_t depth_next, int slot, typename HeavySharedOf<KIND>::type& s) {
+    // Both slots are loaded beside the phase base, not after it.
+    const unsigned long long alloc0 =
+        __hip_atomic_load(&a.ctr->heavy_alloc[0], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    const unsigned long long alloc1 =
+        __hip_atomic_load(&a.ctr->heavy_alloc[1], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     resolve_phase(a, ph, depth_next);
-    const unsigned long long alloc =
-        __hip_atomic_load(&a.ctr->heavy_alloc[ph & 1], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    const unsigned long long alloc = (ph & 1) ? alloc1 : alloc0;
     const uint32_t H = min((uint32_t)(alloc >> 32), a.heavy_cap);
     const uint32_t C = min((uint32_t)alloc, a.chunk_cap);
     if (H == 0 || C == 0) return;
@@ -847,136 +1113,14 @@ __device__ void heavy_body(BfsArgs a, int ph, int32_t depth_next, int slot, type
         __syncthreads();
     }
     const GlobalQueue out = out_queue(a, ph);
-    // HEAVY_ROUND chunks per iteration (grid-strided), each load stage issued
-    // for all of them before the next, so that many dependent chains
-    // (chunk map -> entry -> offsets -> columns) are in flight per workgroup.
-    constexpr int R = HEAVY_ROUND;
-    const uint32_t stride = gridDim.x;
-    auto chunks = [&](uint32_t c0, int32_t (&u)[R], int32_t (&v)[R], bool (&valid)[R]) {
-        int32_t entry[R], start[R], len[R];
-#pragma unroll
-        for (int r = 0; r < R; ++r) {
-            const uint32_t c = c0 + (uint32_t)r * stride;
-            entry[r] = c < C ? coh_ld(&a.chunk_map[c], a.coh_out != 0) : -1;
-        }
-        int2 eu[R];
-#pragma unroll
-        for (int r = 0; r < R; ++r)
-            eu[r] = (uint32_t)entry[r] < H ? coh_ld2(&a.heavy[entry[r]], a.coh_out != 0) : make_int2(-1, 0);
-#pragma unroll
-        for (int r = 0; r < R; ++r) {
-            const uint32_t c = c0 + (uint32_t)r * stride;
-            u[r] = -1;
-            start[r] = 0;
-            len[r] = 0;
-            if ((uint32_t)entry[r] < H && valid_vertex(a, eu[r].x) && (uint32_t)eu[r].y <= c) {
-                const int32_t s0 = a.offs[eu[r].x], deg = a.offs[eu[r].x + 1] - s0;
-                const long long off = (long long)(c - (uint32_t)eu[r].y) * HEAVY_CHUNK;
-                if (off < deg) {
-                    u[r] = eu[r].x;
-                    start[r] = s0 + (int32_t)off;
-                    len[r] = min((int32_t)HEAVY_CHUNK, deg - (int32_t)off);
-                }
-            }
-        }
-        const int32_t k = (int32_t)threadIdx.x;
-#pragma unroll
-        for (int r = 0; r < R; ++r) {
-            valid[r] = k < len[r];
-            v[r] = valid[r] ? a.cols[start[r] + k] : 0;
-        }
-    };
     if constexpr (KIND == HK_PAIRS) {
-        // Every edge of a pair chunk is output, so a chunk's output size is
-        // its length.  Per batch of HEAVY_BATCH of this workgroup's chunks
-        // (c = blockIdx.x + i * stride): each thread measures the chunks
-        // i = 4*tid .. 4*tid+3, a workgroup scan gives every chunk its offset,
-        // one atomic reserves the batch, and the edges are written in place
-        // (consecutive lanes, consecutive slots), HEAVY_ROUND chunks at a time.
-        (void)chunks;
-        const int tid = (int)threadIdx.x;
-        // chunks of this workgroup: c = blockIdx.x + j * stride < C
-        const uint32_t mine = blockIdx.x < C ? (C - blockIdx.x + stride - 1) / stride : 0u;
-        constexpr int PER = HEAVY_BATCH / BFS_THREADS;
-        for (uint32_t b0 = 0; b0 < mine; b0 += HEAVY_BATCH) {
-            const uint32_t nb = min((uint32_t)HEAVY_BATCH, mine - b0);
-            int32_t lens[PER];
-            int32_t mysum = 0;
-#pragma unroll
-            for (int q = 0; q < PER; ++q) {
-                const uint32_t i = (uint32_t)(tid * PER + q);
-                int32_t u = -1, start = 0, len = 0;
-                if (i < nb) {
-                    const uint32_t c = blockIdx.x + (b0 + i) * stride;
-                    const int32_t entry = coh_ld(&a.chunk_map[c], a.coh_out != 0);
-                    if ((uint32_t)entry < H) {
-                        const int2 eu = coh_ld2(&a.heavy[entry], a.coh_out != 0);
-                        if (valid_vertex(a, eu.x) && (uint32_t)eu.y <= c) {
-                            const int32_t s0 = a.offs[eu.x], deg = a.offs[eu.x + 1] - s0;
-                            const long long off = (long long)(c - (uint32_t)eu.y) * HEAVY_CHUNK;
-                            if (off < deg) {
-                                u = eu.x;
-                                start = s0 + (int32_t)off;
-                                len = min((int32_t)HEAVY_CHUNK, deg - (int32_t)off);
-                            }
-                        }
-                    }
-                    s.u[i] = u;
-                    s.start[i] = start;
-                }
-                lens[q] = len;
-                mysum += len;
-            }
-            int total;
-            int run = wg_exclusive_scan<BFS_THREADS>(mysum, total, s.s_wave);
-#pragma unroll
-            for (int q = 0; q < PER; ++q) {
-                const uint32_t i = (uint32_t)(tid * PER + q);
-                if (i < nb) s.off[i] = (uint32_t)run;
-                run += lens[q];
-            }
-            if (tid == 0) {
-                s.off[nb] = (uint32_t)total;
-                s.base = total ? atomic_add_u32(out.len, (uint32_t)total) : 0u;
-                if (total && (uint64_t)s.base + (uint64_t)total > out.cap) st_relaxed(out.overflow, 1u);
-            }
-            __syncthreads();
-            const uint32_t base = s.base;
-            for (uint32_t i0 = 0; i0 < nb; i0 += R) {
-                int32_t v[R];
-                bool valid[R];
-#pragma unroll
-                for (int r = 0; r < R; ++r) {
-                    const uint32_t i = i0 + r;
-                    const int32_t len = i < nb ? (int32_t)(s.off[i + 1] - s.off[i]) : 0;
-                    valid[r] = tid < len;
-                    v[r] = valid[r] ? a.cols[s.start[i] + tid] : 0;
-                }
-#pragma unroll
-                for (int r = 0; r < R; ++r) {
-                    if (!valid[r]) continue;
-                    const uint32_t i = i0 + r;
-                    const uint64_t pos = (uint64_t)base + s.off[i] + (uint32_t)tid;
-                    if (pos < out.cap) {
-                        coh_st(&out.keys[pos], v[r], out.coh);
-                        coh_st(&out.vals[pos], s.u[i], out.coh);
-                    }
-                }
-            }
-            __syncthreads();
-        }
+        InPlaceSink sink{out, s.l};
+        gather_chunks(a, H, C, s.l, sink);
     } else {
-        TdSink<1> tds{a, s.qv, out, (KIND == HK_TD_DO) ? a.fbm[(ph + 1) % 3] : nullptr, depth_next, KIND == HK_TD_DO,
-                   false, 0ull};
-        for (uint32_t c0 = blockIdx.x; c0 < C; c0 += stride * R) {
-            int32_t u[R], v[R];
-            bool valid[R];
-            chunks(c0, u, v, valid);
-#pragma unroll
-            for (int r = 0; r < R; ++r) tds(valid[r], v[r], u[r]);
-            lq_flush<false>(s.qv, out, LQ_CAP / 2);
-        }
-        td_finish(a, ph, tds, s.red);
+        TdSink<1> sink{a, s.qv, out, (KIND == HK_TD_DO && !a.by_label) ? a.fbm[(ph + 1) % 3] : nullptr, depth_next,
+                       KIND == HK_TD_DO, 0ull};
+        gather_chunks(a, H, C, s.l, sink);
+        td_finish(a, ph, sink, s.red);
     }
     stats_end(t0, a, slot);
 }
@@ -1004,7 +1148,20 @@ struct FusedHeavy {
 };
 
 template <int KIND>
-__device__ void fused_body(const BfsArgs& a, int ph, int32_t depth, int max_levels, uint32_t sat_limit, LevelShared& s,
+struct FusedShared {
+    typedef LevelShared type;
+};
+template <>
+struct FusedShared<FK_TP> {
+    typedef PairLevelShared type;
+};
+template <>
+struct FusedShared<FK_TD> {
+    typedef TdLevelShared type;
+};
+
+template <int KIND, typename Shared>
+__device__ void fused_body(const BfsArgs& a, int ph, int32_t depth, int max_levels, uint32_t sat_limit, Shared& s,
                            typename FusedHeavy<KIND>::shared& hs) {
     unsigned long long t0 = 0, busy = 0;
     if (a.wg_stats && threadIdx.x == 0) t0 = wg_clock();
@@ -1047,14 +1204,14 @@ __device__ void fused_body(const BfsArgs& a, int ph, int32_t depth, int max_leve
         int heavy_ph = ph;          // phase whose deferred lists the grid tier takes
         int32_t heavy_depth = depth;  // depth label of what it discovers (top-down)
         uint32_t word = 0;
-        if (KIND == FK_TD) {
-            td_phase(a, ph, depth + 1, nullptr, false, s.q, s.g, s.red, gridDim.x, a.grid_th, n_in);
+        if constexpr (KIND == FK_TD) {
+            td_phase<GATHER_K>(a, ph, depth + 1, nullptr, false, s.q, s.l, s.red, gridDim.x, a.grid_th, n_in);
             heavy_depth = depth + 1;
             ph += 1;
-        } else if (KIND == FK_CE) {
+        } else if constexpr (KIND == FK_CE) {
             ce_phase(a, ph, depth, s, n_in);
             ph += 1;
-        } else {
+        } else if constexpr (KIND == FK_TP) {
             tp_contract_phase(a, ph, depth, s, n_in);
             if (a.wg_stats && threadIdx.x == 0) busy += wg_clock() - tb;
             if (!grid_sync(bar, ++epoch, payload_for(ph + 1, -1), &s.ctl, word)) break;
@@ -1063,7 +1220,7 @@ __device__ void fused_body(const BfsArgs& a, int ph, int32_t depth, int max_leve
             // has it); the overflow flag ends the search.
             uint32_t n_mid = word & 0x7FFFFFFFu;
             if (n_mid > a.qcap[(ph + 1) & 1]) n_mid = 0;
-            tp_expand_phase(a, ph + 1, s, n_mid);
+            tp_expand_phase(a, ph + 1, depth, s.l, n_mid);
             heavy_ph = ph + 1;
             ph += 2;
         }
@@ -1077,10 +1234,10 @@ __device__ void fused_body(const BfsArgs& a, int ph, int32_t depth, int max_leve
             if (!grid_sync(bar, ++epoch, payload_for(ph, -1), &s.ctl, word)) break;
         }
         n_in = word & 0x7FFFFFFFu;
-        // Top-down: the level claimed vertices (at `depth`) iff the next
-        // frontier is not empty (td_finish leaves this to workgroup 0).
-        if (KIND == FK_TD && n_in != 0 && blockIdx.x == 0 && threadIdx.x == 0)
-            atomic_max_u32(a.max_depth, (uint32_t)depth);
+        // A nonempty next frontier tells that the level claimed vertices: those
+        // on it (top-down, at `depth`), or those whose edges are on it.
+        if (KIND != FK_TP && n_in != 0 && blockIdx.x == 0 && threadIdx.x == 0)
+            atomic_max_u32(a.max_depth, (uint32_t)(KIND == FK_TD ? depth : depth - 1));
     }
     if (blockIdx.x == 0 && threadIdx.x == 0) {
         a.ctr->levels_run = (uint32_t)level;

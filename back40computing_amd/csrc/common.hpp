@@ -48,16 +48,12 @@ struct alignas(256) DevCounters {
     uint32_t levels_run;         // persistent kernels: levels executed
     uint32_t saturated;          // persistent kernels: quit because the frontier got wide
     unsigned long long queued;   // total elements taken from input frontiers
-    unsigned long long next_edges;  // degree sum of the vertices discovered this level
-    unsigned long long next_edges_prev;
     // Grid barrier release word: low 32 bits the epoch of the last completed
     // barrier (never reset by a search), high 32 bits the word workgroup 0
     // published with it.
     unsigned long long bar_release;
     uint32_t bar_abort;          // set when a barrier wait timed out
     uint32_t corrupt;            // set when a frontier held an id outside [0, n)
-    unsigned long long level_edges[4];  // rotating per-level degree sums (direction switch)
-    uint32_t level_verts[4];            // rotating per-level discovered-vertex counts
     unsigned long long vis_edges[4];    // degree sum of vertices visited before the level
     uint32_t dir[4];                    // direction chosen per level (0 top-down, 1 bottom-up)
     uint32_t ph_base;                   // graph-replayed level loops: phase of the replay's first step
