@@ -101,6 +101,11 @@ __global__ __launch_bounds__(BFS_THREADS) void k_fused(BfsArgs a, int ph, int32_
     fused_body<KIND>(a, ph, depth, max_levels, sat_limit, s, hs);
 }
 
+__global__ __launch_bounds__(BFS_THREADS) void k_fused_narrow(BfsArgs a, int ph, int32_t depth) {
+    __shared__ NarrowShared s;
+    fused_narrow_body(a, ph, depth, s);
+}
+
 __global__ __launch_bounds__(BFS_THREADS) void k_gbarrier_bench(GridBarrier bar, int iterations) {
     __shared__ uint32_t s_word;
     gbarrier_bench_body(bar, iterations, &s_word);

@@ -1249,6 +1249,176 @@ __device__ void fused_body(const BfsArgs& a, int ph, int32_t depth, int max_leve
     }
 }
 
+// Narrow persistent kernel: expand-contract for grids of at most kAllToAllMax
+// workgroups, which high-diameter and small graphs use.  Their levels are a
+// chain of dependent accesses, and the two longest links were the barrier
+// (three hops through workgroup 0, 2.2 us) and the frontier queue's counter
+// (every workgroup's reservation at one address, 11.4 ns each: 2.9 us for
+// 256).  Here a workgroup writes what it finds to its own piece of the
+// frontier as soon as it is claimed (no shared counter, no LDS queue), and the
+// piece's length travels in its arrival word of the all-to-all barrier: every
+// workgroup gets all the lengths with the barrier itself, and finds any entry
+// by a search over their prefix sums.  What does not fit a piece goes to the
+// shared queue as before and comes first in the next frontier.
+struct NarrowShared {
+    ListSmem l;
+    uint32_t first[kAllToAllMax];  // entries before each workgroup's piece
+    uint32_t count;                // entries found by this workgroup
+    uint32_t spilled, deferred;
+    int s_wave[BFS_WAVES];
+};
+static_assert(kAllToAllMax == BFS_THREADS, "one piece per thread");
+
+constexpr uint32_t kNarrowSpilled = 0x40000000u, kNarrowDeferred = 0x80000000u, kNarrowCount = 0x3FFFFFFFu;
+
+struct NarrowSink {
+    const BfsArgs& a;
+    NarrowShared& s;
+    int32_t* piece;  // REGION entries
+    const GlobalQueue& out;
+    int32_t depth_next;
+    __device__ __forceinline__ void reserve(uint32_t, ListSmem&) {}
+    __device__ __forceinline__ void step_end() {}
+    template <int K>
+    __device__ __forceinline__ void step(uint32_t, const bool (&valid)[K], const int32_t (&v)[K],
+                                         const int32_t (&src)[K]) {
+        bool won[K];
+        td_claim(a, valid, v, src, depth_next, won);
+        uint64_t m[K];
+        uint32_t cnt = 0;
+#pragma unroll
+        for (int r = 0; r < K; ++r) {
+            m[r] = __ballot(won[r]);
+            cnt += (uint32_t)__popcll(m[r]);
+        }
+        if (cnt == 0) return;
+        uint32_t base = 0;
+        if (lane_id() == 0) base = atomicAdd(&s.count, cnt);
+        base = (uint32_t)wave_bcast((int)base, 0);
+        const uint32_t spill_start = base > (uint32_t)REGION ? base : (uint32_t)REGION;
+        uint32_t gb = 0;
+        if (base + cnt > (uint32_t)REGION) {
+            if (lane_id() == 0) {
+                gb = atomic_add_u32(out.len, base + cnt - spill_start);
+                s.spilled = 1u;
+            }
+            gb = (uint32_t)wave_bcast((int)gb, 0);
+        }
+        uint32_t at = base;
+#pragma unroll
+        for (int r = 0; r < K; ++r) {
+            const uint32_t pos = at + (uint32_t)lane_prefix(m[r]);
+            at += (uint32_t)__popcll(m[r]);
+            if (!won[r]) continue;
+            if (pos < (uint32_t)REGION) {
+                coh_st(&piece[pos], v[r], true);
+            } else if (gb + (pos - spill_start) < out.cap) {
+                coh_st(&out.keys[gb + (pos - spill_start)], v[r], true);
+            } else {
+                st_relaxed(out.overflow, 1u);
+            }
+        }
+    }
+};
+
+__device__ void fused_narrow_body(const BfsArgs& a, int ph, int32_t depth, NarrowShared& s) {
+    unsigned long long t0 = 0, busy = 0;
+    if (a.wg_stats && threadIdx.x == 0) t0 = wg_clock();
+    const GridBarrier base_of{a.bar_arrive, &a.ctr->bar_release, &a.ctr->bar_abort, 1u};
+    uint32_t epoch = barrier_base_epoch(base_of);
+    const bool grid_tier = a.grid_th != INT_MAX;
+    const bool lead = blockIdx.x == 0 && threadIdx.x == 0;
+    // The first frontier is the source, in the shared queue.
+    uint32_t n_main = ld_relaxed(&a.ctr->qlen[ph & 3]), n_in = n_main;
+    s.first[threadIdx.x] = 0u;
+    int level = 0;
+    for (;; ++level) {
+        if (n_in == 0) break;
+        if (n_in > a.qcap[ph & 1]) {
+            // A frontier the queue could not hold is an overflow here too,
+            // wherever its entries are.
+            if (lead) st_relaxed(&a.ctr->overflow, 1u);
+            break;
+        }
+        unsigned long long tb = 0;
+        if (a.wg_stats && threadIdx.x == 0) tb = wg_clock();
+        phase_begin(a, ph, n_in);
+        if (threadIdx.x == 0) s.count = s.spilled = s.deferred = 0u;
+        __syncthreads();  // also: `first` is complete
+        const int32_t* qin = a.qk[ph & 1];
+        const int32_t* pieces = a.regions + (size_t)(ph & 1) * kAllToAllMax * REGION;
+        const GlobalQueue out = out_queue(a, ph);
+        NarrowSink sink{a, s, a.regions + ((size_t)((ph + 1) & 1) * kAllToAllMax + blockIdx.x) * REGION, out,
+                        depth + 1};
+        const Deal deal = deal_out(n_in, gridDim.x, false);
+        for (uint32_t base = 0; base < n_in; base += gridDim.x * BFS_THREADS) {
+            const uint32_t i = deal.entry(base, blockIdx.x);
+            int32_t u = -1, start = 0, deg = 0;
+            if (i < n_in) {
+                if (i < n_main) {
+                    u = coh_ld(&qin[i], true);
+                } else {
+                    const uint32_t j = i - n_main;
+                    uint32_t w = 0;  // last piece with first <= j
+#pragma unroll
+                    for (uint32_t h = kAllToAllMax / 2; h >= 1; h >>= 1)
+                        if (s.first[w + h] <= j) w += h;
+                    u = coh_ld(&pieces[w * (uint32_t)REGION + (j - s.first[w])], true);
+                }
+                if (valid_vertex(a, u)) {
+                    start = a.offs[u];
+                    deg = a.offs[u + 1] - start;
+                }
+            }
+            if (grid_tier) {
+                if (deg >= a.grid_th) s.deferred = 1u;
+                defer_heavy(a, ph, u, deg, a.grid_th);
+            }
+            positional_gather<GATHER_K>(a.cols, u, start, deg, s.l, sink);
+        }
+        depth += 1;
+        ph += 1;
+        __syncthreads();
+        if (a.wg_stats && threadIdx.x == 0) busy += wg_clock() - tb;
+        uint32_t word = 0;
+        auto mine = [&] {
+            return min(s.count, (uint32_t)REGION) | (s.spilled ? kNarrowSpilled : 0u) |
+                   (s.deferred ? kNarrowDeferred : 0u);
+        };
+        if (!grid_sync_words(a.bar_words, &a.ctr->bar_abort, ++epoch, mine(), word)) break;
+        bool spilled = false;
+        if (__syncthreads_or((word & ~kNarrowCount) != 0u)) {
+            if (__syncthreads_or((word & kNarrowDeferred) != 0u)) {
+                // Lists this level deferred: the whole grid takes them in
+                // chunks, appending to the same pieces.
+                const unsigned long long alloc = __hip_atomic_load(&a.ctr->heavy_alloc[(ph - 1) & 1], __ATOMIC_RELAXED,
+                                                                   __HIP_MEMORY_SCOPE_AGENT);
+                gather_chunks(a, min((uint32_t)(alloc >> 32), a.heavy_cap), min((uint32_t)alloc, a.chunk_cap), s.l,
+                              sink);
+                __syncthreads();
+                if (!grid_sync_words(a.bar_words, &a.ctr->bar_abort, ++epoch, mine(), word)) break;
+            }
+            spilled = __syncthreads_or((word & kNarrowSpilled) != 0u) != 0;
+        }
+        n_main = spilled ? ld_relaxed(&a.ctr->qlen[ph & 3]) : 0u;
+        int total;
+        s.first[threadIdx.x] =
+            (uint32_t)wg_exclusive_scan<BFS_THREADS>((int)(word & kNarrowCount), total, s.s_wave);
+        n_in = n_main + (uint32_t)total;
+        if (n_in != 0 && lead) atomic_max_u32(a.max_depth, (uint32_t)depth);
+    }
+    if (lead) {
+        a.ctr->levels_run = (uint32_t)level;
+        a.ctr->last_level = (uint32_t)ph;
+        // Later launches continue the epochs.
+        __hip_atomic_store(&a.ctr->bar_release, (unsigned long long)epoch, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    }
+    if (a.wg_stats && threadIdx.x == 0) {
+        atomic_add_u64(&a.wg_stats[0], busy);
+        atomic_add_u64(&a.wg_stats[1], wg_clock() - t0);
+    }
+}
+
 // Global-barrier benchmark (test/gbarrier/test_gbarrier.cu:43-50): the
 // kernel does nothing but pass `iterations` barriers.
 __device__ void gbarrier_bench_body(const GridBarrier& bar, int iterations, uint32_t* s_word) {

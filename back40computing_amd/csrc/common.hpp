@@ -255,6 +255,44 @@ __device__ __forceinline__ bool grid_sync(const GridBarrier& b, uint32_t epoch, 
     return ok;
 }
 
+// All-to-all form for grids of at most one workgroup per thread of a
+// workgroup (light mode only): every workgroup stores one 64-bit arrival word,
+// (word << 32) | epoch, and thread t of every workgroup polls workgroup t's.
+// That saves the hop through workgroup 0, and each workgroup leaves with every
+// other's word: thread t gets workgroup t's in `word` (0 past the grid).
+// Arrival words alternate by epoch parity, since a workgroup that leaves
+// early may arrive at the next barrier while a slow one still polls this one.
+constexpr uint32_t kAllToAllMax = 256;
+__device__ __forceinline__ bool grid_sync_words(unsigned long long* arrive, uint32_t* abort_flag, uint32_t epoch,
+                                                uint32_t mine, uint32_t& word) {
+    __atomic_signal_fence(__ATOMIC_SEQ_CST);
+    __builtin_amdgcn_s_waitcnt(0);
+    __atomic_signal_fence(__ATOMIC_SEQ_CST);
+    __syncthreads();
+    unsigned long long* slots = arrive + (epoch & 1u) * kAllToAllMax;
+    if (threadIdx.x == 0)
+        __hip_atomic_store(&slots[blockIdx.x], ((unsigned long long)mine << 32) | epoch, __ATOMIC_RELAXED,
+                           __HIP_MEMORY_SCOPE_AGENT);
+    bool aborted = false;
+    word = 0;
+    if (threadIdx.x < gridDim.x) {
+        uint32_t spins = 0;
+        unsigned long long w;
+        while ((uint32_t)(w = __hip_atomic_load(&slots[threadIdx.x], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)) !=
+               epoch) {
+            if (ld_relaxed(abort_flag) || ++spins > kBarrierSpinLimit) {
+                st_relaxed(abort_flag, 1u);
+                aborted = true;
+                break;
+            }
+            __builtin_amdgcn_s_sleep(1);
+        }
+        word = (uint32_t)(w >> 32);
+    }
+    __atomic_signal_fence(__ATOMIC_SEQ_CST);
+    return __syncthreads_or(aborted) == 0;
+}
+
 // Barrier without a payload.
 __device__ __forceinline__ bool grid_sync(const GridBarrier& b, uint32_t epoch, uint32_t* s_word) {
     uint32_t unused = 0;

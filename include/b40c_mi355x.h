@@ -74,7 +74,8 @@ typedef struct b40c_tuning {
     int32_t saturation_quit;       /* hybrid: fused kernel quits when frontier > grid * this */
     int32_t do_alpha;              /* direction-optimizing: switch to bottom-up when m_f > m_u / alpha */
     int32_t do_beta;               /* direction-optimizing: back to top-down when n_f < n / beta   */
-    int32_t persistent_wgs_per_cu; /* persistent kernels: resident workgroups per CU        */
+    int32_t persistent_wgs_per_cu; /* persistent kernels: resident workgroups per CU (never set: */
+                                   /* at most 2, 1 on small and low-degree graphs)               */
     int32_t grid_gather_threshold; /* degree >= this: list split over all workgroups (grid tier) */
     int32_t bottom_up_grid_size;   /* direction-optimizing: workgroups per level launch, for its   */
                                    /* bottom-up steps; top-down steps use grid_size of them       */
