@@ -1,36 +1,45 @@
-// Stable LSD radix sort for gfx950: one upsweep -> spine -> downsweep triple
-// per 8-bit digit place, replacing b40c's radix_sort enactor
-// (b40c/radix_sort/enactor.cuh:520-622) and its upsweep/spine/downsweep
-// kernels (radix_sort/upsweep/kernel.cuh:90, scan/spine/kernel.cuh:92,
-// radix_sort/downsweep/kernel.cuh:236).
+// Stable LSD radix sort for gfx950, one kernel per 8-bit digit place, in the
+// place of b40c's radix_sort enactor (b40c/radix_sort/enactor.cuh:520-622) and
+// its upsweep/spine/downsweep kernels (radix_sort/upsweep/kernel.cuh:90,
+// scan/spine/kernel.cuh:92, radix_sort/downsweep/kernel.cuh:236).
 //
 // Design (MI355X-first rather than a translation):
 //  * 8-bit digits (256 bins) instead of the reference's 4-bit digits: half the
 //    passes, and 160 KB of LDS per CU easily holds the per-wave histograms.
-//  * Each workgroup owns a contiguous run of 2048-key tiles, so the spine is
-//    256 x G counters (digit-major, like partition/upsweep/cta.cuh:302-305).
+//  * The digit totals of every place do not change while keys are permuted, so
+//    one kernel (k_histogram) counts them all in one read of the keys.
+//  * A place is then one kernel (k_place).  A workgroup owns a block of
+//    consecutive keys: it counts the block's digits, publishes the counts,
+//    finds the counts of all blocks before it by looking back over their
+//    published words (chained scan with decoupled look-back, Merrill and
+//    Garland 2016), and scatters.  Counting and scattering read the block
+//    twice within microseconds, so the second read comes from the caches: HBM
+//    moves each key once in and once out per place.  The three-kernel form
+//    this replaces read the keys twice from HBM.  Blocks, not tiles, look
+//    back: the words read for that shrink with the block size.
 //  * Stable local ranking uses wave64 "match" masks built from 8 ballots (one
 //    per digit bit) and per-wave running digit counters in LDS; keys are
 //    processed in (wave, round, lane) order which equals index order inside a
 //    tile, so ranks are stable.  The tile is exchanged through LDS into digit
 //    order and written out as contiguous per-digit runs (two-phase scatter,
 //    partition/downsweep/tile.cuh:779-1030).
+//  * Sorts of at most SMALL_KEYS keys run every place in one workgroup and one
+//    launch (k_small_sort).
 //  * Signed and floating-point keys (KeyTraits, radix_sort/sort_utils.cuh:
 //    87-183) are ordered by the reference's bit twiddles, applied in
 //    registers whenever a digit is extracted: memory always holds the
 //    caller's keys, so no pass rewrites them and the trivial-pass skip stays
 //    valid for every key type.
 //  * The trivial-pass early exit (downsweep/kernel.cuh DownsweepPass) is
-//    decided on the device: the spine kernel flags a pass whose keys all share
-//    one digit, the downsweep then does nothing and a device-side selector
-//    (DoubleBuffer::selector) is left unflipped.
-//  * Scratch (spine, digit totals, selector, trivial flag) comes from the
-//    caller as a SortScratch view: a per-call allocation for the stateless
-//    entry points, the sort enactor's own buffer, or a fixed device array for
-//    the allocation-free entry point.  Launching a sort allocates nothing and
-//    does not synchronize; only reading the selector back does.
+//    decided on the device: k_plan flags places whose keys all share one digit;
+//    they move nothing, and which buffer a place reads follows from the number
+//    of places before it that did (DoubleBuffer::selector).
+//  * Scratch comes from the caller as one array of words: a per-call
+//    allocation for the stateless entry points, the sort enactor's own buffer,
+//    or a fixed device array for the allocation-free entry point; the block
+//    size grows until the look-back words fit it.  Launching a sort allocates
+//    nothing and does not synchronize; only waiting for the selector does.
 #include <mutex>
-#include <vector>
 
 #include "common.hpp"
 #include "internal.hpp"
@@ -38,10 +47,12 @@
 namespace b40c {
 namespace {
 
-constexpr int RS_THREADS = 256;
-constexpr int RS_WAVES = RS_THREADS / kWave;
 constexpr int RS_BINS = 256;
 constexpr int RS_MAX_WGS_PER_CU = 8;
+// Tiles per block of a large sort: more make fewer blocks look back, but the
+// second read of a block then misses the caches more (2^26 64-bit keys, 1 / 2 /
+// 3 / 4 / 8 / 16 tiles: 4.4 / 3.55 / 3.53 / 3.53 / 3.8 / 4.1 ms).
+constexpr int kBlockTiles = 4;
 
 // Order-preserving views of the key bits (sort_utils.cuh:87-183):
 // CONV 0 unsigned (as is), 1 signed (flip the sign bit), 2 IEEE float
@@ -61,248 +72,527 @@ __device__ __forceinline__ uint32_t digit_of(K key, int shift, uint32_t mask) {
     return (uint32_t)(ordered_bits<K, CONV>(key) >> shift) & mask;
 }
 
-// Start of a sort: digit totals of the first pass, selector and trivial flag
-// cleared (kernels, not memsets, so a caller may capture the launches).
-__global__ void k_sort_init(uint32_t* digit_total0, int32_t* sel, uint32_t* trivial) {
-    digit_total0[threadIdx.x] = 0;
-    if (threadIdx.x == 0) {
-        *sel = 0;
-        *trivial = 0;
+// A value the compiler knows nothing about: what is computed from it inside a
+// loop stays there.  Otherwise the dozens of offsets and masks that depend on
+// the lane alone are kept in registers across the whole tile loop (162 instead
+// of 97 VGPRs for 64-bit keys, one workgroup less per CU).
+__device__ __forceinline__ int opaque(int x) {
+    asm volatile("" : "+v"(x));
+    return x;
+}
+
+// Ranks of a tile's keys within (wave, digit), in index order; hist (this
+// wave's, zeroed) receives the wave's digit counts.  Keys past tile_n get
+// 0xFFFFFFFF.  Key j of a lane is tile element wid * 64 * ITEMS + j * 64 + lane.
+template <typename K, int CONV, int ITEMS>
+__device__ __forceinline__ void rank_tile(const K (&key)[ITEMS], uint32_t (&rank)[ITEMS], uint32_t* hist, int wid,
+                                          int tile_n, int shift, uint32_t mask) {
+    const int lane = opaque(lane_id());
+#pragma unroll
+    for (int j = 0; j < ITEMS; ++j) {
+        const bool valid = wid * (kWave * ITEMS) + j * kWave + lane < tile_n;
+        const uint32_t d = digit_of<K, CONV>(key[j], shift, mask);
+        uint64_t peers = __ballot(valid);
+#pragma unroll
+        for (int b = 0; b < 8; ++b) {
+            const bool bit = (d >> b) & 1u;
+            const uint64_t bal = __ballot(bit);
+            peers &= bit ? bal : ~bal;
+        }
+        const uint32_t before = hist[d];
+        rank[j] = before + (uint32_t)lane_prefix(peers);
+        const bool leader = valid && lane_prefix(peers) == 0;
+        if (leader) hist[d] = before + (uint32_t)__popcll(peers);
+        if (!valid) rank[j] = 0xFFFFFFFFu;
     }
 }
 
-// Per-workgroup digit histogram of its tile range; counts go to the spine
-// (digit-major) and to the global digit totals.
+constexpr int OS_THREADS = 512;
+constexpr int OS_WAVES = OS_THREADS / kWave;
+constexpr int MAX_PLACES = 8;
+constexpr int HIST_COPIES = 8;
+constexpr int SMALL_THREADS = 1024;
+constexpr int SMALL_ITEMS = 8;
+constexpr int SMALL_KEYS = SMALL_THREADS * SMALL_ITEMS;
+
+// Device state of one sort, carved out of its scratch words.
+struct SortState {
+    uint32_t* copies;   // [HIST_COPIES][MAX_PLACES][RS_BINS] digit totals, spread over copies
+    uint32_t* base;     // [MAX_PLACES][RS_BINS] first output position of each digit
+    uint32_t* trivial;  // [MAX_PLACES] place whose keys all share one digit
+    uint32_t* status;   // [2][blocks][RS_BINS] look-back words (by place parity), 32 or 64 bits each
+    int32_t* out;       // report: selector, failure
+    int32_t blocks;
+    int32_t wide;       // 64-bit look-back words (n >= 2^30)
+    int32_t places;
+};
+constexpr size_t kReportWords = 16;  // the report, where it is in the scratch (first words)
+constexpr size_t kStateWords = kReportWords + (size_t)(HIST_COPIES + 1) * MAX_PLACES * RS_BINS + 64;
+
+// Clears the totals and the first place's look-back words.
+__global__ __launch_bounds__(256) void k_sort_init(SortState st) {
+    const int64_t step = (int64_t)gridDim.x * 256;
+    const int64_t i0 = (int64_t)blockIdx.x * 256 + threadIdx.x;
+    for (int64_t i = i0; i < HIST_COPIES * MAX_PLACES * RS_BINS; i += step) st.copies[i] = 0;
+    const int64_t words = (int64_t)st.blocks * RS_BINS * (st.wide ? 2 : 1);
+    for (int64_t i = i0; i < words; i += step) st.status[i] = 0;
+    if (i0 < 2) st.out[i0] = 0;
+}
+
+// Digit totals of every place in one read, eight keys per thread at a time.
+// Where a wave's keys of such a step all share a place's digit (high bits,
+// mostly), the place is added once: same-address LDS atomics would cost 64
+// times that.  The test is one XOR per key and one ballot per place and step;
+// a test per key and place made the kernel issue-bound (300 us instead of
+// 125 us for 2^26 64-bit keys).  The workgroups' totals go to HIST_COPIES
+// copies: same-line atomics are serialised (11.4 ns).
 template <typename K, int CONV>
-__global__ __launch_bounds__(RS_THREADS) void k_upsweep(const K* k0, const K* k1, const int32_t* sel, int64_t n,
-                                                        int shift, uint32_t mask, int64_t keys_per_wg,
-                                                        uint32_t* spine, uint32_t* digit_total, int G) {
-    __shared__ uint32_t hist[RS_WAVES][RS_BINS];
-    const int tid = threadIdx.x, wid = tid / kWave;
-    for (int i = tid; i < RS_WAVES * RS_BINS; i += RS_THREADS) (&hist[0][0])[i] = 0;
+__global__ __launch_bounds__(OS_THREADS) void k_histogram(const K* keys, int64_t n, int begin_bit, int end_bit,
+                                                          SortState st) {
+    __shared__ uint32_t hist[2][MAX_PLACES][RS_BINS];
+    const int tid = threadIdx.x, lane = lane_id();
+    uint32_t(&mine)[MAX_PLACES][RS_BINS] = hist[(tid / kWave) & 1];
+    for (int i = tid; i < 2 * MAX_PLACES * RS_BINS; i += OS_THREADS) (&hist[0][0][0])[i] = 0;
     __syncthreads();
-    const K* keys = *sel ? k1 : k0;
-    const int64_t begin = (int64_t)blockIdx.x * keys_per_wg;
-    const int64_t end = min(n, begin + keys_per_wg);
-    // RS_UP keys per thread per round, their loads issued together.
-    constexpr int RS_UP = 8;
-    int64_t i = begin + tid;
-    for (; i + (int64_t)(RS_UP - 1) * RS_THREADS < end; i += (int64_t)RS_UP * RS_THREADS) {
-        K kk[RS_UP];
+    constexpr int R = 8;
+    const int64_t step = (int64_t)gridDim.x * OS_THREADS * R;
+    for (int64_t base = (int64_t)blockIdx.x * OS_THREADS * R; base < n; base += step) {
+        const K* kt = keys + base;
+        const uint32_t tn = (uint32_t)min((int64_t)(OS_THREADS * R), n - base);
+        K k[R];
 #pragma unroll
-        for (int j = 0; j < RS_UP; ++j) kk[j] = keys[i + (int64_t)j * RS_THREADS];
+        for (int j = 0; j < R; ++j) k[j] = kt[min((uint32_t)(j * OS_THREADS + tid), tn - 1u)];
+        K differ = 0;
 #pragma unroll
-        for (int j = 0; j < RS_UP; ++j) atomicAdd(&hist[wid][digit_of<K, CONV>(kk[j], shift, mask)], 1u);
+        for (int j = 0; j < R; ++j) {
+            k[j] = ordered_bits<K, CONV>(k[j]);
+            differ |= k[j] ^ k[0];
+        }
+        const bool whole = tn == (uint32_t)(OS_THREADS * R);
+        const K k0 = __shfl(k[0], 0, kWave);
+        differ |= k[0] ^ k0;
+#pragma unroll
+        for (int p = 0; p < (int)sizeof(K); ++p) {
+            const int shift = begin_bit + 8 * p;
+            if (shift >= end_bit) break;
+            const uint32_t mask = (1u << min(8, end_bit - shift)) - 1u;
+            if (whole && __ballot(((uint32_t)(differ >> shift) & mask) != 0u) == 0ull) {
+                if (lane == 0) atomicAdd(&mine[p][(uint32_t)(k0 >> shift) & mask], (uint32_t)(R * kWave));
+                continue;
+            }
+#pragma unroll
+            for (int j = 0; j < R; ++j)
+                if (whole || (uint32_t)(j * OS_THREADS + tid) < tn)
+                    atomicAdd(&mine[p][(uint32_t)(k[j] >> shift) & mask], 1u);
+        }
     }
-    for (; i < end; i += RS_THREADS) atomicAdd(&hist[wid][digit_of<K, CONV>(keys[i], shift, mask)], 1u);
     __syncthreads();
+    uint32_t* out = st.copies + (size_t)(blockIdx.x % HIST_COPIES) * MAX_PLACES * RS_BINS;
+    for (int i = tid; i < st.places * RS_BINS; i += OS_THREADS) {
+        const uint32_t c = (&hist[0][0][0])[i] + (&hist[1][0][0])[i];
+        if (c) atomic_add_u32(&out[i], c);
+    }
+}
+
+// One workgroup per place: the digits' first output positions, and whether
+// the place is trivial.
+__global__ __launch_bounds__(RS_BINS) void k_plan(SortState st, int64_t n) {
+    __shared__ int s_wave[RS_BINS / kWave];
+    const int p = blockIdx.x, d = threadIdx.x;
     uint32_t c = 0;
 #pragma unroll
-    for (int w = 0; w < RS_WAVES; ++w) c += hist[w][tid];
-    spine[(int64_t)tid * G + blockIdx.x] = c;
-    if (c) atomic_add_u32(&digit_total[tid], c);
+    for (int k = 0; k < HIST_COPIES; ++k) c += st.copies[((size_t)k * MAX_PLACES + p) * RS_BINS + d];
+    int total;
+    const int excl = wg_exclusive_scan<RS_BINS>((int)c, total, s_wave);
+    st.base[p * RS_BINS + d] = (uint32_t)excl;
+    const int triv = __syncthreads_or((int64_t)c == n);
+    if (d == 0) st.trivial[p] = triv ? 1u : 0u;
 }
 
-// Exclusive scan of the spine, one workgroup per digit.  Digit d's base is the
-// sum of the totals of the smaller digits.  Flags a trivial pass, and
-// workgroup 0 clears the other digit-total buffer for the next pass.
-__global__ __launch_bounds__(RS_THREADS) void k_spine(uint32_t* spine, const uint32_t* digit_total,
-                                                      uint32_t* next_digit_total, int G, int64_t n,
-                                                      uint32_t* trivial) {
-    __shared__ int s_wave[RS_WAVES];
-    const int d = blockIdx.x, tid = threadIdx.x;
-    const uint32_t t = digit_total[tid];
-    if (d == 0) next_digit_total[tid] = 0;
-    int total_below;
-    int contrib = (tid < d) ? (int)t : 0;
-    (void)wg_exclusive_scan<RS_THREADS>(contrib, total_below, s_wave);
-    if (tid == 0 && (int64_t)digit_total[d] == n) st_relaxed(trivial, 1u);
-    uint32_t carry = (uint32_t)total_below;
-    uint32_t* row = spine + (int64_t)d * G;
-    for (int base = 0; base < G; base += RS_THREADS) {
-        const int i = base + tid;
-        const int v = (i < G) ? (int)row[i] : 0;
-        int chunk_total;
-        const int excl = wg_exclusive_scan<RS_THREADS>(v, chunk_total, s_wave);
-        if (i < G) row[i] = carry + (uint32_t)excl;
-        carry += (uint32_t)chunk_total;
+// Look-back over the published words of the blocks before `block` for digit d:
+// the sum of their counts.  LOOK words are loaded together per round: a round
+// trip past the caches is about 0.7 us and a word is often found only tens of
+// blocks back.  Blocks are dispatched in order, so every block waited for is
+// running; should that fail, the bounded wait ends the sort with an error.
+constexpr uint32_t kLookSpins = 1u << 22;
+template <typename W>
+struct LookWord {
+    static constexpr W COUNT = (W)1 << (8 * sizeof(W) - 2);  // the block's own count
+    static constexpr W PREFIX = (W)2 << (8 * sizeof(W) - 2); // count of this and all blocks before
+    static constexpr W VALUE = COUNT - 1;
+};
+template <typename W>
+__device__ __forceinline__ void publish(W* status, int block, int d, uint32_t value, W flag) {
+    __hip_atomic_store(&status[(size_t)block * RS_BINS + d], flag | (W)value, __ATOMIC_RELAXED,
+                       __HIP_MEMORY_SCOPE_AGENT);
+}
+template <typename W, int LOOK>
+__device__ __forceinline__ uint32_t look_back(const W* status, int block, int d, int32_t* failed) {
+    uint32_t sum = 0, spins = 0;
+    int j = block - 1;
+    while (true) {
+        W w[LOOK];
+        // Word of block j - k, or, before the first block, of block 0, whose
+        // word is a prefix and ends the walk (j >= 0 here).
+#pragma unroll
+        for (int k = 0; k < LOOK; ++k)
+            w[k] = __hip_atomic_load(&status[(uint32_t)(max(j - k, 0) * RS_BINS + d)], __ATOMIC_RELAXED,
+                                     __HIP_MEMORY_SCOPE_AGENT);
+        int used = 0;
+        bool ready = true, done = false;
+#pragma unroll
+        for (int k = 0; k < LOOK; ++k) {
+            ready = ready && !done && w[k] >= LookWord<W>::COUNT;
+            if (ready) {
+                sum += (uint32_t)(w[k] & LookWord<W>::VALUE);
+                ++used;
+                done = w[k] >= LookWord<W>::PREFIX;
+            }
+        }
+        if (done) return sum;
+        j -= used;
+        if (used == 0) {
+            if (++spins > kLookSpins) {
+                *failed = 1;
+                return sum;
+            }
+            __builtin_amdgcn_s_sleep(1);
+        }
     }
 }
 
-// ITEMS keys per thread: a tile of RS_THREADS * ITEMS keys is ranked and
-// staged in LDS at once.  Larger tiles give longer per-digit runs in the
-// scatter (about ITEMS keys per digit on uniform keys), so fewer partial
-// cache lines are written, for more LDS per workgroup.
+// One digit place.  ITEMS keys per thread: a tile of OS_THREADS * ITEMS keys
+// is ranked and staged in LDS at once.  Bound by what passes the caches: 2^26
+// 64-bit keys take 412 us, 1.09 GB read (each key twice) and 0.69 GB written
+// (0.54 GB of keys, partial lines), 4.3 TB/s; the counting and scattering
+// kernels this replaces took 590 us.
 template <typename K, int CONV, bool VALS, int ITEMS>
-__global__ __launch_bounds__(RS_THREADS) void k_downsweep(K* k0, K* k1, uint32_t* v0, uint32_t* v1,
-                                                          const int32_t* sel, int64_t n, int shift, uint32_t mask,
-                                                          int64_t keys_per_wg, const uint32_t* spine, int G,
-                                                          const uint32_t* trivial) {
-    constexpr int RS_TILE = RS_THREADS * ITEMS;
-    if (*trivial) return;
-    __shared__ K stage_k[RS_TILE];
-    __shared__ uint32_t stage_v[VALS ? RS_TILE : 1];
-    __shared__ uint32_t wave_hist[RS_WAVES][RS_BINS];
-    __shared__ uint32_t carry[RS_BINS];
+__global__ __launch_bounds__(OS_THREADS) void k_place(K* k0, K* k1, uint32_t* v0, uint32_t* v1, int64_t n, int place,
+                                                      int shift, uint32_t mask, int64_t block_keys, SortState st) {
+    constexpr int TILE = OS_THREADS * ITEMS;
+    __shared__ K stage_k[TILE];
+    __shared__ uint32_t stage_v[VALS ? TILE : 1];
+    __shared__ uint32_t wave_hist[OS_WAVES][RS_BINS];
+    __shared__ uint32_t next_out[RS_BINS];   // next output position of each digit
+    __shared__ uint32_t out_shift[RS_BINS];  // output position minus tile position
     __shared__ uint32_t tile_excl[RS_BINS];
-    __shared__ int s_wave[RS_WAVES];
+    __shared__ int s_wave[OS_WAVES];
 
-    const int tid = threadIdx.x, lane = lane_id(), wid = tid / kWave;
-    const int s = *sel;
-    const K* kin = s ? k1 : k0;
-    K* kout = s ? k0 : k1;
-    const uint32_t* vin = VALS ? (s ? v1 : v0) : nullptr;
-    uint32_t* vout = VALS ? (s ? v0 : v1) : nullptr;
-
-    carry[tid] = spine[(int64_t)tid * G + blockIdx.x];
-    const int64_t begin = (int64_t)blockIdx.x * keys_per_wg;
-    const int64_t end = min(n, begin + keys_per_wg);
-    const uint64_t lt_mask = (lane == 0) ? 0ull : (~0ull >> (64 - lane));
+    const int tid = threadIdx.x, lane = lane_id(), wid = __builtin_amdgcn_readfirstlane(tid / kWave);
+    const int block = blockIdx.x;
+    const size_t words = (size_t)st.blocks * RS_BINS * (st.wide ? 2 : 1);
+    // The other parity's words of this block, for the next place (its last
+    // user, the place before this one, has finished).
+    uint32_t* status = st.status + (place & 1) * words;
+    uint32_t* next_status = st.status + ((place + 1) & 1) * words;
+    for (int i = tid; i < RS_BINS * (st.wide ? 2 : 1); i += OS_THREADS)
+        next_status[(size_t)block * RS_BINS * (st.wide ? 2 : 1) + i] = 0;
+    int moved = 0;  // places before this one that moved the keys
+    for (int p = 0; p < place; ++p) moved += st.trivial[p] ? 0 : 1;
+    const bool skip = st.trivial[place] != 0;
+    if (place == st.places - 1 && block == 0 && tid == 0) st.out[0] = (moved + (skip ? 0 : 1)) & 1;
+    if (skip) return;
+    const K* kin = (moved & 1) ? k1 : k0;
+    K* kout = (moved & 1) ? k0 : k1;
+    const uint32_t* vin = VALS ? ((moved & 1) ? v1 : v0) : nullptr;
+    uint32_t* vout = VALS ? ((moved & 1) ? v0 : v1) : nullptr;
+    const int64_t begin = (int64_t)block * block_keys;
+    const int64_t end = min(n, begin + block_keys);
+    const bool one_tile = end - begin <= TILE;
 
     // The next tile's keys (and values) are loaded into registers while the
     // current tile is ranked and scattered.
+    // (Positions past the end read the last key instead: no branch per load.)
     K nkey[ITEMS];
     uint32_t nval[ITEMS];
     auto load_tile = [&](int64_t tb) {
-        const int tn = (int)min((int64_t)RS_TILE, end - tb);
+        const uint32_t first = (uint32_t)(wid * (kWave * ITEMS) + opaque(lane));
+        const uint32_t last = (uint32_t)min((int64_t)TILE, end - tb) - 1u;
+        const K* kt = kin + tb;
+        const uint32_t* vt = VALS ? vin + tb : nullptr;
 #pragma unroll
         for (int j = 0; j < ITEMS; ++j) {
-            const int idx = wid * (kWave * ITEMS) + j * kWave + lane;
-            const bool valid = idx < tn;
-            nkey[j] = valid ? kin[tb + idx] : (K)0;
-            if (VALS) nval[j] = valid ? vin[tb + idx] : 0u;
+            const uint32_t idx = min(first + (uint32_t)(j * kWave), last);
+            nkey[j] = kt[idx];
+            if (VALS) nval[j] = vt[idx];
         }
     };
-    if (begin < end) load_tile(begin);
-    for (int64_t tile_base = begin; tile_base < end; tile_base += RS_TILE) {
-        const int tile_n = (int)min((int64_t)RS_TILE, end - tile_base);
+    auto announce = [&](uint32_t count) {  // threads 0 .. RS_BINS - 1
+        if (st.wide)
+            publish((unsigned long long*)status, block, tid, count,
+                    block ? LookWord<unsigned long long>::COUNT : LookWord<unsigned long long>::PREFIX);
+        else
+            publish(status, block, tid, count, block ? LookWord<uint32_t>::COUNT : LookWord<uint32_t>::PREFIX);
+    };
+    uint32_t block_count = 0;
+    if (!one_tile) {
         for (int i = lane; i < RS_BINS; i += kWave) wave_hist[wid][i] = 0;
         __syncthreads();
-
+        for (int64_t tb = begin; tb < end; tb += TILE) {
+            const uint32_t tn = (uint32_t)min((int64_t)TILE, end - tb);
+            const K* kt = kin + tb;
+            K key[ITEMS];
+#pragma unroll
+            for (int j = 0; j < ITEMS; ++j) key[j] = kt[min((uint32_t)(j * OS_THREADS + tid), tn - 1u)];
+#pragma unroll
+            for (int j = 0; j < ITEMS; ++j)
+                if ((uint32_t)(j * OS_THREADS + tid) < tn)
+                    atomicAdd(&wave_hist[wid][digit_of<K, CONV>(key[j], shift, mask)], 1u);
+        }
+        __syncthreads();
+        if (tid < RS_BINS) {
+#pragma unroll
+            for (int w = 0; w < OS_WAVES; ++w) block_count += wave_hist[w][tid];
+            announce(block_count);
+        }
+        __syncthreads();
+    }
+    load_tile(begin);
+    for (int64_t tile_base = begin; tile_base < end; tile_base += TILE) {
+        const int tile_n = (int)min((int64_t)TILE, end - tile_base);
+        const int tid = opaque((int)threadIdx.x);
+        const int lane = tid % kWave;
+        for (int i = lane; i < RS_BINS; i += kWave) wave_hist[wid][i] = 0;
+        __syncthreads();
         K key[ITEMS];
         uint32_t val[ITEMS];
         uint32_t rank[ITEMS];
-        uint32_t dig[ITEMS];
 #pragma unroll
         for (int j = 0; j < ITEMS; ++j) {
             key[j] = nkey[j];
             if (VALS) val[j] = nval[j];
         }
-        if (tile_base + RS_TILE < end) load_tile(tile_base + RS_TILE);
-#pragma unroll
-        for (int j = 0; j < ITEMS; ++j) {
-            const int idx = wid * (kWave * ITEMS) + j * kWave + lane;
-            const bool valid = idx < tile_n;
-            const uint32_t d = digit_of<K, CONV>(key[j], shift, mask);
-            dig[j] = d;
-            uint64_t peers = __ballot(valid);
-#pragma unroll
-            for (int b = 0; b < 8; ++b) {
-                const bool bit = (d >> b) & 1u;
-                const uint64_t bal = __ballot(bit);
-                peers &= bit ? bal : ~bal;
-            }
-            const uint32_t before = wave_hist[wid][d];
-            rank[j] = before + (uint32_t)__popcll(peers & lt_mask);
-            const bool leader = valid && ((peers & lt_mask) == 0);
-            if (leader) wave_hist[wid][d] = before + (uint32_t)__popcll(peers);
-            if (!valid) rank[j] = 0xFFFFFFFFu;
-        }
+        if (tile_base + TILE < end) load_tile(tile_base + TILE);
+        rank_tile<K, CONV, ITEMS>(key, rank, wave_hist[wid], wid, tile_n, shift, mask);
         __syncthreads();
         // Per digit: offsets of each wave inside the digit, and tile totals.
         uint32_t cnt = 0;
+        if (tid < RS_BINS) {
 #pragma unroll
-        for (int w = 0; w < RS_WAVES; ++w) {
-            const uint32_t c = wave_hist[w][tid];
-            wave_hist[w][tid] = cnt;
-            cnt += c;
+            for (int w = 0; w < OS_WAVES; ++w) {
+                const uint32_t c = wave_hist[w][tid];
+                wave_hist[w][tid] = cnt;
+                cnt += c;
+            }
+            if (one_tile) {
+                block_count = cnt;
+                announce(cnt);
+            }
         }
         int tot;
-        const int excl = wg_exclusive_scan<RS_THREADS>((int)cnt, tot, s_wave);
-        tile_excl[tid] = (uint32_t)excl;
+        const int excl = wg_exclusive_scan<OS_THREADS>((int)cnt, tot, s_wave);
+        if (tid < RS_BINS) tile_excl[tid] = (uint32_t)excl;
         __syncthreads();
 #pragma unroll
         for (int j = 0; j < ITEMS; ++j) {
             if (rank[j] != 0xFFFFFFFFu) {
-                const uint32_t pos = tile_excl[dig[j]] + wave_hist[wid][dig[j]] + rank[j];
+                const uint32_t d = digit_of<K, CONV>(key[j], shift, mask);
+                const uint32_t pos = tile_excl[d] + wave_hist[wid][d] + rank[j];
+                stage_k[pos] = key[j];
+                if (VALS) stage_v[pos] = val[j];
+            }
+        }
+        if (tid < RS_BINS) {
+            uint32_t at;
+            if (tile_base == begin) {
+                uint32_t before = 0;
+                if (block) {
+                    if (st.wide) {
+                        before = look_back<unsigned long long, 4>((const unsigned long long*)status, block, tid, &st.out[1]);
+                        publish((unsigned long long*)status, block, tid, before + block_count,
+                                LookWord<unsigned long long>::PREFIX);
+                    } else {
+                        before = look_back<uint32_t, 8>((const uint32_t*)status, block, tid, &st.out[1]);
+                        publish(status, block, tid, before + block_count, LookWord<uint32_t>::PREFIX);
+                    }
+                }
+                at = st.base[place * RS_BINS + tid] + before;
+            } else {
+                at = next_out[tid];
+            }
+            out_shift[tid] = at - (uint32_t)excl;
+            next_out[tid] = at + cnt;
+        }
+        __syncthreads();
+#pragma unroll
+        for (int j = 0; j < ITEMS; ++j) {
+            const int k = j * OS_THREADS + tid;
+            if (k < tile_n) {
+                const K kk = stage_k[k];
+                const uint32_t out = out_shift[digit_of<K, CONV>(kk, shift, mask)] + (uint32_t)k;
+                kout[out] = kk;
+                if (VALS) vout[out] = stage_v[k];
+            }
+        }
+        __syncthreads();
+    }
+}
+
+// Every place of a small sort in one workgroup: the keys stay in registers
+// and LDS between the places.  A launch costs 2.5 us or more and a place of a
+// few thousand keys about as much, so the launches of the large form would be
+// most of such a sort (6,001 32-bit pairs: 31 us against 100 us in 17
+// launches).
+template <typename K, int CONV, bool VALS>
+__global__ __launch_bounds__(SMALL_THREADS) void k_small_sort(K* k0, K* k1, uint32_t* v0, uint32_t* v1, int n,
+                                                              int begin_bit, int end_bit, int32_t* out) {
+    constexpr int WAVES = SMALL_THREADS / kWave;
+    __shared__ K stage_k[SMALL_KEYS];
+    __shared__ uint32_t stage_v[VALS ? SMALL_KEYS : 1];
+    __shared__ uint32_t wave_hist[WAVES][RS_BINS];
+    __shared__ uint32_t tile_excl[RS_BINS];
+    __shared__ int s_wave[WAVES];
+    const int tid = threadIdx.x, lane = lane_id(), wid = tid / kWave;
+    K key[SMALL_ITEMS];
+    uint32_t val[SMALL_ITEMS], rank[SMALL_ITEMS];
+#pragma unroll
+    for (int j = 0; j < SMALL_ITEMS; ++j) {
+        const int idx = wid * (kWave * SMALL_ITEMS) + j * kWave + lane;
+        key[j] = idx < n ? k0[idx] : (K)0;
+        if (VALS) val[j] = idx < n ? v0[idx] : 0u;
+    }
+    int moved = 0;
+    for (int shift = begin_bit; shift < end_bit; shift += 8) {
+        const uint32_t mask = (1u << min(8, end_bit - shift)) - 1u;
+        for (int i = lane; i < RS_BINS; i += kWave) wave_hist[wid][i] = 0;
+        __syncthreads();
+        rank_tile<K, CONV, SMALL_ITEMS>(key, rank, wave_hist[wid], wid, n, shift, mask);
+        __syncthreads();
+        uint32_t cnt = 0;
+        if (tid < RS_BINS) {
+#pragma unroll
+            for (int w = 0; w < WAVES; ++w) {
+                const uint32_t c = wave_hist[w][tid];
+                wave_hist[w][tid] = cnt;
+                cnt += c;
+            }
+        }
+        int tot;
+        const int excl = wg_exclusive_scan<SMALL_THREADS>((int)cnt, tot, s_wave);
+        if (tid < RS_BINS) tile_excl[tid] = (uint32_t)excl;
+        if (__syncthreads_or(tid < RS_BINS && cnt == (uint32_t)n)) continue;  // all keys share one digit
+        ++moved;
+#pragma unroll
+        for (int j = 0; j < SMALL_ITEMS; ++j) {
+            if (rank[j] != 0xFFFFFFFFu) {
+                const uint32_t d = digit_of<K, CONV>(key[j], shift, mask);
+                const uint32_t pos = tile_excl[d] + wave_hist[wid][d] + rank[j];
                 stage_k[pos] = key[j];
                 if (VALS) stage_v[pos] = val[j];
             }
         }
         __syncthreads();
-        for (int k = tid; k < tile_n; k += RS_THREADS) {
-            const K kk = stage_k[k];
-            const uint32_t d = digit_of<K, CONV>(kk, shift, mask);
-            const uint32_t out = carry[d] + (uint32_t)k - tile_excl[d];
-            kout[out] = kk;
-            if (VALS) vout[out] = stage_v[k];
+#pragma unroll
+        for (int j = 0; j < SMALL_ITEMS; ++j) {
+            const int idx = wid * (kWave * SMALL_ITEMS) + j * kWave + lane;
+            if (idx < n) {
+                key[j] = stage_k[idx];
+                if (VALS) val[j] = stage_v[idx];
+            }
         }
-        __syncthreads();
-        carry[tid] += cnt;
-        __syncthreads();
+    }
+    if (moved) {
+        K* ko = (moved & 1) ? k1 : k0;
+        uint32_t* vo = (moved & 1) ? v1 : v0;
+#pragma unroll
+        for (int j = 0; j < SMALL_ITEMS; ++j) {
+            const int idx = wid * (kWave * SMALL_ITEMS) + j * kWave + lane;
+            if (idx < n) {
+                ko[idx] = key[j];
+                if (VALS) vo[idx] = val[j];
+            }
+        }
+    }
+    if (tid == 0) {
+        out[0] = moved & 1;
+        out[1] = 0;
     }
 }
 
-__global__ void k_flip_selector(int32_t* sel, uint32_t* trivial) {
-    if (*trivial == 0) *sel ^= 1;
-    *trivial = 0;
-}
-
-// Launch shape for n keys on a device with `num_cus` CUs: at most
-// policy.wgs_per_cu workgroups per CU, each owning a whole number of tiles.
+// Block size and count for n keys: whole tiles, at most `max_blocks` blocks.
 struct SortPlan {
-    int64_t keys_per_wg = 1;
-    int G = 1;
+    int64_t block_keys = 1;
+    int blocks = 1;
     int items = 8;
+    bool wide = false;
+    int hist_wgs = 1;
 };
 
-SortPlan sort_plan(int64_t n, int num_cus, const SortPolicy& pol) {
+size_t look_words(const SortPlan& p) { return (size_t)2 * p.blocks * RS_BINS * (p.wide ? 2 : 1); }
+
+// max_words: scratch words there are (0: as many as the plan wants).
+SortPlan sort_plan(int64_t n, int num_cus, const SortPolicy& pol, size_t max_words = 0) {
     SortPlan p;
     p.items = pol.items;
-    const int64_t tile = (int64_t)RS_THREADS * pol.items;
-    const int64_t num_tiles = std::max<int64_t>(1, (n + tile - 1) / tile);
-    const int64_t max_grid = (int64_t)num_cus * pol.wgs_per_cu;
-    const int64_t tiles_per_wg = (num_tiles + max_grid - 1) / max_grid;
-    p.keys_per_wg = tiles_per_wg * tile;
-    p.G = (int)((num_tiles + tiles_per_wg - 1) / tiles_per_wg);
+    p.wide = n >= (1ll << 30);
+    const int64_t tile = (int64_t)OS_THREADS * pol.items;
+    const int64_t tiles = std::max<int64_t>(1, (n + tile - 1) / tile);
+    int64_t max_blocks = pol.wgs_per_cu > 0 ? (int64_t)num_cus * pol.wgs_per_cu : tiles;
+    int64_t per = std::max<int64_t>((tiles + max_blocks - 1) / max_blocks, 1);
+    if (pol.wgs_per_cu == 0) per = std::max<int64_t>(1, std::min<int64_t>(kBlockTiles, tiles / ((int64_t)num_cus * 4)));
+    if (max_words) {
+        const int64_t fit = (int64_t)((max_words - kStateWords) / (2 * RS_BINS * (p.wide ? 2 : 1)));
+        per = std::max(per, (tiles + fit - 1) / fit);
+    }
+    p.block_keys = per * tile;
+    p.blocks = (int)((tiles + per - 1) / per);
+    p.hist_wgs = (int)std::min<int64_t>((n + OS_THREADS * 8 - 1) / (OS_THREADS * 8), (int64_t)num_cus * 2);
     return p;
 }
 
+SortState sort_state(const SortScratch& sc, const SortPlan& plan, int places, int32_t* out) {
+    SortState st;
+    st.copies = sc.base + kReportWords;
+    st.base = st.copies + (size_t)HIST_COPIES * MAX_PLACES * RS_BINS;
+    st.trivial = st.base + (size_t)MAX_PLACES * RS_BINS;
+    st.status = sc.base + kStateWords;
+    st.out = out;
+    st.blocks = plan.blocks;
+    st.wide = plan.wide ? 1 : 0;
+    st.places = places;
+    return st;
+}
+
 template <typename K, int CONV, bool VALS, int ITEMS>
-void launch_passes(K* k0, K* k1, uint32_t* v0, uint32_t* v1, int64_t n, int begin_bit, int end_bit,
-                   const SortPlan& plan, const SortScratch& sc, hipStream_t stream) {
-    uint32_t* dtot[2] = {sc.digit_total, sc.digit_total + RS_BINS};
-    hipLaunchKernelGGL(k_sort_init, dim3(1), dim3(RS_BINS), 0, stream, dtot[0], sc.sel, sc.trivial);
-    int pass = 0;
-    for (int shift = begin_bit; shift < end_bit; shift += 8, ++pass) {
-        const int bits = std::min(8, end_bit - shift);
-        const uint32_t mask = (1u << bits) - 1u;
-        uint32_t* cur = dtot[pass & 1];
-        uint32_t* next = dtot[(pass + 1) & 1];
-        hipLaunchKernelGGL((k_upsweep<K, CONV>), dim3(plan.G), dim3(RS_THREADS), 0, stream, k0, k1, sc.sel, n, shift,
-                           mask, plan.keys_per_wg, sc.spine, cur, plan.G);
-        hipLaunchKernelGGL(k_spine, dim3(RS_BINS), dim3(RS_THREADS), 0, stream, sc.spine, cur, next, plan.G, n,
-                           sc.trivial);
-        hipLaunchKernelGGL((k_downsweep<K, CONV, VALS, ITEMS>), dim3(plan.G), dim3(RS_THREADS), 0, stream, k0, k1, v0,
-                           v1, sc.sel, n, shift, mask, plan.keys_per_wg, sc.spine, plan.G, sc.trivial);
-        hipLaunchKernelGGL(k_flip_selector, dim3(1), dim3(1), 0, stream, sc.sel, sc.trivial);
+void launch_places(K* k0, K* k1, uint32_t* v0, uint32_t* v1, int64_t n, int begin_bit, int end_bit,
+                   const SortPlan& plan, const SortState& st, hipStream_t stream) {
+    const int64_t clear = (int64_t)HIST_COPIES * MAX_PLACES * RS_BINS + (int64_t)look_words(plan) / 2;
+    hipLaunchKernelGGL(k_sort_init, dim3((unsigned)std::min<int64_t>((clear + 1023) / 1024, 512)), dim3(256), 0, stream,
+                       st);
+    hipLaunchKernelGGL((k_histogram<K, CONV>), dim3(plan.hist_wgs), dim3(OS_THREADS), 0, stream, (const K*)k0, n,
+                       begin_bit, end_bit, st);
+    hipLaunchKernelGGL(k_plan, dim3(st.places), dim3(RS_BINS), 0, stream, st, n);
+    for (int place = 0, shift = begin_bit; shift < end_bit; shift += 8, ++place) {
+        const uint32_t mask = (1u << std::min(8, end_bit - shift)) - 1u;
+        hipLaunchKernelGGL((k_place<K, CONV, VALS, ITEMS>), dim3(plan.blocks), dim3(OS_THREADS), 0, stream, k0, k1, v0,
+                           v1, n, place, shift, mask, plan.block_keys, st);
     }
 }
 
 template <typename K, int CONV>
 void launch_typed(void* k0, void* k1, uint32_t* v0, uint32_t* v1, int64_t n, int begin_bit, int end_bit,
-                  const SortPlan& plan, const SortScratch& sc, hipStream_t stream) {
+                  const SortPlan& plan, const SortScratch& sc, int32_t* out, hipStream_t stream) {
+    if (n <= SMALL_KEYS) {
+        if (v0)
+            hipLaunchKernelGGL((k_small_sort<K, CONV, true>), dim3(1), dim3(SMALL_THREADS), 0, stream, (K*)k0, (K*)k1,
+                               v0, v1, (int)n, begin_bit, end_bit, out);
+        else
+            hipLaunchKernelGGL((k_small_sort<K, CONV, false>), dim3(1), dim3(SMALL_THREADS), 0, stream, (K*)k0, (K*)k1,
+                               v0, v1, (int)n, begin_bit, end_bit, out);
+        return;
+    }
+    const SortState st = sort_state(sc, plan, (end_bit - begin_bit + 7) / 8, out);
     if (v0) {
         if (plan.items == 16)
-            launch_passes<K, CONV, true, 16>((K*)k0, (K*)k1, v0, v1, n, begin_bit, end_bit, plan, sc, stream);
+            launch_places<K, CONV, true, 16>((K*)k0, (K*)k1, v0, v1, n, begin_bit, end_bit, plan, st, stream);
         else
-            launch_passes<K, CONV, true, 8>((K*)k0, (K*)k1, v0, v1, n, begin_bit, end_bit, plan, sc, stream);
+            launch_places<K, CONV, true, 8>((K*)k0, (K*)k1, v0, v1, n, begin_bit, end_bit, plan, st, stream);
     } else {
         if (plan.items == 16)
-            launch_passes<K, CONV, false, 16>((K*)k0, (K*)k1, nullptr, nullptr, n, begin_bit, end_bit, plan, sc,
+            launch_places<K, CONV, false, 16>((K*)k0, (K*)k1, nullptr, nullptr, n, begin_bit, end_bit, plan, st,
                                               stream);
         else
-            launch_passes<K, CONV, false, 8>((K*)k0, (K*)k1, nullptr, nullptr, n, begin_bit, end_bit, plan, sc,
+            launch_places<K, CONV, false, 8>((K*)k0, (K*)k1, nullptr, nullptr, n, begin_bit, end_bit, plan, st,
                                              stream);
     }
 }
@@ -336,68 +626,120 @@ b40c_status validate(const char* who, int32_t key_type, const void* k0, const vo
 
 }  // namespace
 
-// Defaults: 8 keys per thread and 4 workgroups per CU.
+// Default: 8 keys per thread; blocks as sort_plan sizes them.
 SortPolicy resolve_sort_policy(SortPolicy p, int64_t n, int key_bytes) {
     (void)n;
     (void)key_bytes;
     if (p.items != 8 && p.items != 16) p.items = 8;
-    if (p.wgs_per_cu < 1 || p.wgs_per_cu > RS_MAX_WGS_PER_CU) p.wgs_per_cu = 4;
+    if (p.wgs_per_cu < 0 || p.wgs_per_cu > RS_MAX_WGS_PER_CU) p.wgs_per_cu = 0;
     return p;
 }
 
 size_t sort_scratch_words(int64_t n, int num_cus, const SortPolicy& pol) {
-    const SortPlan p = sort_plan(n, num_cus, pol);
-    return (size_t)RS_BINS * (size_t)p.G + 2 * RS_BINS + 2;
+    if (n <= SMALL_KEYS) return kReportWords;
+    return kStateWords + look_words(sort_plan(n, num_cus, pol));
 }
 
-SortScratch sort_scratch_view(uint32_t* words, size_t count) {
-    SortScratch sc;
-    sc.words = count;
-    sc.digit_total = words;
-    sc.sel = (int32_t*)(words + 2 * RS_BINS);
-    sc.trivial = words + 2 * RS_BINS + 1;
-    sc.spine = words + 2 * RS_BINS + 2;
-    return sc;
-}
+// Pinned host words that sorts report through (selector, failure): one page
+// per process, a slot per sort in flight, so no copy follows a sort.  Held
+// until the process ends.  A sort beyond the slots reads its report back with
+// a copy instead.
+namespace {
+class SortReports {
+  public:
+    static constexpr int kSlots = 64;
+    // Null when the page could not be had or every slot is taken.
+    int32_t* take() {
+        std::lock_guard<std::mutex> lock(mu_);
+        if (!tried_) {
+            tried_ = true;
+            if (hipHostMalloc((void**)&page_, kSlots * kStride * sizeof(int32_t),
+                              hipHostMallocCoherent | hipHostMallocPortable | hipHostMallocMapped) != hipSuccess) {
+                page_ = nullptr;
+                (void)hipGetLastError();
+            }
+        }
+        if (!page_) return nullptr;
+        for (int i = 0; i < kSlots; ++i)
+            if (!used_[i]) {
+                used_[i] = true;
+                return page_ + i * kStride;
+            }
+        return nullptr;
+    }
+    void give(int32_t* slot) {
+        std::lock_guard<std::mutex> lock(mu_);
+        used_[(slot - page_) / kStride] = false;
+    }
 
-b40c_status radix_sort_async(int32_t key_type, void* k0, void* k1, uint32_t* v0, uint32_t* v1, int64_t n,
-                             int begin_bit, int end_bit, int num_cus, const SortPolicy& policy,
-                             const SortScratch& sc, hipStream_t stream, bool& launched) {
-    launched = false;
-    if (n <= 1 || begin_bit == end_bit) return B40C_OK;
-    const SortPolicy pol = resolve_sort_policy(policy, n, key_bits(key_type) / 8);
-    const SortPlan plan = sort_plan(n, num_cus, pol);
-    if (sort_scratch_words(n, num_cus, pol) > sc.words)
-        return fail(B40C_ERR_INVALID_ARG, "radix sort: scratch of %zu words is smaller than the %zu needed", sc.words,
-                    sort_scratch_words(n, num_cus, pol));
+  private:
+    static constexpr int kStride = 16;
+    std::mutex mu_;
+    bool tried_ = false;
+    int32_t* page_ = nullptr;
+    bool used_[kSlots] = {};
+};
+SortReports g_reports;
+
+// One sort's report words: a pinned slot, or, without one, the first words of
+// the scratch, copied back after the sort.
+struct SortReport {
+    int32_t* slot = nullptr;
+    int32_t* dev = nullptr;
+    ~SortReport() {
+        if (slot) g_reports.give(slot);
+    }
+    b40c_status take(const SortScratch& sc, bool pinned) {
+        if (pinned) slot = g_reports.take();
+        if (slot)
+            B40C_HIP(hipHostGetDevicePointer((void**)&dev, slot, 0));
+        else
+            dev = reinterpret_cast<int32_t*>(sc.base);
+        return B40C_OK;
+    }
+    b40c_status wait(int32_t (&words)[2], hipStream_t stream) {
+        if (!slot) B40C_HIP(hipMemcpyAsync(words, dev, sizeof(words), hipMemcpyDeviceToHost, stream));
+        B40C_HIP(hipStreamSynchronize(stream));
+        if (slot) {
+            words[0] = slot[0];
+            words[1] = slot[1];
+        }
+        return B40C_OK;
+    }
+};
+}  // namespace
+
+// Launches the sort (no allocation, no synchronization).
+static b40c_status radix_sort_launch(int32_t key_type, void* k0, void* k1, uint32_t* v0, uint32_t* v1, int64_t n,
+                                     int begin_bit, int end_bit, int num_cus, const SortPolicy& pol,
+                                     const SortScratch& sc, int32_t* report, hipStream_t stream) {
+    const SortPlan plan = sort_plan(n, num_cus, pol, sc.words);
     switch (key_type) {
-        case B40C_KEY_U32: launch_typed<uint32_t, KC_UNSIGNED>(k0, k1, v0, v1, n, begin_bit, end_bit, plan, sc, stream); break;
-        case B40C_KEY_I32: launch_typed<uint32_t, KC_SIGNED>(k0, k1, v0, v1, n, begin_bit, end_bit, plan, sc, stream); break;
-        case B40C_KEY_F32: launch_typed<uint32_t, KC_FLOAT>(k0, k1, v0, v1, n, begin_bit, end_bit, plan, sc, stream); break;
-        case B40C_KEY_U64: launch_typed<uint64_t, KC_UNSIGNED>(k0, k1, v0, v1, n, begin_bit, end_bit, plan, sc, stream); break;
-        case B40C_KEY_I64: launch_typed<uint64_t, KC_SIGNED>(k0, k1, v0, v1, n, begin_bit, end_bit, plan, sc, stream); break;
-        case B40C_KEY_F64: launch_typed<uint64_t, KC_FLOAT>(k0, k1, v0, v1, n, begin_bit, end_bit, plan, sc, stream); break;
+        case B40C_KEY_U32: launch_typed<uint32_t, KC_UNSIGNED>(k0, k1, v0, v1, n, begin_bit, end_bit, plan, sc, report, stream); break;
+        case B40C_KEY_I32: launch_typed<uint32_t, KC_SIGNED>(k0, k1, v0, v1, n, begin_bit, end_bit, plan, sc, report, stream); break;
+        case B40C_KEY_F32: launch_typed<uint32_t, KC_FLOAT>(k0, k1, v0, v1, n, begin_bit, end_bit, plan, sc, report, stream); break;
+        case B40C_KEY_U64: launch_typed<uint64_t, KC_UNSIGNED>(k0, k1, v0, v1, n, begin_bit, end_bit, plan, sc, report, stream); break;
+        case B40C_KEY_I64: launch_typed<uint64_t, KC_SIGNED>(k0, k1, v0, v1, n, begin_bit, end_bit, plan, sc, report, stream); break;
+        case B40C_KEY_F64: launch_typed<uint64_t, KC_FLOAT>(k0, k1, v0, v1, n, begin_bit, end_bit, plan, sc, report, stream); break;
         default: return fail(B40C_ERR_INVALID_ARG, "radix sort: unknown key type %d", key_type);
     }
     B40C_HIP(hipGetLastError());
-    launched = true;
     return B40C_OK;
 }
 
-// Runs a sort with its scratch and reads the selector back (one stream
-// synchronization).
-b40c_status radix_sort_sync(int32_t key_type, void* k0, void* k1, uint32_t* v0, uint32_t* v1, int64_t n, int begin_bit,
-                            int end_bit, int num_cus, const SortPolicy& policy, const SortScratch& sc,
-                            int32_t* selector, hipStream_t stream) {
-    bool launched = false;
-    B40C_TRY(radix_sort_async(key_type, k0, k1, v0, v1, n, begin_bit, end_bit, num_cus, policy, sc, stream,
-                              launched));
-    int32_t h_sel = 0;
-    if (launched) {
-        B40C_HIP(hipMemcpyAsync(&h_sel, sc.sel, sizeof(int32_t), hipMemcpyDeviceToHost, stream));
-        B40C_HIP(hipStreamSynchronize(stream));
-    }
-    *selector = h_sel;
+// Runs a sort with its scratch and waits for the selector (one stream
+// synchronization).  `pinned` false: nothing is allocated, not even the
+// report page of the process's first sort.
+static b40c_status radix_sort_sync(int32_t key_type, void* k0, void* k1, uint32_t* v0, uint32_t* v1, int64_t n,
+                                   int begin_bit, int end_bit, int num_cus, const SortPolicy& pol,
+                                   const SortScratch& sc, int32_t* selector, hipStream_t stream, bool pinned = true) {
+    SortReport report;
+    B40C_TRY(report.take(sc, pinned));
+    B40C_TRY(radix_sort_launch(key_type, k0, k1, v0, v1, n, begin_bit, end_bit, num_cus, pol, sc, report.dev, stream));
+    int32_t words[2] = {0, 0};
+    B40C_TRY(report.wait(words, stream));
+    if (words[1]) return fail(B40C_ERR_HIP, "radix sort: a block waited too long for the blocks before it");
+    *selector = words[0];
     return B40C_OK;
 }
 
@@ -413,7 +755,7 @@ b40c_status radix_sort_once(int32_t key_type, void* k0, void* k1, uint32_t* v0, 
     const size_t words = sort_scratch_words(n, info.num_cus, pol);
     B40C_TRY(mem.alloc(words * sizeof(uint32_t)));
     return radix_sort_sync(key_type, k0, k1, v0, v1, n, begin_bit, end_bit, info.num_cus, pol,
-                           sort_scratch_view(mem.as<uint32_t>(), words), selector, stream);
+                           SortScratch{mem.as<uint32_t>(), words}, selector, stream);
 }
 
 b40c_status radix_sort_u64(uint64_t* k0, uint64_t* k1, int64_t n, int begin_bit, int end_bit, int32_t* selector,
@@ -433,16 +775,16 @@ b40c_status radix_sort_pairs_u32(uint32_t* k0, uint32_t* k1, uint32_t* v0, uint3
 // ---------------------------------------------------------------------------
 // Allocation-free sort (no counterpart in the reference): its scratch is this
 // fixed device array, one copy per GPU, which the GPU keeps until the
-// process ends.  The grid is capped at RS_MAX_WGS_PER_CU workgroups per CU,
-// so kNoAllocWords covers a sort of any n <= 2^32 - 1 under any policy on a
-// device with up to kNoAllocMaxCus CUs (256 on MI355X): 2 MiB + 2 KiB.  In host code `scratch`
+// process ends: 2 MiB + 2 KiB, enough for the look-back words of 950 blocks
+// (475 from 2^30 keys on); blocks are as large as n <= 2^32 - 1 keys then need.
+// In host code `scratch`
 // is only a stand-in for the device array; its device address comes from
 // hipGetSymbolAddress, once per device, and only that address is used.
 // ---------------------------------------------------------------------------
 namespace b40c {
 namespace {
-constexpr int kNoAllocMaxCus = 256;
-constexpr size_t kNoAllocWords = (size_t)RS_BINS * RS_MAX_WGS_PER_CU * kNoAllocMaxCus + 2 * RS_BINS + 64;
+constexpr size_t kNoAllocWords = (size_t)RS_BINS * 2048 + 2 * RS_BINS + 64;
+static_assert(kNoAllocWords > kStateWords + 400 * 2 * RS_BINS * 2, "room for the state and hundreds of blocks");
 }  // namespace
 }  // namespace b40c
 
@@ -524,13 +866,8 @@ b40c_status b40c_radix_sort_u64_noalloc(uint64_t* d_keys0, uint64_t* d_keys1, in
     NoAllocSlot* slot = nullptr;
     B40C_TRY(noalloc_slot(slot));
     const SortPolicy pol = resolve_sort_policy(SortPolicy{}, n, 8);
-    const size_t need = sort_scratch_words(n, slot->num_cus, pol);
-    if (need > kNoAllocWords)
-        return fail(B40C_ERR_UNSUPPORTED,
-                    "b40c_radix_sort_u64_noalloc: n=%lld on %d CUs needs %zu scratch words; the fixed array holds %zu",
-                    (long long)n, slot->num_cus, need, kNoAllocWords);
     return radix_sort_sync(B40C_KEY_U64, d_keys0, d_keys1, nullptr, nullptr, n, begin_bit, end_bit, slot->num_cus,
-                           pol, sort_scratch_view(slot->ptr, kNoAllocWords), selector, nullptr);
+                           pol, SortScratch{slot->ptr, kNoAllocWords}, selector, nullptr, false);
 }
 
 b40c_status b40c_sort_enactor_create(b40c_sort_enactor** out) {
@@ -560,7 +897,7 @@ b40c_status b40c_sort_enactor_sort(b40c_sort_enactor* e, int32_t key_type, void*
     // Grow-only: later sorts of at most this size allocate nothing.
     B40C_TRY(e->scratch.reserve(words * sizeof(uint32_t)));
     return radix_sort_sync(key_type, d_keys0, d_keys1, d_vals0, d_vals1, n, begin_bit, end_bit, info.num_cus, pol,
-                           sort_scratch_view(e->scratch.as<uint32_t>(), e->scratch.bytes / sizeof(uint32_t)), selector,
+                           SortScratch{e->scratch.as<uint32_t>(), e->scratch.bytes / sizeof(uint32_t)}, selector,
                            e->stream);
 }
 

@@ -60,7 +60,7 @@ KEY_TYPES = {
 class Enactor:
     """radix_sort::Enactor::Sort(DoubleBuffer&, num_elements) for any key type
     of the reference's KeyTraits (radix_sort/sort_utils.cuh:87-183), keys
-    only or with uint32 values.  The enactor owns its scratch (the spine)
+    only or with uint32 values.  The enactor owns its scratch
     across calls, as the reference Enactor owns its spine storage."""
 
     def __init__(self):
@@ -70,7 +70,7 @@ class Enactor:
 
     def set_policy(self, items_per_thread=0, wgs_per_cu=0):
         """Launch policy (0 = the tuned default): keys per thread of a
-        downsweep tile (8 or 16) and workgroups per CU (1-8)."""
+        tile (8 or 16) and workgroups per CU (1-8)."""
         check(lib().b40c_sort_enactor_set_policy(self._h, int(items_per_thread), int(wgs_per_cu)))
 
     def Sort(self, storage, num_elements, begin_bit=0, end_bit=None):

@@ -55,7 +55,7 @@ template <> struct KeyTypeCode<uint64_t> { static constexpr int32_t value = B40C
 template <> struct KeyTypeCode<int64_t> { static constexpr int32_t value = B40C_KEY_I64; };
 template <> struct KeyTypeCode<double> { static constexpr int32_t value = B40C_KEY_F64; };
 
-// Owns its scratch (the spine) across calls, like the reference Enactor
+// Owns its scratch across calls, like the reference Enactor
 // (radix_sort/enactor.cuh:96-140).  Not copyable.
 class Enactor {
 public:

@@ -172,7 +172,7 @@ b40c_status b40c_scan_u32(const uint32_t* d_in, uint32_t* d_out, int64_t n, int3
 
 /* ---- radix sort (b40c/radix_sort/enactor.cuh:153-266) ------------------- */
 /* Stable LSD sort of device keys over bits [begin_bit, end_bit) with 8-bit
- * digits (upsweep -> spine -> downsweep per digit place).  d_keys[0] holds the
+ * digits (one histogram of every place, then one kernel per place).  d_keys[0] holds the
  * input; d_keys[1] must have room for n keys.  On return *selector says which
  * buffer holds the result (DoubleBuffer::selector, util/multiple_buffering.cuh:
  * 65-80).  Digit places whose keys all share one digit are skipped. */
@@ -184,9 +184,9 @@ b40c_status b40c_radix_sort_pairs_u32(uint32_t* d_keys0, uint32_t* d_keys1, uint
 /* b40c_radix_sort_u64 without any allocation.  No counterpart in the
  * reference: for callers that cannot allocate device memory (code that must
  * not call hipMalloc, tight serving loops, harnesses that forbid it).  The
- * scratch is a fixed 1 MiB device array per GPU, held until the process
- * ends, which covers any n <= 2^32 - 1 on a device of up to 256 CUs (larger
- * requests fail with B40C_ERR_UNSUPPORTED).  All calls on one GPU share that
+ * scratch is a fixed 2 MiB device array per GPU, held until the process
+ * ends, which covers any n <= 2^32 - 1 (larger requests fail with
+ * B40C_ERR_UNSUPPORTED).  All calls on one GPU share that
  * array, so calls that overlap in time on one GPU (other host threads) race
  * and must be serialized by the caller.  Synchronous, on the default stream. */
 b40c_status b40c_radix_sort_u64_noalloc(uint64_t* d_keys0, uint64_t* d_keys1, int64_t n, int32_t begin_bit,
@@ -208,7 +208,7 @@ b40c_status b40c_radix_sort_u64_noalloc(uint64_t* d_keys0, uint64_t* d_keys1, in
  * (radix_sort/enactor.cuh:153-266).  Scratch is allocated for the call. */
 b40c_status b40c_radix_sort(int32_t key_type, void* d_keys0, void* d_keys1, uint32_t* d_vals0, uint32_t* d_vals1,
                             int64_t n, int32_t begin_bit, int32_t end_bit, int32_t* selector);
-/* A sort enactor owns its scratch (the spine) across calls, like the
+/* A sort enactor owns its scratch across calls, like the
  * reference Enactor's spine storage (radix_sort/enactor.cuh:96-140): a sort
  * no larger than an earlier one on the same enactor allocates nothing.  One
  * HIP stream per enactor; calls are synchronous (the selector is read back). */
@@ -219,8 +219,8 @@ b40c_status b40c_sort_enactor_sort(b40c_sort_enactor* e, int32_t key_type, void*
                                    int32_t end_bit, int32_t* selector);
 /* The enactor's launch policy, the run-time form of the reference's
  * per-architecture sort policies (radix_sort/autotuned_policy.cuh:190-230):
- * keys per thread of a downsweep tile (8 or 16; 0 = default) and
- * workgroups per CU (1-8; 0 = default).  The defaults are the tuned values
+ * keys per thread of a tile (8 or 16; 0 = default) and workgroups per CU
+ * (1-8, each then sorting one block of keys per digit place; 0 = default).  The defaults are the tuned values
  * the stateless sorts and the CSR builds use. */
 b40c_status b40c_sort_enactor_set_policy(b40c_sort_enactor* e, int32_t items_per_thread, int32_t wgs_per_cu);
 void b40c_sort_enactor_destroy(b40c_sort_enactor* e);
