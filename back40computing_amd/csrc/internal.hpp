@@ -38,6 +38,21 @@ struct DeviceBuffer {
     T* as() const { return static_cast<T*>(ptr); }
 };
 
+// runtime.hip.  A call's report: a few pinned host words that its kernels
+// write and the host reads after one stream synchronization, in place of a copy
+// (about 10 us).  One page of slots per process, held until it ends; take()
+// is false when the page could not be had or every slot is in use.
+struct ReportSlot {
+    void* host = nullptr;  // kBytes bytes, zeroed by take()
+    void* dev = nullptr;   // the same words as kernels address them
+    static constexpr size_t kBytes = 64;
+    ReportSlot() = default;
+    ReportSlot(const ReportSlot&) = delete;
+    ReportSlot& operator=(const ReportSlot&) = delete;
+    ~ReportSlot();
+    bool take();
+};
+
 // radix_sort.hip.  A sort's device scratch: one block of `words` uint32 words.
 struct SortScratch {
     uint32_t* base = nullptr;

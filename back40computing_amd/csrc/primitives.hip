@@ -1,14 +1,19 @@
-// Device primitives next to the CSR build, each a chunked three-pass
-// (count or reduce per chunk, one-workgroup spine, ordered scatter) over
-// coalesced 256-element tiles:
+// Device primitives next to the CSR build:
 //  * consecutive removal — consecutive_removal::Enactor::Trim
 //    (b40c/consecutive_removal/enactor.cuh:119-126): the first element of
 //    every run of equal keys (and its value), in input order;
 //  * prefix sum — scan::Enactor::Scan (b40c/scan/enactor.cuh:122-136),
 //    exclusive or inclusive, unsigned 32-bit arithmetic.
-// Chunks are contiguous, so each workgroup streams its own slice; the chunk
-// count is a few workgroups per CU, enough to fill the chip while keeping the
-// spine to one workgroup.
+// Each is one kernel: a workgroup holds a block of the input in registers and
+// waits for the sum of the blocks before it, which one workgroup keeps, so the
+// input is read once.  Scans of arrays that are not 16-byte aligned or longer
+// than the chain's words can sum (2^30 elements) take three passes over
+// contiguous chunks instead: reduce per chunk, one-workgroup spine, ordered
+// scan.
+#include <algorithm>
+#include <climits>
+#include <cstring>
+
 #include "internal.hpp"
 
 namespace b40c {
@@ -47,18 +52,6 @@ __device__ __forceinline__ T wg_scan_excl(T x, T& total, T* s_wave) {
     return base + incl - x;
 }
 
-__device__ __forceinline__ bool run_head(const uint64_t* keys, int64_t i) { return i == 0 || keys[i - 1] != keys[i]; }
-
-__global__ __launch_bounds__(PT) void k_trim_count(const uint64_t* keys, int64_t n, int64_t chunk, uint64_t* counts) {
-    __shared__ uint64_t s_wave[PW];
-    const int64_t begin = (int64_t)blockIdx.x * chunk, end = min(n, begin + chunk);
-    uint64_t c = 0;
-    for (int64_t i = begin + threadIdx.x; i < end; i += PT) c += run_head(keys, i) ? 1u : 0u;
-    uint64_t total;
-    (void)wg_scan_excl<uint64_t>(c, total, s_wave);
-    if (threadIdx.x == 0) counts[blockIdx.x] = total;
-}
-
 // Exclusive scan, in place, of the G per-chunk values (one workgroup);
 // *total receives their sum.
 __global__ __launch_bounds__(PT) void k_spine_u64(uint64_t* v, int G, uint64_t* total) {
@@ -73,25 +66,6 @@ __global__ __launch_bounds__(PT) void k_spine_u64(uint64_t* v, int G, uint64_t* 
         carry += tot;
     }
     if (threadIdx.x == 0) *total = carry;
-}
-
-__global__ __launch_bounds__(PT) void k_trim_scatter(const uint64_t* keys, const uint32_t* vals, int64_t n,
-                                                     int64_t chunk, const uint64_t* offsets, uint64_t* keys_out,
-                                                     uint32_t* vals_out) {
-    __shared__ uint32_t s_wave[PW];
-    const int64_t begin = (int64_t)blockIdx.x * chunk, end = min(n, begin + chunk);
-    uint64_t carry = offsets[blockIdx.x];
-    for (int64_t base = begin; base < end; base += PT) {
-        const int64_t i = base + threadIdx.x;
-        const bool keep = i < end && run_head(keys, i);
-        uint32_t tot;
-        const uint32_t ex = wg_scan_excl<uint32_t>(keep ? 1u : 0u, tot, s_wave);
-        if (keep) {
-            keys_out[carry + ex] = keys[i];
-            if (vals) vals_out[carry + ex] = vals[i];
-        }
-        carry += tot;
-    }
 }
 
 __global__ __launch_bounds__(PT) void k_scan_reduce(const uint32_t* in, int64_t n, int64_t chunk, uint64_t* sums) {
@@ -128,9 +102,6 @@ __global__ __launch_bounds__(PT) void k_scan_down(const uint32_t* in, uint32_t* 
 constexpr int VEC32 = 4;                   // uint32 per uint4
 constexpr int SUB32 = 4;
 constexpr int64_t STEP32 = (int64_t)PT * VEC32 * SUB32;  // 4096 elements
-constexpr int VEC64 = 4;                   // uint64 per two uint4
-constexpr int SUB64 = 2;
-constexpr int64_t STEP64 = (int64_t)PT * VEC64 * SUB64;  // 2048 keys
 
 __device__ __forceinline__ void load4_u32(const uint32_t* p, int64_t i, int64_t end, uint32_t (&x)[4]) {
     if (i + 4 <= end) {
@@ -139,18 +110,6 @@ __device__ __forceinline__ void load4_u32(const uint32_t* p, int64_t i, int64_t 
     } else {
 #pragma unroll
         for (int j = 0; j < 4; ++j) x[j] = (i + j < end) ? p[i + j] : 0u;
-    }
-}
-
-__device__ __forceinline__ void load4_u64(const uint64_t* p, int64_t i, int64_t end, uint64_t (&x)[4]) {
-    if (i + 4 <= end) {
-        const uint4 a = *reinterpret_cast<const uint4*>(p + i);
-        const uint4 b = *reinterpret_cast<const uint4*>(p + i + 2);
-        x[0] = ((uint64_t)a.y << 32) | a.x, x[1] = ((uint64_t)a.w << 32) | a.z;
-        x[2] = ((uint64_t)b.y << 32) | b.x, x[3] = ((uint64_t)b.w << 32) | b.z;
-    } else {
-#pragma unroll
-        for (int j = 0; j < 4; ++j) x[j] = (i + j < end) ? p[i + j] : 0ull;
     }
 }
 
@@ -202,63 +161,254 @@ __global__ __launch_bounds__(PT) void k_scan_down_v(const uint32_t* in, uint32_t
     }
 }
 
-// Run heads of the VEC64 keys at i (the key before i is read separately).
-__device__ __forceinline__ uint32_t heads4(const uint64_t* keys, int64_t i, int64_t end, const uint64_t (&x)[4]) {
-    uint64_t prev = (i > 0 && i < end) ? keys[i - 1] : ~x[0];
-    uint32_t h = 0;
-#pragma unroll
-    for (int j = 0; j < 4; ++j) {
-        if (i + j < end && (i + j == 0 || x[j] != prev)) h |= 1u << j;
-        prev = x[j];
-    }
-    return h;
-}
+// ---- chained single-pass forms ---------------------------------------------
+// One 64-bit word per block: its own sum (CHAIN_SUM), which the serving
+// workgroup replaces by the sum of all blocks before it (CHAIN_PREFIX).  Words
+// are CHAIN_STRIDE apart, one per 64-byte line: stores to one line are
+// serialised (33 ns each), and blocks in order store in order, so packed words
+// limited a scan to one block per 55 ns (2^28 elements in 3.6 ms).
+constexpr unsigned long long CHAIN_SUM = 1ull << 62, CHAIN_PREFIX = 2ull << 62, CHAIN_VALUE = CHAIN_SUM - 1;
+constexpr int CHAIN_STRIDE = 8;
+constexpr uint32_t kChainSpins = 1u << 22;
 
-__global__ __launch_bounds__(PT) void k_trim_count_v(const uint64_t* keys, int64_t n, int64_t chunk,
-                                                     uint64_t* counts) {
-    __shared__ uint64_t s_wave[PW];
-    const int64_t begin = (int64_t)blockIdx.x * chunk, end = min(n, begin + chunk);
-    uint64_t c = 0;
-    for (int64_t base = begin; base < end; base += STEP64) {
-        uint64_t x[SUB64][4];
-#pragma unroll
-        for (int k = 0; k < SUB64; ++k) load4_u64(keys, base + (int64_t)k * PT * VEC64 + threadIdx.x * VEC64, end, x[k]);
-#pragma unroll
-        for (int k = 0; k < SUB64; ++k)
-            c += __popc(heads4(keys, base + (int64_t)k * PT * VEC64 + threadIdx.x * VEC64, end, x[k]));
-    }
+// Report of a chained call.
+struct ChainReport {
     uint64_t total;
-    (void)wg_scan_excl<uint64_t>(c, total, s_wave);
-    if (threadIdx.x == 0) counts[blockIdx.x] = total;
+    uint32_t failed;
+};
+
+__device__ __forceinline__ unsigned long long chain_load(const unsigned long long* chain, int b) {
+    return __hip_atomic_load(&chain[(size_t)b * CHAIN_STRIDE], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+__device__ __forceinline__ void chain_store(unsigned long long* chain, int b, unsigned long long w) {
+    __hip_atomic_store(&chain[(size_t)b * CHAIN_STRIDE], w, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
 
-__global__ __launch_bounds__(PT) void k_trim_scatter_v(const uint64_t* keys, const uint32_t* vals, int64_t n,
-                                                       int64_t chunk, const uint64_t* offsets, uint64_t* keys_out,
-                                                       uint32_t* vals_out) {
-    __shared__ uint32_t s_wave[PW];
-    const int64_t begin = (int64_t)blockIdx.x * chunk, end = min(n, begin + chunk);
-    uint64_t carry = offsets[blockIdx.x];
-    for (int64_t base = begin; base < end; base += STEP64) {
-        uint64_t x[SUB64][4];
+__global__ __launch_bounds__(PT) void k_chain_init(unsigned long long* chain, int blocks) {
+    for (int i = blockIdx.x * PT + threadIdx.x; i < blocks; i += gridDim.x * PT) chain[(size_t)i * CHAIN_STRIDE] = 0;
+}
+
+struct ChainServeShared {
+    uint64_t sum[PW];
+    uint32_t ready[PW];
+};
+
+// Workgroup 0 of a chained kernel: turns the blocks' sums into prefixes, up to
+// PT of them per round trip (0.7 us), and reports the total.  The blocks poll one
+// line each; when every block looked back over its predecessors' words itself,
+// the polling alone took 20 to 45 us of a scan of 2^26 elements.  Workgroups
+// are dispatched in order, so the lowest block without a sum is running or
+// next to run; should that fail, the bounded wait sets failed and the
+// remaining blocks go on with what there is.
+__device__ __forceinline__ void chain_serve(unsigned long long* chain, int blocks, ChainReport* report,
+                                            ChainServeShared& s) {
+    const int tid = threadIdx.x, lane = lane_id(), wid = tid / kWave;
+    uint64_t before = 0;
+    int base = 0;
+    uint32_t spins = 0;
+    while (base < blocks) {
+        const int b = base + tid;
+        const unsigned long long w = b < blocks ? chain_load(chain, b) : 0ull;
+        const uint64_t waiting = __ballot(w < CHAIN_SUM);
+        const int ready = waiting ? __ffsll((unsigned long long)waiting) - 1 : kWave;
+        const uint64_t v = lane < ready ? (w & CHAIN_VALUE) : 0ull;
+        uint64_t incl = v;
 #pragma unroll
-        for (int k = 0; k < SUB64; ++k) load4_u64(keys, base + (int64_t)k * PT * VEC64 + threadIdx.x * VEC64, end, x[k]);
+        for (int d = 1; d < kWave; d <<= 1) {
+            const uint64_t o = __shfl_up(incl, d, kWave);
+            if (lane >= d) incl += o;
+        }
+        if (lane == kWave - 1) {
+            s.sum[wid] = incl;
+            s.ready[wid] = (uint32_t)ready;
+        }
+        __syncthreads();
+        uint64_t mine = before;
+        bool open = true;
+        int taken = 0;
 #pragma unroll
-        for (int k = 0; k < SUB64; ++k) {
-            const int64_t i = base + (int64_t)k * PT * VEC64 + threadIdx.x * VEC64;
-            const uint32_t h = heads4(keys, i, end, x[k]);
-            uint32_t tot;
-            uint64_t pos = carry + wg_scan_excl<uint32_t>((uint32_t)__popc(h), tot, s_wave);
-            uint32_t v[4] = {0u, 0u, 0u, 0u};
-            if (vals && h) load4_u32(vals, i, end, v);
+        for (int k = 0; k < PW; ++k) {
+            if (k == wid && open && lane < ready) chain_store(chain, b, CHAIN_PREFIX | (mine + incl - v));
+            if (open) {
+                mine += s.sum[k];
+                taken += (int)s.ready[k];
+                open = s.ready[k] == kWave;
+            }
+        }
+        __syncthreads();
+        before = mine;
+        base += taken;
+        if (taken == 0 && base < blocks) {
+            if (++spins > kChainSpins) {
+                if (tid == 0) report->failed = 1;
+                for (int i = base + tid; i < blocks; i += PT) chain_store(chain, i, CHAIN_PREFIX | before);
+                return;
+            }
+            __builtin_amdgcn_s_sleep(1);
+        }
+    }
+    if (tid == 0) report->total = before;
+}
+
+// Sum of the blocks before `block`, which publishes `mine`; one lane.
+__device__ __forceinline__ uint64_t chain_before(unsigned long long* chain, int block, uint64_t mine,
+                                                 ChainReport* report) {
+    chain_store(chain, block, CHAIN_SUM | mine);
+    unsigned long long w;
+    uint32_t spins = 0;
+    while ((w = chain_load(chain, block)) < CHAIN_PREFIX) {
+        if (++spins > kChainSpins) {
+            report->failed = 1;
+            return 0;
+        }
+        __builtin_amdgcn_s_sleep(1);
+    }
+    return w & CHAIN_VALUE;
+}
+
+// Prefix sum in one pass, bound by its read and its write: 2^26 elements in 113
+// us (4.75 TB/s, as a large copy), where a reduce, a spine and a scan took 176.
+// A workgroup holds SCAN_SUB sub-tiles of 1,024 elements (a thread four
+// consecutive ones of each), so every load and store of a wave covers 1 KiB;
+// 4, 12 or 16 sub-tiles measured 114, 117 and 144 us.  Each sub-tile is scanned
+// per wave, and one wave scans the waves' totals while another waits for the
+// blocks before.  Nothing here reads the output again, so its stores bypass the
+// caches (with ordinary stores the reads lose 25 us).  `out` may equal `in`: a
+// block is in registers before its first store, and blocks are disjoint.
+constexpr int64_t kChainScanMax = 1ll << 30;  // sums of 32-bit values stay below 2^62
+constexpr int SCAN_SUB = 8;
+constexpr int64_t SCAN_BLOCK = (int64_t)PT * VEC32 * SCAN_SUB;
+
+__global__ __launch_bounds__(PT) void k_scan_chained(const uint32_t* in, uint32_t* out, int64_t n, int inclusive,
+                                                     unsigned long long* chain, ChainReport* report) {
+    static_assert(SCAN_SUB * PW <= kWave, "one wave scans the waves' totals");
+    __shared__ uint32_t s_tot[SCAN_SUB * PW];
+    __shared__ uint64_t s_sum[PW];
+    __shared__ uint32_t s_before;
+    __shared__ ChainServeShared s_serve;
+    if (blockIdx.x == 0) {
+        chain_serve(chain, gridDim.x - 1, report, s_serve);
+        return;
+    }
+    const int block = blockIdx.x - 1;
+    const int64_t begin = (int64_t)block * SCAN_BLOCK;
+    const int tid = threadIdx.x, lane = lane_id(), wid = tid / kWave;
+    uint32_t x[SCAN_SUB][4];
+#pragma unroll
+    for (int k = 0; k < SCAN_SUB; ++k) load4_u32(in, begin + (int64_t)k * PT * VEC32 + tid * VEC32, n, x[k]);
+    uint64_t sum = 0;
+    uint32_t ex[SCAN_SUB];
+#pragma unroll
+    for (int k = 0; k < SCAN_SUB; ++k) {
+        sum += (uint64_t)x[k][0] + x[k][1] + x[k][2] + x[k][3];
+        const uint32_t run = x[k][0] + x[k][1] + x[k][2] + x[k][3];
+        const uint32_t incl = wave_scan_incl(run);
+        ex[k] = incl - run;
+        if (lane == kWave - 1) s_tot[k * PW + wid] = incl;
+    }
+#pragma unroll
+    for (int d = kWave / 2; d >= 1; d >>= 1) sum += __shfl_xor(sum, d, kWave);
+    if (lane == 0) s_sum[wid] = sum;
+    __syncthreads();
+    if (wid == 0) {
+        uint64_t mine = 0;
+#pragma unroll
+        for (int w = 0; w < PW; ++w) mine += s_sum[w];
+        if (lane == 0) s_before = (uint32_t)chain_before(chain, block, mine, report);
+    } else if (wid == 1) {
+        const uint32_t t = lane < SCAN_SUB * PW ? s_tot[lane] : 0u;
+        const uint32_t incl = wave_scan_incl(t);
+        if (lane < SCAN_SUB * PW) s_tot[lane] = incl - t;
+    }
+    __syncthreads();
+    const uint32_t before = s_before;
+#pragma unroll
+    for (int k = 0; k < SCAN_SUB; ++k) {
+        const int64_t i = begin + (int64_t)k * PT * VEC32 + tid * VEC32;
+        uint32_t run = before + s_tot[k * PW + wid] + ex[k];
+        uint32_t y[4];
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+            y[j] = run + (inclusive ? x[k][j] : 0u);
+            run += x[k][j];
+        }
+        if (i + 4 <= n) {
+            typedef uint32_t vec4 __attribute__((ext_vector_type(4)));
+            __builtin_nontemporal_store(vec4{y[0], y[1], y[2], y[3]}, reinterpret_cast<vec4*>(out + i));
+        } else {
 #pragma unroll
             for (int j = 0; j < 4; ++j)
-                if ((h >> j) & 1u) {
-                    keys_out[pos] = x[k][j];
-                    if (vals) vals_out[pos] = v[j];
-                    ++pos;
-                }
-            carry += tot;
+                if (i + j < n) out[i + j] = y[j];
         }
+    }
+}
+
+// Run heads in one pass, bound by its reads and writes: 2^25 pairs, half of them
+// kept, in 118 us (4.9 TB/s), where a count, a spine and a scatter took 235.  A
+// wave holds TRIM_ITEMS rows of 64 consecutive keys (and values), so that every
+// load, and every store of a row's kept entries, covers consecutive entries;
+// four consecutive keys per thread scattered the stores (161 us).  8 or 32 rows
+// measured 141 and 129 us.
+constexpr int TRIM_ITEMS = 16;
+constexpr int64_t TRIM_BLOCK = (int64_t)PT * TRIM_ITEMS;
+
+template <bool VALS>
+__global__ __launch_bounds__(PT) void k_trim_chained(const uint64_t* keys, const uint32_t* vals, int64_t n,
+                                                     uint64_t* keys_out, uint32_t* vals_out,
+                                                     unsigned long long* chain, ChainReport* report) {
+    __shared__ uint32_t s_tot[PW];
+    __shared__ uint64_t s_before;
+    __shared__ ChainServeShared s_serve;
+    if (blockIdx.x == 0) {
+        chain_serve(chain, gridDim.x - 1, report, s_serve);
+        return;
+    }
+    const int block = blockIdx.x - 1;
+    const int lane = lane_id(), wid = threadIdx.x / kWave;
+    const int64_t begin = (int64_t)block * TRIM_BLOCK + (int64_t)wid * kWave * TRIM_ITEMS;
+    uint64_t x[TRIM_ITEMS];
+    uint32_t v[TRIM_ITEMS];
+    uint64_t last = 0;  // the key before the row; lane 0
+    if (lane == 0 && begin > 0 && begin < n) last = keys[begin - 1];
+#pragma unroll
+    for (int k = 0; k < TRIM_ITEMS; ++k) {
+        const int64_t i = begin + k * kWave + lane;
+        x[k] = i < n ? keys[i] : 0ull;
+        if (VALS) v[k] = i < n ? vals[i] : 0u;
+    }
+    uint64_t heads[TRIM_ITEMS];
+    uint32_t count = 0;
+#pragma unroll
+    for (int k = 0; k < TRIM_ITEMS; ++k) {
+        const int64_t i = begin + k * kWave + lane;
+        const uint64_t left = __shfl_up(x[k], 1, kWave);
+        const uint64_t prev = lane == 0 ? last : left;
+        heads[k] = __ballot(i < n && (i == 0 || x[k] != prev));
+        count += (uint32_t)__popcll(heads[k]);
+        last = __shfl(x[k], kWave - 1, kWave);
+    }
+    if (lane == 0) s_tot[wid] = count;
+    __syncthreads();
+    if (threadIdx.x == 0) {
+        uint64_t mine = 0;
+#pragma unroll
+        for (int w = 0; w < PW; ++w) {
+            const uint32_t t = s_tot[w];
+            s_tot[w] = (uint32_t)mine;
+            mine += t;
+        }
+        s_before = chain_before(chain, block, mine, report);
+    }
+    __syncthreads();
+    uint64_t pos = s_before + s_tot[wid];
+#pragma unroll
+    for (int k = 0; k < TRIM_ITEMS; ++k) {
+        if ((heads[k] >> lane) & 1u) {
+            const uint64_t at = pos + __popcll(heads[k] & ((1ull << lane) - 1));
+            keys_out[at] = x[k];
+            if (VALS) vals_out[at] = v[k];
+        }
+        pos += (uint64_t)__popcll(heads[k]);
     }
 }
 
@@ -274,6 +424,40 @@ void chunking(int64_t n, int64_t step, int64_t& chunk, int& G) {
     G = (int)((n + chunk - 1) / chunk);
     if (G < 1) G = 1;
 }
+
+// Chained calls: chain words, then a report for when there is no pinned slot.
+size_t chain_bytes(int64_t blocks) { return (size_t)blocks * CHAIN_STRIDE * 8 + sizeof(ChainReport); }
+
+// One chained call's scratch and report.
+struct ChainCall {
+    ReportSlot slot;
+    DeviceBuffer mem;  // freed before the slot is given back
+    unsigned long long* chain = nullptr;
+    ChainReport* report = nullptr;
+    b40c_status start(int64_t blocks, hipStream_t stream) {
+        B40C_TRY(mem.alloc(chain_bytes(blocks)));
+        chain = mem.as<unsigned long long>();
+        report = reinterpret_cast<ChainReport*>(chain + (size_t)blocks * CHAIN_STRIDE);
+        if (slot.take())
+            report = static_cast<ChainReport*>(slot.dev);
+        else
+            B40C_TRY(fill_u32(reinterpret_cast<uint32_t*>(report), 0, sizeof(ChainReport) / 4, stream));
+        hipLaunchKernelGGL(k_chain_init, dim3((unsigned)std::min<int64_t>((blocks + PT - 1) / PT, 256)), dim3(PT), 0,
+                           stream, chain, (int)blocks);
+        return B40C_OK;
+    }
+    b40c_status finish(const char* who, uint64_t& total, hipStream_t stream) {
+        B40C_HIP(hipGetLastError());
+        ChainReport h;
+        if (!slot.host) B40C_HIP(hipMemcpyAsync(&h, report, sizeof(h), hipMemcpyDeviceToHost, stream));
+        B40C_HIP(hipStreamSynchronize(stream));
+        if (slot.host) std::memcpy(&h, slot.host, sizeof(h));
+        if (h.failed) return fail(B40C_ERR_HIP, "%s: a block waited too long for the blocks before it", who);
+        total = h.total;
+        return B40C_OK;
+    }
+};
+static_assert(sizeof(ChainReport) <= ReportSlot::kBytes, "a report fits its slot");
 
 }  // namespace
 
@@ -321,28 +505,19 @@ b40c_status b40c_consecutive_removal_u64(const uint64_t* d_keys_in, const uint32
         return fail(B40C_ERR_INVALID_ARG, "b40c_consecutive_removal_u64: output must not alias input");
     *num_compacted = 0;
     if (n == 0) return B40C_OK;
-    const bool vec = aligned16(d_keys_in) && (!d_values_in || aligned16(d_values_in));
-    int64_t chunk;
-    int G;
-    chunking(n, vec ? STEP64 : PT, chunk, G);
-    DeviceBuffer counts, total;
-    B40C_TRY(counts.alloc((size_t)G * 8));
-    B40C_TRY(total.alloc(8));
-    if (vec)
-        hipLaunchKernelGGL(k_trim_count_v, dim3(G), dim3(PT), 0, nullptr, d_keys_in, n, chunk, counts.as<uint64_t>());
+    const int64_t blocks = (n + TRIM_BLOCK - 1) / TRIM_BLOCK;
+    if (blocks >= INT32_MAX) return fail(B40C_ERR_INVALID_ARG, "b40c_consecutive_removal_u64: n out of range");
+    ChainCall call;
+    B40C_TRY(call.start(blocks, nullptr));
+    if (d_values_in)
+        hipLaunchKernelGGL(k_trim_chained<true>, dim3((unsigned)blocks + 1), dim3(PT), 0, nullptr, d_keys_in,
+                           d_values_in, n, d_keys_out, d_values_out, call.chain, call.report);
     else
-        hipLaunchKernelGGL(k_trim_count, dim3(G), dim3(PT), 0, nullptr, d_keys_in, n, chunk, counts.as<uint64_t>());
-    hipLaunchKernelGGL(k_spine_u64, dim3(1), dim3(PT), 0, nullptr, counts.as<uint64_t>(), G, total.as<uint64_t>());
-    if (vec)
-        hipLaunchKernelGGL(k_trim_scatter_v, dim3(G), dim3(PT), 0, nullptr, d_keys_in, d_values_in, n, chunk,
-                           counts.as<uint64_t>(), d_keys_out, d_values_out);
-    else
-        hipLaunchKernelGGL(k_trim_scatter, dim3(G), dim3(PT), 0, nullptr, d_keys_in, d_values_in, n, chunk,
-                           counts.as<uint64_t>(), d_keys_out, d_values_out);
-    B40C_HIP(hipGetLastError());
-    uint64_t h = 0;
-    B40C_HIP(hipMemcpy(&h, total.ptr, 8, hipMemcpyDeviceToHost));
-    *num_compacted = (int64_t)h;
+        hipLaunchKernelGGL(k_trim_chained<false>, dim3((unsigned)blocks + 1), dim3(PT), 0, nullptr, d_keys_in,
+                           d_values_in, n, d_keys_out, d_values_out, call.chain, call.report);
+    uint64_t total = 0;
+    B40C_TRY(call.finish("b40c_consecutive_removal_u64", total, nullptr));
+    *num_compacted = (int64_t)total;
     return B40C_OK;
 }
 
@@ -352,6 +527,17 @@ b40c_status b40c_scan_u32(const uint32_t* d_in, uint32_t* d_out, int64_t n, int3
         return fail(B40C_ERR_INVALID_ARG, "b40c_scan_u32: bad arguments");
     if (total) *total = 0;
     if (n == 0) return B40C_OK;
+    if (aligned16(d_in) && aligned16(d_out) && n <= kChainScanMax) {
+        const int64_t blocks = (n + SCAN_BLOCK - 1) / SCAN_BLOCK;
+        ChainCall call;
+        B40C_TRY(call.start(blocks, nullptr));
+        hipLaunchKernelGGL(k_scan_chained, dim3((unsigned)blocks + 1), dim3(PT), 0, nullptr, d_in, d_out, n,
+                           exclusive ? 0 : 1, call.chain, call.report);
+        uint64_t sum = 0;
+        B40C_TRY(call.finish("b40c_scan_u32", sum, nullptr));
+        if (total) *total = sum;
+        return B40C_OK;
+    }
     DeviceBuffer sums, tot;
     B40C_TRY(sums.alloc((size_t)scan_u32_max_partials() * 8));
     B40C_TRY(tot.alloc(8));

@@ -39,6 +39,7 @@
 //    or a fixed device array for the allocation-free entry point; the block
 //    size grows until the look-back words fit it.  Launching a sort allocates
 //    nothing and does not synchronize; only waiting for the selector does.
+#include <cstring>
 #include <mutex>
 
 #include "common.hpp"
@@ -640,70 +641,19 @@ size_t sort_scratch_words(int64_t n, int num_cus, const SortPolicy& pol) {
     return kStateWords + look_words(sort_plan(n, num_cus, pol));
 }
 
-// Pinned host words that sorts report through (selector, failure): one page
-// per process, a slot per sort in flight, so no copy follows a sort.  Held
-// until the process ends.  A sort beyond the slots reads its report back with
-// a copy instead.
 namespace {
-class SortReports {
-  public:
-    static constexpr int kSlots = 64;
-    // Null when the page could not be had or every slot is taken.
-    int32_t* take() {
-        std::lock_guard<std::mutex> lock(mu_);
-        if (!tried_) {
-            tried_ = true;
-            if (hipHostMalloc((void**)&page_, kSlots * kStride * sizeof(int32_t),
-                              hipHostMallocCoherent | hipHostMallocPortable | hipHostMallocMapped) != hipSuccess) {
-                page_ = nullptr;
-                (void)hipGetLastError();
-            }
-        }
-        if (!page_) return nullptr;
-        for (int i = 0; i < kSlots; ++i)
-            if (!used_[i]) {
-                used_[i] = true;
-                return page_ + i * kStride;
-            }
-        return nullptr;
-    }
-    void give(int32_t* slot) {
-        std::lock_guard<std::mutex> lock(mu_);
-        used_[(slot - page_) / kStride] = false;
-    }
-
-  private:
-    static constexpr int kStride = 16;
-    std::mutex mu_;
-    bool tried_ = false;
-    int32_t* page_ = nullptr;
-    bool used_[kSlots] = {};
-};
-SortReports g_reports;
-
-// One sort's report words: a pinned slot, or, without one, the first words of
-// the scratch, copied back after the sort.
+// One sort's report words (selector, failure): a pinned slot, or, without one,
+// the first words of the scratch, copied back after the sort.
 struct SortReport {
-    int32_t* slot = nullptr;
+    ReportSlot slot;
     int32_t* dev = nullptr;
-    ~SortReport() {
-        if (slot) g_reports.give(slot);
-    }
-    b40c_status take(const SortScratch& sc, bool pinned) {
-        if (pinned) slot = g_reports.take();
-        if (slot)
-            B40C_HIP(hipHostGetDevicePointer((void**)&dev, slot, 0));
-        else
-            dev = reinterpret_cast<int32_t*>(sc.base);
-        return B40C_OK;
+    void take(const SortScratch& sc, bool pinned) {
+        dev = static_cast<int32_t*>(pinned && slot.take() ? slot.dev : sc.base);
     }
     b40c_status wait(int32_t (&words)[2], hipStream_t stream) {
-        if (!slot) B40C_HIP(hipMemcpyAsync(words, dev, sizeof(words), hipMemcpyDeviceToHost, stream));
+        if (!slot.host) B40C_HIP(hipMemcpyAsync(words, dev, sizeof(words), hipMemcpyDeviceToHost, stream));
         B40C_HIP(hipStreamSynchronize(stream));
-        if (slot) {
-            words[0] = slot[0];
-            words[1] = slot[1];
-        }
+        if (slot.host) std::memcpy(words, slot.host, sizeof(words));
         return B40C_OK;
     }
 };
@@ -734,7 +684,7 @@ static b40c_status radix_sort_sync(int32_t key_type, void* k0, void* k1, uint32_
                                    int begin_bit, int end_bit, int num_cus, const SortPolicy& pol,
                                    const SortScratch& sc, int32_t* selector, hipStream_t stream, bool pinned = true) {
     SortReport report;
-    B40C_TRY(report.take(sc, pinned));
+    report.take(sc, pinned);
     B40C_TRY(radix_sort_launch(key_type, k0, k1, v0, v1, n, begin_bit, end_bit, num_cus, pol, sc, report.dev, stream));
     int32_t words[2] = {0, 0};
     B40C_TRY(report.wait(words, stream));

@@ -47,6 +47,46 @@ b40c_status device_info(DeviceInfo& info) {
 }
 
 namespace {
+constexpr int kReportSlots = 64;
+std::mutex g_report_mu;
+bool g_report_tried = false;
+char* g_report_page = nullptr;
+bool g_report_used[kReportSlots] = {};
+}  // namespace
+
+bool ReportSlot::take() {
+    std::lock_guard<std::mutex> lock(g_report_mu);
+    if (!g_report_tried) {
+        g_report_tried = true;
+        if (hipHostMalloc((void**)&g_report_page, kReportSlots * kBytes,
+                          hipHostMallocCoherent | hipHostMallocPortable | hipHostMallocMapped) != hipSuccess) {
+            g_report_page = nullptr;
+            (void)hipGetLastError();
+        }
+    }
+    if (!g_report_page) return false;
+    for (int i = 0; i < kReportSlots; ++i) {
+        if (g_report_used[i]) continue;
+        char* slot = g_report_page + i * kBytes;
+        if (hipHostGetDevicePointer(&dev, slot, 0) != hipSuccess) {
+            (void)hipGetLastError();
+            return false;
+        }
+        g_report_used[i] = true;
+        host = slot;
+        std::memset(host, 0, kBytes);
+        return true;
+    }
+    return false;
+}
+
+ReportSlot::~ReportSlot() {
+    if (!host) return;
+    std::lock_guard<std::mutex> lock(g_report_mu);
+    g_report_used[((char*)host - g_report_page) / kBytes] = false;
+}
+
+namespace {
 __global__ void k_fill_u32(uint32_t* p, uint32_t v, size_t n) {
     for (size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += (size_t)gridDim.x * blockDim.x) p[i] = v;
 }
