@@ -66,10 +66,11 @@ struct SortPolicy {
     int items = 0;
     int wgs_per_cu = 0;
 };
-// Policy with its zero fields filled in for n keys of key_bytes bytes.
-SortPolicy resolve_sort_policy(SortPolicy p, int64_t n, int key_bytes);
-// Words of scratch a sort of n keys wants on a device with num_cus CUs.
-size_t sort_scratch_words(int64_t n, int num_cus, const SortPolicy& p);
+// Policy with its zero fields filled in for n keys (with their values
+// pair_bytes bytes each).
+SortPolicy resolve_sort_policy(SortPolicy p, int64_t n, int pair_bytes, int num_cus);
+// Words of scratch a sort of n keys wants.
+size_t sort_scratch_words(int64_t n);
 b40c_status radix_sort_u64(uint64_t* k0, uint64_t* k1, int64_t n, int begin_bit, int end_bit, int32_t* selector,
                            hipStream_t stream);
 b40c_status radix_sort_pairs_u32(uint32_t* k0, uint32_t* k1, uint32_t* v0, uint32_t* v1, int64_t n, int begin_bit,

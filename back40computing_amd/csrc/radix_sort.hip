@@ -8,15 +8,15 @@
 //    passes, and 160 KB of LDS per CU easily holds the per-wave histograms.
 //  * The digit totals of every place do not change while keys are permuted, so
 //    one kernel (k_histogram) counts them all in one read of the keys.
-//  * A place is then one kernel (k_place).  A workgroup owns a block of
-//    consecutive keys: it counts the block's digits, publishes the counts,
-//    finds the counts of all blocks before it by looking back over their
-//    published words (chained scan with decoupled look-back, Merrill and
-//    Garland 2016), and scatters.  Counting and scattering read the block
-//    twice within microseconds, so the second read comes from the caches: HBM
-//    moves each key once in and once out per place.  The three-kernel form
-//    this replaces read the keys twice from HBM.  Blocks, not tiles, look
-//    back: the words read for that shrink with the block size.
+//  * A place is then one kernel (k_place).  A workgroup owns a tile of
+//    consecutive keys: it ranks them, publishes its digit counts, learns where
+//    its digits start in the output, and scatters, so HBM moves each key once in
+//    and once out per place.  Sixteen more workgroups chain the tiles: they turn
+//    the published counts into starts, each for 16 digits.  Workgroups that
+//    look back over their predecessors' words by themselves (Merrill and Garland
+//    2016) poll 256 words of each and spend more on that than on the keys (2^26
+//    64-bit keys: 4.4 ms a sort; with blocks of four tiles, which read their keys
+//    twice, 3.5 ms; served, 2.75 ms).
 //  * Stable local ranking uses wave64 "match" masks built from 8 ballots (one
 //    per digit bit) and per-wave running digit counters in LDS; keys are
 //    processed in (wave, round, lane) order which equals index order inside a
@@ -37,7 +37,7 @@
 //  * Scratch comes from the caller as one array of words: a per-call
 //    allocation for the stateless entry points, the sort enactor's own buffer,
 //    or a fixed device array for the allocation-free entry point; the block
-//    size grows until the look-back words fit it.  Launching a sort allocates
+//    size grows until the chain words fit it.  Launching a sort allocates
 //    nothing and does not synchronize; only waiting for the selector does.
 #include <cstring>
 #include <mutex>
@@ -50,10 +50,8 @@ namespace {
 
 constexpr int RS_BINS = 256;
 constexpr int RS_MAX_WGS_PER_CU = 8;
-// Tiles per block of a large sort: more make fewer blocks look back, but the
-// second read of a block then misses the caches more (2^26 64-bit keys, 1 / 2 /
-// 3 / 4 / 8 / 16 tiles: 4.4 / 3.55 / 3.53 / 3.53 / 3.8 / 4.1 ms).
-constexpr int kBlockTiles = 4;
+// Most blocks of a place: 64 MB of chain words (128 MB from 2^30 keys on).
+constexpr int64_t kMaxBlocks = 1 << 15;
 
 // Order-preserving views of the key bits (sort_utils.cuh:87-183):
 // CONV 0 unsigned (as is), 1 signed (flip the sign bit), 2 IEEE float
@@ -121,16 +119,16 @@ struct SortState {
     uint32_t* copies;   // [HIST_COPIES][MAX_PLACES][RS_BINS] digit totals, spread over copies
     uint32_t* base;     // [MAX_PLACES][RS_BINS] first output position of each digit
     uint32_t* trivial;  // [MAX_PLACES] place whose keys all share one digit
-    uint32_t* status;   // [2][blocks][RS_BINS] look-back words (by place parity), 32 or 64 bits each
+    uint32_t* status;   // [2][blocks][RS_BINS] chain words (by place parity), 32 or 64 bits each
     int32_t* out;       // report: selector, failure
     int32_t blocks;
-    int32_t wide;       // 64-bit look-back words (n >= 2^30)
+    int32_t wide;       // 64-bit chain words (n >= 2^30)
     int32_t places;
 };
 constexpr size_t kReportWords = 16;  // the report, where it is in the scratch (first words)
 constexpr size_t kStateWords = kReportWords + (size_t)(HIST_COPIES + 1) * MAX_PLACES * RS_BINS + 64;
 
-// Clears the totals and the first place's look-back words.
+// Clears the totals and the first place's chain words.
 __global__ __launch_bounds__(256) void k_sort_init(SortState st) {
     const int64_t step = (int64_t)gridDim.x * 256;
     const int64_t i0 = (int64_t)blockIdx.x * 256 + threadIdx.x;
@@ -210,63 +208,157 @@ __global__ __launch_bounds__(RS_BINS) void k_plan(SortState st, int64_t n) {
     if (d == 0) st.trivial[p] = triv ? 1u : 0u;
 }
 
-// Look-back over the published words of the blocks before `block` for digit d:
-// the sum of their counts.  LOOK words are loaded together per round: a round
-// trip past the caches is about 0.7 us and a word is often found only tens of
-// blocks back.  Blocks are dispatched in order, so every block waited for is
-// running; should that fail, the bounded wait ends the sort with an error.
-constexpr uint32_t kLookSpins = 1u << 22;
+// Chain of the blocks of a place: one word per block and digit, the block's
+// count first (COUNT), then the digit's next output position where the block
+// starts (START), which a serving workgroup puts in its place.
+constexpr uint32_t kChainSpins = 1u << 22;
 template <typename W>
-struct LookWord {
-    static constexpr W COUNT = (W)1 << (8 * sizeof(W) - 2);  // the block's own count
-    static constexpr W PREFIX = (W)2 << (8 * sizeof(W) - 2); // count of this and all blocks before
+struct ChainWord {
+    static constexpr W COUNT = (W)1 << (8 * sizeof(W) - 2);
+    static constexpr W START = (W)2 << (8 * sizeof(W) - 2);
     static constexpr W VALUE = COUNT - 1;
 };
 template <typename W>
-__device__ __forceinline__ void publish(W* status, int block, int d, uint32_t value, W flag) {
-    __hip_atomic_store(&status[(size_t)block * RS_BINS + d], flag | (W)value, __ATOMIC_RELAXED,
-                       __HIP_MEMORY_SCOPE_AGENT);
+__device__ __forceinline__ W chain_load(const W* status, int block, int d) {
+    return __hip_atomic_load(&status[(size_t)block * RS_BINS + d], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
-template <typename W, int LOOK>
-__device__ __forceinline__ uint32_t look_back(const W* status, int block, int d, int32_t* failed) {
-    uint32_t sum = 0, spins = 0;
-    int j = block - 1;
-    while (true) {
-        W w[LOOK];
-        // Word of block j - k, or, before the first block, of block 0, whose
-        // word is a prefix and ends the walk (j >= 0 here).
+template <typename W>
+__device__ __forceinline__ void chain_store(W* status, int block, int d, W w) {
+    __hip_atomic_store(&status[(size_t)block * RS_BINS + d], w, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+
+// Workgroups 0 .. SERVERS - 1 of a place each serve SERVE_DIGITS digits: they turn
+// the blocks' counts into starts, a window of OS_WAVES * SERVE_SUBS * ROW blocks
+// per round trip past the caches (0.7 us).  A thread has ROW consecutive blocks of
+// one digit.  Workgroups are dispatched in order, so the servers run, and the
+// lowest block without counts is running or next to run; should that fail, the
+// bounded wait sets *failed and the remaining blocks go on with the starts there
+// are (which lie in the output).
+constexpr int SERVE_DIGITS = 16;  // one 64-byte line of 32-bit words
+constexpr int SERVERS = RS_BINS / SERVE_DIGITS;
+constexpr int SERVE_SUBS = kWave / SERVE_DIGITS;
+// Blocks per thread.  Of few blocks most publish their counts at the same time
+// and a wide window takes them in one step (1.3 M 64-bit keys, 318 blocks, 44
+// bits: 132 us with 8, 146 with 4); many come a few at a time and a short step
+// answers sooner (2^26 keys: 2.92 and 2.75 ms; 4 M 12-byte pairs, 977 blocks:
+// 336 and 314 us).
+constexpr int SERVE_FEW_BLOCKS = 512;
+constexpr int SERVE_ROW_FEW = 8;
+constexpr int SERVE_ROW_MANY = 4;
+
+struct ServeShared {
+    unsigned long long sum[OS_WAVES][SERVE_DIGITS];
+    int lead[OS_WAVES];
+};
+
+template <typename W, int ROW>
+__device__ __forceinline__ void serve_place(W* status, int blocks, const uint32_t* base, int32_t* failed,
+                                            ServeShared& s) {
+    constexpr int WAVE_BLOCKS = SERVE_SUBS * ROW;
+    const int tid = threadIdx.x, lane = lane_id(), wid = tid / kWave;
+    const int col = lane % SERVE_DIGITS, sub = lane / SERVE_DIGITS;
+    const int d = (int)blockIdx.x * SERVE_DIGITS + col;
+    W start = (W)base[d];
+    uint32_t spins = 0;
+    for (int first = 0; first < blocks;) {
+        const int mine = first + wid * WAVE_BLOCKS + sub * ROW;
+        W w[ROW];
 #pragma unroll
-        for (int k = 0; k < LOOK; ++k)
-            w[k] = __hip_atomic_load(&status[(uint32_t)(max(j - k, 0) * RS_BINS + d)], __ATOMIC_RELAXED,
-                                     __HIP_MEMORY_SCOPE_AGENT);
-        int used = 0;
-        bool ready = true, done = false;
+        for (int r = 0; r < ROW; ++r) w[r] = chain_load(status, min(mine + r, blocks - 1), d);
+        int lead = 0;  // leading blocks of the row whose counts are there, for all the digits
 #pragma unroll
-        for (int k = 0; k < LOOK; ++k) {
-            ready = ready && !done && w[k] >= LookWord<W>::COUNT;
-            if (ready) {
-                sum += (uint32_t)(w[k] & LookWord<W>::VALUE);
-                ++used;
-                done = w[k] >= LookWord<W>::PREFIX;
-            }
+        for (int r = 0; r < ROW; ++r)
+            if (lead == r && mine + r < blocks && w[r] >= ChainWord<W>::COUNT) ++lead;
+#pragma unroll
+        for (int m = 1; m < SERVE_DIGITS; m <<= 1) lead = min(lead, __shfl_xor(lead, m, kWave));
+        int wave_lead = 0;
+        bool open = true;
+#pragma unroll
+        for (int k = 0; k < SERVE_SUBS; ++k) {
+            const int l = __shfl(lead, k * SERVE_DIGITS, kWave);
+            if (k == sub && !open) lead = 0;
+            if (open) wave_lead += l;
+            open = open && l == ROW;
         }
-        if (done) return sum;
-        j -= used;
-        if (used == 0) {
-            if (++spins > kLookSpins) {
-                *failed = 1;
-                return sum;
+        W row = 0, excl[ROW];
+#pragma unroll
+        for (int r = 0; r < ROW; ++r) {
+            excl[r] = row;
+            if (r < lead) row += w[r] & ChainWord<W>::VALUE;
+        }
+        W incl = row;
+#pragma unroll
+        for (int m = SERVE_DIGITS; m < kWave; m <<= 1) {
+            const W o = __shfl_up(incl, m, kWave);
+            if (lane >= m) incl += o;
+        }
+        if (sub == SERVE_SUBS - 1) s.sum[wid][col] = incl;
+        if (lane == 0) s.lead[wid] = wave_lead;
+        __syncthreads();
+        int taken = 0;
+        open = true;
+        W next = start;
+#pragma unroll
+        for (int k = 0; k < OS_WAVES; ++k) {
+            if (k == wid && open) {
+                const W at = next + incl - row;
+#pragma unroll
+                for (int r = 0; r < ROW; ++r)
+                    if (r < lead) chain_store(status, mine + r, d, (W)(ChainWord<W>::START | (at + excl[r])));
+            }
+            if (open) {
+                taken += s.lead[k];
+                next += (W)s.sum[k][col];
+            }
+            open = open && s.lead[k] == WAVE_BLOCKS;
+        }
+        __syncthreads();
+        start = next;
+        first += taken;
+        if (taken == 0) {
+            if (++spins > kChainSpins) {
+                if (tid == 0) *failed = 1;
+                for (int b = first + tid / SERVE_DIGITS; b < blocks; b += OS_THREADS / SERVE_DIGITS)
+                    chain_store(status, b, (int)blockIdx.x * SERVE_DIGITS + tid % SERVE_DIGITS,
+                                (W)(ChainWord<W>::START | start));
+                return;
             }
             __builtin_amdgcn_s_sleep(1);
         }
     }
 }
 
+// Where digit d of a block goes: waits for its server.
+template <typename W>
+__device__ __forceinline__ uint32_t await_start(const W* status, int block, int d, int32_t* failed) {
+    W w;
+    uint32_t spins = 0;
+    while ((w = chain_load(status, block, d)) < ChainWord<W>::START) {
+        if (++spins > kChainSpins) {
+            *failed = 1;
+            return 0;
+        }
+        __builtin_amdgcn_s_sleep(2);
+    }
+    return (uint32_t)(w & ChainWord<W>::VALUE);
+}
+
+// Block of the i-th working workgroup.  Workgroups go to the XCDs in turn; of
+// every XCD_RUN * 8 blocks each XCD takes XCD_RUN consecutive ones, whose runs
+// of a digit meet in the middle of a line: its L2 then writes the line once.
+constexpr int XCDS = 8;
+constexpr int XCD_RUN = 8;
+__device__ __forceinline__ int place_block(int i, int blocks) {
+    constexpr int GROUP = XCDS * XCD_RUN;
+    if (i < 0 || i / GROUP * GROUP + GROUP > blocks) return i;
+    return i / GROUP * GROUP + i % XCDS * XCD_RUN + i % GROUP / XCDS;
+}
+
 // One digit place.  ITEMS keys per thread: a tile of OS_THREADS * ITEMS keys
-// is ranked and staged in LDS at once.  Bound by what passes the caches: 2^26
-// 64-bit keys take 412 us, 1.09 GB read (each key twice) and 0.69 GB written
-// (0.54 GB of keys, partial lines), 4.3 TB/s; the counting and scattering
-// kernels this replaces took 590 us.
+// is ranked and staged in LDS at once.  Bound by memory and by waiting for the
+// starts: 2^26 64-bit keys take 320 us (1.07 GB of keys in and out, 3.4 TB/s; 295
+// us with the wait left out), where counting and scattering kernels took 590.
+// The order of the XCDs (place_block) gives 20 to 30 us of that.
 template <typename K, int CONV, bool VALS, int ITEMS>
 __global__ __launch_bounds__(OS_THREADS) void k_place(K* k0, K* k1, uint32_t* v0, uint32_t* v1, int64_t n, int place,
                                                       int shift, uint32_t mask, int64_t block_keys, SortState st) {
@@ -278,21 +370,34 @@ __global__ __launch_bounds__(OS_THREADS) void k_place(K* k0, K* k1, uint32_t* v0
     __shared__ uint32_t out_shift[RS_BINS];  // output position minus tile position
     __shared__ uint32_t tile_excl[RS_BINS];
     __shared__ int s_wave[OS_WAVES];
+    __shared__ ServeShared s_serve;
 
     const int tid = threadIdx.x, lane = lane_id(), wid = __builtin_amdgcn_readfirstlane(tid / kWave);
-    const int block = blockIdx.x;
+    const int block = place_block((int)blockIdx.x - SERVERS, st.blocks);
     const size_t words = (size_t)st.blocks * RS_BINS * (st.wide ? 2 : 1);
     // The other parity's words of this block, for the next place (its last
     // user, the place before this one, has finished).
     uint32_t* status = st.status + (place & 1) * words;
     uint32_t* next_status = st.status + ((place + 1) & 1) * words;
-    for (int i = tid; i < RS_BINS * (st.wide ? 2 : 1); i += OS_THREADS)
-        next_status[(size_t)block * RS_BINS * (st.wide ? 2 : 1) + i] = 0;
+    if (block >= 0)
+        for (int i = tid; i < RS_BINS * (st.wide ? 2 : 1); i += OS_THREADS)
+            next_status[(size_t)block * RS_BINS * (st.wide ? 2 : 1) + i] = 0;
     int moved = 0;  // places before this one that moved the keys
     for (int p = 0; p < place; ++p) moved += st.trivial[p] ? 0 : 1;
     const bool skip = st.trivial[place] != 0;
     if (place == st.places - 1 && block == 0 && tid == 0) st.out[0] = (moved + (skip ? 0 : 1)) & 1;
     if (skip) return;
+    if (block < 0) {
+        const uint32_t* base = st.base + place * RS_BINS;
+        if (st.wide)
+            serve_place<unsigned long long, SERVE_ROW_MANY>((unsigned long long*)status, st.blocks, base, &st.out[1],
+                                                            s_serve);
+        else if (st.blocks <= SERVE_FEW_BLOCKS)
+            serve_place<uint32_t, SERVE_ROW_FEW>(status, st.blocks, base, &st.out[1], s_serve);
+        else
+            serve_place<uint32_t, SERVE_ROW_MANY>(status, st.blocks, base, &st.out[1], s_serve);
+        return;
+    }
     const K* kin = (moved & 1) ? k1 : k0;
     K* kout = (moved & 1) ? k0 : k1;
     const uint32_t* vin = VALS ? ((moved & 1) ? v1 : v0) : nullptr;
@@ -301,31 +406,12 @@ __global__ __launch_bounds__(OS_THREADS) void k_place(K* k0, K* k1, uint32_t* v0
     const int64_t end = min(n, begin + block_keys);
     const bool one_tile = end - begin <= TILE;
 
-    // The next tile's keys (and values) are loaded into registers while the
-    // current tile is ranked and scattered.
-    // (Positions past the end read the last key instead: no branch per load.)
-    K nkey[ITEMS];
-    uint32_t nval[ITEMS];
-    auto load_tile = [&](int64_t tb) {
-        const uint32_t first = (uint32_t)(wid * (kWave * ITEMS) + opaque(lane));
-        const uint32_t last = (uint32_t)min((int64_t)TILE, end - tb) - 1u;
-        const K* kt = kin + tb;
-        const uint32_t* vt = VALS ? vin + tb : nullptr;
-#pragma unroll
-        for (int j = 0; j < ITEMS; ++j) {
-            const uint32_t idx = min(first + (uint32_t)(j * kWave), last);
-            nkey[j] = kt[idx];
-            if (VALS) nval[j] = vt[idx];
-        }
-    };
     auto announce = [&](uint32_t count) {  // threads 0 .. RS_BINS - 1
         if (st.wide)
-            publish((unsigned long long*)status, block, tid, count,
-                    block ? LookWord<unsigned long long>::COUNT : LookWord<unsigned long long>::PREFIX);
+            chain_store((unsigned long long*)status, block, tid, ChainWord<unsigned long long>::COUNT | count);
         else
-            publish(status, block, tid, count, block ? LookWord<uint32_t>::COUNT : LookWord<uint32_t>::PREFIX);
+            chain_store(status, block, tid, ChainWord<uint32_t>::COUNT | count);
     };
-    uint32_t block_count = 0;
     if (!one_tile) {
         for (int i = lane; i < RS_BINS; i += kWave) wave_hist[wid][i] = 0;
         __syncthreads();
@@ -342,28 +428,31 @@ __global__ __launch_bounds__(OS_THREADS) void k_place(K* k0, K* k1, uint32_t* v0
         }
         __syncthreads();
         if (tid < RS_BINS) {
+            uint32_t count = 0;
 #pragma unroll
-            for (int w = 0; w < OS_WAVES; ++w) block_count += wave_hist[w][tid];
-            announce(block_count);
+            for (int w = 0; w < OS_WAVES; ++w) count += wave_hist[w][tid];
+            announce(count);
         }
         __syncthreads();
     }
-    load_tile(begin);
     for (int64_t tile_base = begin; tile_base < end; tile_base += TILE) {
         const int tile_n = (int)min((int64_t)TILE, end - tile_base);
         const int tid = opaque((int)threadIdx.x);
         const int lane = tid % kWave;
-        for (int i = lane; i < RS_BINS; i += kWave) wave_hist[wid][i] = 0;
-        __syncthreads();
+        // Positions past the end read the last key instead: no branch per load.
         K key[ITEMS];
         uint32_t val[ITEMS];
         uint32_t rank[ITEMS];
+        const K* kt = kin + tile_base;
+        const uint32_t* vt = VALS ? vin + tile_base : nullptr;
 #pragma unroll
         for (int j = 0; j < ITEMS; ++j) {
-            key[j] = nkey[j];
-            if (VALS) val[j] = nval[j];
+            const uint32_t idx = min((uint32_t)(wid * (kWave * ITEMS) + j * kWave + lane), (uint32_t)tile_n - 1u);
+            key[j] = kt[idx];
+            if (VALS) val[j] = vt[idx];
         }
-        if (tile_base + TILE < end) load_tile(tile_base + TILE);
+        for (int i = lane; i < RS_BINS; i += kWave) wave_hist[wid][i] = 0;
+        __syncthreads();
         rank_tile<K, CONV, ITEMS>(key, rank, wave_hist[wid], wid, tile_n, shift, mask);
         __syncthreads();
         // Per digit: offsets of each wave inside the digit, and tile totals.
@@ -375,10 +464,7 @@ __global__ __launch_bounds__(OS_THREADS) void k_place(K* k0, K* k1, uint32_t* v0
                 wave_hist[w][tid] = cnt;
                 cnt += c;
             }
-            if (one_tile) {
-                block_count = cnt;
-                announce(cnt);
-            }
+            if (one_tile) announce(cnt);
         }
         int tot;
         const int excl = wg_exclusive_scan<OS_THREADS>((int)cnt, tot, s_wave);
@@ -395,22 +481,12 @@ __global__ __launch_bounds__(OS_THREADS) void k_place(K* k0, K* k1, uint32_t* v0
         }
         if (tid < RS_BINS) {
             uint32_t at;
-            if (tile_base == begin) {
-                uint32_t before = 0;
-                if (block) {
-                    if (st.wide) {
-                        before = look_back<unsigned long long, 4>((const unsigned long long*)status, block, tid, &st.out[1]);
-                        publish((unsigned long long*)status, block, tid, before + block_count,
-                                LookWord<unsigned long long>::PREFIX);
-                    } else {
-                        before = look_back<uint32_t, 8>((const uint32_t*)status, block, tid, &st.out[1]);
-                        publish(status, block, tid, before + block_count, LookWord<uint32_t>::PREFIX);
-                    }
-                }
-                at = st.base[place * RS_BINS + tid] + before;
-            } else {
+            if (tile_base != begin)
                 at = next_out[tid];
-            }
+            else if (st.wide)
+                at = await_start((const unsigned long long*)status, block, tid, &st.out[1]);
+            else
+                at = await_start((const uint32_t*)status, block, tid, &st.out[1]);
             out_shift[tid] = at - (uint32_t)excl;
             next_out[tid] = at + cnt;
         }
@@ -519,22 +595,22 @@ struct SortPlan {
     int hist_wgs = 1;
 };
 
-size_t look_words(const SortPlan& p) { return (size_t)2 * p.blocks * RS_BINS * (p.wide ? 2 : 1); }
+bool wide_words(int64_t n) { return n >= (1ll << 30); }
+size_t look_words(int64_t blocks, bool wide) { return (size_t)2 * blocks * RS_BINS * (wide ? 2 : 1); }
 
-// max_words: scratch words there are (0: as many as the plan wants).
-SortPlan sort_plan(int64_t n, int num_cus, const SortPolicy& pol, size_t max_words = 0) {
+// Blocks of one tile: longer ones read their keys twice, and are for sorts
+// whose chain words would exceed the scratch or kMaxBlocks, and for a policy
+// that names a number of workgroups.
+SortPlan sort_plan(int64_t n, int num_cus, const SortPolicy& pol, size_t max_words) {
     SortPlan p;
     p.items = pol.items;
-    p.wide = n >= (1ll << 30);
+    p.wide = wide_words(n);
     const int64_t tile = (int64_t)OS_THREADS * pol.items;
     const int64_t tiles = std::max<int64_t>(1, (n + tile - 1) / tile);
-    int64_t max_blocks = pol.wgs_per_cu > 0 ? (int64_t)num_cus * pol.wgs_per_cu : tiles;
-    int64_t per = std::max<int64_t>((tiles + max_blocks - 1) / max_blocks, 1);
-    if (pol.wgs_per_cu == 0) per = std::max<int64_t>(1, std::min<int64_t>(kBlockTiles, tiles / ((int64_t)num_cus * 4)));
-    if (max_words) {
-        const int64_t fit = (int64_t)((max_words - kStateWords) / (2 * RS_BINS * (p.wide ? 2 : 1)));
-        per = std::max(per, (tiles + fit - 1) / fit);
-    }
+    int64_t most = kMaxBlocks;
+    if (pol.wgs_per_cu > 0) most = (int64_t)num_cus * pol.wgs_per_cu;
+    if (n > SMALL_KEYS) most = std::min<int64_t>(most, (max_words - kStateWords) / look_words(1, p.wide));
+    const int64_t per = (tiles + most - 1) / most;
     p.block_keys = per * tile;
     p.blocks = (int)((tiles + per - 1) / per);
     p.hist_wgs = (int)std::min<int64_t>((n + OS_THREADS * 8 - 1) / (OS_THREADS * 8), (int64_t)num_cus * 2);
@@ -557,7 +633,7 @@ SortState sort_state(const SortScratch& sc, const SortPlan& plan, int places, in
 template <typename K, int CONV, bool VALS, int ITEMS>
 void launch_places(K* k0, K* k1, uint32_t* v0, uint32_t* v1, int64_t n, int begin_bit, int end_bit,
                    const SortPlan& plan, const SortState& st, hipStream_t stream) {
-    const int64_t clear = (int64_t)HIST_COPIES * MAX_PLACES * RS_BINS + (int64_t)look_words(plan) / 2;
+    const int64_t clear = (int64_t)HIST_COPIES * MAX_PLACES * RS_BINS + (int64_t)look_words(plan.blocks, plan.wide) / 2;
     hipLaunchKernelGGL(k_sort_init, dim3((unsigned)std::min<int64_t>((clear + 1023) / 1024, 512)), dim3(256), 0, stream,
                        st);
     hipLaunchKernelGGL((k_histogram<K, CONV>), dim3(plan.hist_wgs), dim3(OS_THREADS), 0, stream, (const K*)k0, n,
@@ -565,7 +641,7 @@ void launch_places(K* k0, K* k1, uint32_t* v0, uint32_t* v1, int64_t n, int begi
     hipLaunchKernelGGL(k_plan, dim3(st.places), dim3(RS_BINS), 0, stream, st, n);
     for (int place = 0, shift = begin_bit; shift < end_bit; shift += 8, ++place) {
         const uint32_t mask = (1u << std::min(8, end_bit - shift)) - 1u;
-        hipLaunchKernelGGL((k_place<K, CONV, VALS, ITEMS>), dim3(plan.blocks), dim3(OS_THREADS), 0, stream, k0, k1, v0,
+        hipLaunchKernelGGL((k_place<K, CONV, VALS, ITEMS>), dim3(plan.blocks + SERVERS), dim3(OS_THREADS), 0, stream, k0, k1, v0,
                            v1, n, place, shift, mask, plan.block_keys, st);
     }
 }
@@ -627,18 +703,26 @@ b40c_status validate(const char* who, int32_t key_type, const void* k0, const vo
 
 }  // namespace
 
-// Default: 8 keys per thread; blocks as sort_plan sizes them.
-SortPolicy resolve_sort_policy(SortPolicy p, int64_t n, int key_bytes) {
-    (void)n;
-    (void)key_bytes;
-    if (p.items != 8 && p.items != 16) p.items = 8;
+// Default keys per thread: 16 where key and value are at most 8 bytes (the tile
+// is 64 KB of LDS, two workgroups per CU) and the sort gives the CUs almost two
+// (1.75) of these workgroups each; else 8.  Longer runs of a digit waste fewer
+// partial lines (16 against 8, 2^26 64-bit keys: 2.91 and 3.15 ms; 32-bit pairs
+// 1.58 and 1.70; 4 M 64-bit keys 230 and 246 us), but shorter sorts lack
+// workgroups (3 M 64-bit keys: 216 and 208 us; 1.3 M 32-bit pairs 80 and 74) and
+// 12-byte pairs the LDS (4 M pairs: 413 and 336 us).
+SortPolicy resolve_sort_policy(SortPolicy p, int64_t n, int pair_bytes, int num_cus) {
+    if (p.items != 8 && p.items != 16)
+        p.items = pair_bytes <= 8 && 4 * n >= 7 * (int64_t)num_cus * OS_THREADS * 16 ? 16 : 8;
     if (p.wgs_per_cu < 0 || p.wgs_per_cu > RS_MAX_WGS_PER_CU) p.wgs_per_cu = 0;
     return p;
 }
 
-size_t sort_scratch_words(int64_t n, int num_cus, const SortPolicy& pol) {
+// Never less for more keys, whatever the policy: an enactor's scratch serves
+// every sort of at most as many keys as the one that sized it.
+size_t sort_scratch_words(int64_t n) {
     if (n <= SMALL_KEYS) return kReportWords;
-    return kStateWords + look_words(sort_plan(n, num_cus, pol));
+    const int64_t blocks = std::min<int64_t>((n + OS_THREADS * 8 - 1) / (OS_THREADS * 8), kMaxBlocks);
+    return kStateWords + look_words(blocks, wide_words(n));
 }
 
 namespace {
@@ -701,8 +785,8 @@ b40c_status radix_sort_once(int32_t key_type, void* k0, void* k1, uint32_t* v0, 
     DeviceInfo info;
     B40C_TRY(device_info(info));
     DeviceBuffer mem;
-    const SortPolicy pol = resolve_sort_policy(SortPolicy{}, n, key_bits(key_type) / 8);
-    const size_t words = sort_scratch_words(n, info.num_cus, pol);
+    const SortPolicy pol = resolve_sort_policy(SortPolicy{}, n, key_bits(key_type) / 8 + (v0 ? 4 : 0), info.num_cus);
+    const size_t words = sort_scratch_words(n);
     B40C_TRY(mem.alloc(words * sizeof(uint32_t)));
     return radix_sort_sync(key_type, k0, k1, v0, v1, n, begin_bit, end_bit, info.num_cus, pol,
                            SortScratch{mem.as<uint32_t>(), words}, selector, stream);
@@ -725,7 +809,7 @@ b40c_status radix_sort_pairs_u32(uint32_t* k0, uint32_t* k1, uint32_t* v0, uint3
 // ---------------------------------------------------------------------------
 // Allocation-free sort (no counterpart in the reference): its scratch is this
 // fixed device array, one copy per GPU, which the GPU keeps until the
-// process ends: 2 MiB + 2 KiB, enough for the look-back words of 950 blocks
+// process ends: 2 MiB + 2 KiB, enough for the chain words of 950 blocks
 // (475 from 2^30 keys on); blocks are as large as n <= 2^32 - 1 keys then need.
 // In host code `scratch`
 // is only a stand-in for the device array; its device address comes from
@@ -815,7 +899,7 @@ b40c_status b40c_radix_sort_u64_noalloc(uint64_t* d_keys0, uint64_t* d_keys1, in
     if (n <= 1 || begin_bit == end_bit) return B40C_OK;
     NoAllocSlot* slot = nullptr;
     B40C_TRY(noalloc_slot(slot));
-    const SortPolicy pol = resolve_sort_policy(SortPolicy{}, n, 8);
+    const SortPolicy pol = resolve_sort_policy(SortPolicy{}, n, 8, slot->num_cus);
     return radix_sort_sync(B40C_KEY_U64, d_keys0, d_keys1, nullptr, nullptr, n, begin_bit, end_bit, slot->num_cus,
                            pol, SortScratch{slot->ptr, kNoAllocWords}, selector, nullptr, false);
 }
@@ -842,8 +926,8 @@ b40c_status b40c_sort_enactor_sort(b40c_sort_enactor* e, int32_t key_type, void*
     if (n <= 1 || begin_bit == end_bit) return B40C_OK;
     DeviceInfo info;
     B40C_TRY(device_info(info));
-    const SortPolicy pol = resolve_sort_policy(e->policy, n, key_bits(key_type) / 8);
-    const size_t words = sort_scratch_words(n, info.num_cus, pol);
+    const SortPolicy pol = resolve_sort_policy(e->policy, n, key_bits(key_type) / 8 + (d_vals0 ? 4 : 0), info.num_cus);
+    const size_t words = sort_scratch_words(n);
     // Grow-only: later sorts of at most this size allocate nothing.
     B40C_TRY(e->scratch.reserve(words * sizeof(uint32_t)));
     return radix_sort_sync(key_type, d_keys0, d_keys1, d_vals0, d_vals1, n, begin_bit, end_bit, info.num_cus, pol,

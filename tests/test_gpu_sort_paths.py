@@ -155,3 +155,12 @@ def test_concurrent_enactors():
     for t in threads:
         t.join()
     assert not errors, errors
+
+
+# Tiles of 4,096 keys around an XCD group (64), a serving step (256 and 128), the
+# change of the step (512), and the keys from which tiles hold 8,192 on.
+@pytest.mark.parametrize("n", [64 * 4096, 64 * 4096 + 1, 128 * 4096 + 1, 256 * 4096 + 1, 512 * 4096, 512 * 4096 + 1,
+                               3_670_015, 3_670_016])
+@pytest.mark.parametrize("dtype,values", [(np.uint32, True), (np.uint64, False), (np.float64, True)])
+def test_chained_tiles(dtype, values, n):
+    _check(_keys(dtype, n, n % 1000), values)
