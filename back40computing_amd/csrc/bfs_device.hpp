@@ -6,12 +6,11 @@
 //    (replaces CooperativeTileScan::ScanTileWithEnqueue's per-tile atomic,
 //    b40c/util/scan/cooperative_scan.cuh:173-229).  A wave that finds the LDS
 //    buffer full spills straight to the global queue (one atomic per wave).
-//  * tiered_gather: neighbour gathering in three tiers (whole workgroup for
-//    degree >= cta threshold, whole wave for degree >= wave threshold,
-//    scan-ranked gather staged in LDS for the rest), replacing
+//  * positional_gather: neighbour gathering by edge position over a tile's
+//    lists laid end to end, several edges per thread in flight, replacing
 //    ExpandByCta / ExpandByWarp / ExpandByScan
-//    (b40c/graph/bfs/two_phase/expand_atomic/cta.cuh:215-423, 606-719).
-//    Thresholds are runtime values.
+//    (b40c/graph/bfs/two_phase/expand_atomic/cta.cuh:215-423, 606-719): one
+//    form for every degree.
 //  * claim_exact: the visited bitmask with an agent-scope atomicOr, so each
 //    vertex has exactly one discoverer (the reference's best-effort bitmask
 //    RMW, contract_expand_atomic/cta.cuh:237-252, lets duplicates through).
@@ -30,7 +29,6 @@ namespace b40c {
 constexpr int BFS_THREADS = 256;
 constexpr int BFS_WAVES = BFS_THREADS / kWave;
 constexpr int LQ_CAP = 2048;          // LDS queue entries
-constexpr int GATHER_ELEMS = 1024;    // fine-tier staging window
 constexpr int HIST_SIZE = 1024;       // history hash entries
 
 struct BfsArgs {
@@ -317,97 +315,6 @@ __device__ __forceinline__ bool history_seen(HistoryHash& h, int32_t v) {
     if (h.slot[idx] == v) return true;
     h.slot[idx] = v;
     return false;
-}
-
-// ---------------------------------------------------------------------------
-// Tiered neighbour gather.  `sink(valid, neighbour, source)` is called
-// wave-uniformly (all lanes active) for every edge of every input vertex.
-// `deg` is consumed (zeroed) as vertices are handled.  Workgroup-uniform call.
-// ---------------------------------------------------------------------------
-struct GatherSmem {
-    int32_t owner;
-    int32_t o_start, o_deg, o_src;
-    int32_t goff[GATHER_ELEMS];
-    int32_t gsrc[GATHER_ELEMS];
-    int32_t s_wave[BFS_WAVES];
-};
-
-__device__ __forceinline__ void gather_init(GatherSmem& g) {
-    if (threadIdx.x == 0) g.owner = -1;
-}
-
-template <typename Sink>
-__device__ __forceinline__ void tiered_gather(const int32_t* __restrict__ cols, int32_t src, int32_t start,
-                                              int32_t deg, int32_t cta_th, int32_t wave_th, GatherSmem& g,
-                                              Sink& sink) {
-    const int tid = threadIdx.x;
-    const int lane = lane_id();
-    // Whole-workgroup tier: threads vie for the workgroup; the winner's list
-    // is strided by all threads.
-    while (true) {
-        if (deg >= cta_th) g.owner = tid;
-        __syncthreads();
-        const int owner = g.owner;
-        if (owner < 0) break;
-        if (tid == owner) {
-            g.o_start = start;
-            g.o_deg = deg;
-            g.o_src = src;
-            deg = 0;
-        }
-        __syncthreads();
-        const int32_t os = g.o_start, od = g.o_deg, osrc = g.o_src;
-        for (int32_t e0 = 0; e0 < od; e0 += BFS_THREADS) {
-            const int32_t e = e0 + tid;
-            const bool valid = e < od;
-            const int32_t v = valid ? cols[os + e] : 0;
-            sink(valid, v, osrc);
-        }
-        __syncthreads();
-        if (tid == 0) g.owner = -1;
-        __syncthreads();
-    }
-    // Whole-wave tier: lanes vie through a ballot; the wave strides the list.
-    while (true) {
-        const uint64_t m = __ballot(deg >= wave_th);
-        if (m == 0) break;
-        const int leader = __ffsll((unsigned long long)m) - 1;
-        const int32_t ls = wave_bcast(start, leader);
-        const int32_t ld = wave_bcast(deg, leader);
-        const int32_t lsrc = wave_bcast(src, leader);
-        if (lane == leader) deg = 0;
-        for (int32_t e0 = 0; e0 < ld; e0 += kWave) {
-            const int32_t e = e0 + lane;
-            const bool valid = e < ld;
-            const int32_t v = valid ? cols[ls + e] : 0;
-            sink(valid, v, lsrc);
-        }
-    }
-    // Fine tier: workgroup scan of the remaining (small) degrees, gather
-    // offsets staged in LDS, then a coalesced sweep of the staged window.
-    int total;
-    const int rank = wg_exclusive_scan<BFS_THREADS>(deg, total, g.s_wave);
-    for (int w0 = 0; w0 < total; w0 += GATHER_ELEMS) {
-        const int lo = max(rank, w0);
-        const int hi = min(rank + deg, w0 + GATHER_ELEMS);
-        for (int j = lo; j < hi; ++j) {
-            g.goff[j - w0] = start + (j - rank);
-            g.gsrc[j - w0] = src;
-        }
-        __syncthreads();
-        const int cnt = min(GATHER_ELEMS, total - w0);
-        for (int k0 = 0; k0 < cnt; k0 += BFS_THREADS) {
-            const int k = k0 + tid;
-            const bool valid = k < cnt;
-            int32_t v = 0, s = 0;
-            if (valid) {
-                v = cols[g.goff[k]];
-                s = g.gsrc[k];
-            }
-            sink(valid, v, s);
-        }
-        __syncthreads();
-    }
 }
 
 // ---------------------------------------------------------------------------

@@ -2,7 +2,7 @@
 // over a packed multi-graph CSR, with per-query label slots and admission at
 // level boundaries (continuous batching).  No counterpart in the reference;
 // it stands beside the single-source enactors and shares their device
-// building blocks (LDS-buffered queues, tiered gather).
+// building blocks (LDS-buffered queues, positional gather).
 //
 // Layout:
 //  * packed CSR: graphs concatenated, vertex ids global, graph g owns
@@ -94,8 +94,6 @@ struct MsArgs {
     int32_t G;
     int32_t alpha;
     int32_t beta;
-    int32_t cta_th;
-    int32_t wave_th;
     int32_t grid_th;
 };
 
@@ -146,16 +144,18 @@ constexpr int kMsMaxFusedGrid = 4096;  // grid-barrier arrival words of the pers
 
 struct MsShared {
     LdsKeyQueue q;
-    GatherSmem g;
-    unsigned long long red[BFS_WAVES];
+    ListSmem l;                        // lists of the tile's vertices; l.src is the vertex's thread
+    unsigned long long w[BFS_THREADS]; // the vertex's bits in top-down mode
+    int32_t u[BFS_THREADS];
+    int32_t g[BFS_THREADS];
 };
 
 // Labels for every newly reached (query, v) bit; `src` is the discovering
 // neighbour (global id) or -1 for a source.  One bit at a time: unrolling
 // the slot lookups four bits at a time measured the same and doubled the
 // pull's code.
-__device__ __forceinline__ void ms_record(const MsArgs& a, int ph, int32_t v, int32_t src, unsigned long long bits) {
-    const int32_t g = a.gid[v];
+__device__ __forceinline__ void ms_record(const MsArgs& a, int ph, int32_t g, int32_t v, int32_t src,
+                                          unsigned long long bits) {
     const int32_t vb = a.vbase[g];
     while (bits) {
         const int b = __ffsll(bits) - 1;
@@ -166,6 +166,9 @@ __device__ __forceinline__ void ms_record(const MsArgs& a, int ph, int32_t v, in
         a.depth_out[idx] = ph + 1 - a.qstart[q];
         a.pred_out[idx] = src - vb;
     }
+}
+__device__ __forceinline__ void ms_record(const MsArgs& a, int ph, int32_t v, int32_t src, unsigned long long bits) {
+    ms_record(a, ph, a.gid[v], v, src, bits);
 }
 
 __device__ __forceinline__ GlobalQueue ms_out_queue(const MsArgs& a, int ph) {
@@ -178,26 +181,46 @@ __device__ __forceinline__ GlobalQueue ms_out_queue(const MsArgs& a, int ph) {
     return out;
 }
 
-// Top-down edge (src -> v) for the bits of src in top-down mode: exact
-// claim by atomic OR on visited[v], labels, and the first OR into next[v]
-// enqueues v.  Wave-collective (the LDS queue append).
-__device__ __forceinline__ void ms_push_edge(const MsArgs& a, int ph, MsShared& s, const GlobalQueue& out,
-                                             bool valid, int32_t v, int32_t src) {
-    const unsigned long long* cur = a.front[ph % 3];
-    unsigned long long nb = 0;
-    if (valid) {
-        const unsigned long long w = cur[src] & ~a.bu[a.gid[src]] & ~a.visited[v];
-        if (w) {
-            const unsigned long long old = atomic_or_u64(&a.visited[v], w);
-            nb = w & ~old;
-        }
+// Top-down edges of one gather step, for the bits of each source in top-down
+// mode: exact claim by atomic OR on visited[v], labels, and the first OR into
+// next[v] enqueues v.  The K edges' probes, claims and ORs are in flight together.
+// Edges stay within a graph, so the source's graph is the neighbour's.
+constexpr int MS_GATHER_K = 4;
+struct MsPushSink {
+    const MsArgs& a;
+    int ph;
+    MsShared& s;
+    const GlobalQueue& out;
+    __device__ __forceinline__ void reserve(uint32_t, ListSmem&) {}
+    template <int K>
+    __device__ __forceinline__ void step(uint32_t, const bool (&valid)[K], const int32_t (&v)[K],
+                                         const int32_t (&from)[K]) {
+        unsigned long long* next = a.front[(ph + 1) % 3];
+        unsigned long long w[K], nb[K];
+        bool enq[K];
+#pragma unroll
+        for (int r = 0; r < K; ++r) w[r] = valid[r] ? s.w[from[r]] & ~a.visited[v[r]] : 0ull;
+#pragma unroll
+        for (int r = 0; r < K; ++r) nb[r] = w[r] ? w[r] & ~atomic_or_u64(&a.visited[v[r]], w[r]) : 0ull;
+#pragma unroll
+        for (int r = 0; r < K; ++r) enq[r] = nb[r] && atomic_or_u64(&next[v[r]], nb[r]) == 0ull;
+#pragma unroll
+        for (int r = 0; r < K; ++r)
+            if (nb[r]) ms_record(a, ph, s.g[from[r]], v[r], s.u[from[r]], nb[r]);
+        lq_append_batch<false>(s.q, out, enq, v, v);
     }
-    bool enq = false;
-    if (nb) {
-        ms_record(a, ph, v, src, nb);
-        enq = atomic_or_u64(&a.front[(ph + 1) % 3][v], nb) == 0ull;
-    }
-    lq_append<false>(s.q, out, enq, v, 0);
+    __device__ __forceinline__ void step_end() { lq_flush<false>(s.q, out, LQ_CAP / 2); }
+};
+
+// Frontier vertex x and its list as this thread's entry of a gather tile; false
+// where no bit of x is in top-down mode.
+__device__ __forceinline__ bool ms_push_entry(const MsArgs& a, int ph, MsShared& s, int32_t x) {
+    const int32_t g = a.gid[x];
+    const unsigned long long w = a.front[ph % 3][x] & ~a.bu[g];
+    s.w[threadIdx.x] = w;
+    s.u[threadIdx.x] = x;
+    s.g[threadIdx.x] = g;
+    return w != 0ull;
 }
 
 // Grid tier: a list of at least grid_th edges is cut into HEAVY_CHUNK-edge
@@ -263,20 +286,26 @@ __device__ void ms_push_body(const MsArgs& a, int ph, MsShared& s) {
     }
     if (n_f == 0) return;  // no vertex carries a bit: nothing can be found
     if (threadIdx.x == 0) s.q.count = 0;
-    gather_init(s.g);
     __syncthreads();
     const GlobalQueue out = ms_out_queue(a, ph);
-    const unsigned long long* cur = a.front[ph % 3];
 
-    // Top-down push over the frontier queue, for the bits in top-down mode.
+    // Top-down push over the frontier queue, for the bits in top-down mode.  A
+    // level's frontier is often shorter than the grid has threads, and its
+    // lists differ by orders of magnitude: each workgroup takes an equal number
+    // of vertices, at most one per thread.  Latency of the chain probe, claim,
+    // OR, slot lookup, labels bounds a step, so K edges per thread share it (256
+    // queries over 64 graphs: the first two levels' pushes 79 and 109 us in
+    // tiles of 256 vertices and one edge per thread, now 10 and 14).
     const int32_t* qin = a.queue[ph % 3];
-    for (uint32_t base = blockIdx.x * BFS_THREADS; base < n_f; base += gridDim.x * BFS_THREADS) {
+    const uint32_t per = min((n_f + gridDim.x - 1) / gridDim.x, (uint32_t)BFS_THREADS);
+    MsPushSink sink{a, ph, s, out};
+    for (uint32_t base = blockIdx.x * per; base < n_f; base += gridDim.x * per) {
         const uint32_t i = base + threadIdx.x;
         int32_t u = -1, start = 0, deg = 0;
-        if (i < n_f) {
+        if (threadIdx.x < per && i < n_f) {
             const int32_t x = qin[i];
             if ((uint32_t)x < (uint32_t)a.n) {
-                if (cur[x] & ~a.bu[a.gid[x]]) {
+                if (ms_push_entry(a, ph, s, x)) {
                     u = x;
                     start = a.offs[x];
                     deg = a.offs[x + 1] - start;
@@ -286,8 +315,7 @@ __device__ void ms_push_body(const MsArgs& a, int ph, MsShared& s) {
             }
         }
         ms_defer_heavy(a, ph, u, deg);
-        auto sink = [&](bool valid, int32_t v, int32_t src) { ms_push_edge(a, ph, s, out, valid, v, src); };
-        tiered_gather(a.cols, u, start, deg, a.cta_th, a.wave_th, s.g, sink);
+        positional_gather<MS_GATHER_K>(a.cols, (int32_t)threadIdx.x, start, deg, s.l, sink);
         lq_flush<false>(s.q, out, LQ_CAP / 2);
     }
     lq_flush<false>(s.q, out, 1);
@@ -778,9 +806,9 @@ __device__ void ms_pull_narrow_body(const MsArgs& a, int ph, MsPullNarrowShared&
     lq_flush<false>(s.q, out, 1);
 }
 
-// Grid tier of level ph's push: workgroups take chunks grid-stride, one edge
-// per thread.  Each chunk is checked against the entry it names, so a stale
-// map word never indexes outside a list.
+// Grid tier of level ph's push: workgroups take chunks grid-stride, up to one
+// per thread, and gather them together.  Each chunk is checked against the entry
+// it names, so a stale map word never indexes outside a list.
 __device__ void ms_heavy_body(const MsArgs& a, int ph, MsShared& s) {
     const unsigned long long alloc =
         __hip_atomic_load(&a.ctr->heavy_alloc[ph & 1], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
@@ -790,38 +818,71 @@ __device__ void ms_heavy_body(const MsArgs& a, int ph, MsShared& s) {
     if (threadIdx.x == 0) s.q.count = 0;
     __syncthreads();
     const GlobalQueue out = ms_out_queue(a, ph);
-    for (uint32_t c = blockIdx.x; c < C; c += gridDim.x) {
-        const int32_t entry = a.chunk_map[c];
-        int32_t u = -1, e = 0;
-        bool valid = false;
+    MsPushSink sink{a, ph, s, out};
+    for (uint64_t base = 0; base + blockIdx.x < C; base += (uint64_t)gridDim.x * BFS_THREADS) {
+        const uint64_t c = base + (uint64_t)threadIdx.x * gridDim.x + blockIdx.x;
+        int32_t start = 0, len = 0;
+        const int32_t entry = c < C ? a.chunk_map[c] : -1;
         if ((uint32_t)entry < H) {
             const int2 eu = a.heavy[entry];
             if ((uint32_t)eu.x < (uint32_t)a.n && (uint32_t)eu.y <= c) {
                 const int32_t s0 = a.offs[eu.x], deg = a.offs[eu.x + 1] - s0;
-                const long long off = (long long)(c - (uint32_t)eu.y) * HEAVY_CHUNK + threadIdx.x;
-                if (off < deg) {
-                    u = eu.x;
-                    e = s0 + (int32_t)off;
-                    valid = true;
+                const long long off = (long long)((uint32_t)c - (uint32_t)eu.y) * HEAVY_CHUNK;
+                if (off < deg && ms_push_entry(a, ph, s, eu.x)) {
+                    start = s0 + (int32_t)off;
+                    len = min((int32_t)HEAVY_CHUNK, deg - (int32_t)off);
                 }
             } else {
                 st_relaxed(&a.ctr->corrupt, 1u);
             }
         }
-        const int32_t v = valid ? a.cols[e] : -1;
-        ms_push_edge(a, ph, s, out, valid, v, u);
+        positional_gather<MS_GATHER_K>(a.cols, (int32_t)threadIdx.x, start, len, s.l, sink);
         lq_flush<false>(s.q, out, LQ_CAP / 2);
     }
     lq_flush<false>(s.q, out, 1);
 }
 
 // Per (graph, slot) count and degree sum of the vertices discovered by level
-// ph (the next frontier queue; next[v] holds exactly v's new bits).  Each
-// wave takes one contiguous stretch of the queue (entries appended together
-// mostly share a graph) and, per chunk of 64 entries and per graph present in
-// it, transposes the lanes' bit masks so that lane b holds the set of lanes
-// carrying bit b.  Running totals are kept while the graph stays the same.
-__device__ void ms_count_body(const MsArgs& a, int ph) {
+// ph (the next frontier queue; next[v] holds exactly v's new bits).  A
+// workgroup takes one contiguous stretch of the queue, of at least
+// MS_COUNT_STRETCH entries: every workgroup ends with atomics on its graphs'
+// counters, and those of one line are serialised (256 entries: 8 queries on one
+// graph of 2^18 vertices 465 us a run for 413; 1,024 or more: slower batches).
+//
+// Chunks of 64 entries whose vertices have few new bits each add them one by one
+// to a table in LDS, keyed by graph and slot: a chunk may hold many graphs.  In
+// other chunks the lanes' bit masks are transposed, per graph present, so that
+// lane b holds the set of lanes carrying bit b, and running totals are kept
+// while the graph stays the same.  Transposing every chunk took 20 to 60 us of a
+// level of 256 queries over 64 graphs, now 10 to 19; adding one by one loses from
+// more than 32 bits on (64 queries on each of 4 graphs: 883 us a run for 833).
+constexpr int MS_COUNT_FEW = 16;
+constexpr int MS_COUNT_STRETCH = 512;
+constexpr int MS_COUNT_TABLE = 512;
+constexpr int MS_COUNT_PROBES = 4;
+struct MsCountShared {
+    uint32_t key[MS_COUNT_TABLE];  // graph * 64 + slot, or MS_COUNT_FREE
+    uint32_t n[MS_COUNT_TABLE];
+    unsigned long long m[MS_COUNT_TABLE];
+};
+constexpr uint32_t MS_COUNT_FREE = 0xFFFFFFFFu;
+
+__device__ __forceinline__ void ms_count_add(const MsArgs& a, MsCountShared& s, uint32_t key, uint32_t deg) {
+    uint32_t at = (key * 2654435761u) >> (32 - 9);
+    static_assert(MS_COUNT_TABLE == 1 << 9, "the hash's width");
+    for (int k = 0; k < MS_COUNT_PROBES; ++k, at = (at + 1) & (MS_COUNT_TABLE - 1)) {
+        const uint32_t old = atomicCAS(&s.key[at], MS_COUNT_FREE, key);
+        if (old == MS_COUNT_FREE || old == key) {
+            atomicAdd(&s.n[at], 1u);
+            atomicAdd(&s.m[at], (unsigned long long)deg);
+            return;
+        }
+    }
+    atomic_add_u32(&a.cnt_n[key], 1u);
+    atomic_add_u64(&a.cnt_m[key], (unsigned long long)deg);
+}
+
+__device__ void ms_count_body(const MsArgs& a, int ph, MsCountShared& s) {
     uint32_t n_q = ld_relaxed(&a.ctr->qlen[(ph + 1) & 3]);
     // Frontier bitmap of level ph + 1: set entry by entry from the queue while
     // it is short (the array is all zero: its bits were those of level ph - 1,
@@ -833,56 +894,78 @@ __device__ void ms_count_body(const MsArgs& a, int ph) {
     const unsigned long long* nxt = a.front[(ph + 1) % 3];
     uint32_t* fbm_next = a.fbm[(ph + 1) & 1];
     const int lane = lane_id();
-    const int64_t wave = (int64_t)blockIdx.x * BFS_WAVES + threadIdx.x / kWave;
+    const int wid = threadIdx.x / kWave;
+    const int64_t wave = (int64_t)blockIdx.x * BFS_WAVES + wid;
     const int64_t nwaves = (int64_t)gridDim.x * BFS_WAVES;
-    const int64_t per = (((int64_t)n_q + nwaves - 1) / nwaves + kWave - 1) / kWave * kWave;
-    const int64_t lo = wave * per, hi = min((int64_t)n_q, lo + per);
-    int32_t accg = -1;
-    uint32_t accn = 0;
-    unsigned long long accm = 0;
-    for (int64_t base = lo; base < hi; base += kWave) {
-        const int64_t i = base + lane;
-        int32_t g = -1, deg = 0;
-        unsigned long long bits = 0;
-        if (i < hi) {
-            const int32_t v = q[i];
-            if ((uint32_t)v < (uint32_t)a.n) {
-                g = a.gid[v];
-                bits = nxt[v];
-                deg = a.offs[v + 1] - a.offs[v];
-                if (!dense) atomicOr(&fbm_next[v >> 5], 1u << (v & 31));
-            } else {
-                st_relaxed(&a.ctr->corrupt, 1u);
-            }
+    const int64_t per = max(((int64_t)n_q + gridDim.x - 1) / gridDim.x, (int64_t)MS_COUNT_STRETCH);
+    const int64_t lo = (int64_t)blockIdx.x * per, hi = min((int64_t)n_q, lo + per);
+    if (lo < hi) {
+        for (int i = threadIdx.x; i < MS_COUNT_TABLE; i += BFS_THREADS) {
+            s.key[i] = MS_COUNT_FREE;
+            s.n[i] = 0u;
+            s.m[i] = 0ull;
         }
-        bool todo = g >= 0;
-        for (uint64_t rest = __ballot(todo); rest; rest = __ballot(todo)) {
-            const int32_t g1 = __shfl(g, __ffsll((unsigned long long)rest) - 1, kWave);
-            const bool mine = todo && g == g1;
-            todo = todo && !mine;
-            const unsigned long long y = wave_transpose64(mine ? bits : 0ull);
-            unsigned long long m = 0;
-#pragma unroll 8
-            for (int l = 0; l < kWave; ++l) {
-                const int d = __shfl(deg, l, kWave);
-                if ((y >> l) & 1ull) m += (unsigned long long)d;
+        __syncthreads();
+        int32_t accg = -1;
+        uint32_t accn = 0;
+        unsigned long long accm = 0;
+        auto flush = [&]() {
+            if (accg >= 0 && accn) {
+                atomic_add_u32(&a.cnt_n[(size_t)accg * 64 + lane], accn);
+                atomic_add_u64(&a.cnt_m[(size_t)accg * 64 + lane], accm);
             }
-            if (g1 != accg) {
-                if (accg >= 0 && accn) {
-                    atomic_add_u32(&a.cnt_n[(size_t)accg * 64 + lane], accn);
-                    atomic_add_u64(&a.cnt_m[(size_t)accg * 64 + lane], accm);
+        };
+        for (int64_t base = lo + wid * kWave; base < hi; base += BFS_THREADS) {
+            const int64_t i = base + lane;
+            int32_t g = -1, deg = 0;
+            unsigned long long bits = 0;
+            if (i < hi) {
+                const int32_t v = q[i];
+                if ((uint32_t)v < (uint32_t)a.n) {
+                    g = a.gid[v];
+                    bits = nxt[v];
+                    deg = a.offs[v + 1] - a.offs[v];
+                    if (!dense) atomicOr(&fbm_next[v >> 5], 1u << (v & 31));
+                } else {
+                    st_relaxed(&a.ctr->corrupt, 1u);
                 }
-                accg = g1;
-                accn = 0;
-                accm = 0;
             }
-            accn += (uint32_t)__popcll(y);
-            accm += m;
+            if (__ballot(__popcll(bits) > MS_COUNT_FEW) == 0ull) {
+                for (; bits; bits &= bits - 1)
+                    ms_count_add(a, s, (uint32_t)g * 64u + (uint32_t)(__ffsll(bits) - 1), (uint32_t)deg);
+                continue;
+            }
+            bool todo = g >= 0;
+            for (uint64_t rest = __ballot(todo); rest; rest = __ballot(todo)) {
+                const int32_t g1 = __shfl(g, __ffsll((unsigned long long)rest) - 1, kWave);
+                const bool mine = todo && g == g1;
+                todo = todo && !mine;
+                const unsigned long long y = wave_transpose64(mine ? bits : 0ull);
+                unsigned long long m = 0;
+#pragma unroll 8
+                for (int l = 0; l < kWave; ++l) {
+                    const int d = __shfl(deg, l, kWave);
+                    if ((y >> l) & 1ull) m += (unsigned long long)d;
+                }
+                if (g1 != accg) {
+                    flush();
+                    accg = g1;
+                    accn = 0;
+                    accm = 0;
+                }
+                accn += (uint32_t)__popcll(y);
+                accm += m;
+            }
         }
-    }
-    if (accg >= 0 && accn) {
-        atomic_add_u32(&a.cnt_n[(size_t)accg * 64 + lane], accn);
-        atomic_add_u64(&a.cnt_m[(size_t)accg * 64 + lane], accm);
+        flush();
+        __syncthreads();
+        for (int i = threadIdx.x; i < MS_COUNT_TABLE; i += BFS_THREADS) {
+            if (s.n[i]) {
+                atomic_add_u32(&a.cnt_n[s.key[i]], s.n[i]);
+                atomic_add_u64(&a.cnt_m[s.key[i]], s.m[i]);
+            }
+        }
+        __syncthreads();
     }
     const int64_t words = ((int64_t)a.n + 31) / 32;
     if (dense) {
@@ -999,7 +1082,10 @@ __global__ __launch_bounds__(BFS_THREADS) void k_ms_pull_narrow(MsArgs a, int ph
     __shared__ MsPullNarrowShared s;
     ms_pull_narrow_body(a, ms_phase(a, ph), s);
 }
-__global__ __launch_bounds__(BFS_THREADS) void k_ms_count(MsArgs a, int ph) { ms_count_body(a, ms_phase(a, ph)); }
+__global__ __launch_bounds__(BFS_THREADS) void k_ms_count(MsArgs a, int ph) {
+    __shared__ MsCountShared s;
+    ms_count_body(a, ms_phase(a, ph), s);
+}
 __global__ __launch_bounds__(BFS_THREADS) void k_ms_direction(MsArgs a, int ph) {
     ms_direction_body(a, ms_phase(a, ph));
 }
@@ -1013,6 +1099,7 @@ union MsFusedShared {
     MsShared push;
     MsPullShared pull;
     MsPullNarrowShared pull_n;
+    MsCountShared count;
 };
 __global__ __launch_bounds__(BFS_THREADS) void k_ms_fused(MsArgs a, int ph0, int levels) {
     __shared__ MsFusedShared s;
@@ -1029,7 +1116,7 @@ __global__ __launch_bounds__(BFS_THREADS) void k_ms_fused(MsArgs a, int ph0, int
         if (!grid_sync(bar, ++epoch, &s_word)) break;
         ms_pull_body(a, ph, s.pull);
         if (!grid_sync(bar, ++epoch, &s_word)) break;
-        ms_count_body(a, ph);
+        ms_count_body(a, ph, s.count);
         if (!grid_sync(bar, ++epoch, &s_word)) break;
         ms_direction_body(a, ph);
         if (!grid_sync(bar, ++epoch, &s_word)) break;
@@ -1340,9 +1427,7 @@ MsArgs ms_args(b40c_msbfs* m) {
     a.G = m->G;
     a.alpha = m->alpha;
     a.beta = m->beta;
-    a.cta_th = 256;
-    a.wave_th = 64;
-    a.grid_th = 128;
+    a.grid_th = 128;  // 512 and 1,024: 678 and 723 us for 256 queries over 64 graphs, 128: 666
     return a;
 }
 
