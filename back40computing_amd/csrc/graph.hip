@@ -9,9 +9,11 @@
 // rand() and std::stable_sort; here every step runs on the GPU with a
 // counter-based generator so the stream is identical for any launch shape.
 #include <cstring>
+#include <string>
+#include <utility>
 #include <vector>
 
-#include "internal.hpp"
+#include "chain.hpp"
 
 namespace b40c {
 
@@ -150,59 +152,102 @@ __global__ __launch_bounds__(GB_THREADS) void k_lattice_keys(int w, const int32_
     }
 }
 
-__device__ __forceinline__ bool keep_key(const uint64_t* keys, int64_t i, uint64_t sentinel) {
-    const uint64_t k = keys[i];
-    return k != sentinel && (i == 0 || keys[i - 1] != k);
-}
+// Sorted packed keys to CSR in one pass: the columns of the distinct keys in
+// order, and the row offsets.  A key that opens a new row writes its position as
+// the offset of that row and of the empty rows before it, the rule of
+// CsrGraph::FromCoo (csr_graph.cuh:127-147); dropped keys (the sentinel, above all
+// others) count as row n, and the last key closes the trailing rows.  A wave
+// holds rows of 64 consecutive keys, so loads and the stores of a row's kept
+// columns cover consecutive entries, and a long run of empty rows is filled by
+// the whole wave.  Bound by its read of the keys and, below a few million, by the
+// round trips of the chain: 33.5 M keys of RMAT-20 in 127 us (with its stores
+// 3.2 TB/s), 2 M keys in 16 us.  A count, a one-workgroup scan, a scatter of
+// columns and rows and a pass over the rows took 404 and 30 us, and a copy of the
+// total to the host between them 30 us more.
+constexpr int CSR_ITEMS = 16;
+constexpr int64_t CSR_BLOCK = (int64_t)CHAIN_THREADS * CSR_ITEMS;
+constexpr int64_t CSR_LONG_GAP = 16;  // rows opened by one key that the wave fills together
 
-// Pass 1 of the unique compaction: kept keys per workgroup chunk.
-__global__ __launch_bounds__(GB_THREADS) void k_unique_count(const uint64_t* keys, int64_t nkeys, uint64_t sentinel,
-                                                             int64_t chunk, uint32_t* wg_counts) {
-    __shared__ int s_wave[GB_THREADS / kWave];
-    const int64_t begin = (int64_t)blockIdx.x * chunk;
-    const int64_t end = min(nkeys, begin + chunk);
-    int c = 0;
-    for (int64_t i = begin + threadIdx.x; i < end; i += GB_THREADS) c += keep_key(keys, i, sentinel) ? 1 : 0;
-    int total;
-    (void)wg_exclusive_scan<GB_THREADS>(c, total, s_wave);
-    if (threadIdx.x == 0) wg_counts[blockIdx.x] = (uint32_t)total;
-}
-
-// Exclusive scan of up to a few thousand workgroup counts (one workgroup).
-__global__ __launch_bounds__(GB_THREADS) void k_scan_counts(uint32_t* counts, int G, uint32_t* total_out) {
-    __shared__ int s_wave[GB_THREADS / kWave];
-    uint32_t carry = 0;
-    for (int base = 0; base < G; base += GB_THREADS) {
-        const int i = base + threadIdx.x;
-        const int v = (i < G) ? (int)counts[i] : 0;
-        int tot;
-        const int ex = wg_exclusive_scan<GB_THREADS>(v, tot, s_wave);
-        if (i < G) counts[i] = carry + (uint32_t)ex;
-        carry += (uint32_t)tot;
+__global__ __launch_bounds__(CHAIN_THREADS) void k_csr_chained(const uint64_t* keys, int64_t nkeys, int shift,
+                                                               uint64_t sentinel, int32_t n, int32_t* cols,
+                                                               int32_t* offsets, unsigned long long* chain,
+                                                               ChainReport* report) {
+    __shared__ uint32_t s_tot[CHAIN_WAVES];
+    __shared__ uint64_t s_before;
+    __shared__ ChainServeShared s_serve;
+    if (blockIdx.x == 0) {
+        chain_serve(chain, gridDim.x - 1, report, s_serve);
+        return;
     }
-    if (threadIdx.x == 0) *total_out = carry;
-}
-
-// Pass 2: write the kept keys' columns and rows in order.
-__global__ __launch_bounds__(GB_THREADS) void k_unique_scatter(const uint64_t* keys, int64_t nkeys, uint64_t sentinel,
-                                                               int64_t chunk, const uint32_t* wg_offsets, int shift,
-                                                               int32_t* cols, uint32_t* rows) {
-    __shared__ int s_wave[GB_THREADS / kWave];
-    const int64_t begin = (int64_t)blockIdx.x * chunk;
-    const int64_t end = min(nkeys, begin + chunk);
-    const uint64_t mask = (1ull << shift) - 1;
-    uint32_t carry = wg_offsets[blockIdx.x];
-    for (int64_t base = begin; base < end; base += GB_THREADS) {
-        const int64_t i = base + threadIdx.x;
-        const bool keep = (i < end) && keep_key(keys, i, sentinel);
-        int tot;
-        const int ex = wg_exclusive_scan<GB_THREADS>(keep ? 1 : 0, tot, s_wave);
-        if (keep) {
-            const uint64_t k = keys[i];
-            cols[carry + ex] = (int32_t)(k & mask);
-            rows[carry + ex] = (uint32_t)(k >> shift);
+    const int block = blockIdx.x - 1;
+    const int lane = lane_id(), wid = threadIdx.x / kWave;
+    const int64_t begin = (int64_t)block * CSR_BLOCK + (int64_t)wid * kWave * CSR_ITEMS;
+    uint64_t x[CSR_ITEMS];
+    uint64_t first_left = 0;  // the key before the wave's first; lane 0
+    if (lane == 0 && begin > 0 && begin < nkeys) first_left = keys[begin - 1];
+#pragma unroll
+    for (int k = 0; k < CSR_ITEMS; ++k) {
+        const int64_t i = begin + k * kWave + lane;
+        x[k] = i < nkeys ? keys[i] : sentinel;
+    }
+    uint64_t heads[CSR_ITEMS];
+    uint32_t count = 0;
+    uint64_t last = first_left;
+#pragma unroll
+    for (int k = 0; k < CSR_ITEMS; ++k) {
+        const int64_t i = begin + k * kWave + lane;
+        const uint64_t left = __shfl_up(x[k], 1, kWave);
+        const uint64_t prev = lane == 0 ? last : left;
+        heads[k] = __ballot(x[k] != sentinel && (i == 0 || x[k] != prev));
+        count += (uint32_t)__popcll(heads[k]);
+        last = __shfl(x[k], kWave - 1, kWave);
+    }
+    if (lane == 0) s_tot[wid] = count;
+    __syncthreads();
+    if (threadIdx.x == 0) {
+        uint64_t mine = 0;
+#pragma unroll
+        for (int w = 0; w < CHAIN_WAVES; ++w) {
+            const uint32_t t = s_tot[w];
+            s_tot[w] = (uint32_t)mine;
+            mine += t;
         }
-        carry += (uint32_t)tot;
+        s_before = chain_before(chain, block, mine, report);
+    }
+    __syncthreads();
+    uint64_t pos = s_before + s_tot[wid];
+    const uint64_t mask = (1ull << shift) - 1;
+    last = first_left;
+#pragma unroll
+    for (int k = 0; k < CSR_ITEMS; ++k) {
+        const int64_t i = begin + k * kWave + lane;
+        const uint64_t left = __shfl_up(x[k], 1, kWave);
+        const uint64_t prev = lane == 0 ? last : left;
+        last = __shfl(x[k], kWave - 1, kWave);
+        const bool head = (heads[k] >> lane) & 1u;
+        const uint64_t at = pos + __popcll(heads[k] & ((1ull << lane) - 1));
+        pos += (uint64_t)__popcll(heads[k]);
+        if (head) cols[at] = (int32_t)(x[k] & mask);
+        // Rows this key opens, and after the last key those it closes.
+        const int64_t row = x[k] == sentinel ? (int64_t)n : (int64_t)(x[k] >> shift);
+        const int64_t prev_row = i == 0 ? -1 : prev == sentinel ? (int64_t)n : (int64_t)(prev >> shift);
+        const bool tail = i == nkeys - 1;
+        int64_t open = i < nkeys ? row - prev_row : 0;
+        if (open > 0 && open <= CSR_LONG_GAP)
+            for (int64_t r = prev_row + 1; r <= row; ++r) offsets[r] = (int32_t)at;
+        for (uint64_t wide = __ballot(open > CSR_LONG_GAP); wide; wide &= wide - 1) {
+            const int from = __ffsll((unsigned long long)wide) - 1;
+            const int64_t lo = __shfl(prev_row, from, kWave) + 1, hi = __shfl(row, from, kWave);
+            const int32_t v = (int32_t)__shfl(at, from, kWave);
+            for (int64_t r = lo + lane; r <= hi; r += kWave) offsets[r] = v;
+        }
+        const uint64_t ends = __ballot(tail && row < n);
+        if (ends) {
+            const int from = __ffsll((unsigned long long)ends) - 1;
+            const int64_t lo = __shfl(row, from, kWave) + 1;
+            const int32_t v = (int32_t)__shfl(at + (head ? 1 : 0), from, kWave);
+            for (int64_t r = lo + lane; r <= n; r += kWave) offsets[r] = v;
+        }
     }
 }
 
@@ -276,72 +321,101 @@ unsigned grid_for(int64_t n, int64_t cap = 16384) {
     return (unsigned)b;
 }
 
-// Sorted packed keys -> deduplicated CSR in g (sentinel keys dropped).
-b40c_status csr_from_sorted_keys(const uint64_t* keys, int64_t nkeys, int shift, uint64_t sentinel, int32_t n,
-                                 b40c_graph* g, hipStream_t stream) {
-    DeviceInfo info;
-    B40C_TRY(device_info(info));
-    int64_t G = (int64_t)info.num_cus * 4;
-    int64_t chunk = (nkeys + G - 1) / G;
-    if (chunk < 1) chunk = 1;
-    G = (nkeys + chunk - 1) / chunk;
-    if (G < 1) G = 1;
-    DeviceBuffer counts, total;
-    B40C_TRY(counts.alloc(G * sizeof(uint32_t)));
-    B40C_TRY(total.alloc(sizeof(uint32_t)));
-    hipLaunchKernelGGL(k_unique_count, dim3((unsigned)G), dim3(GB_THREADS), 0, stream, keys, nkeys, sentinel, chunk,
-                       counts.as<uint32_t>());
-    hipLaunchKernelGGL(k_scan_counts, dim3(1), dim3(GB_THREADS), 0, stream, counts.as<uint32_t>(), (int)G,
-                       total.as<uint32_t>());
-    B40C_HIP(hipGetLastError());
-    uint32_t E = 0;
-    B40C_HIP(hipMemcpyAsync(&E, total.ptr, sizeof(uint32_t), hipMemcpyDeviceToHost, stream));
-    B40C_HIP(hipStreamSynchronize(stream));
-    if ((int64_t)E > 0x7FFFFFFFll) return fail(B40C_ERR_UNSUPPORTED, "CSR with %u edges exceeds int32 offsets", E);
-    g->nodes = n;
-    g->edges = E;
-    DeviceBuffer rows;
-    B40C_TRY(g->cols.alloc((size_t)E * sizeof(int32_t)));
-    B40C_TRY(rows.alloc((size_t)E * sizeof(uint32_t)));
-    B40C_TRY(g->offsets.alloc(((size_t)n + 1) * sizeof(int32_t)));
-    hipLaunchKernelGGL(k_unique_scatter, dim3((unsigned)G), dim3(GB_THREADS), 0, stream, keys, nkeys, sentinel, chunk,
-                       counts.as<uint32_t>(), shift, g->cols.as<int32_t>(), rows.as<uint32_t>());
-    if (E == 0) {
-        B40C_HIP(hipMemsetAsync(g->offsets.ptr, 0, ((size_t)n + 1) * sizeof(int32_t), stream));
-    } else {
-        hipLaunchKernelGGL(k_row_offsets, dim3(grid_for(E)), dim3(GB_THREADS), 0, stream, rows.as<uint32_t>(),
-                           (int64_t)E, n, g->offsets.as<int32_t>());
+// Device memory of a packed-key build, one allocation: two key arrays, the
+// sort's scratch, and the chain words of the CSR pass (over the scratch, which
+// the sort no longer needs); `extra` bytes more for the caller.
+struct KeyArena {
+    DeviceBuffer mem;
+    uint64_t* k0 = nullptr;
+    uint64_t* k1 = nullptr;
+    uint32_t* scratch = nullptr;
+    size_t scratch_words = 0;
+    char* extra = nullptr;
+    b40c_status alloc(int64_t nkeys, size_t extra_bytes) {
+        auto up = [](size_t b) { return (b + 255) / 256 * 256; };
+        const size_t keys = up((size_t)std::max<int64_t>(nkeys, 1) * 8);
+        scratch_words = sort_scratch_words(std::max<int64_t>(nkeys, 1));
+        const size_t work = up(std::max(scratch_words * 4, chain_bytes((nkeys + CSR_BLOCK - 1) / CSR_BLOCK)));
+        B40C_TRY(mem.alloc(2 * keys + work + extra_bytes));
+        char* p = mem.as<char>();
+        k0 = reinterpret_cast<uint64_t*>(p);
+        k1 = reinterpret_cast<uint64_t*>(p + keys);
+        scratch = reinterpret_cast<uint32_t*>(p + 2 * keys);
+        extra = p + 2 * keys + work;
+        return B40C_OK;
     }
-    B40C_HIP(hipGetLastError());
-    B40C_HIP(hipStreamSynchronize(stream));
+    // Sorts k0 by bits [0, end_bit); afterwards k0 holds the result.
+    b40c_status sort(int64_t n, int end_bit, hipStream_t stream) {
+        int32_t sel = 0;
+        B40C_TRY(radix_sort_u64(k0, k1, n, 0, end_bit, &sel, stream, scratch, scratch_words));
+        if (sel) std::swap(k0, k1);
+        return B40C_OK;
+    }
+};
+
+// Sorted packed keys (a.k0) -> deduplicated CSR in g (sentinel keys dropped).
+// The columns are written over a.k1 and copied from there once their number is
+// known.
+b40c_status csr_from_sorted_keys(const KeyArena& a, int64_t nkeys, int shift, uint64_t sentinel, int32_t n,
+                                 b40c_graph* g, hipStream_t stream) {
+    B40C_TRY(g->offsets.alloc(((size_t)n + 1) * sizeof(int32_t)));
+    uint64_t E = 0;
+    if (nkeys == 0) {
+        B40C_TRY(fill_u32(g->offsets.as<uint32_t>(), 0, (size_t)n + 1, stream));
+        B40C_HIP(hipStreamSynchronize(stream));
+    } else {
+        const int64_t blocks = (nkeys + CSR_BLOCK - 1) / CSR_BLOCK;
+        ChainCall call;
+        B40C_TRY(call.start(blocks, stream, a.scratch));
+        hipLaunchKernelGGL(k_csr_chained, dim3((unsigned)blocks + 1), dim3(CHAIN_THREADS), 0, stream, a.k0, nkeys,
+                           shift, sentinel, n, reinterpret_cast<int32_t*>(a.k1), g->offsets.as<int32_t>(), call.chain,
+                           call.report);
+        B40C_TRY(call.finish("CSR build", E, stream));
+    }
+    if (E > 0x7FFFFFFFull)
+        return fail(B40C_ERR_UNSUPPORTED, "CSR with %llu edges exceeds int32 offsets", (unsigned long long)E);
+    g->nodes = n;
+    g->edges = (int64_t)E;
+    B40C_TRY(g->cols.alloc((size_t)E * sizeof(int32_t)));
+    if (E) {
+        B40C_HIP(hipMemcpyAsync(g->cols.ptr, a.k1, (size_t)E * sizeof(int32_t), hipMemcpyDeviceToDevice, stream));
+        B40C_HIP(hipStreamSynchronize(stream));
+    }
     return B40C_OK;
 }
 
 // COO edge e -> packed key (row << shift) | col, plus its reverse at m + e
-// when symmetrizing; dropped self-loops become the sentinel.
+// when symmetrizing; dropped self-loops become the sentinel.  Edges with an id
+// outside [0, n) are dropped too and raise *bad.
 __global__ __launch_bounds__(GB_THREADS) void k_pack_coo(const int32_t* rows, const int32_t* cols, int64_t m,
-                                                         int shift, int drop_loops, int symmetrize, uint64_t sentinel,
-                                                         uint64_t* keys) {
+                                                         uint32_t n, int shift, int drop_loops, int symmetrize,
+                                                         uint64_t sentinel, uint64_t* keys, uint32_t* bad) {
     for (int64_t e = (int64_t)blockIdx.x * GB_THREADS + threadIdx.x; e < m; e += (int64_t)gridDim.x * GB_THREADS) {
         const uint64_t r = (uint32_t)rows[e], c = (uint32_t)cols[e];
-        const bool loop = drop_loops && r == c;
-        keys[e] = loop ? sentinel : ((r << shift) | c);
-        if (symmetrize) keys[m + e] = loop ? sentinel : ((c << shift) | r);
+        const bool outside = r >= n || c >= n;
+        const bool drop = outside || (drop_loops && r == c);
+        if (outside) *bad = 1;
+        keys[e] = drop ? sentinel : ((r << shift) | c);
+        if (symmetrize) keys[m + e] = drop ? sentinel : ((c << shift) | r);
     }
+}
+
+b40c_status check_coo_ids(int32_t n, int64_t m, const int32_t* rows, const int32_t* cols) {
+    for (int64_t e = 0; e < m; ++e)
+        if (rows[e] < 0 || rows[e] >= n || cols[e] < 0 || cols[e] >= n)
+            return fail(B40C_ERR_INVALID_ARG, "from_coo_unique: edge %lld (%d,%d) out of range [0,%d)",
+                        (long long)e, rows[e], cols[e], n);
+    return B40C_OK;
 }
 
 // COO -> CSR with sorted, unique columns per row: pack, GPU radix sort of the
 // packed keys, consecutive removal, row offsets (the steps around the sort
 // that the reference does with consecutive_removal::Enactor::Trim and
-// scan::Enactor::Scan).
-b40c_status build_from_coo_unique(int32_t n, int64_t m, const int32_t* rows, const int32_t* cols, int32_t flags,
-                                  b40c_graph* g) {
-    if (n < 1 || m < 0 || (m > 0 && (!rows || !cols)) || (flags & ~(B40C_COO_DROP_SELF_LOOPS | B40C_COO_SYMMETRIZE)))
-        return fail(B40C_ERR_INVALID_ARG, "from_coo_unique: bad arguments");
-    for (int64_t e = 0; e < m; ++e)
-        if (rows[e] < 0 || rows[e] >= n || cols[e] < 0 || cols[e] >= n)
-            return fail(B40C_ERR_INVALID_ARG, "from_coo_unique: edge %lld (%d,%d) out of range [0,%d)",
-                        (long long)e, rows[e], cols[e], n);
+// scan::Enactor::Scan).  The ids are checked where they are packed (a host loop
+// over 1 M edges took 275 us); the host looks for the edge to name only if one
+// is outside, or if the device could not say.
+b40c_status build_from_coo_unique_on_device(int32_t n, int64_t m, const int32_t* rows, const int32_t* cols,
+                                            int32_t flags, b40c_graph* g, bool& checked) {
     const bool sym = (flags & B40C_COO_SYMMETRIZE) != 0;
     const int64_t nkeys = sym ? 2 * m : m;
     if (nkeys > 0xFFFFFFFFll) return fail(B40C_ERR_UNSUPPORTED, "from_coo_unique: %lld keys exceed the sorter",
@@ -349,25 +423,48 @@ b40c_status build_from_coo_unique(int32_t n, int64_t m, const int32_t* rows, con
     hipStream_t stream = nullptr;
     const int shift = std::max(1, ceil_log2_u64((uint64_t)n));
     const uint64_t sentinel = 1ull << (2 * shift);  // above every real key
-    DeviceBuffer r_d, c_d, k0, k1;
-    B40C_TRY(r_d.alloc((size_t)std::max<int64_t>(m, 1) * 4));
-    B40C_TRY(c_d.alloc((size_t)std::max<int64_t>(m, 1) * 4));
-    B40C_TRY(k0.alloc((size_t)std::max<int64_t>(nkeys, 1) * 8));
-    B40C_TRY(k1.alloc((size_t)std::max<int64_t>(nkeys, 1) * 8));
+    ReportSlot bad;
+    KeyArena a;
+    B40C_TRY(a.alloc(nkeys, (size_t)m * 8 + 4));
+    int32_t* r_d = reinterpret_cast<int32_t*>(a.extra);
+    int32_t* c_d = r_d + m;
     if (m > 0) {
-        B40C_HIP(hipMemcpy(r_d.ptr, rows, (size_t)m * 4, hipMemcpyHostToDevice));
-        B40C_HIP(hipMemcpy(c_d.ptr, cols, (size_t)m * 4, hipMemcpyHostToDevice));
-        hipLaunchKernelGGL(k_pack_coo, dim3(grid_for(m)), dim3(GB_THREADS), 0, stream, r_d.as<int32_t>(),
-                           c_d.as<int32_t>(), m, shift, (flags & B40C_COO_DROP_SELF_LOOPS) ? 1 : 0, sym ? 1 : 0,
-                           sentinel, k0.as<uint64_t>());
+        const bool pinned = bad.take();
+        if (!pinned) {
+            checked = true;
+            B40C_TRY(check_coo_ids(n, m, rows, cols));
+        }
+        B40C_HIP(hipMemcpy(r_d, rows, (size_t)m * 4, hipMemcpyHostToDevice));
+        B40C_HIP(hipMemcpy(c_d, cols, (size_t)m * 4, hipMemcpyHostToDevice));
+        hipLaunchKernelGGL(k_pack_coo, dim3(grid_for(m)), dim3(GB_THREADS), 0, stream, r_d, c_d, m, (uint32_t)n, shift,
+                           (flags & B40C_COO_DROP_SELF_LOOPS) ? 1 : 0, sym ? 1 : 0, sentinel, a.k0,
+                           pinned ? static_cast<uint32_t*>(bad.dev) : reinterpret_cast<uint32_t*>(c_d + m));
         B40C_HIP(hipGetLastError());
+        B40C_TRY(a.sort(nkeys, 2 * shift + 1, stream));
     }
-    int32_t sel = 0;
-    if (nkeys > 0) B40C_TRY(radix_sort_u64(k0.as<uint64_t>(), k1.as<uint64_t>(), nkeys, 0, 2 * shift + 1, &sel, stream));
-    const uint64_t* sorted = sel ? k1.as<uint64_t>() : k0.as<uint64_t>();
-    B40C_TRY(csr_from_sorted_keys(sorted, nkeys, shift, sentinel, n, g, stream));
+    B40C_TRY(csr_from_sorted_keys(a, nkeys, shift, sentinel, n, g, stream));
+    if (bad.host) {
+        uint32_t outside = 0;
+        std::memcpy(&outside, bad.host, sizeof(outside));
+        checked = outside == 0;
+        if (!checked) return fail(B40C_ERR_INVALID_ARG, "from_coo_unique: an edge is out of range [0,%d)", n);
+    }
     if (sym) g->symmetric.store(1);
     return B40C_OK;
+}
+
+b40c_status build_from_coo_unique(int32_t n, int64_t m, const int32_t* rows, const int32_t* cols, int32_t flags,
+                                  b40c_graph* g) {
+    if (n < 1 || m < 0 || (m > 0 && (!rows || !cols)) || (flags & ~(B40C_COO_DROP_SELF_LOOPS | B40C_COO_SYMMETRIZE)))
+        return fail(B40C_ERR_INVALID_ARG, "from_coo_unique: bad arguments");
+    bool checked = false;
+    const b40c_status s = build_from_coo_unique_on_device(n, m, rows, cols, flags, g, checked);
+    if (s != B40C_OK && !checked) {
+        const std::string why = b40c_last_error_string();
+        B40C_TRY(check_coo_ids(n, m, rows, cols));
+        return fail(s, "%s", why.c_str());
+    }
+    return s;
 }
 
 b40c_status build_rmat(int scale, int edge_factor, double a, double b, double c, uint64_t seed, b40c_graph* g) {
@@ -379,18 +476,14 @@ b40c_status build_rmat(int scale, int edge_factor, double a, double b, double c,
     const int64_t nkeys = 2 * m;
     if (nkeys > 0xFFFFFFFFll) return fail(B40C_ERR_UNSUPPORTED, "rmat: %lld keys exceed the sorter", (long long)nkeys);
     hipStream_t stream = nullptr;
-    DeviceBuffer k0, k1;
-    B40C_TRY(k0.alloc((size_t)nkeys * sizeof(uint64_t)));
-    B40C_TRY(k1.alloc((size_t)nkeys * sizeof(uint64_t)));
+    KeyArena arena;
+    B40C_TRY(arena.alloc(nkeys, 0));
     const uint64_t sentinel = (scale * 2 >= 64) ? ~0ull : ((1ull << (2 * scale)) - 1);
     hipLaunchKernelGGL(k_rmat_keys, dim3(grid_for(m)), dim3(GB_THREADS), 0, stream, scale, m, prob_threshold(a),
-                       prob_threshold(a + b), prob_threshold(a + b + c), splitmix64(seed), k0.as<uint64_t>(),
-                       sentinel);
+                       prob_threshold(a + b), prob_threshold(a + b + c), splitmix64(seed), arena.k0, sentinel);
     B40C_HIP(hipGetLastError());
-    int32_t sel = 0;
-    B40C_TRY(radix_sort_u64(k0.as<uint64_t>(), k1.as<uint64_t>(), nkeys, 0, 2 * scale, &sel, stream));
-    const uint64_t* sorted = sel ? k1.as<uint64_t>() : k0.as<uint64_t>();
-    B40C_TRY(csr_from_sorted_keys(sorted, nkeys, scale, sentinel, n, g, stream));
+    B40C_TRY(arena.sort(nkeys, 2 * scale, stream));
+    B40C_TRY(csr_from_sorted_keys(arena, nkeys, scale, sentinel, n, g, stream));
     g->symmetric.store(1);  // both directions of every sampled edge were emitted
     return B40C_OK;
 }
@@ -403,23 +496,21 @@ b40c_status build_lattice(int w, uint64_t seed, int32_t* h_perm, b40c_graph* g) 
     const uint64_t lowmask = (1ull << bits) - 1;
     hipStream_t stream = nullptr;
     const int64_t nkeys = 6 * n;
-    DeviceBuffer k0, k1, perm;
-    B40C_TRY(k0.alloc((size_t)nkeys * sizeof(uint64_t)));
-    B40C_TRY(k1.alloc((size_t)nkeys * sizeof(uint64_t)));
+    DeviceBuffer perm;
+    KeyArena arena;
+    B40C_TRY(arena.alloc(nkeys, 0));
     B40C_TRY(perm.alloc((size_t)n * sizeof(int32_t)));
     hipLaunchKernelGGL(k_perm_keys, dim3(grid_for(n)), dim3(GB_THREADS), 0, stream, n, lowmask, splitmix64(seed),
-                       k0.as<uint64_t>());
-    int32_t sel = 0;
-    B40C_TRY(radix_sort_u64(k0.as<uint64_t>(), k1.as<uint64_t>(), n, 0, 64, &sel, stream));
-    hipLaunchKernelGGL(k_perm_from_sorted, dim3(grid_for(n)), dim3(GB_THREADS), 0, stream,
-                       sel ? k1.as<uint64_t>() : k0.as<uint64_t>(), n, lowmask, perm.as<int32_t>());
+                       arena.k0);
+    B40C_TRY(arena.sort(n, 64, stream));
+    hipLaunchKernelGGL(k_perm_from_sorted, dim3(grid_for(n)), dim3(GB_THREADS), 0, stream, arena.k0, n, lowmask,
+                       perm.as<int32_t>());
     const uint64_t sentinel = (1ull << (2 * bits)) - 1;
     hipLaunchKernelGGL(k_lattice_keys, dim3(grid_for(n)), dim3(GB_THREADS), 0, stream, w, perm.as<int32_t>(), bits,
-                       k0.as<uint64_t>(), sentinel);
+                       arena.k0, sentinel);
     B40C_HIP(hipGetLastError());
-    B40C_TRY(radix_sort_u64(k0.as<uint64_t>(), k1.as<uint64_t>(), nkeys, 0, 2 * bits, &sel, stream));
-    B40C_TRY(csr_from_sorted_keys(sel ? k1.as<uint64_t>() : k0.as<uint64_t>(), nkeys, bits, sentinel, (int32_t)n, g,
-                                  stream));
+    B40C_TRY(arena.sort(nkeys, 2 * bits, stream));
+    B40C_TRY(csr_from_sorted_keys(arena, nkeys, bits, sentinel, (int32_t)n, g, stream));
     if (h_perm) B40C_HIP(hipMemcpy(h_perm, perm.ptr, (size_t)n * sizeof(int32_t), hipMemcpyDeviceToHost));
     g->symmetric.store(1);  // every lattice edge is emitted from both endpoints
     return B40C_OK;

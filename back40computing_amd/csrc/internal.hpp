@@ -71,8 +71,9 @@ struct SortPolicy {
 SortPolicy resolve_sort_policy(SortPolicy p, int64_t n, int pair_bytes, int num_cus);
 // Words of scratch a sort of n keys wants.
 size_t sort_scratch_words(int64_t n);
+// With `scratch` null, or less than sort_scratch_words(n), it is allocated for the call.
 b40c_status radix_sort_u64(uint64_t* k0, uint64_t* k1, int64_t n, int begin_bit, int end_bit, int32_t* selector,
-                           hipStream_t stream);
+                           hipStream_t stream, uint32_t* scratch = nullptr, size_t scratch_words = 0);
 b40c_status radix_sort_pairs_u32(uint32_t* k0, uint32_t* k1, uint32_t* v0, uint32_t* v1, int64_t n, int begin_bit,
                                  int end_bit, int32_t* selector, hipStream_t stream);
 

@@ -777,9 +777,11 @@ static b40c_status radix_sort_sync(int32_t key_type, void* k0, void* k1, uint32_
     return B40C_OK;
 }
 
-// Stateless form: scratch allocated for this call.
+// Stateless form: with the caller's scratch if it is large enough, else
+// allocated for this call.
 b40c_status radix_sort_once(int32_t key_type, void* k0, void* k1, uint32_t* v0, uint32_t* v1, int64_t n, int begin_bit,
-                            int end_bit, int32_t* selector, hipStream_t stream) {
+                            int end_bit, int32_t* selector, hipStream_t stream, uint32_t* scratch = nullptr,
+                            size_t scratch_words = 0) {
     *selector = 0;
     if (n <= 1 || begin_bit == end_bit) return B40C_OK;
     DeviceInfo info;
@@ -787,15 +789,20 @@ b40c_status radix_sort_once(int32_t key_type, void* k0, void* k1, uint32_t* v0, 
     DeviceBuffer mem;
     const SortPolicy pol = resolve_sort_policy(SortPolicy{}, n, key_bits(key_type) / 8 + (v0 ? 4 : 0), info.num_cus);
     const size_t words = sort_scratch_words(n);
-    B40C_TRY(mem.alloc(words * sizeof(uint32_t)));
+    if (!scratch || scratch_words < words) {
+        B40C_TRY(mem.alloc(words * sizeof(uint32_t)));
+        scratch = mem.as<uint32_t>();
+        scratch_words = words;
+    }
     return radix_sort_sync(key_type, k0, k1, v0, v1, n, begin_bit, end_bit, info.num_cus, pol,
-                           SortScratch{mem.as<uint32_t>(), words}, selector, stream);
+                           SortScratch{scratch, scratch_words}, selector, stream);
 }
 
 b40c_status radix_sort_u64(uint64_t* k0, uint64_t* k1, int64_t n, int begin_bit, int end_bit, int32_t* selector,
-                           hipStream_t stream) {
+                           hipStream_t stream, uint32_t* scratch_mem, size_t scratch_words) {
     B40C_TRY(validate("radix sort", B40C_KEY_U64, k0, k1, nullptr, nullptr, n, begin_bit, end_bit, selector));
-    return radix_sort_once(B40C_KEY_U64, k0, k1, nullptr, nullptr, n, begin_bit, end_bit, selector, stream);
+    return radix_sort_once(B40C_KEY_U64, k0, k1, nullptr, nullptr, n, begin_bit, end_bit, selector, stream, scratch_mem,
+                           scratch_words);
 }
 
 b40c_status radix_sort_pairs_u32(uint32_t* k0, uint32_t* k1, uint32_t* v0, uint32_t* v1, int64_t n, int begin_bit,
