@@ -94,3 +94,27 @@ def test_paths_against_oracle(orc, name):
                 assert autotune.verify_bfs_labels(off, cols, src, depth, pred, edge_keys, depth_verified=True)
                 assert st["search_depth"] == int(ref.max()) + 1
     g.close()
+
+
+@pytest.mark.parametrize("edges", [(1 << 19) - 2, 1 << 19])
+def test_default_grid_tier_line(orc, edges):
+    """Both sides of the number of edges from which lists of 128 edges go to
+    the grid tier, with lists of 127, 128 and 129 edges and a few longer ones."""
+    from back40computing_amd import autotune, bfs
+    rng = np.random.default_rng(edges)
+    n = 6000
+    deg = np.concatenate([[400, 127, 128, 129, 2047, 2048, 2049, 5000], rng.choice([0, 1, 60, 127, 128, 129], n)])
+    deg = np.concatenate([deg, np.full(n, (edges - int(deg.sum())) // n)])
+    deg[-1] += edges - int(deg.sum())
+    off = np.concatenate([[0], np.cumsum(deg)]).astype(np.int32)
+    assert off[-1] == edges
+    cols = rng.integers(0, deg.size, edges).astype(np.int32)
+    g = bfs.Graph.from_host_csr(off, cols)
+    edge_keys = autotune.sorted_edge_keys(off, cols)
+    ref = orc.bfs(off, cols, 0, with_pred=False)[0]
+    for strategy, mode in FORMS:
+        print("grid tier line", edges, strategy, mode, flush=True)
+        depth, pred, st = bfs.bfs(g, 0, strategy=strategy, mode=mode)
+        np.testing.assert_array_equal(depth, ref)
+        assert autotune.verify_bfs_labels(off, cols, 0, depth, pred, edge_keys, depth_verified=True)
+    g.close()
