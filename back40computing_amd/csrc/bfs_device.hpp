@@ -48,7 +48,8 @@ struct BfsArgs {
     DevCounters* ctr;
     uint32_t* bar_arrive;    // persistent kernels: grid-barrier arrival word per workgroup
     unsigned long long* bar_words;  // ... of the all-to-all barrier, [2][kAllToAllMax]
-    int32_t* regions;        // narrow persistent kernel: frontier pieces, [2][kAllToAllMax][REGION]
+    int32_t* regions;        // narrow persistent kernel: frontier pieces, [2][kAllToAllMax][region]
+    uint32_t region;         // entries of a piece
     DevCounters* hctr;       // device address of the pinned host mirror of *ctr
     uint32_t* max_depth;     // deepest depth label written
     unsigned long long* wg_stats;  // instrumented: [grid][2] (busy clocks, lifetime clocks)
@@ -115,7 +116,6 @@ __device__ __forceinline__ int2 coh_ld2(const int2* p, bool coh) {
     return make_int2((int32_t)(uint32_t)w, (int32_t)(uint32_t)(w >> 32));
 }
 
-constexpr int REGION = 4096;       // frontier entries a workgroup of the narrow persistent kernel keeps in its own piece
 constexpr int HEAVY_CHUNK = 256;     // most grid-tier edges per work item
 
 // ---------------------------------------------------------------------------

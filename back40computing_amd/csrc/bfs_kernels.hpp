@@ -1274,7 +1274,7 @@ constexpr uint32_t kNarrowSpilled = 0x40000000u, kNarrowDeferred = 0x80000000u, 
 struct NarrowSink {
     const BfsArgs& a;
     NarrowShared& s;
-    int32_t* piece;  // REGION entries
+    int32_t* piece;  // a.region entries
     const GlobalQueue& out;
     int32_t depth_next;
     __device__ __forceinline__ void reserve(uint32_t, ListSmem&) {}
@@ -1295,9 +1295,9 @@ struct NarrowSink {
         uint32_t base = 0;
         if (lane_id() == 0) base = atomicAdd(&s.count, cnt);
         base = (uint32_t)wave_bcast((int)base, 0);
-        const uint32_t spill_start = base > (uint32_t)REGION ? base : (uint32_t)REGION;
+        const uint32_t spill_start = base > a.region ? base : a.region;
         uint32_t gb = 0;
-        if (base + cnt > (uint32_t)REGION) {
+        if (base + cnt > a.region) {
             if (lane_id() == 0) {
                 gb = atomic_add_u32(out.len, base + cnt - spill_start);
                 s.spilled = 1u;
@@ -1310,7 +1310,7 @@ struct NarrowSink {
             const uint32_t pos = at + (uint32_t)lane_prefix(m[r]);
             at += (uint32_t)__popcll(m[r]);
             if (!won[r]) continue;
-            if (pos < (uint32_t)REGION) {
+            if (pos < a.region) {
                 coh_st(&piece[pos], v[r], true);
             } else if (gb + (pos - spill_start) < out.cap) {
                 coh_st(&out.keys[gb + (pos - spill_start)], v[r], true);
@@ -1346,9 +1346,9 @@ __device__ void fused_narrow_body(const BfsArgs& a, int ph, int32_t depth, Narro
         if (threadIdx.x == 0) s.count = s.spilled = s.deferred = 0u;
         __syncthreads();  // also: `first` is complete
         const int32_t* qin = a.qk[ph & 1];
-        const int32_t* pieces = a.regions + (size_t)(ph & 1) * kAllToAllMax * REGION;
+        const int32_t* pieces = a.regions + (size_t)(ph & 1) * kAllToAllMax * a.region;
         const GlobalQueue out = out_queue(a, ph);
-        NarrowSink sink{a, s, a.regions + ((size_t)((ph + 1) & 1) * kAllToAllMax + blockIdx.x) * REGION, out,
+        NarrowSink sink{a, s, a.regions + ((size_t)((ph + 1) & 1) * kAllToAllMax + blockIdx.x) * a.region, out,
                         depth + 1};
         const Deal deal = deal_out(n_in, gridDim.x, false);
         for (uint32_t base = 0; base < n_in; base += gridDim.x * BFS_THREADS) {
@@ -1363,7 +1363,7 @@ __device__ void fused_narrow_body(const BfsArgs& a, int ph, int32_t depth, Narro
 #pragma unroll
                     for (uint32_t h = kAllToAllMax / 2; h >= 1; h >>= 1)
                         if (s.first[w + h] <= j) w += h;
-                    u = coh_ld(&pieces[w * (uint32_t)REGION + (j - s.first[w])], true);
+                    u = coh_ld(&pieces[w * a.region + (j - s.first[w])], true);
                 }
                 if (valid_vertex(a, u)) {
                     start = a.offs[u];
@@ -1382,7 +1382,7 @@ __device__ void fused_narrow_body(const BfsArgs& a, int ph, int32_t depth, Narro
         if (a.wg_stats && threadIdx.x == 0) busy += wg_clock() - tb;
         uint32_t word = 0;
         auto mine = [&] {
-            return min(s.count, (uint32_t)REGION) | (s.spilled ? kNarrowSpilled : 0u) |
+            return min(s.count, a.region) | (s.spilled ? kNarrowSpilled : 0u) |
                    (s.deferred ? kNarrowDeferred : 0u);
         };
         if (!grid_sync_words(a.bar_words, &a.ctr->bar_abort, ++epoch, mine(), word)) break;
