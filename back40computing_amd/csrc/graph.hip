@@ -321,11 +321,13 @@ unsigned grid_for(int64_t n, int64_t cap = 16384) {
     return (unsigned)b;
 }
 
-// Device memory of a packed-key build, one allocation: two key arrays, the
-// sort's scratch, and the chain words of the CSR pass (over the scratch, which
-// the sort no longer needs); `extra` bytes more for the caller.
+// Device memory of a packed-key build: two key arrays, the sort's scratch, and
+// the chain words of the CSR pass (over the scratch, which the sort no longer
+// needs); `extra` bytes more for the caller.  One allocation, except that
+// arrays of at most 1 MB are allocated one by one: the runtime serves those from
+// chunks it keeps (1 us each), and larger ones by mapping memory (20 to 130 us).
 struct KeyArena {
-    DeviceBuffer mem;
+    DeviceBuffer mem, small[3];
     uint64_t* k0 = nullptr;
     uint64_t* k1 = nullptr;
     uint32_t* scratch = nullptr;
@@ -336,6 +338,17 @@ struct KeyArena {
         const size_t keys = up((size_t)std::max<int64_t>(nkeys, 1) * 8);
         scratch_words = sort_scratch_words(std::max<int64_t>(nkeys, 1));
         const size_t work = up(std::max(scratch_words * 4, chain_bytes((nkeys + CSR_BLOCK - 1) / CSR_BLOCK)));
+        if (std::max(std::max(keys, work), extra_bytes) <= (1u << 20)) {
+            B40C_TRY(mem.alloc(keys));
+            B40C_TRY(small[0].alloc(keys));
+            B40C_TRY(small[1].alloc(work));
+            B40C_TRY(small[2].alloc(extra_bytes));
+            k0 = mem.as<uint64_t>();
+            k1 = small[0].as<uint64_t>();
+            scratch = small[1].as<uint32_t>();
+            extra = small[2].as<char>();
+            return B40C_OK;
+        }
         B40C_TRY(mem.alloc(2 * keys + work + extra_bytes));
         char* p = mem.as<char>();
         k0 = reinterpret_cast<uint64_t*>(p);
