@@ -282,9 +282,9 @@ def tune_and_record(graph, strategy, sources, path=TABLE_PATH, log=None, **kw):
 
 
 # Radix-sort policies (b40c_sort_enactor_set_policy): keys per thread of a
-# downsweep tile and workgroups per CU, the run-time form of the reference's
+# tile and workgroups per CU (0: a block per tile), the run-time form of the reference's
 # per-architecture sort policies (radix_sort/autotuned_policy.cuh:190-230).
-SORT_SPACE = [(items, wgs) for items in (8, 16) for wgs in (1, 2, 3, 4, 6, 8)]
+SORT_SPACE = [(items, wgs) for items in (8, 16) for wgs in (0, 1, 2, 3, 4, 6, 8)]
 
 SORT_KEY_DTYPES = {"u32": np.uint32, "i32": np.int32, "f32": np.float32, "u64": np.uint64, "i64": np.int64,
                    "f64": np.float64}
