@@ -48,16 +48,12 @@ SPACE = {
 
 # Knobs that matter per strategy.
 KNOBS = {
-    _lib.EXPAND_CONTRACT: ["persistent_wgs_per_cu", "grid_gather_threshold", "cta_gather_threshold",
-                           "wave_gather_threshold", "grid_size", "levels_per_sync"],
-    _lib.CONTRACT_EXPAND: ["persistent_wgs_per_cu", "grid_gather_threshold", "cta_gather_threshold",
-                           "wave_gather_threshold", "grid_size", "levels_per_sync"],
-    _lib.TWO_PHASE: ["persistent_wgs_per_cu", "grid_gather_threshold", "cta_gather_threshold",
-                     "wave_gather_threshold", "grid_size", "levels_per_sync"],
-    _lib.HYBRID: ["saturation_quit", "persistent_wgs_per_cu", "grid_gather_threshold", "cta_gather_threshold",
-                  "wave_gather_threshold", "grid_size"],
+    _lib.EXPAND_CONTRACT: ["persistent_wgs_per_cu", "grid_gather_threshold", "grid_size", "levels_per_sync"],
+    _lib.CONTRACT_EXPAND: ["persistent_wgs_per_cu", "grid_gather_threshold", "grid_size", "levels_per_sync"],
+    _lib.TWO_PHASE: ["persistent_wgs_per_cu", "grid_gather_threshold", "grid_size", "levels_per_sync"],
+    _lib.HYBRID: ["saturation_quit", "persistent_wgs_per_cu", "grid_gather_threshold", "grid_size"],
     _lib.DIRECTION_OPTIMIZING: ["bottom_up_grid_size", "do_alpha", "do_beta", "grid_gather_threshold",
-                                "grid_size", "levels_per_sync", "wave_gather_threshold"],
+                                "grid_size", "levels_per_sync"],
 }
 
 

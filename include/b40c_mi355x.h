@@ -68,8 +68,8 @@ typedef struct b40c_enactor b40c_enactor;
  * default / autotuned". */
 typedef struct b40c_tuning {
     int32_t grid_size;             /* workgroups per level launch (0: 4 x CUs)              */
-    int32_t cta_gather_threshold;  /* degree >= this: whole-workgroup gather                */
-    int32_t wave_gather_threshold; /* degree >= this: whole-wavefront gather                */
+    int32_t cta_gather_threshold;  /* kept for callers that set it; lists below the grid tier  */
+    int32_t wave_gather_threshold; /* are gathered by edge position whatever their degree       */
     int32_t levels_per_sync;       /* iterative enactors: levels launched between host checks */
     int32_t saturation_quit;       /* hybrid: fused kernel quits when frontier > grid * this */
     int32_t do_alpha;              /* direction-optimizing: switch to bottom-up when m_f > m_u / alpha */
