@@ -55,6 +55,8 @@ struct BfsArgs {
     unsigned long long* wg_stats;  // instrumented: [grid][2] (busy clocks, lifetime clocks)
     int32_t n;
     int32_t words;           // ceil(n / 32)
+    int32_t cta_th;          // set by callers that drive the bodies themselves; no body reads them
+    int32_t wave_th;
     int32_t grid_th;         // degree >= this: grid tier (split across workgroups)
     int32_t symmetric;       // graph has every reverse edge (bottom-up allowed)
     int32_t do_alpha;
