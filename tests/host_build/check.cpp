@@ -1,0 +1,408 @@
+// Checks of the library's own entry points on the host build (test
+// infrastructure only): check CASE [ARGUMENT...].  Each case prints what it runs
+// and exits 0 if everything held; results are compared with the serial
+// references below.
+#include <hip/hip_runtime.h>
+
+#include <algorithm>
+#include <cstdarg>
+#include <random>
+#include <set>
+
+#include "b40c_mi355x.h"
+
+namespace {
+
+[[noreturn]] void die(const char* fmt, ...) {
+    va_list ap;
+    va_start(ap, fmt);
+    std::fprintf(stderr, "check failed: ");
+    std::vfprintf(stderr, fmt, ap);
+    std::fprintf(stderr, " [last error: %s]\n", b40c_last_error_string());
+    va_end(ap);
+    std::fflush(nullptr);
+    _Exit(1);
+}
+#define REQUIRE(cond, ...)                                        \
+    do {                                                          \
+        if (!(cond)) {                                            \
+            std::fprintf(stderr, "%s:%d: ", __FILE__, __LINE__);  \
+            die(__VA_ARGS__);                                     \
+        }                                                         \
+    } while (0)
+#define OK(expr)                                                                \
+    do {                                                                        \
+        const b40c_status s_ = (expr);                                          \
+        REQUIRE(s_ == B40C_OK, "%s returned %d", #expr, (int)s_);               \
+    } while (0)
+
+// ---- graphs -----------------------------------------------------------------
+
+struct HostGraph {
+    std::string name;
+    int32_t n = 0;
+    std::vector<int32_t> off, cols;
+    int64_t m() const { return (int64_t)cols.size(); }
+};
+
+HostGraph make_graph(const std::string& name, int32_t n, std::vector<std::pair<int32_t, int32_t>> edges, bool undirected) {
+    if (undirected) {
+        const size_t k = edges.size();
+        for (size_t i = 0; i < k; ++i) edges.emplace_back(edges[i].second, edges[i].first);
+    }
+    std::sort(edges.begin(), edges.end());
+    edges.erase(std::unique(edges.begin(), edges.end()), edges.end());
+    HostGraph g;
+    g.name = name;
+    g.n = n;
+    g.off.assign((size_t)n + 1, 0);
+    for (auto& e : edges) ++g.off[(size_t)e.first + 1];
+    for (int32_t v = 0; v < n; ++v) g.off[(size_t)v + 1] += g.off[(size_t)v];
+    for (auto& e : edges) g.cols.push_back(e.second);
+    return g;
+}
+
+HostGraph path_graph(int32_t n) {
+    std::vector<std::pair<int32_t, int32_t>> e;
+    for (int32_t v = 0; v + 1 < n; ++v) e.emplace_back(v, v + 1);
+    return make_graph("path" + std::to_string(n), n, e, true);
+}
+HostGraph star_graph(int32_t leaves) {
+    std::vector<std::pair<int32_t, int32_t>> e;
+    for (int32_t v = 1; v <= leaves; ++v) e.emplace_back(0, v);
+    return make_graph("star" + std::to_string(leaves), leaves + 1, e, true);
+}
+// A skewed graph of 2^scale vertices: ids drawn bit by bit with P(0) = 0.7.
+HostGraph skewed_graph(int scale, int factor, bool undirected, unsigned seed) {
+    std::mt19937 rng(seed);
+    std::bernoulli_distribution one(0.3);
+    std::vector<std::pair<int32_t, int32_t>> e;
+    for (int i = 0; i < factor << scale; ++i) {
+        int32_t a = 0, b = 0;
+        for (int k = 0; k < scale; ++k) {
+            a = a * 2 + (one(rng) ? 1 : 0);
+            b = b * 2 + (one(rng) ? 1 : 0);
+        }
+        if (a != b) e.emplace_back(a, b);
+    }
+    return make_graph((undirected ? "skewed" : "directed") + std::to_string(scale), 1 << scale, e, undirected);
+}
+HostGraph grid_graph(int32_t w) {
+    std::vector<std::pair<int32_t, int32_t>> e;
+    auto id = [&](int x, int y, int z) { return (int32_t)(((z * w + y) * w + x) * 2654435761ull % (uint64_t)(w * w * w)); };
+    std::set<int32_t> seen;
+    for (int z = 0; z < w; ++z)
+        for (int y = 0; y < w; ++y)
+            for (int x = 0; x < w; ++x) {
+                seen.insert(id(x, y, z));
+                if (x + 1 < w) e.emplace_back(id(x, y, z), id(x + 1, y, z));
+                if (y + 1 < w) e.emplace_back(id(x, y, z), id(x, y + 1, z));
+                if (z + 1 < w) e.emplace_back(id(x, y, z), id(x, y, z + 1));
+            }
+    REQUIRE((int32_t)seen.size() == w * w * w, "grid ids collide");
+    return make_graph("grid" + std::to_string(w), w * w * w, e, true);
+}
+
+std::vector<int32_t> serial_bfs(const HostGraph& g, int32_t src) {
+    std::vector<int32_t> d((size_t)g.n, -1), q{src};
+    d[(size_t)src] = 0;
+    for (size_t h = 0; h < q.size(); ++h)
+        for (int32_t i = g.off[(size_t)q[h]]; i < g.off[(size_t)q[h] + 1]; ++i)
+            if (d[(size_t)g.cols[(size_t)i]] < 0) {
+                d[(size_t)g.cols[(size_t)i]] = d[(size_t)q[h]] + 1;
+                q.push_back(g.cols[(size_t)i]);
+            }
+    return d;
+}
+
+struct DeviceGraph {
+    b40c_graph* g = nullptr;
+    explicit DeviceGraph(const HostGraph& h) { OK(b40c_graph_from_host_csr(h.n, h.m(), h.off.data(), h.cols.data(), &g)); }
+    ~DeviceGraph() { b40c_graph_destroy(g); }
+};
+struct Problem {
+    b40c_problem* p = nullptr;
+    explicit Problem(b40c_graph* g) { OK(b40c_problem_create_from_graph(g, 0, &p)); }
+    ~Problem() { b40c_problem_destroy(p); }
+};
+struct Enactor {
+    b40c_enactor* e = nullptr;
+    explicit Enactor(int32_t strategy, const b40c_tuning* t = nullptr, int32_t instrument = 0) {
+        OK(b40c_enactor_create(strategy, instrument, &e));
+        if (t) OK(b40c_enactor_set_tuning(e, t));
+    }
+    ~Enactor() { b40c_enactor_destroy(e); }
+};
+
+const char* kStrategies[] = {"expand-contract", "contract-expand", "two-phase", "hybrid", "persistent", "direction-optimizing"};
+
+// Reset and search; labels, predecessors and search depth against the serial search.
+void search(const HostGraph& h, b40c_problem* p, b40c_enactor* e, int32_t src, int32_t mode) {
+    OK(b40c_problem_reset(p, b40c_enactor_frontier_type(e), 1.3));
+    OK(b40c_enact_search(e, p, src, 0, mode));
+    std::vector<int32_t> depth((size_t)h.n), pred((size_t)h.n);
+    OK(b40c_problem_extract(p, depth.data(), pred.data()));
+    const std::vector<int32_t> want = serial_bfs(h, src);
+    int32_t deepest = 0;
+    for (int32_t v = 0; v < h.n; ++v) {
+        REQUIRE(depth[(size_t)v] == want[(size_t)v], "%s source %d: depth[%d] is %d, not %d", h.name.c_str(), src, v,
+                depth[(size_t)v], want[(size_t)v]);
+        deepest = std::max(deepest, want[(size_t)v]);
+        const int32_t u = pred[(size_t)v];
+        if (v == src || want[(size_t)v] < 0) {
+            REQUIRE(u == (v == src ? -2 : -1), "%s: pred[%d] is %d", h.name.c_str(), v, u);
+            continue;
+        }
+        REQUIRE(u >= 0 && u < h.n && want[(size_t)u] == want[(size_t)v] - 1 &&
+                    std::binary_search(h.cols.begin() + h.off[(size_t)u], h.cols.begin() + h.off[(size_t)u + 1], v),
+                "%s: pred[%d] is %d", h.name.c_str(), v, u);
+    }
+    int32_t sd = 0;
+    OK(b40c_get_statistics(e, nullptr, &sd, nullptr));
+    REQUIRE(sd == deepest + 1, "%s source %d: search depth %d, not %d", h.name.c_str(), src, sd, deepest + 1);
+}
+
+std::vector<HostGraph> search_graphs() {
+    return {path_graph(1), path_graph(7), star_graph(3000), skewed_graph(9, 8, true, 1), skewed_graph(9, 6, false, 2), grid_graph(7)};
+}
+
+// Every strategy and mode on every graph: claims on labels (marks 1) or on the
+// bitmask (marks 0), `wgs` persistent workgroups per CU, grid tier from `tier`.
+void case_searches(int marks, int wgs, int tier) {
+    emu::dev().label_claim_nodes = marks ? 1 << 20 : 0;
+    for (const HostGraph& h : search_graphs()) {
+        DeviceGraph g(h);
+        for (int32_t strategy = 0; strategy < 6; ++strategy)
+            for (int32_t mode = 0; mode < 3; ++mode) {
+                std::printf("%s %s mode %d\n", h.name.c_str(), kStrategies[strategy], mode);
+                std::fflush(stdout);
+                Problem p(g.g);
+                b40c_tuning t{};
+                t.persistent_wgs_per_cu = wgs;
+                t.grid_gather_threshold = tier;
+                t.saturation_quit = 8;
+                t.levels_per_sync = 1 + strategy % 3;
+                Enactor e(strategy, &t);
+                for (int32_t src : {0, h.n / 2, h.n - 1}) search(h, p.p, e.e, src, mode);
+            }
+    }
+}
+
+// A grid of more than 256 workgroups: the persistent kernel with the shared queue.
+void case_wide_persistent() {
+    emu::dev().cus = 260;
+    emu::dev().resident = 300;
+    for (const HostGraph& h : {star_graph(3000), skewed_graph(9, 8, true, 1)}) {
+        DeviceGraph g(h);
+        Problem p(g.g);
+        Enactor e(B40C_EXPAND_CONTRACT);
+        search(h, p.p, e.e, 0, B40C_MODE_FUSED);
+        const auto& last = emu::dev().launches.back();
+        REQUIRE(last.first == "k_fused<FK_TD>" && last.second == 260, "%s with %u workgroups was launched", last.first.c_str(),
+                last.second);
+    }
+}
+
+// ---- sort, scan, removal, CSR builds -------------------------------------------
+
+template <class T>
+struct DeviceArray {
+    void* p = nullptr;
+    size_t n;
+    explicit DeviceArray(size_t k) : n(k) { OK(b40c_device_alloc(&p, (int64_t)(k * sizeof(T)))); }
+    explicit DeviceArray(const std::vector<T>& h) : DeviceArray(h.size()) { put(h); }
+    DeviceArray(const DeviceArray&) = delete;
+    ~DeviceArray() { b40c_device_free(p); }
+    void put(const std::vector<T>& h) { OK(b40c_memcpy_h2d(p, h.data(), (int64_t)(h.size() * sizeof(T)))); }
+    std::vector<T> get(size_t k) const {
+        std::vector<T> h(k);
+        OK(b40c_memcpy_d2h(h.data(), p, (int64_t)(k * sizeof(T))));
+        return h;
+    }
+    T* ptr() const { return static_cast<T*>(p); }
+};
+
+// Keys whose bits [0, bits) are random; every fifth equals its neighbour.
+std::vector<uint64_t> random_keys(size_t n, int bits, unsigned seed) {
+    std::mt19937_64 rng(seed);
+    std::vector<uint64_t> k(n);
+    for (size_t i = 0; i < n; ++i) k[i] = i % 5 == 1 ? k[i - 1] : rng() & (bits == 64 ? ~0ull : (1ull << bits) - 1);
+    return k;
+}
+
+void sort_u64(size_t n, int bits, b40c_sort_enactor* e = nullptr) {
+    std::printf("sort %zu keys of %d bits\n", n, bits);
+    std::fflush(stdout);
+    std::vector<uint64_t> k = random_keys(n, bits, (unsigned)n);
+    DeviceArray<uint64_t> a(k), b(n);
+    int32_t sel = -1;
+    if (e)
+        OK(b40c_sort_enactor_sort(e, B40C_KEY_U64, a.ptr(), b.ptr(), nullptr, nullptr, (int64_t)n, 0, 64, &sel));
+    else
+        OK(b40c_radix_sort_u64(a.ptr(), b.ptr(), (int64_t)n, 0, 64, &sel));
+    std::sort(k.begin(), k.end());
+    REQUIRE((sel ? b : a).get(n) == k, "%zu keys are not in order", n);
+}
+
+void sort_pairs(size_t n, int bits) {
+    std::printf("sort %zu pairs of %d bits\n", n, bits);
+    std::fflush(stdout);
+    const std::vector<uint64_t> k = random_keys(n, bits, (unsigned)n + 1);
+    std::vector<uint32_t> key(k.begin(), k.end()), val(n);
+    for (size_t i = 0; i < n; ++i) val[i] = (uint32_t)i;
+    DeviceArray<uint32_t> a(key), b(n), va(val), vb(n);
+    int32_t sel = -1;
+    OK(b40c_radix_sort_pairs_u32(a.ptr(), b.ptr(), va.ptr(), vb.ptr(), (int64_t)n, 0, 32, &sel));
+    std::stable_sort(val.begin(), val.end(), [&](uint32_t x, uint32_t y) { return key[x] < key[y]; });
+    const std::vector<uint32_t> gk = (sel ? b : a).get(n), gv = (sel ? vb : va).get(n);
+    for (size_t i = 0; i < n; ++i)
+        REQUIRE(gv[i] == val[i] && gk[i] == key[val[i]], "pair %zu of %zu is wrong", i, n);
+}
+
+void case_sorts() {
+    for (size_t n : {2, 63, 8192, 8193, 40000}) sort_u64(n, 64);
+    for (size_t n : {1000, 9000, 30001}) sort_pairs(n, 20);
+}
+
+void case_primitives() {
+    for (size_t n : {1, 1023, 8192, 8193, 50001}) {
+        std::printf("scan and removal %zu\n", n);
+        std::fflush(stdout);
+        const std::vector<uint64_t> k = random_keys(n, 40, (unsigned)n);
+        std::vector<uint32_t> x(k.begin(), k.end()), y(n);
+        uint64_t sum = 0, total = 0;
+        for (size_t i = 0; i < n; ++i) {
+            y[i] = (uint32_t)sum;
+            sum += x[i];
+        }
+        DeviceArray<uint32_t> in(x), out(n);
+        OK(b40c_scan_u32(in.ptr(), out.ptr(), (int64_t)n, 1, &total));
+        REQUIRE(out.get(n) == y && total == sum, "scan of %zu", n);
+        DeviceArray<uint64_t> ka(k), kb(n);
+        DeviceArray<uint32_t> vb(n);
+        int64_t kept = 0;
+        OK(b40c_consecutive_removal_u64(ka.ptr(), in.ptr(), kb.ptr(), vb.ptr(), (int64_t)n, &kept));
+        std::vector<uint64_t> wk;
+        std::vector<uint32_t> wv;
+        for (size_t i = 0; i < n; ++i)
+            if (i == 0 || k[i] != k[i - 1]) {
+                wk.push_back(k[i]);
+                wv.push_back(x[i]);
+            }
+        REQUIRE(kept == (int64_t)wk.size() && kb.get(wk.size()) == wk && vb.get(wk.size()) == wv, "removal of %zu", n);
+    }
+}
+
+void case_builds() {
+    for (const HostGraph& h : {path_graph(7), star_graph(3000), skewed_graph(11, 6, false, 3)}) {
+        std::printf("build %s\n", h.name.c_str());
+        std::fflush(stdout);
+        std::vector<int32_t> r, c;
+        for (int32_t v = 0; v < h.n; ++v)
+            for (int32_t i = h.off[(size_t)v]; i < h.off[(size_t)v + 1]; ++i) {
+                r.push_back(v);
+                c.push_back(h.cols[(size_t)i]);
+                if (i % 3 == 0) {
+                    r.push_back(v);
+                    c.push_back(h.cols[(size_t)i]);
+                }
+            }
+        for (size_t i = r.size(); i > 1; --i) {
+            const size_t j = (i * 2654435761u) % i;
+            std::swap(r[i - 1], r[j]);
+            std::swap(c[i - 1], c[j]);
+        }
+        b40c_graph* g = nullptr;
+        OK(b40c_graph_from_coo_unique(h.n, (int64_t)r.size(), r.data(), c.data(), 0, &g));
+        int32_t n = 0;
+        int64_t m = 0;
+        OK(b40c_graph_info(g, &n, &m));
+        REQUIRE(n == h.n && m == h.m(), "%d vertices and %lld edges", n, (long long)m);
+        std::vector<int32_t> off((size_t)n + 1), cols((size_t)m);
+        OK(b40c_graph_copy_to_host(g, off.data(), cols.data()));
+        REQUIRE(off == h.off && cols == h.cols, "the CSR differs");
+        b40c_graph_destroy(g);
+        r[r.size() / 2] = h.n;
+        REQUIRE(b40c_graph_from_coo_unique(h.n, (int64_t)r.size(), r.data(), c.data(), 0, &g) == B40C_ERR_INVALID_ARG,
+                "an id outside the graph was accepted");
+    }
+    b40c_graph* g = nullptr;
+    OK(b40c_graph_build_rmat(10, 8, 0.57, 0.19, 0.19, 1, &g));
+    b40c_graph_destroy(g);
+    OK(b40c_graph_build_lattice3d(9, 1, nullptr, &g));
+    b40c_graph_destroy(g);
+}
+
+// ---- batched queries -----------------------------------------------------------
+
+void case_batched(int levels, int persistent) {
+    const std::vector<HostGraph> hs = {path_graph(9), star_graph(700), skewed_graph(9, 8, true, 1), grid_graph(6)};
+    std::vector<b40c_graph*> gs;
+    for (const HostGraph& h : hs) {
+        b40c_graph* g = nullptr;
+        OK(b40c_graph_from_host_csr(h.n, h.m(), h.off.data(), h.cols.data(), &g));
+        gs.push_back(g);
+    }
+    b40c_multigraph* mg = nullptr;
+    OK(b40c_multigraph_pack(gs.data(), (int32_t)gs.size(), &mg));
+    for (b40c_graph* g : gs) b40c_graph_destroy(g);
+    b40c_msbfs* m = nullptr;
+    OK(b40c_msbfs_create(mg, 1 << 22, 256, &m));
+    OK(b40c_msbfs_set_levels_per_step(m, levels));
+    OK(b40c_msbfs_set_persistent(m, persistent));
+    std::vector<std::pair<int, int32_t>> asked;
+    std::vector<int32_t> ids;
+    for (int k = 0; k < 40; ++k) {
+        const int gi = k % (int)hs.size();
+        const int32_t src = (int32_t)((k * 37) % hs[(size_t)gi].n);
+        int32_t id = -1;
+        OK(b40c_msbfs_submit(m, gi, src, &id));
+        asked.emplace_back(gi, src);
+        ids.push_back(id);
+    }
+    OK(b40c_msbfs_run(m));
+    std::printf("batched: %d levels a step, persistent %d: run\n", levels, persistent);
+    std::fflush(stdout);
+    for (size_t k = 0; k < ids.size(); ++k) {
+        const size_t q = k < 20 ? k : ids.size() - 1 - (k - 20);  // in order, then from the end
+        const HostGraph& h = hs[(size_t)asked[q].first];
+        std::vector<int32_t> depth((size_t)h.n), pred((size_t)h.n);
+        int32_t sd = 0;
+        OK(b40c_msbfs_result(m, ids[q], depth.data(), q % 3 ? pred.data() : nullptr, &sd));
+        const std::vector<int32_t> want = serial_bfs(h, asked[q].second);
+        REQUIRE(depth == want, "query %zu on %s", q, h.name.c_str());
+        for (int32_t v = 0; q % 3 && v < h.n; ++v)
+            if (v != asked[q].second && want[(size_t)v] >= 0)
+                REQUIRE(pred[(size_t)v] >= 0 && want[(size_t)pred[(size_t)v]] == want[(size_t)v] - 1, "query %zu pred[%d]", q, v);
+    }
+    b40c_msbfs_destroy(m);
+    b40c_multigraph_destroy(mg);
+}
+
+}  // namespace
+
+int main(int argc, char** argv) {
+    if (argc < 2) return 2;
+    const std::string name = argv[1];
+    auto arg = [&](int i) {
+        REQUIRE(argc > 2 + i, "%s wants more arguments", name.c_str());
+        return std::atoi(argv[2 + i]);
+    };
+    if (name == "searches")
+        case_searches(arg(0), arg(1), arg(2));
+    else if (name == "wide_persistent")
+        case_wide_persistent();
+    else if (name == "sorts")
+        case_sorts();
+    else if (name == "primitives")
+        case_primitives();
+    else if (name == "builds")
+        case_builds();
+    else if (name == "batched")
+        case_batched(arg(0), arg(1));
+    else
+        die("unknown case %s", name.c_str());
+    std::printf("ok\n");
+    std::fflush(nullptr);
+    _Exit(0);  // the workgroup threads never end
+}

@@ -1,0 +1,63 @@
+"""The library's sources built for the host under AddressSanitizer (no GPU).
+
+tests/host_build compiles csrc/*.hip with the host compiler against a stand-in
+for the HIP runtime (lanes are fibers, a workgroup is a host thread, device
+allocations have exactly the asked size), so the library's own C entry points
+run end to end: every launch form of every search, sorts, CSR builds and
+batched queries.  tests/host_build/check.cpp holds the cases and compares with
+serial references.
+"""
+import fcntl
+import os
+import shutil
+import subprocess
+
+import pytest
+
+HERE = os.path.join(os.path.dirname(os.path.abspath(__file__)), "host_build")
+CXX = "/opt/rocm/llvm/bin/clang++"
+
+
+@pytest.fixture(scope="module")
+def check():
+    if shutil.which(CXX) is None:
+        pytest.skip("%s is not available" % CXX)
+    with open(os.path.join(HERE, ".build.lock"), "w") as lk:
+        fcntl.flock(lk, fcntl.LOCK_EX)
+        subprocess.run(["make", "-s", "-j8", "-C", HERE], check=True)
+
+    def run(*args):
+        cmd = [os.path.join(HERE, "_build", "check")] + [str(a) for a in args]
+        r = subprocess.run(cmd, capture_output=True, text=True, timeout=300,
+                           env=dict(os.environ, ASAN_OPTIONS="detect_leaks=0"))
+        assert r.returncode == 0, "%s\n%s\n%s" % (" ".join(cmd[1:]), r.stdout[-1000:], r.stderr[-4000:])
+        return r.stdout
+    return run
+
+
+@pytest.mark.parametrize("marks,wgs,tier", [(1, 1, 16), (0, 2, 100000), (1, 2, 100000), (0, 1, 16)])
+def test_searches(check, marks, wgs, tier):
+    """Every strategy and mode on paths, stars, skewed graphs (symmetric and
+    directed) and a grid: claims on labels (marks 1) or on the bitmask, the
+    narrow persistent kernel with pieces that spill (the star), the grid tier
+    from `tier` edges on."""
+    check("searches", marks, wgs, tier)
+
+
+def test_wide_persistent(check):
+    """More than 256 persistent workgroups: the form with the shared queue."""
+    check("wide_persistent")
+
+
+@pytest.mark.parametrize("case", ["sorts", "primitives", "builds"])
+def test_arrays_and_builds(check, case):
+    """Sorts on both sides of the one-workgroup limit, scans, consecutive
+    removals and CSR builds."""
+    check(case)
+
+
+@pytest.mark.parametrize("levels,persistent", [(0, 0), (3, 0), (2, 1)])
+def test_batched(check, levels, persistent):
+    """40 queries over four graphs in each form of a step, results taken in
+    and against the order of submission."""
+    check("batched", levels, persistent)
