@@ -52,16 +52,17 @@ __global__ __launch_bounds__(256) void k_isolated(const int32_t* offs, int32_t n
 
 // Last node of a captured level loop: advances the phase base and publishes
 // the counters to the pinned host mirror, so the host's per-replay check
-// needs no separate device-to-host copy.  The length published for the next
-// phase (`ph_rel` phases after the old base) includes the vertices that a
-// bottom-up step found, which are in no queue.
+// needs no separate device-to-host copy.  In a direction-optimizing search
+// (`spread` set) the length published for the next phase (`ph_rel` phases after
+// the old base) includes the vertices that a bottom-up step found, which are in
+// no queue.
 __global__ void k_advance(BfsArgs a, int steps, int ph_rel) {
     constexpr int kWords = (int)(sizeof(DevCounters) / 4);
     constexpr int kPhWord = (int)(offsetof(DevCounters, ph_base) / 4);
     const uint32_t* src = reinterpret_cast<const uint32_t*>(a.ctr);
     uint32_t* dst = reinterpret_cast<uint32_t*>(a.hctr);
     const int slot = (int)((src[kPhWord] + (uint32_t)ph_rel) & 3u);
-    unsigned long long sum = threadIdx.x < SPREAD ? *spread_at(a.spread, slot, threadIdx.x) : 0ull;
+    unsigned long long sum = a.spread && threadIdx.x < SPREAD ? *spread_at(a.spread, slot, threadIdx.x) : 0ull;
     for (int d = SPREAD / 2; d >= 1; d >>= 1) sum += __shfl_xor(sum, d, kWave);
     const uint32_t found = (uint32_t)__shfl(sum, 0, kWave);
     for (int i = threadIdx.x; i < kWords; i += blockDim.x) {

@@ -69,7 +69,7 @@ struct BfsArgs {
     int32_t coh_out;         // persistent: outputs (queue, grid-tier entries) are written with coh_st
     long long edges;
     int32_t by_label;        // small graphs: the depth labels mark visited vertices, not the bitmask (mark_claim)
-    unsigned long long* spread;  // direction-optimizing: per-level sums of what the steps found (spread_at)
+    unsigned long long* spread;  // direction-optimizing (else null): per-level sums of what the steps found (spread_at)
 };
 
 // Same-address traffic is serialised at memory: every workgroup's atomic add

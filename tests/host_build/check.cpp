@@ -203,6 +203,29 @@ void case_wide_persistent() {
     }
 }
 
+// Several strategies in turn on one problem: what one leaves behind is not the
+// next one's input.  `first_sync` levels per host check for direction-optimizing.
+void case_shared_problem(int first_sync) {
+    for (const HostGraph& h : {path_graph(5), path_graph(9), skewed_graph(9, 8, true, 1)}) {
+        DeviceGraph g(h);
+        Problem p(g.g);
+        b40c_tuning t{};
+        t.levels_per_sync = first_sync;
+        Enactor dir(B40C_DIRECTION_OPTIMIZING, &t);
+        t.levels_per_sync = 4;
+        for (int32_t src : {0, h.n / 2, h.n - 1})
+            for (int32_t strategy = 0; strategy < 6; ++strategy)
+                for (int32_t mode : {B40C_MODE_ITERATIVE, B40C_MODE_DEFAULT}) {
+                    std::printf("%s source %d: direction-optimizing, then %s mode %d\n", h.name.c_str(), src,
+                                kStrategies[strategy], mode);
+                    std::fflush(stdout);
+                    search(h, p.p, dir.e, src, B40C_MODE_DEFAULT);
+                    Enactor e(strategy, &t);
+                    search(h, p.p, e.e, src, mode);
+                }
+    }
+}
+
 // ---- sort, scan, removal, CSR builds -------------------------------------------
 
 template <class T>
@@ -392,6 +415,8 @@ int main(int argc, char** argv) {
         case_searches(arg(0), arg(1), arg(2));
     else if (name == "wide_persistent")
         case_wide_persistent();
+    else if (name == "shared_problem")
+        case_shared_problem(arg(0));
     else if (name == "sorts")
         case_sorts();
     else if (name == "primitives")

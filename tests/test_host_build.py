@@ -61,3 +61,11 @@ def test_batched(check, levels, persistent):
     """40 queries over four graphs in each form of a step, results taken in
     and against the order of submission."""
     check("batched", levels, persistent)
+
+
+@pytest.mark.parametrize("levels", [1, 2, 3, 6, 8])
+def test_strategies_share_a_problem(check, levels):
+    """A direction-optimizing search with `levels` levels per host check, then
+    every other strategy, on one problem: its partial sums, left behind, made
+    captured expand-contract loops replay for ever."""
+    check("shared_problem", levels)
