@@ -97,11 +97,13 @@ __device__ __forceinline__ uint32_t input_len(const BfsArgs& a, int ph, uint32_t
 }
 
 // `frontier_depth` >= 0: the phase's input vertices carry that label, so a
-// nonempty input makes it the deepest one so far (one store by workgroup 0;
-// a maximum taken by every workgroup would be serialised at one address).
+// nonempty input makes it the deepest one before this phase (told by workgroup
+// 0 alone: updates by every workgroup would be serialised at one address).  A
+// maximum and not a store: another workgroup of the launch may have raised it to
+// this phase's own label already (raise_max_depth).
 __device__ __forceinline__ void phase_begin(const BfsArgs& a, int ph, uint32_t n_in, int32_t frontier_depth = -1) {
     if (blockIdx.x == 0 && threadIdx.x == 0) {
-        if (frontier_depth >= 0 && n_in) st_relaxed(a.max_depth, (uint32_t)frontier_depth);
+        if (frontier_depth >= 0 && n_in) atomic_max_u32(a.max_depth, (uint32_t)frontier_depth);
         st_relaxed(&a.ctr->qlen[(ph + 2) & 3], 0u);
         __hip_atomic_store(&a.ctr->heavy_alloc[(ph + 1) & 1], 0ull, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
         if (n_in) atomic_add_u64(&a.ctr->queued, n_in);

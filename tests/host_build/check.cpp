@@ -226,6 +226,35 @@ void case_shared_problem(int first_sync) {
     }
 }
 
+// Contract-expand launches whose first workgroup starts when all the others have
+// ended: the search depth does not depend on it.  Vertices 1 and 2 list the same
+// 448 sinks, the latter after 128 vertices of its own level, so the last level's
+// 1,024 pairs are four tiles and all of the first one's are culled.
+void case_late_first_workgroup() {
+    std::vector<std::pair<int32_t, int32_t>> e;
+    for (int32_t v = 1; v < 131; ++v) e.emplace_back(0, v);
+    for (int32_t v = 3; v < 579; ++v) {
+        if (v >= 131) e.emplace_back(1, v);
+        e.emplace_back(2, v);
+    }
+    const HostGraph h = make_graph("sinks", 579, e, false);
+    std::atomic<int> ended{0};
+    b40c_tuning t{};
+    t.grid_size = 8;
+    emu::dev().on_start = [&](const std::string& k, unsigned id) {
+        if (k != "k_phase<PK_CE>" || id != 0) return;
+        while (ended.load() < 7) sched_yield();
+        ended = 0;
+    };
+    emu::dev().on_end = [&](const std::string& k, unsigned id) {
+        if (k == "k_phase<PK_CE>" && id != 0) ++ended;
+    };
+    DeviceGraph g(h);
+    Problem p(g.g);
+    Enactor x(B40C_CONTRACT_EXPAND, &t);
+    search(h, p.p, x.e, 0, B40C_MODE_ITERATIVE);
+}
+
 // ---- sort, scan, removal, CSR builds -------------------------------------------
 
 template <class T>
@@ -415,6 +444,8 @@ int main(int argc, char** argv) {
         case_searches(arg(0), arg(1), arg(2));
     else if (name == "wide_persistent")
         case_wide_persistent();
+    else if (name == "late_first_workgroup")
+        case_late_first_workgroup();
     else if (name == "shared_problem")
         case_shared_problem(arg(0));
     else if (name == "sorts")

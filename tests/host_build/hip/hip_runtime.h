@@ -461,7 +461,7 @@ inline hipError_t set(hipError_t e) {
     return e;
 }
 
-// Kernels launched through hipLaunchKernel, or whose occupancy a test sets.
+// Kernels launched through hipLaunchKernel, or that a test names.
 struct Kernel {
     std::string name;
     std::function<std::function<void()>(void**)> bind;
@@ -492,7 +492,8 @@ inline int occupancy_of(const void* k) {
 template <class... P, class... A>
 void launch(const char* text, void (*k)(P...), dim3 grid, dim3 block, Stream* s, A&&... a) {
     std::tuple<std::decay_t<P>...> t{static_cast<std::decay_t<P>>(a)...};
-    Launch job{text, grid, block, [k, t] { std::apply(k, t); }};
+    auto named = kernels().find((const void*)k);
+    Launch job{named == kernels().end() ? text : named->second.name, grid, block, [k, t] { std::apply(k, t); }};
     enqueue(s, [job] { Pool::get().run(job); });
 }
 

@@ -69,3 +69,9 @@ def test_strategies_share_a_problem(check, levels):
     every other strategy, on one problem: its partial sums, left behind, made
     captured expand-contract loops replay for ever."""
     check("shared_problem", levels)
+
+
+def test_search_depth_with_a_late_first_workgroup(check):
+    """Contract-expand in launches per level where workgroup 0 starts last: its
+    plain store of the level before overwrote what the others had found."""
+    check("late_first_workgroup")
