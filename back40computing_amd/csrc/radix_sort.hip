@@ -119,6 +119,7 @@ struct SortState {
     uint32_t* copies;   // [HIST_COPIES][MAX_PLACES][RS_BINS] digit totals, spread over copies
     uint32_t* base;     // [MAX_PLACES][RS_BINS] first output position of each digit
     uint32_t* trivial;  // [MAX_PLACES] place whose keys all share one digit
+    uint32_t* failed;   // first place + 1 whose waits ran out, beside `trivial`
     uint32_t* status;   // [2][blocks][RS_BINS] chain words (by place parity), 32 or 64 bits each
     int32_t* out;       // report: selector, failure
     int32_t blocks;
@@ -136,6 +137,7 @@ __global__ __launch_bounds__(256) void k_sort_init(SortState st) {
     const int64_t words = (int64_t)st.blocks * RS_BINS * (st.wide ? 2 : 1);
     for (int64_t i = i0; i < words; i += step) st.status[i] = 0;
     if (i0 < 2) st.out[i0] = 0;
+    if (i0 == 0) *st.failed = 0;
 }
 
 // Digit totals of every place in one read, eight keys per thread at a time.
@@ -212,6 +214,13 @@ __global__ __launch_bounds__(RS_BINS) void k_plan(SortState st, int64_t n) {
 // count first (COUNT), then the digit's next output position where the block
 // starts (START), which a serving workgroup puts in its place.
 constexpr uint32_t kChainSpins = 1u << 22;
+// A bounded wait of `place` has run out.  What the place then writes lies in the
+// output, but is no permutation of the keys: the digit totals do not hold for
+// it, and later places that went by them would write past the arrays.
+__device__ __forceinline__ void place_failed(const SortState& st, int place) {
+    st.out[1] = 1;
+    st.failed[0] = (uint32_t)place + 1;
+}
 template <typename W>
 struct ChainWord {
     static constexpr W COUNT = (W)1 << (8 * sizeof(W) - 2);
@@ -232,8 +241,8 @@ __device__ __forceinline__ void chain_store(W* status, int block, int d, W w) {
 // per round trip past the caches (0.7 us).  A thread has ROW consecutive blocks of
 // one digit.  Workgroups are dispatched in order, so the servers run, and the
 // lowest block without counts is running or next to run; should that fail, the
-// bounded wait sets *failed and the remaining blocks go on with the starts there
-// are (which lie in the output).
+// bounded wait records it (place_failed) and the remaining blocks go on with the
+// starts there are (which lie in the output).
 constexpr int SERVE_DIGITS = 16;  // one 64-byte line of 32-bit words
 constexpr int SERVERS = RS_BINS / SERVE_DIGITS;
 constexpr int SERVE_SUBS = kWave / SERVE_DIGITS;
@@ -252,13 +261,13 @@ struct ServeShared {
 };
 
 template <typename W, int ROW>
-__device__ __forceinline__ void serve_place(W* status, int blocks, const uint32_t* base, int32_t* failed,
-                                            ServeShared& s) {
+__device__ __forceinline__ void serve_place(W* status, const SortState& st, int place, ServeShared& s) {
     constexpr int WAVE_BLOCKS = SERVE_SUBS * ROW;
     const int tid = threadIdx.x, lane = lane_id(), wid = tid / kWave;
     const int col = lane % SERVE_DIGITS, sub = lane / SERVE_DIGITS;
     const int d = (int)blockIdx.x * SERVE_DIGITS + col;
-    W start = (W)base[d];
+    const int blocks = st.blocks;
+    W start = (W)st.base[place * RS_BINS + d];
     uint32_t spins = 0;
     for (int first = 0; first < blocks;) {
         const int mine = first + wid * WAVE_BLOCKS + sub * ROW;
@@ -317,7 +326,7 @@ __device__ __forceinline__ void serve_place(W* status, int blocks, const uint32_
         first += taken;
         if (taken == 0) {
             if (++spins > kChainSpins) {
-                if (tid == 0) *failed = 1;
+                if (tid == 0) place_failed(st, place);
                 for (int b = first + tid / SERVE_DIGITS; b < blocks; b += OS_THREADS / SERVE_DIGITS)
                     chain_store(status, b, (int)blockIdx.x * SERVE_DIGITS + tid % SERVE_DIGITS,
                                 (W)(ChainWord<W>::START | start));
@@ -330,12 +339,12 @@ __device__ __forceinline__ void serve_place(W* status, int blocks, const uint32_
 
 // Where digit d of a block goes: waits for its server.
 template <typename W>
-__device__ __forceinline__ uint32_t await_start(const W* status, int block, int d, int32_t* failed) {
+__device__ __forceinline__ uint32_t await_start(const W* status, int block, int d, const SortState& st, int place) {
     W w;
     uint32_t spins = 0;
     while ((w = chain_load(status, block, d)) < ChainWord<W>::START) {
         if (++spins > kChainSpins) {
-            *failed = 1;
+            place_failed(st, place);
             return 0;
         }
         __builtin_amdgcn_s_sleep(2);
@@ -385,17 +394,16 @@ __global__ __launch_bounds__(OS_THREADS) void k_place(K* k0, K* k1, uint32_t* v0
     int moved = 0;  // places before this one that moved the keys
     for (int p = 0; p < place; ++p) moved += st.trivial[p] ? 0 : 1;
     const bool skip = st.trivial[place] != 0;
+    const uint32_t failed = st.failed[0];
     if (place == st.places - 1 && block == 0 && tid == 0) st.out[0] = (moved + (skip ? 0 : 1)) & 1;
-    if (skip) return;
+    if (skip || (failed && failed <= (uint32_t)place)) return;  // (failed == place + 1: in this launch, go on)
     if (block < 0) {
-        const uint32_t* base = st.base + place * RS_BINS;
         if (st.wide)
-            serve_place<unsigned long long, SERVE_ROW_MANY>((unsigned long long*)status, st.blocks, base, &st.out[1],
-                                                            s_serve);
+            serve_place<unsigned long long, SERVE_ROW_MANY>((unsigned long long*)status, st, place, s_serve);
         else if (st.blocks <= SERVE_FEW_BLOCKS)
-            serve_place<uint32_t, SERVE_ROW_FEW>(status, st.blocks, base, &st.out[1], s_serve);
+            serve_place<uint32_t, SERVE_ROW_FEW>(status, st, place, s_serve);
         else
-            serve_place<uint32_t, SERVE_ROW_MANY>(status, st.blocks, base, &st.out[1], s_serve);
+            serve_place<uint32_t, SERVE_ROW_MANY>(status, st, place, s_serve);
         return;
     }
     const K* kin = (moved & 1) ? k1 : k0;
@@ -484,9 +492,9 @@ __global__ __launch_bounds__(OS_THREADS) void k_place(K* k0, K* k1, uint32_t* v0
             if (tile_base != begin)
                 at = next_out[tid];
             else if (st.wide)
-                at = await_start((const unsigned long long*)status, block, tid, &st.out[1]);
+                at = await_start((const unsigned long long*)status, block, tid, st, place);
             else
-                at = await_start((const uint32_t*)status, block, tid, &st.out[1]);
+                at = await_start((const uint32_t*)status, block, tid, st, place);
             out_shift[tid] = at - (uint32_t)excl;
             next_out[tid] = at + cnt;
         }
@@ -622,6 +630,7 @@ SortState sort_state(const SortScratch& sc, const SortPlan& plan, int places, in
     st.copies = sc.base + kReportWords;
     st.base = st.copies + (size_t)HIST_COPIES * MAX_PLACES * RS_BINS;
     st.trivial = st.base + (size_t)MAX_PLACES * RS_BINS;
+    st.failed = st.trivial + MAX_PLACES;
     st.status = sc.base + kStateWords;
     st.out = out;
     st.blocks = plan.blocks;

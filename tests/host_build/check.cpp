@@ -316,6 +316,28 @@ void case_sorts() {
     for (size_t n : {1000, 9000, 30001}) sort_pairs(n, 20);
 }
 
+// A place whose second block starts after the bounded waits have run out: the
+// sort fails, and the places after it, whose digit totals no longer hold, write
+// nothing outside the arrays.
+void case_sort_wait_runs_out() {
+    emu::dev().chain_spins = 50;
+    std::atomic<int> places{0};
+    emu::dev().on_start = [&](const std::string& k, unsigned id) {
+        if (k.find("k_place") == std::string::npos || id != 16 + 1) return;
+        if (places++ == 0) std::this_thread::sleep_for(std::chrono::milliseconds(1500));
+    };
+    const size_t n = 20000;
+    const std::vector<uint64_t> k = random_keys(n, 64, 5);
+    DeviceArray<uint64_t> a(k), b(n);
+    int32_t sel = -1;
+    const b40c_status s = b40c_radix_sort_u64(a.ptr(), b.ptr(), (int64_t)n, 0, 64, &sel);
+    REQUIRE(places > 1, "the sort took no second place");
+    REQUIRE(s == B40C_ERR_HIP, "the sort returned %d", (int)s);
+    emu::dev().chain_spins = 1u << 22;
+    emu::dev().on_start = nullptr;
+    sort_u64(n, 64);
+}
+
 void case_primitives() {
     for (size_t n : {1, 1023, 8192, 8193, 50001}) {
         std::printf("scan and removal %zu\n", n);
@@ -450,6 +472,8 @@ int main(int argc, char** argv) {
         case_shared_problem(arg(0));
     else if (name == "sorts")
         case_sorts();
+    else if (name == "sort_wait_runs_out")
+        case_sort_wait_runs_out();
     else if (name == "primitives")
         case_primitives();
     else if (name == "builds")

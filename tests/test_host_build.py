@@ -75,3 +75,9 @@ def test_search_depth_with_a_late_first_workgroup(check):
     """Contract-expand in launches per level where workgroup 0 starts last: its
     plain store of the level before overwrote what the others had found."""
     check("late_first_workgroup")
+
+
+def test_sort_whose_wait_runs_out(check):
+    """A sort that fails in its first place writes nothing outside its arrays in
+    the later ones, and the next sort is right."""
+    check("sort_wait_runs_out")
