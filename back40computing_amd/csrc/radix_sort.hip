@@ -124,6 +124,7 @@ struct SortState {
     int32_t* out;       // report: selector, failure
     int32_t blocks;
     int32_t wide;       // 64-bit chain words (n >= 2^30)
+    int32_t grouped;    // blocks in the order of place_block, else in the workgroups'
     int32_t places;
 };
 constexpr size_t kReportWords = 16;  // the report, where it is in the scratch (first words)
@@ -240,7 +241,9 @@ __device__ __forceinline__ void chain_store(W* status, int block, int d, W w) {
 // the blocks' counts into starts, a window of OS_WAVES * SERVE_SUBS * ROW blocks
 // per round trip past the caches (0.7 us).  A thread has ROW consecutive blocks of
 // one digit.  Workgroups are dispatched in order, so the servers run, and the
-// lowest block without counts is running or next to run; should that fail, the
+// lowest block without counts runs, or will as soon as there is room for it beside
+// the workgroups dispatched before it that wait for it (none in plain order, up to
+// GROUPED_AHEAD in that of place_block).  Should other kernels leave less room, the
 // bounded wait records it (place_failed) and the remaining blocks go on with the
 // starts there are (which lie in the output).
 constexpr int SERVE_DIGITS = 16;  // one 64-byte line of 32-bit words
@@ -355,11 +358,17 @@ __device__ __forceinline__ uint32_t await_start(const W* status, int block, int 
 // Block of the i-th working workgroup.  Workgroups go to the XCDs in turn; of
 // every XCD_RUN * 8 blocks each XCD takes XCD_RUN consecutive ones, whose runs
 // of a digit meet in the middle of a line: its L2 then writes the line once.
+// Blocks then wait for others that are dispatched after them: before block 7 of a
+// group, 49 later ones are (7 of each other XCD).  A device that may not hold
+// those, the servers and the block itself, at one workgroup per CU, keeps plain
+// order.
 constexpr int XCDS = 8;
 constexpr int XCD_RUN = 8;
-__device__ __forceinline__ int place_block(int i, int blocks) {
+constexpr int GROUPED_AHEAD = (XCDS - 1) * (XCD_RUN - 1);
+constexpr int GROUPED_CUS = SERVERS + GROUPED_AHEAD + 1;
+__device__ __forceinline__ int place_block(int i, int blocks, bool grouped) {
     constexpr int GROUP = XCDS * XCD_RUN;
-    if (i < 0 || i / GROUP * GROUP + GROUP > blocks) return i;
+    if (i < 0 || !grouped || i / GROUP * GROUP + GROUP > blocks) return i;
     return i / GROUP * GROUP + i % XCDS * XCD_RUN + i % GROUP / XCDS;
 }
 
@@ -382,7 +391,7 @@ __global__ __launch_bounds__(OS_THREADS) void k_place(K* k0, K* k1, uint32_t* v0
     __shared__ ServeShared s_serve;
 
     const int tid = threadIdx.x, lane = lane_id(), wid = __builtin_amdgcn_readfirstlane(tid / kWave);
-    const int block = place_block((int)blockIdx.x - SERVERS, st.blocks);
+    const int block = place_block((int)blockIdx.x - SERVERS, st.blocks, st.grouped != 0);
     const size_t words = (size_t)st.blocks * RS_BINS * (st.wide ? 2 : 1);
     // The other parity's words of this block, for the next place (its last
     // user, the place before this one, has finished).
@@ -600,6 +609,7 @@ struct SortPlan {
     int blocks = 1;
     int items = 8;
     bool wide = false;
+    bool grouped = false;
     int hist_wgs = 1;
 };
 
@@ -613,6 +623,7 @@ SortPlan sort_plan(int64_t n, int num_cus, const SortPolicy& pol, size_t max_wor
     SortPlan p;
     p.items = pol.items;
     p.wide = wide_words(n);
+    p.grouped = num_cus >= GROUPED_CUS;
     const int64_t tile = (int64_t)OS_THREADS * pol.items;
     const int64_t tiles = std::max<int64_t>(1, (n + tile - 1) / tile);
     int64_t most = kMaxBlocks;
@@ -635,6 +646,7 @@ SortState sort_state(const SortScratch& sc, const SortPlan& plan, int places, in
     st.out = out;
     st.blocks = plan.blocks;
     st.wide = plan.wide ? 1 : 0;
+    st.grouped = plan.grouped ? 1 : 0;
     st.places = places;
     return st;
 }

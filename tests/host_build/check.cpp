@@ -338,6 +338,22 @@ void case_sort_wait_runs_out() {
     sort_u64(n, 64);
 }
 
+// A small device that runs 20 workgroups at a time: every block of a place whose
+// turn has come can start, whatever the others wait for.
+void case_sort_few_resident() {
+    emu::dev().resident = 20;
+    emu::dev().chain_spins = 30000;
+    sort_u64(70 * 4096 + 17, 16);
+    sort_pairs(66 * 4096, 8);
+}
+// The fewest workgroups at a time with which blocks are grouped by XCD.
+void case_sort_grouped() {
+    emu::dev().cus = 66;
+    emu::dev().resident = 66;
+    emu::dev().chain_spins = 30000;
+    sort_u64(140 * 4096 + 17, 16);
+}
+
 void case_primitives() {
     for (size_t n : {1, 1023, 8192, 8193, 50001}) {
         std::printf("scan and removal %zu\n", n);
@@ -474,6 +490,10 @@ int main(int argc, char** argv) {
         case_sorts();
     else if (name == "sort_wait_runs_out")
         case_sort_wait_runs_out();
+    else if (name == "sort_few_resident")
+        case_sort_few_resident();
+    else if (name == "sort_grouped")
+        case_sort_grouped();
     else if (name == "primitives")
         case_primitives();
     else if (name == "builds")

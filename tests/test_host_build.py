@@ -81,3 +81,11 @@ def test_sort_whose_wait_runs_out(check):
     """A sort that fails in its first place writes nothing outside its arrays in
     the later ones, and the next sort is right."""
     check("sort_wait_runs_out")
+
+
+@pytest.mark.parametrize("case", ["sort_few_resident", "sort_grouped"])
+def test_sort_progress(check, case):
+    """A place ends whatever waits for whatever: 20 workgroups at a time on a
+    small device (blocks grouped by XCD ran into the bounded wait there), and the
+    fewest with which blocks are grouped."""
+    check(case)
