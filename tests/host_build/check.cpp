@@ -255,6 +255,25 @@ void case_late_first_workgroup() {
     search(h, p.p, x.e, 0, B40C_MODE_ITERATIVE);
 }
 
+// Fewer of the narrow persistent kernel's workgroups fit a CU than of the general
+// one's: the grid is sized by the kernel that is launched.
+void case_narrow_occupancy() {
+    emu::dev().occupancies["k_fused_narrow"] = 1;
+    const HostGraph h = skewed_graph(9, 8, true, 1);
+    DeviceGraph g(h);
+    Problem p(g.g);
+    b40c_tuning t{};
+    t.persistent_wgs_per_cu = 8;
+    for (int grid : {0, 7, 1}) {
+        t.grid_size = grid;
+        Enactor e(B40C_EXPAND_CONTRACT, &t);
+        search(h, p.p, e.e, 0, B40C_MODE_FUSED);
+        const auto& last = emu::dev().launches.back();
+        REQUIRE(last.first == "k_fused_narrow" && last.second == (grid == 1 ? 1u : 4u), "%s with %u workgroups was launched",
+                last.first.c_str(), last.second);
+    }
+}
+
 // ---- sort, scan, removal, CSR builds -------------------------------------------
 
 template <class T>
@@ -484,6 +503,8 @@ int main(int argc, char** argv) {
         case_wide_persistent();
     else if (name == "late_first_workgroup")
         case_late_first_workgroup();
+    else if (name == "narrow_occupancy")
+        case_narrow_occupancy();
     else if (name == "shared_problem")
         case_shared_problem(arg(0));
     else if (name == "sorts")

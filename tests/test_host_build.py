@@ -89,3 +89,8 @@ def test_sort_progress(check, case):
     small device (blocks grouped by XCD ran into the bounded wait there), and the
     fewest with which blocks are grouped."""
     check(case)
+
+
+def test_narrow_persistent_grid(check):
+    """The narrow persistent kernel's grid follows its own occupancy."""
+    check("narrow_occupancy")
