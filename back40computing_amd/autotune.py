@@ -207,7 +207,8 @@ class LabelsInvalid(AssertionError):
 
 def tune(graph, strategy, sources, rounds=2, repeats=2, log=None, knobs=None, space=None, start=None):
     """Coordinate descent from the library defaults (overridden by `start`,
-    e.g. an earlier table entry).  Returns (tuning, ms, history).  The
+    e.g. an earlier table entry); what the library chooses per graph stays open
+    (0) unless a set value is faster.  Returns (tuning, ms, history).  The
     starting point's labels are verified as BFS labels first; every
     candidate must reproduce them."""
     from . import bfs

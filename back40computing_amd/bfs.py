@@ -243,6 +243,8 @@ class _Enactor:
 
     @property
     def tuning(self):
+        """The tuning in force (b40c_tuning's fields); 0 for those left open,
+        which the library chooses per graph."""
         t = Tuning()
         check(lib().b40c_enactor_get_tuning(self._h, ctypes.byref(t)))
         return t.as_dict()

@@ -254,6 +254,8 @@ void b40c_problem_destroy(b40c_problem* p);
 /* Enactor construction (enactor_*.cuh constructors; INSTRUMENT template flag). */
 b40c_status b40c_enactor_create(int32_t strategy, int32_t instrument, b40c_enactor** out);
 b40c_status b40c_enactor_set_tuning(b40c_enactor* e, const b40c_tuning* t);
+/* The tuning in force; 0 in persistent_wgs_per_cu and grid_gather_threshold where
+ * they were never set and the library chooses them per graph. */
 b40c_status b40c_enactor_get_tuning(const b40c_enactor* e, b40c_tuning* t);
 /* The frontier type a problem must be Reset with for this enactor
  * (GetFrontierType, e.g. enactor_contract_expand.cuh:205). */

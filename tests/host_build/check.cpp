@@ -274,6 +274,36 @@ void case_narrow_occupancy() {
     }
 }
 
+// A tuning that is read and set again changes nothing: fields that the caller left
+// open, which the library chooses per graph, stay open.
+void case_tuning_round_trip() {
+    const HostGraph h = grid_graph(7);
+    DeviceGraph g(h);
+    Problem p(g.g);
+    for (int32_t strategy = 0; strategy < 6; ++strategy) {
+        Enactor fresh(strategy);
+        b40c_tuning t{}, again{};
+        OK(b40c_enactor_get_tuning(fresh.e, &t));
+        Enactor copy(strategy, &t);
+        OK(b40c_enactor_get_tuning(copy.e, &again));
+        REQUIRE(std::memcmp(&t, &again, sizeof(t)) == 0, "%s: the tuning read back differs", kStrategies[strategy]);
+        const int32_t mode = strategy == B40C_HYBRID ? B40C_MODE_DEFAULT : B40C_MODE_FUSED;
+        emu::dev().launches.clear();
+        search(h, p.p, fresh.e, 0, mode);
+        const auto want = emu::dev().launches;
+        emu::dev().launches.clear();
+        search(h, p.p, copy.e, 0, mode);
+        REQUIRE(emu::dev().launches == want, "%s: other persistent launches", kStrategies[strategy]);
+        t = b40c_tuning{};
+        t.persistent_wgs_per_cu = 3;
+        t.grid_gather_threshold = 100;
+        OK(b40c_enactor_set_tuning(copy.e, &t));
+        OK(b40c_enactor_get_tuning(copy.e, &again));
+        REQUIRE(again.persistent_wgs_per_cu == 3 && again.grid_gather_threshold == 100, "%s: what was set is not reported",
+                kStrategies[strategy]);
+    }
+}
+
 // ---- sort, scan, removal, CSR builds -------------------------------------------
 
 template <class T>
@@ -505,6 +535,8 @@ int main(int argc, char** argv) {
         case_late_first_workgroup();
     else if (name == "narrow_occupancy")
         case_narrow_occupancy();
+    else if (name == "tuning_round_trip")
+        case_tuning_round_trip();
     else if (name == "shared_problem")
         case_shared_problem(arg(0));
     else if (name == "sorts")

@@ -94,3 +94,8 @@ def test_sort_progress(check, case):
 def test_narrow_persistent_grid(check):
     """The narrow persistent kernel's grid follows its own occupancy."""
     check("narrow_occupancy")
+
+
+def test_tuning_round_trip(check):
+    """Setting the tuning that was read leaves the choices per graph alone."""
+    check("tuning_round_trip")
