@@ -141,7 +141,9 @@ struct ChainCall {
         return B40C_OK;
     }
     b40c_status finish(const char* who, uint64_t& total, hipStream_t stream) {
-        B40C_HIP(hipGetLastError());
+        const hipError_t launched = hipGetLastError();
+        if (launched != hipSuccess) (void)hipStreamSynchronize(stream);  // the report and `words` are in use until then
+        B40C_HIP(launched);
         ChainReport h;
         if (!slot.host) B40C_HIP(hipMemcpyAsync(&h, report, sizeof(h), hipMemcpyDeviceToHost, stream));
         B40C_HIP(hipStreamSynchronize(stream));

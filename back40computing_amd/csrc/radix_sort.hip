@@ -790,7 +790,13 @@ static b40c_status radix_sort_sync(int32_t key_type, void* k0, void* k1, uint32_
                                    const SortScratch& sc, int32_t* selector, hipStream_t stream, bool pinned = true) {
     SortReport report;
     report.take(sc, pinned);
-    B40C_TRY(radix_sort_launch(key_type, k0, k1, v0, v1, n, begin_bit, end_bit, num_cus, pol, sc, report.dev, stream));
+    const b40c_status launched =
+        radix_sort_launch(key_type, k0, k1, v0, v1, n, begin_bit, end_bit, num_cus, pol, sc, report.dev, stream);
+    if (launched != B40C_OK) {
+        // Some kernels may be on their way: the report is theirs until they end.
+        (void)hipStreamSynchronize(stream);
+        return launched;
+    }
     int32_t words[2] = {0, 0};
     B40C_TRY(report.wait(words, stream));
     if (words[1]) return fail(B40C_ERR_HIP, "radix sort: a block waited too long for the blocks before it");

@@ -403,6 +403,30 @@ void case_sort_grouped() {
     sort_u64(140 * 4096 + 17, 16);
 }
 
+// A sort that returns an error after its kernels were launched, then another one:
+// the second one's report is its own, though the first one's kernels run late.
+void case_sort_after_error() {
+    emu::dev().lazy = true;
+    b40c_sort_enactor *e = nullptr, *f = nullptr;
+    OK(b40c_sort_enactor_create(&e));
+    OK(b40c_sort_enactor_create(&f));
+    const size_t n = 500;
+    const std::vector<uint64_t> one = random_keys(n, 8, 1), two = random_keys(n, 16, 2);
+    DeviceArray<uint64_t> a(one), b(n), c(two), d(n);
+    int32_t sel = -1;
+    sort_u64(n, 8, e);  // the scratch is allocated
+    sort_u64(n, 8, f);
+    emu::last_error = hipErrorUnknown;
+    REQUIRE(b40c_sort_enactor_sort(e, B40C_KEY_U64, a.ptr(), b.ptr(), nullptr, nullptr, (int64_t)n, 0, 64, &sel) == B40C_ERR_HIP,
+            "the planted error was not returned");
+    OK(b40c_sort_enactor_sort(f, B40C_KEY_U64, c.ptr(), d.ptr(), nullptr, nullptr, (int64_t)n, 0, 64, &sel));
+    std::vector<uint64_t> want = two;
+    std::sort(want.begin(), want.end());
+    REQUIRE((sel ? d : c).get(n) == want, "selector %d is not this sort's", sel);
+    b40c_sort_enactor_destroy(e);
+    b40c_sort_enactor_destroy(f);
+}
+
 void case_primitives() {
     for (size_t n : {1, 1023, 8192, 8193, 50001}) {
         std::printf("scan and removal %zu\n", n);
@@ -547,6 +571,8 @@ int main(int argc, char** argv) {
         case_sort_few_resident();
     else if (name == "sort_grouped")
         case_sort_grouped();
+    else if (name == "sort_after_error")
+        case_sort_after_error();
     else if (name == "primitives")
         case_primitives();
     else if (name == "builds")

@@ -99,3 +99,9 @@ def test_narrow_persistent_grid(check):
 def test_tuning_round_trip(check):
     """Setting the tuning that was read leaves the choices per graph alone."""
     check("tuning_round_trip")
+
+
+def test_sort_after_a_failed_one(check):
+    """A sort that fails after its launches keeps its report words until its
+    kernels have run; they were given to the next sort at once."""
+    check("sort_after_error")
