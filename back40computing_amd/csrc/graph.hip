@@ -337,7 +337,7 @@ struct KeyArena {
         auto up = [](size_t b) { return (b + 255) / 256 * 256; };
         const size_t keys = up((size_t)std::max<int64_t>(nkeys, 1) * 8);
         scratch_words = sort_scratch_words(std::max<int64_t>(nkeys, 1));
-        const size_t work = up(std::max(scratch_words * 4, chain_bytes((nkeys + CSR_BLOCK - 1) / CSR_BLOCK)));
+        size_t work = up(std::max(scratch_words * 4, chain_bytes((nkeys + CSR_BLOCK - 1) / CSR_BLOCK)));
         if (std::max(std::max(keys, work), extra_bytes) <= (1u << 20)) {
             B40C_TRY(mem.alloc(keys));
             B40C_TRY(small[0].alloc(keys));
@@ -349,7 +349,15 @@ struct KeyArena {
             extra = small[2].as<char>();
             return B40C_OK;
         }
-        B40C_TRY(mem.alloc(2 * keys + work + extra_bytes));
+        b40c_status s = mem.alloc(2 * keys + work + extra_bytes);
+        if (s == B40C_ERR_OOM) {
+            // The sort looks for its scratch itself, and can do with less.
+            (void)hipGetLastError();
+            scratch_words = 0;
+            work = up(chain_bytes((nkeys + CSR_BLOCK - 1) / CSR_BLOCK));
+            s = mem.alloc(2 * keys + work + extra_bytes);
+        }
+        B40C_TRY(s);
         char* p = mem.as<char>();
         k0 = reinterpret_cast<uint64_t*>(p);
         k1 = reinterpret_cast<uint64_t*>(p + keys);

@@ -747,6 +747,20 @@ size_t sort_scratch_words(int64_t n) {
 }
 
 namespace {
+// Scratch that any sort can do with, in fewer and longer blocks: that of the
+// allocation-free entry point.
+constexpr size_t kNoAllocWords = (size_t)RS_BINS * 2048 + 2 * RS_BINS + 64;
+static_assert((kNoAllocWords - kStateWords) / (2 * RS_BINS) == 988 && (kNoAllocWords - kStateWords) / (4 * RS_BINS) == 494,
+              "the blocks that its comment names");
+
+// A sort's scratch in device memory of at least `words` words, or what there is room for.
+b40c_status reserve_scratch(DeviceBuffer& mem, size_t words) {
+    const b40c_status s = mem.reserve(words * sizeof(uint32_t));
+    if (s != B40C_ERR_OOM || words <= kNoAllocWords) return s;
+    (void)hipGetLastError();
+    return mem.reserve(kNoAllocWords * sizeof(uint32_t));
+}
+
 // One sort's report words (selector, failure): a pinned slot, or, without one,
 // the first words of the scratch, copied back after the sort.
 struct SortReport {
@@ -817,9 +831,9 @@ b40c_status radix_sort_once(int32_t key_type, void* k0, void* k1, uint32_t* v0, 
     const SortPolicy pol = resolve_sort_policy(SortPolicy{}, n, key_bits(key_type) / 8 + (v0 ? 4 : 0), info.num_cus);
     const size_t words = sort_scratch_words(n);
     if (!scratch || scratch_words < words) {
-        B40C_TRY(mem.alloc(words * sizeof(uint32_t)));
+        B40C_TRY(reserve_scratch(mem, words));
         scratch = mem.as<uint32_t>();
-        scratch_words = words;
+        scratch_words = mem.bytes / sizeof(uint32_t);
     }
     return radix_sort_sync(key_type, k0, k1, v0, v1, n, begin_bit, end_bit, info.num_cus, pol,
                            SortScratch{scratch, scratch_words}, selector, stream);
@@ -843,19 +857,12 @@ b40c_status radix_sort_pairs_u32(uint32_t* k0, uint32_t* k1, uint32_t* v0, uint3
 // ---------------------------------------------------------------------------
 // Allocation-free sort (no counterpart in the reference): its scratch is this
 // fixed device array, one copy per GPU, which the GPU keeps until the
-// process ends: 2 MiB + 2 KiB, enough for the chain words of 950 blocks
-// (475 from 2^30 keys on); blocks are as large as n <= 2^32 - 1 keys then need.
-// In host code `scratch`
-// is only a stand-in for the device array; its device address comes from
-// hipGetSymbolAddress, once per device, and only that address is used.
+// process ends: 2 MiB + 2 KiB, enough for the chain words of 988 blocks
+// (494 from 2^30 keys on); blocks are as large as n <= 2^32 - 1 keys then need.
+// In host code `scratch` is only a stand-in for the device array; its device
+// address comes from hipGetSymbolAddress, once per device, and only that address
+// is used.
 // ---------------------------------------------------------------------------
-namespace b40c {
-namespace {
-constexpr size_t kNoAllocWords = (size_t)RS_BINS * 2048 + 2 * RS_BINS + 64;
-static_assert(kNoAllocWords > kStateWords + 400 * 2 * RS_BINS * 2, "room for the state and hundreds of blocks");
-}  // namespace
-}  // namespace b40c
-
 static __device__ __align__(256) uint32_t scratch[b40c::kNoAllocWords];
 
 namespace b40c {
@@ -963,7 +970,7 @@ b40c_status b40c_sort_enactor_sort(b40c_sort_enactor* e, int32_t key_type, void*
     const SortPolicy pol = resolve_sort_policy(e->policy, n, key_bits(key_type) / 8 + (d_vals0 ? 4 : 0), info.num_cus);
     const size_t words = sort_scratch_words(n);
     // Grow-only: later sorts of at most this size allocate nothing.
-    B40C_TRY(e->scratch.reserve(words * sizeof(uint32_t)));
+    B40C_TRY(reserve_scratch(e->scratch, words));
     return radix_sort_sync(key_type, d_keys0, d_keys1, d_vals0, d_vals1, n, begin_bit, end_bit, info.num_cus, pol,
                            SortScratch{e->scratch.as<uint32_t>(), e->scratch.bytes / sizeof(uint32_t)}, selector,
                            e->stream);

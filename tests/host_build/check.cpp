@@ -427,6 +427,42 @@ void case_sort_after_error() {
     b40c_sort_enactor_destroy(f);
 }
 
+// Device memory too short for the scratch that a sort or a build wants: they make
+// do with less.
+void case_short_of_memory() {
+    const size_t n = 1100 * 4096;
+    {
+        std::vector<uint64_t> k = random_keys(n, 8, 3);
+        DeviceArray<uint64_t> a(k), b(n);
+        b40c_sort_enactor* e = nullptr;
+        OK(b40c_sort_enactor_create(&e));
+        emu::dev().largest_alloc = 2200000;
+        int32_t sel = -1;
+        OK(b40c_radix_sort_u64(a.ptr(), b.ptr(), (int64_t)n, 0, 8, &sel));
+        std::vector<uint64_t> want = k;
+        std::sort(want.begin(), want.end());
+        REQUIRE((sel ? b : a).get(n) == want, "the keys are not in order");
+        a.put(k);
+        OK(b40c_sort_enactor_sort(e, B40C_KEY_U64, a.ptr(), b.ptr(), nullptr, nullptr, (int64_t)n, 0, 8, &sel));
+        REQUIRE((sel ? b : a).get(n) == want, "the enactor's keys are not in order");
+        b40c_sort_enactor_destroy(e);
+    }
+    // A build whose arrays fit but not with the sort's scratch beside them.
+    const int32_t m = 140000;
+    std::vector<int32_t> r((size_t)m), c((size_t)m);
+    for (int32_t i = 0; i < m; ++i) {
+        r[(size_t)i] = i / 8;
+        c[(size_t)i] = i % 8;
+    }
+    emu::dev().largest_alloc = (size_t)m * (2 * 8 + 8) + 50000;
+    b40c_graph* g = nullptr;
+    OK(b40c_graph_from_coo_unique(m / 8, m, r.data(), c.data(), 0, &g));
+    int64_t edges = 0;
+    OK(b40c_graph_info(g, nullptr, &edges));
+    REQUIRE(edges == m, "%lld edges", (long long)edges);
+    b40c_graph_destroy(g);
+}
+
 void case_primitives() {
     for (size_t n : {1, 1023, 8192, 8193, 50001}) {
         std::printf("scan and removal %zu\n", n);
@@ -573,6 +609,8 @@ int main(int argc, char** argv) {
         case_sort_grouped();
     else if (name == "sort_after_error")
         case_sort_after_error();
+    else if (name == "short_of_memory")
+        case_short_of_memory();
     else if (name == "primitives")
         case_primitives();
     else if (name == "builds")

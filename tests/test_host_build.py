@@ -105,3 +105,9 @@ def test_sort_after_a_failed_one(check):
     """A sort that fails after its launches keeps its report words until its
     kernels have run; they were given to the next sort at once."""
     check("sort_after_error")
+
+
+def test_short_of_device_memory(check):
+    """Sorts and builds that find no memory for the scratch they want go on with
+    the little they need."""
+    check("short_of_memory")
