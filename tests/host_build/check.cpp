@@ -304,6 +304,24 @@ void case_tuning_round_trip() {
     }
 }
 
+// No memory for the narrow persistent kernel's frontier pieces: the search runs
+// the general form.
+void case_no_frontier_pieces() {
+    const HostGraph h = skewed_graph(9, 8, true, 1);
+    DeviceGraph g(h);
+    Problem p(g.g);
+    Enactor e(B40C_EXPAND_CONTRACT);
+    search(h, p.p, e.e, 0, B40C_MODE_ITERATIVE);  // the queues are allocated
+    emu::dev().largest_alloc = 200000;
+    for (int k = 0; k < 2; ++k) {
+        search(h, p.p, e.e, 1, B40C_MODE_FUSED);
+        REQUIRE(emu::dev().launches.back().first == "k_fused<FK_TD>", "%s was launched", emu::dev().launches.back().first.c_str());
+    }
+    emu::dev().largest_alloc = ~(size_t)0;
+    search(h, p.p, e.e, 1, B40C_MODE_FUSED);
+    REQUIRE(emu::dev().launches.back().first == "k_fused_narrow", "%s was launched", emu::dev().launches.back().first.c_str());
+}
+
 // ---- sort, scan, removal, CSR builds -------------------------------------------
 
 template <class T>
@@ -597,6 +615,8 @@ int main(int argc, char** argv) {
         case_narrow_occupancy();
     else if (name == "tuning_round_trip")
         case_tuning_round_trip();
+    else if (name == "no_frontier_pieces")
+        case_no_frontier_pieces();
     else if (name == "shared_problem")
         case_shared_problem(arg(0));
     else if (name == "sorts")

@@ -111,3 +111,8 @@ def test_short_of_device_memory(check):
     """Sorts and builds that find no memory for the scratch they want go on with
     the little they need."""
     check("short_of_memory")
+
+
+def test_no_memory_for_frontier_pieces(check):
+    """Expand-contract without room for the narrow kernel's pieces."""
+    check("no_frontier_pieces")
