@@ -32,7 +32,9 @@ from ._lib import check, lib
 
 TABLE_PATH = os.path.join(os.path.dirname(os.path.abspath(__file__)), "tuning_table.json")
 
-# Candidate values per knob (coordinate descent visits them in this order).
+# Candidate values per knob (coordinate descent visits them in this order).  The
+# two gather thresholds below the grid tier are for callers that name them; no
+# kernel reads them, so no strategy's knobs hold them.
 SPACE = {
     "do_alpha": [1, 2, 3, 4, 6, 8, 14, 32, 64, 128, 256, 1024],
     "do_beta": [6, 12, 24, 48, 96, 192],

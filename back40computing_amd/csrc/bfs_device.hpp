@@ -11,9 +11,10 @@
 //    ExpandByCta / ExpandByWarp / ExpandByScan
 //    (b40c/graph/bfs/two_phase/expand_atomic/cta.cuh:215-423, 606-719): one
 //    form for every degree.
-//  * claim_exact: the visited bitmask with an agent-scope atomicOr, so each
-//    vertex has exactly one discoverer (the reference's best-effort bitmask
-//    RMW, contract_expand_atomic/cta.cuh:237-252, lets duplicates through).
+//  * mark_claim: an agent-scope atomic on the visited bitmask, or on the depth
+//    label of a small graph, so each vertex has exactly one discoverer (the
+//    reference's best-effort bitmask RMW, contract_expand_atomic/cta.cuh:237-252,
+//    lets duplicates through).
 //  * HistoryHash: per-workgroup LDS hash of recently seen ids that culls
 //    duplicates before they reach the atomic (the reference's warp/history
 //    culls, contract_expand_atomic/cta.cuh:363-387,
@@ -289,14 +290,6 @@ __device__ __forceinline__ uint32_t mark_claim(const BfsArgs& a, int32_t v, int3
         return __hip_atomic_fetch_min(reinterpret_cast<uint32_t*>(&a.depth[v]), (uint32_t)depth, __ATOMIC_RELAXED,
                                       __HIP_MEMORY_SCOPE_AGENT);
     return atomic_or_u32(&a.visited[v >> 5], 1u << (v & 31));
-}
-
-__device__ __forceinline__ bool visited_test(const BfsArgs& a, int32_t v) { return mark_seen(a, v, mark_load(a, v)); }
-
-// Exactly one caller per vertex returns true.
-__device__ __forceinline__ bool claim_exact(const BfsArgs& a, int32_t v, int32_t depth) {
-    if (visited_test(a, v)) return false;
-    return !mark_seen(a, v, mark_claim(a, v, depth));
 }
 
 struct HistoryHash {

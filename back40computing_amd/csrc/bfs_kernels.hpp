@@ -673,8 +673,7 @@ struct DoTdShared {
 // Start state of a level (do_level_in).
 struct DoLevelIn {
     int32_t ph;
-    uint32_t queued;   // vertices a top-down step left in the queue
-    uint32_t n_f;      // frontier vertices: those and what a bottom-up step found
+    uint32_t n_f;      // frontier vertices: queued by a top-down step, or found by a bottom-up one
     uint32_t prev_dir;
     long long m_f;     // their degree sum
     long long vis;     // degree sum of the vertices visited before them
@@ -986,7 +985,6 @@ __device__ __forceinline__ void do_level_in(const BfsArgs& a, int ph, DoLevelIn&
         const uint32_t lo = __shfl(w, kVis + 2 * (ph & 3), kWave), hi = __shfl(w, kVis + 2 * (ph & 3) + 1, kWave);
         if (lane == 0) {
             in.ph = ph;
-            in.queued = n_q;
             in.n_f = n_q + (uint32_t)part;
             in.prev_dir = dir;
             in.m_f = (long long)(part >> 32);

@@ -64,9 +64,6 @@ struct alignas(256) DevCounters {
 // ---------------------------------------------------------------------------
 // Agent-scope atomics (visible across all XCDs of the device).
 // ---------------------------------------------------------------------------
-__device__ __forceinline__ uint32_t ld_acquire(const uint32_t* p) {
-    return __hip_atomic_load(p, __ATOMIC_ACQUIRE, __HIP_MEMORY_SCOPE_AGENT);
-}
 __device__ __forceinline__ uint32_t ld_relaxed(const uint32_t* p) {
     return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
