@@ -304,6 +304,28 @@ void case_tuning_round_trip() {
     }
 }
 
+// Queues of less than one entry by the sizing factor: every strategy ends with an
+// overflow or, where no frontier is longer than one, with the right labels.
+void case_tiny_queues() {
+    for (const HostGraph& h : {path_graph(2), path_graph(7), star_graph(20)}) {
+        DeviceGraph g(h);
+        for (int32_t strategy = 0; strategy < 6; ++strategy)
+            for (int32_t mode = 0; mode < 3; ++mode) {
+                std::printf("%s %s mode %d\n", h.name.c_str(), kStrategies[strategy], mode);
+                std::fflush(stdout);
+                Problem p(g.g);
+                Enactor e(strategy);
+                OK(b40c_problem_reset(p.p, b40c_enactor_frontier_type(e.e), 0.01));
+                const b40c_status s = b40c_enact_search(e.e, p.p, 0, 0, mode);
+                REQUIRE(s == B40C_OK || s == B40C_ERR_QUEUE_OVERFLOW, "the search returned %d", (int)s);
+                if (s != B40C_OK) continue;
+                std::vector<int32_t> depth((size_t)h.n);
+                OK(b40c_problem_extract(p.p, depth.data(), nullptr));
+                REQUIRE(depth == serial_bfs(h, 0), "wrong labels and no overflow");
+            }
+    }
+}
+
 // No memory for the narrow persistent kernel's frontier pieces: the search runs
 // the general form.
 void case_no_frontier_pieces() {
@@ -617,6 +639,8 @@ int main(int argc, char** argv) {
         case_tuning_round_trip();
     else if (name == "no_frontier_pieces")
         case_no_frontier_pieces();
+    else if (name == "tiny_queues")
+        case_tiny_queues();
     else if (name == "shared_problem")
         case_shared_problem(arg(0));
     else if (name == "sorts")

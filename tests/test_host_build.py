@@ -116,3 +116,9 @@ def test_short_of_device_memory(check):
 def test_no_memory_for_frontier_pieces(check):
     """Expand-contract without room for the narrow kernel's pieces."""
     check("no_frontier_pieces")
+
+
+def test_tiny_queues(check):
+    """A sizing factor that asks for less than one queue entry: no value array
+    was allocated for an edge frontier's single one."""
+    check("tiny_queues")
