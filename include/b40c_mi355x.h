@@ -303,15 +303,13 @@ b40c_status b40c_msbfs_set_tuning(b40c_msbfs* m, int32_t alpha, int32_t beta, in
  * queries arrive in cohorts that share their expensive first levels (1 =
  * admit at every boundary; default 6).  An idle engine admits at once. */
 b40c_status b40c_msbfs_set_admission(b40c_msbfs* m, int32_t cohort_gap);
-/* Launch form of a step (north-star batched form; no counterpart in the
- * reference).  levels >= 1: each b40c_msbfs_step replays one hipGraph that
+/* Launch form of a step (no counterpart in the reference).  levels >= 1: each b40c_msbfs_step replays one hipGraph that
  * holds `levels` levels (six kernels each, the phase read from device
  * memory) and one phase-advance node, then synchronizes once; queries that
  * finish inside the replay are retired on the device and reported at its
  * end.  0 (default): each step launches one level's kernels directly. */
 b40c_status b40c_msbfs_set_levels_per_step(b40c_msbfs* m, int32_t levels);
-/* Persistent form (north-star batched form; no counterpart in the
- * reference): on = 1 runs each step's levels (levels_per_step, at least 1)
+/* Persistent form (no counterpart in the reference): on = 1 runs each step's levels (levels_per_step, at least 1)
  * in one launch of a co-resident grid, the six steps of every level
  * separated by software grid barriers; 0 (default) uses launches or the
  * captured graph.  The grid is the occupancy API's co-resident maximum
