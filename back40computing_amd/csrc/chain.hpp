@@ -52,10 +52,10 @@ struct ChainServeShared {
 // are dispatched in order, so the lowest block without a sum is running or
 // next to run; should that fail, the bounded wait sets failed and the
 // remaining blocks go on with what there is.
+// `before` is what comes before the first block.
 __device__ __forceinline__ void chain_serve(unsigned long long* chain, int blocks, ChainReport* report,
-                                            ChainServeShared& s) {
+                                            ChainServeShared& s, uint64_t before = 0) {
     const int tid = threadIdx.x, lane = lane_id(), wid = tid / kWave;
-    uint64_t before = 0;
     int base = 0;
     uint32_t spins = 0;
     while (base < blocks) {
@@ -136,9 +136,13 @@ struct ChainCall {
             report = static_cast<ChainReport*>(slot.dev);
         else
             B40C_TRY(fill_u32(reinterpret_cast<uint32_t*>(report), 0, sizeof(ChainReport) / 4, stream));
+        clear(blocks, stream);
+        return B40C_OK;
+    }
+    // The words of a kernel's blocks; before every kernel of the call.
+    void clear(int64_t blocks, hipStream_t stream) {
         hipLaunchKernelGGL(k_chain_init, dim3((unsigned)std::min<int64_t>((blocks + CHAIN_THREADS - 1) / CHAIN_THREADS, 256)), dim3(CHAIN_THREADS), 0,
                            stream, chain, (int)blocks);
-        return B40C_OK;
     }
     b40c_status finish(const char* who, uint64_t& total, hipStream_t stream) {
         const hipError_t launched = hipGetLastError();

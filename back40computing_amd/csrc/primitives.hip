@@ -172,15 +172,22 @@ constexpr int64_t kChainScanMax = 1ll << 30;  // sums of 32-bit values stay belo
 constexpr int SCAN_SUB = 8;
 constexpr int64_t SCAN_BLOCK = (int64_t)PT * VEC32 * SCAN_SUB;
 
+// Arrays are scanned in segments of at most kScanSegment elements, one launch
+// each, the total so far in the report: their chain words stay below 2 MB, which
+// the runtime serves from chunks it keeps (8 us after an upload).  More are mapped
+// anew on every call: 2^28 elements in place after an upload took 790 us, with
+// 550 to 610 in segments, as three passes 650 to 730.
+constexpr int64_t kScanSegment = (1ll << 28) - (1ll << 20);
+
 __global__ __launch_bounds__(PT) void k_scan_chained(const uint32_t* in, uint32_t* out, int64_t n, int inclusive,
-                                                     unsigned long long* chain, ChainReport* report) {
+                                                     int first, unsigned long long* chain, ChainReport* report) {
     static_assert(SCAN_SUB * PW <= kWave, "one wave scans the waves' totals");
     __shared__ uint32_t s_tot[SCAN_SUB * PW];
     __shared__ uint64_t s_sum[PW];
     __shared__ uint32_t s_before;
     __shared__ ChainServeShared s_serve;
     if (blockIdx.x == 0) {
-        chain_serve(chain, gridDim.x - 1, report, s_serve);
+        chain_serve(chain, gridDim.x - 1, report, s_serve, first ? 0 : report->total);
         return;
     }
     const int block = blockIdx.x - 1;
@@ -388,11 +395,16 @@ b40c_status b40c_scan_u32(const uint32_t* d_in, uint32_t* d_out, int64_t n, int3
     if (total) *total = 0;
     if (n == 0) return B40C_OK;
     if (aligned16(d_in) && aligned16(d_out) && n <= kChainScanMax) {
-        const int64_t blocks = (n + SCAN_BLOCK - 1) / SCAN_BLOCK;
         ChainCall call;
-        B40C_TRY(call.start(blocks, nullptr));
-        hipLaunchKernelGGL(k_scan_chained, dim3((unsigned)blocks + 1), dim3(PT), 0, nullptr, d_in, d_out, n,
-                           exclusive ? 0 : 1, call.chain, call.report);
+        for (int64_t at = 0; at < n; at += kScanSegment) {
+            const int64_t len = std::min<int64_t>(n - at, kScanSegment), blocks = (len + SCAN_BLOCK - 1) / SCAN_BLOCK;
+            if (at == 0)
+                B40C_TRY(call.start(blocks, nullptr));
+            else
+                call.clear(blocks, nullptr);
+            hipLaunchKernelGGL(k_scan_chained, dim3((unsigned)blocks + 1), dim3(PT), 0, nullptr, d_in + at, d_out + at,
+                               len, exclusive ? 0 : 1, at == 0 ? 1 : 0, call.chain, call.report);
+        }
         uint64_t sum = 0;
         B40C_TRY(call.finish("b40c_scan_u32", sum, nullptr));
         if (total) *total = sum;

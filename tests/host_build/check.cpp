@@ -532,6 +532,31 @@ void case_primitives() {
     }
 }
 
+// Scans of several launches: whole and partial last blocks and segments.
+void case_scan_segments() {
+    const size_t block = 8192;
+    for (size_t blocks : {1, 3}) {
+        emu::dev().scan_segment = (long long)(blocks * block);
+        for (size_t n : {block, blocks * block, blocks * block + 1, 2 * blocks * block - 1, 2 * blocks * block, 7 * block + 5}) {
+            std::printf("scan %zu in segments of %zu blocks\n", n, blocks);
+            std::fflush(stdout);
+            const std::vector<uint64_t> k = random_keys(n, 32, (unsigned)n);
+            std::vector<uint32_t> x(k.begin(), k.end()), excl(n), incl(n);
+            uint64_t sum = 0, total = 0;
+            for (size_t i = 0; i < n; ++i) {
+                excl[i] = (uint32_t)sum;
+                sum += x[i];
+                incl[i] = (uint32_t)sum;
+            }
+            DeviceArray<uint32_t> in(x), out(n);
+            OK(b40c_scan_u32(in.ptr(), out.ptr(), (int64_t)n, 1, &total));
+            REQUIRE(out.get(n) == excl && total == sum, "exclusive scan");
+            OK(b40c_scan_u32(in.ptr(), in.ptr(), (int64_t)n, 0, &total));
+            REQUIRE(in.get(n) == incl && total == sum, "inclusive scan in place");
+        }
+    }
+}
+
 void case_builds() {
     for (const HostGraph& h : {path_graph(7), star_graph(3000), skewed_graph(11, 6, false, 3)}) {
         std::printf("build %s\n", h.name.c_str());
@@ -657,6 +682,8 @@ int main(int argc, char** argv) {
         case_short_of_memory();
     else if (name == "primitives")
         case_primitives();
+    else if (name == "scan_segments")
+        case_scan_segments();
     else if (name == "builds")
         case_builds();
     else if (name == "batched")

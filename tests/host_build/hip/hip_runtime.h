@@ -103,6 +103,7 @@ struct Device {
     bool lazy = false;
     unsigned chain_spins = 1u << 22;    // polls of a bounded wait
     int label_claim_nodes = 1 << 20;
+    long long scan_segment = 1 << 27;   // elements of a scan's launch
     // Called as a workgroup starts (kernel's name, workgroup); may wait.
     std::function<void(const std::string&, unsigned)> on_start;
     std::function<void(const std::string&, unsigned)> on_end;

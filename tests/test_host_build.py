@@ -49,7 +49,7 @@ def test_wide_persistent(check):
     check("wide_persistent")
 
 
-@pytest.mark.parametrize("case", ["sorts", "primitives", "builds"])
+@pytest.mark.parametrize("case", ["sorts", "primitives", "builds", "scan_segments"])
 def test_arrays_and_builds(check, case):
     """Sorts on both sides of the one-workgroup limit, scans, consecutive
     removals and CSR builds."""
