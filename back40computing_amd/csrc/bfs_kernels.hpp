@@ -559,6 +559,14 @@ __device__ void tp_contract_phase(const BfsArgs& a, int ph, int32_t depth_here, 
     lq_flush<false>(s.q, out, 1);
 }
 
+// A workgroup takes at least this many vertices: each reserves its output at one
+// address (11.4 ns apiece), which on narrow levels, dealt out to all workgroups
+// of a persistent launch one vertex each, took longer than the expansion.  One-
+// launch searches with 1 / 4 / 16 vertices at least: 10^3 lattice 308 / 266 / 248 us,
+// 20^3 668 / 640 / 549, a comb of 400 vertices a level 11.9 / 10.8 / 9.1 ms; RMAT-12,
+// whose few vertices have long lists, 104 / 105 / 110 us, RMAT-14 131 / 133 / 136.
+constexpr uint32_t TP_EXPAND_ENTRIES = 16;
+
 // Two-phase expand (vertex frontier -> edge frontier of (neighbour, pred)),
 // two_phase/expand_atomic/cta.cuh:606-719.  No culling: lists below the
 // grid threshold are expanded in place per tile, longer ones by k_heavy.
@@ -569,7 +577,7 @@ __device__ void tp_expand_phase(const BfsArgs& a, int ph, int32_t depth_here, Li
     const int32_t* qin = a.qk[ph & 1];
     const GlobalQueue out = out_queue(a, ph);
     InPlaceSink sink{out, l};
-    const uint32_t wgs = sharing_wgs(a, n_in, gridDim.x);
+    const uint32_t wgs = min(sharing_wgs(a, n_in, gridDim.x), (n_in + TP_EXPAND_ENTRIES - 1) / TP_EXPAND_ENTRIES);
     const Deal deal = deal_out(n_in, wgs, false);
     for (uint32_t base = 0; blockIdx.x < wgs && base < n_in; base += wgs * BFS_THREADS) {
         const uint32_t i = deal.entry(base, blockIdx.x);
