@@ -643,6 +643,52 @@ void case_batched(int levels, int persistent) {
     b40c_multigraph_destroy(mg);
 }
 
+// Which results are copied out: in the order of submission many at a time, in
+// other orders none that is not asked for next.  One workgroup per query copied.
+void case_result_orders() {
+    const HostGraph h = skewed_graph(8, 8, true, 1);
+    DeviceGraph g(h);
+    b40c_multigraph* mg = nullptr;
+    OK(b40c_multigraph_pack(&g.g, 1, &mg));
+    const int Q = 60;
+    for (const char* form : {"submitted", "reversed", "evens first", "shuffled"}) {
+        b40c_msbfs* m = nullptr;
+        OK(b40c_msbfs_create(mg, 1 << 22, Q, &m));
+        std::vector<int32_t> ids((size_t)Q), take;
+        for (int k = 0; k < Q; ++k) OK(b40c_msbfs_submit(m, 0, k, &ids[(size_t)k]));
+        OK(b40c_msbfs_run(m));
+        for (int k = 0; k < Q; ++k) take.push_back(form[0] == 'r' ? Q - 1 - k : form[0] == 'e' ? (2 * k < Q ? 2 * k : 2 * k - Q + 1) : k);
+        if (form[1] == 'h') std::shuffle(take.begin(), take.end(), std::mt19937(1));
+        std::atomic<int> copied{0}, launches{0};
+        emu::dev().on_start = [&](const std::string& k, unsigned id) {
+            if (k != "k_ms_stage") return;
+            ++copied;
+            if (id == 0) ++launches;
+        };
+        for (int32_t k : take) {
+            std::vector<int32_t> depth((size_t)h.n);
+            OK(b40c_msbfs_result(m, ids[(size_t)k], depth.data(), nullptr, nullptr));
+            REQUIRE(depth == serial_bfs(h, k), "query %d", k);
+        }
+        std::printf("%s: %d copied by %d launches\n", form, copied.load(), launches.load());
+        std::fflush(stdout);
+        if (form[0] == 's' && form[1] == 'u') {
+            REQUIRE(copied == Q && launches <= 7, "more copies or launches than a doubling window takes");
+            // The next batch goes on with the window learnt.
+            launches = 0;
+            for (int k = 0; k < Q; ++k) OK(b40c_msbfs_submit(m, 0, k, &ids[(size_t)k]));
+            OK(b40c_msbfs_run(m));
+            for (int k = 0; k < Q; ++k) OK(b40c_msbfs_result(m, ids[(size_t)k], std::vector<int32_t>((size_t)h.n).data(), nullptr, nullptr));
+            REQUIRE(launches <= 2, "%d launches for a second batch", launches.load());
+        } else {
+            REQUIRE(copied <= Q + Q / 10, "results were copied that were not asked for next");
+        }
+        emu::dev().on_start = nullptr;
+        b40c_msbfs_destroy(m);
+    }
+    b40c_multigraph_destroy(mg);
+}
+
 }  // namespace
 
 int main(int argc, char** argv) {
@@ -686,6 +732,8 @@ int main(int argc, char** argv) {
         case_scan_segments();
     else if (name == "builds")
         case_builds();
+    else if (name == "result_orders")
+        case_result_orders();
     else if (name == "batched")
         case_batched(arg(0), arg(1));
     else

@@ -122,3 +122,9 @@ def test_tiny_queues(check):
     """A sizing factor that asks for less than one queue entry: no value array
     was allocated for an edge frontier's single one."""
     check("tiny_queues")
+
+
+def test_orders_of_results(check):
+    """Batched results taken in and out of the order of submission: out of it,
+    every second window held a result that was not asked for next."""
+    check("result_orders")
