@@ -405,15 +405,19 @@ void case_sorts() {
     for (size_t n : {1000, 9000, 30001}) sort_pairs(n, 20);
 }
 
-// A place whose second block starts after the bounded waits have run out: the
+// A place whose second block starts after a server's bounded wait has run out: the
 // sort fails, and the places after it, whose digit totals no longer hold, write
 // nothing outside the arrays.
 void case_sort_wait_runs_out() {
     emu::dev().chain_spins = 50;
-    std::atomic<int> places{0};
+    std::atomic<int> places{0}, servers_ended{0};
     emu::dev().on_start = [&](const std::string& k, unsigned id) {
         if (k.find("k_place") == std::string::npos || id != 16 + 1) return;
-        if (places++ == 0) std::this_thread::sleep_for(std::chrono::milliseconds(1500));
+        if (places++ == 0)
+            while (servers_ended.load() == 0) sched_yield();
+    };
+    emu::dev().on_end = [&](const std::string& k, unsigned id) {
+        if (k.find("k_place") != std::string::npos && id < 16) ++servers_ended;
     };
     const size_t n = 20000;
     const std::vector<uint64_t> k = random_keys(n, 64, 5);
@@ -424,6 +428,7 @@ void case_sort_wait_runs_out() {
     REQUIRE(s == B40C_ERR_HIP, "the sort returned %d", (int)s);
     emu::dev().chain_spins = 1u << 22;
     emu::dev().on_start = nullptr;
+    emu::dev().on_end = nullptr;
     sort_u64(n, 64);
 }
 
