@@ -48,7 +48,8 @@ SPACE = {
     "persistent_wgs_per_cu": [1, 2, 3, 4, 6, 8],
 }
 
-# Knobs that matter per strategy.
+# Knobs that matter per strategy (direction-optimizing reads the grid tier's
+# threshold on graphs that are not symmetric).
 KNOBS = {
     _lib.EXPAND_CONTRACT: ["persistent_wgs_per_cu", "grid_gather_threshold", "grid_size", "levels_per_sync"],
     _lib.CONTRACT_EXPAND: ["persistent_wgs_per_cu", "grid_gather_threshold", "grid_size", "levels_per_sync"],
