@@ -203,6 +203,28 @@ void case_wide_persistent() {
     }
 }
 
+// Instrumented enactors: the average duty is a share of the workgroups' time,
+// whatever launches a search is made of.
+void case_duty() {
+    for (const HostGraph& h : {skewed_graph(9, 8, true, 1), grid_graph(7), star_graph(3000)}) {
+        DeviceGraph g(h);
+        for (int32_t strategy = 0; strategy < 6; ++strategy)
+            for (int32_t mode = 0; mode < 3; ++mode) {
+                Problem p(g.g);
+                b40c_tuning t{};
+                t.saturation_quit = 4;
+                t.grid_gather_threshold = 64;
+                Enactor e(strategy, &t, 1);
+                search(h, p.p, e.e, 0, mode);
+                double duty = 0;
+                OK(b40c_get_statistics(e.e, nullptr, nullptr, &duty));
+                std::printf("%s %s mode %d: duty %.3f\n", h.name.c_str(), kStrategies[strategy], mode, duty);
+                std::fflush(stdout);
+                REQUIRE(duty > 0 && duty <= 1, "a duty of %.3f", duty);
+            }
+    }
+}
+
 // Several strategies in turn on one problem: what one leaves behind is not the
 // next one's input.  `first_sync` levels per host check for direction-optimizing.
 void case_shared_problem(int first_sync) {
@@ -717,6 +739,8 @@ int main(int argc, char** argv) {
         case_no_frontier_pieces();
     else if (name == "tiny_queues")
         case_tiny_queues();
+    else if (name == "duty")
+        case_duty();
     else if (name == "shared_problem")
         case_shared_problem(arg(0));
     else if (name == "sorts")

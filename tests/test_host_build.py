@@ -128,3 +128,9 @@ def test_orders_of_results(check):
     """Batched results taken in and out of the order of submission: out of it,
     every second window held a result that was not asked for next."""
     check("result_orders")
+
+
+def test_average_duty(check):
+    """Instrumented searches of every strategy and mode report a duty of at most
+    one: hybrid's level launches counted as work but not as time."""
+    check("duty")
