@@ -168,18 +168,18 @@ constexpr int CSR_ITEMS = 16;
 constexpr int64_t CSR_BLOCK = (int64_t)CHAIN_THREADS * CSR_ITEMS;
 constexpr int64_t CSR_LONG_GAP = 16;  // rows opened by one key that the wave fills together
 
+template <bool REST>
 __global__ __launch_bounds__(CHAIN_THREADS) void k_csr_chained(const uint64_t* keys, int64_t nkeys, int shift,
                                                                uint64_t sentinel, int32_t n, int32_t* cols,
-                                                               int32_t* offsets, unsigned long long* chain,
-                                                               ChainReport* report) {
+                                                               int32_t* offsets, Chain chain) {
     __shared__ uint32_t s_tot[CHAIN_WAVES];
-    __shared__ uint64_t s_before;
+    __shared__ unsigned long long s_before;
     __shared__ ChainServeShared s_serve;
-    if (blockIdx.x == 0) {
-        chain_serve(chain, gridDim.x - 1, report, s_serve);
+    if (chain_serves<REST>()) {
+        chain_serve(chain, s_serve, chain.before, 0);
         return;
     }
-    const int block = blockIdx.x - 1;
+    const int block = chain_block<REST>(chain);
     const int lane = lane_id(), wid = threadIdx.x / kWave;
     const int64_t begin = (int64_t)block * CSR_BLOCK + (int64_t)wid * kWave * CSR_ITEMS;
     uint64_t x[CSR_ITEMS];
@@ -212,10 +212,11 @@ __global__ __launch_bounds__(CHAIN_THREADS) void k_csr_chained(const uint64_t* k
             s_tot[w] = (uint32_t)mine;
             mine += t;
         }
-        s_before = chain_before(chain, block, mine, report);
+        s_before = chain_before<REST>(chain, block, mine);
     }
     __syncthreads();
-    uint64_t pos = s_before + s_tot[wid];
+    if (!s_before) return;
+    uint64_t pos = (s_before & CHAIN_VALUE) + s_tot[wid];
     const uint64_t mask = (1ull << shift) - 1;
     last = first_left;
 #pragma unroll
@@ -388,10 +389,10 @@ b40c_status csr_from_sorted_keys(const KeyArena& a, int64_t nkeys, int shift, ui
         const int64_t blocks = (nkeys + CSR_BLOCK - 1) / CSR_BLOCK;
         ChainCall call;
         B40C_TRY(call.start(blocks, stream, a.scratch));
-        hipLaunchKernelGGL(k_csr_chained, dim3((unsigned)blocks + 1), dim3(CHAIN_THREADS), 0, stream, a.k0, nkeys,
-                           shift, sentinel, n, reinterpret_cast<int32_t*>(a.k1), g->offsets.as<int32_t>(), call.chain,
-                           call.report);
-        B40C_TRY(call.finish("CSR build", E, stream));
+        B40C_TRY(call.run(blocks, 0, E, stream, [&](const Chain& chain, unsigned wgs, bool rest) {
+            hipLaunchKernelGGL(rest ? k_csr_chained<true> : k_csr_chained<false>, dim3(wgs), dim3(CHAIN_THREADS), 0, stream, a.k0, nkeys, shift, sentinel,
+                               n, reinterpret_cast<int32_t*>(a.k1), g->offsets.as<int32_t>(), chain);
+        }));
     }
     if (E > 0x7FFFFFFFull)
         return fail(B40C_ERR_UNSUPPORTED, "CSR with %llu edges exceeds int32 offsets", (unsigned long long)E);

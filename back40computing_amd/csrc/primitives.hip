@@ -172,25 +172,26 @@ constexpr int64_t kChainScanMax = 1ll << 30;  // sums of 32-bit values stay belo
 constexpr int SCAN_SUB = 8;
 constexpr int64_t SCAN_BLOCK = (int64_t)PT * VEC32 * SCAN_SUB;
 
-// Arrays are scanned in segments of at most kScanSegment elements, one launch
-// each, the total so far in the report: their chain words stay below 2 MB, which
+// Arrays are scanned in segments of at most kScanSegment elements, one after the
+// other: their chain words stay below 2 MB, which
 // the runtime serves from chunks it keeps (8 us after an upload).  More are mapped
 // anew on every call: 2^28 elements in place after an upload took 790 us, with
 // 550 to 610 in segments, as three passes 650 to 730.
 constexpr int64_t kScanSegment = (1ll << 28) - (1ll << 20);
 
+template <bool REST>
 __global__ __launch_bounds__(PT) void k_scan_chained(const uint32_t* in, uint32_t* out, int64_t n, int inclusive,
-                                                     int first, unsigned long long* chain, ChainReport* report) {
+                                                     Chain chain) {
     static_assert(SCAN_SUB * PW <= kWave, "one wave scans the waves' totals");
     __shared__ uint32_t s_tot[SCAN_SUB * PW];
     __shared__ uint64_t s_sum[PW];
-    __shared__ uint32_t s_before;
+    __shared__ unsigned long long s_before;
     __shared__ ChainServeShared s_serve;
-    if (blockIdx.x == 0) {
-        chain_serve(chain, gridDim.x - 1, report, s_serve, first ? 0 : report->total);
+    if (chain_serves<REST>()) {
+        chain_serve(chain, s_serve, chain.before, 0);
         return;
     }
-    const int block = blockIdx.x - 1;
+    const int block = chain_block<REST>(chain);
     const int64_t begin = (int64_t)block * SCAN_BLOCK;
     const int tid = threadIdx.x, lane = lane_id(), wid = tid / kWave;
     uint32_t x[SCAN_SUB][4];
@@ -214,14 +215,15 @@ __global__ __launch_bounds__(PT) void k_scan_chained(const uint32_t* in, uint32_
         uint64_t mine = 0;
 #pragma unroll
         for (int w = 0; w < PW; ++w) mine += s_sum[w];
-        if (lane == 0) s_before = (uint32_t)chain_before(chain, block, mine, report);
+        if (lane == 0) s_before = chain_before<REST>(chain, block, mine);
     } else if (wid == 1) {
         const uint32_t t = lane < SCAN_SUB * PW ? s_tot[lane] : 0u;
         const uint32_t incl = wave_scan_incl(t);
         if (lane < SCAN_SUB * PW) s_tot[lane] = incl - t;
     }
     __syncthreads();
-    const uint32_t before = s_before;
+    if (__builtin_amdgcn_readfirstlane((int)(s_before >> 32)) == 0) return;  // (a set word has its top bit)
+    const uint32_t before = (uint32_t)s_before;
 #pragma unroll
     for (int k = 0; k < SCAN_SUB; ++k) {
         const int64_t i = begin + (int64_t)k * PT * VEC32 + tid * VEC32;
@@ -252,18 +254,18 @@ __global__ __launch_bounds__(PT) void k_scan_chained(const uint32_t* in, uint32_
 constexpr int TRIM_ITEMS = 16;
 constexpr int64_t TRIM_BLOCK = (int64_t)PT * TRIM_ITEMS;
 
-template <bool VALS>
+template <bool VALS, bool REST>
 __global__ __launch_bounds__(PT) void k_trim_chained(const uint64_t* keys, const uint32_t* vals, int64_t n,
                                                      uint64_t* keys_out, uint32_t* vals_out,
-                                                     unsigned long long* chain, ChainReport* report) {
+                                                     Chain chain) {
     __shared__ uint32_t s_tot[PW];
-    __shared__ uint64_t s_before;
+    __shared__ unsigned long long s_before;
     __shared__ ChainServeShared s_serve;
-    if (blockIdx.x == 0) {
-        chain_serve(chain, gridDim.x - 1, report, s_serve);
+    if (chain_serves<REST>()) {
+        chain_serve(chain, s_serve, chain.before, 0);
         return;
     }
-    const int block = blockIdx.x - 1;
+    const int block = chain_block<REST>(chain);
     const int lane = lane_id(), wid = threadIdx.x / kWave;
     const int64_t begin = (int64_t)block * TRIM_BLOCK + (int64_t)wid * kWave * TRIM_ITEMS;
     uint64_t x[TRIM_ITEMS];
@@ -297,10 +299,11 @@ __global__ __launch_bounds__(PT) void k_trim_chained(const uint64_t* keys, const
             s_tot[w] = (uint32_t)mine;
             mine += t;
         }
-        s_before = chain_before(chain, block, mine, report);
+        s_before = chain_before<REST>(chain, block, mine);
     }
     __syncthreads();
-    uint64_t pos = s_before + s_tot[wid];
+    if (!s_before) return;
+    uint64_t pos = (s_before & CHAIN_VALUE) + s_tot[wid];
 #pragma unroll
     for (int k = 0; k < TRIM_ITEMS; ++k) {
         if ((heads[k] >> lane) & 1u) {
@@ -376,14 +379,13 @@ b40c_status b40c_consecutive_removal_u64(const uint64_t* d_keys_in, const uint32
     if (blocks >= INT32_MAX) return fail(B40C_ERR_INVALID_ARG, "b40c_consecutive_removal_u64: n out of range");
     ChainCall call;
     B40C_TRY(call.start(blocks, nullptr));
-    if (d_values_in)
-        hipLaunchKernelGGL(k_trim_chained<true>, dim3((unsigned)blocks + 1), dim3(PT), 0, nullptr, d_keys_in,
-                           d_values_in, n, d_keys_out, d_values_out, call.chain, call.report);
-    else
-        hipLaunchKernelGGL(k_trim_chained<false>, dim3((unsigned)blocks + 1), dim3(PT), 0, nullptr, d_keys_in,
-                           d_values_in, n, d_keys_out, d_values_out, call.chain, call.report);
     uint64_t total = 0;
-    B40C_TRY(call.finish("b40c_consecutive_removal_u64", total, nullptr));
+    B40C_TRY(call.run(blocks, 0, total, nullptr, [&](const Chain& chain, unsigned wgs, bool rest) {
+        auto* kernel = d_values_in ? (rest ? k_trim_chained<true, true> : k_trim_chained<true, false>)
+                                   : (rest ? k_trim_chained<false, true> : k_trim_chained<false, false>);
+        hipLaunchKernelGGL(kernel, dim3(wgs), dim3(PT), 0, nullptr, d_keys_in, d_values_in, n, d_keys_out,
+                           d_values_out, chain);
+    }));
     *num_compacted = (int64_t)total;
     return B40C_OK;
 }
@@ -396,17 +398,17 @@ b40c_status b40c_scan_u32(const uint32_t* d_in, uint32_t* d_out, int64_t n, int3
     if (n == 0) return B40C_OK;
     if (aligned16(d_in) && aligned16(d_out) && n <= kChainScanMax) {
         ChainCall call;
-        for (int64_t at = 0; at < n; at += kScanSegment) {
-            const int64_t len = std::min<int64_t>(n - at, kScanSegment), blocks = (len + SCAN_BLOCK - 1) / SCAN_BLOCK;
-            if (at == 0)
-                B40C_TRY(call.start(blocks, nullptr));
-            else
-                call.clear(blocks, nullptr);
-            hipLaunchKernelGGL(k_scan_chained, dim3((unsigned)blocks + 1), dim3(PT), 0, nullptr, d_in + at, d_out + at,
-                               len, exclusive ? 0 : 1, at == 0 ? 1 : 0, call.chain, call.report);
-        }
+        B40C_TRY(call.start((std::min<int64_t>(n, kScanSegment) + SCAN_BLOCK - 1) / SCAN_BLOCK, nullptr));
         uint64_t sum = 0;
-        B40C_TRY(call.finish("b40c_scan_u32", sum, nullptr));
+        for (int64_t at = 0; at < n; at += kScanSegment) {
+            const int64_t len = std::min<int64_t>(n - at, kScanSegment);
+            B40C_TRY(call.run((len + SCAN_BLOCK - 1) / SCAN_BLOCK, sum, sum, nullptr,
+                              [&](const Chain& chain, unsigned wgs, bool rest) {
+                                  hipLaunchKernelGGL(rest ? k_scan_chained<true> : k_scan_chained<false>, dim3(wgs),
+                                                     dim3(PT), 0, nullptr, d_in + at, d_out + at, len,
+                                                     exclusive ? 0 : 1, chain);
+                              }));
+        }
         if (total) *total = sum;
         return B40C_OK;
     }

@@ -559,6 +559,62 @@ void case_primitives() {
     }
 }
 
+// Calls `f` while the workgroup `late` of every kernel whose name holds `kernel`
+// starts only when a workgroup below `servers` has ended, which it does only by
+// giving up waiting; returns how often that happened.
+int with_late_workgroup(const char* kernel, unsigned late, unsigned servers, const std::function<void()>& f) {
+    std::atomic<int> gave_up{0}, held{0};
+    emu::dev().chain_spins = 50;
+    emu::dev().on_start = [&](const std::string& k, unsigned id) {
+        if (k.find(kernel) == std::string::npos || id != late) return;
+        const int before = gave_up.load();
+        if (held++ == 0)
+            while (gave_up.load() == before) sched_yield();
+    };
+    emu::dev().on_end = [&](const std::string& k, unsigned id) {
+        if (k.find(kernel) != std::string::npos && id < servers) ++gave_up;
+    };
+    f();
+    emu::dev().chain_spins = 1u << 14;
+    emu::dev().on_start = nullptr;
+    emu::dev().on_end = nullptr;
+    return held.load();
+}
+
+// Chained calls one of whose blocks starts after the serving workgroup has given
+// up: what the others then leave undone is finished.
+void case_late_blocks() {
+    const size_t n = 9 * 8192 + 77;
+    const std::vector<uint64_t> k = random_keys(n, 40, 9);
+    std::vector<uint32_t> x(k.begin(), k.end()), y(n);
+    uint64_t sum = 0;
+    for (size_t i = 0; i < n; ++i) {
+        y[i] = (uint32_t)sum;
+        sum += x[i];
+    }
+    std::vector<uint64_t> wk;
+    for (size_t i = 0; i < n; ++i)
+        if (i == 0 || k[i] != k[i - 1]) wk.push_back(k[i]);
+    for (unsigned late : {1u, 2u, 8u}) {
+        std::printf("workgroup %u late\n", late);
+        std::fflush(stdout);
+        DeviceArray<uint32_t> in(x);
+        const int scans = with_late_workgroup("k_scan_chained", late, 1, [&] {
+            uint64_t total = 0;
+            OK(b40c_scan_u32(in.ptr(), in.ptr(), (int64_t)n, 1, &total));
+            REQUIRE(total == sum, "the total");
+        });
+        REQUIRE(scans > 0 && in.get(n) == y, "the scan");
+        DeviceArray<uint64_t> ka(k), kb(n);
+        const int trims = with_late_workgroup("k_trim_chained", late, 1, [&] {
+            int64_t kept = 0;
+            OK(b40c_consecutive_removal_u64(ka.ptr(), nullptr, kb.ptr(), nullptr, (int64_t)n, &kept));
+            REQUIRE(kept == (int64_t)wk.size(), "%lld kept", (long long)kept);
+        });
+        REQUIRE(trims > 0 && kb.get(wk.size()) == wk, "the removal");
+    }
+}
+
 // Scans of several launches: whole and partial last blocks and segments.
 void case_scan_segments() {
     const size_t block = 8192;
@@ -757,6 +813,8 @@ int main(int argc, char** argv) {
         case_short_of_memory();
     else if (name == "primitives")
         case_primitives();
+    else if (name == "late_blocks")
+        case_late_blocks();
     else if (name == "scan_segments")
         case_scan_segments();
     else if (name == "builds")

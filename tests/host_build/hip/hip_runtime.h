@@ -101,7 +101,7 @@ struct Device {
     std::map<std::string, int> occupancies;
     size_t largest_alloc = ~(size_t)0;  // larger device allocations fail
     bool lazy = false;
-    unsigned chain_spins = 1u << 22;    // polls of a bounded wait
+    unsigned chain_spins = 1u << 14;    // polls of a bounded wait
     int label_claim_nodes = 1 << 20;
     long long scan_segment = 1 << 27;   // elements of a scan's launch
     // Called as a workgroup starts (kernel's name, workgroup); may wait.

@@ -134,3 +134,10 @@ def test_average_duty(check):
     """Instrumented searches of every strategy and mode report a duty of at most
     one: hybrid's level launches counted as work but not as time."""
     check("duty")
+
+
+def test_late_blocks(check):
+    """Scans and removals where a block cannot start while the others wait for
+    it (as beside a persistent kernel that holds the GPU): the call finishes what
+    gave up; it failed."""
+    check("late_blocks")
