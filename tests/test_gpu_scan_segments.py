@@ -1,10 +1,12 @@
 """Prefix sums of more than one launch: arrays around one segment (2^28 - 2^20
-elements) and of several, against torch's 64-bit sums on the device."""
+elements) and of several, exclusive and, in place, inclusive."""
 import ctypes
 
+import numpy as np
 import pytest
 
 from back40computing_amd._lib import check, lib
+from back40computing_amd.radix_sort import DeviceArray
 
 pytestmark = pytest.mark.gpu
 
@@ -13,17 +15,17 @@ SEGMENT = (1 << 28) - (1 << 20)
 
 @pytest.mark.parametrize("n", [SEGMENT, SEGMENT + 1, 2 * SEGMENT + 8193])
 def test_scan_segments(n):
-    import torch
     print("scan segments", n, flush=True)
-    x = torch.randint(-2 ** 31, 2 ** 31, (n,), dtype=torch.int64, device="cuda", generator=torch.Generator("cuda").manual_seed(n))
-    sums = torch.cumsum(x.bitwise_and_(0xFFFFFFFF), 0)
-    x = x.to(torch.int32)
-    torch.cuda.synchronize()
+    x = np.random.default_rng(n).integers(0, 1 << 32, n, dtype=np.uint32)
+    incl = np.cumsum(x, dtype=np.uint32)  # modulo 2^32
+    sum64 = int(x.sum(dtype=np.uint64))
+    src, dst = DeviceArray(4 * n), DeviceArray(4 * n)
+    src.upload(x)
     total = ctypes.c_uint64()
-    out = torch.empty_like(x)
-    check(lib().b40c_scan_u32(x.data_ptr(), out.data_ptr(), n, 0, ctypes.byref(total)))
-    assert total.value == int(sums[-1])
-    assert torch.equal(out, sums.to(torch.int32))
-    check(lib().b40c_scan_u32(x.data_ptr(), x.data_ptr(), n, 1, ctypes.byref(total)))
-    assert total.value == int(sums[-1])
-    assert int(x[0]) == 0 and torch.equal(x[1:], out[:-1])
+    check(lib().b40c_scan_u32(src.ptr, dst.ptr, n, 1, ctypes.byref(total)))
+    assert total.value == sum64
+    out = dst.download(np.uint32, n)
+    assert out[0] == 0 and np.array_equal(out[1:], incl[:-1])
+    check(lib().b40c_scan_u32(src.ptr, src.ptr, n, 0, ctypes.byref(total)))
+    assert total.value == sum64
+    assert np.array_equal(src.download(np.uint32, n), incl)
