@@ -119,16 +119,20 @@ struct SortState {
     uint32_t* copies;   // [HIST_COPIES][MAX_PLACES][RS_BINS] digit totals, spread over copies
     uint32_t* base;     // [MAX_PLACES][RS_BINS] first output position of each digit
     uint32_t* trivial;  // [MAX_PLACES] place whose keys all share one digit
-    uint32_t* failed;   // first place + 1 whose waits ran out, beside `trivial`
+    uint32_t* failed;   // beside `trivial`: a place with unfinished blocks (place + 1), and how many it has
+    uint32_t* served;   // where a serving workgroup gave up: blocks served, and each digit's next start
     uint32_t* status;   // [2][blocks][RS_BINS] chain words (by place parity), 32 or 64 bits each
-    int32_t* out;       // report: selector, failure
+    int32_t* out;       // report: selector, unfinished place + 1
     int32_t blocks;
     int32_t wide;       // 64-bit chain words (n >= 2^30)
     int32_t grouped;    // blocks in the order of place_block, else in the workgroups'
     int32_t places;
 };
 constexpr size_t kReportWords = 16;  // the report, where it is in the scratch (first words)
-constexpr size_t kStateWords = kReportWords + (size_t)(HIST_COPIES + 1) * MAX_PLACES * RS_BINS + 64;
+constexpr size_t kStateWords = kReportWords + (size_t)(HIST_COPIES + 1) * MAX_PLACES * RS_BINS + RS_BINS + 64;
+// The unfinished blocks of a place are listed where the totals were, 16 bits each.
+static_assert(kMaxBlocks * 2 <= (int64_t)HIST_COPIES * MAX_PLACES * RS_BINS * 4 && kMaxBlocks <= 1 << 16,
+              "every block fits the list");
 
 // Clears the totals and the first place's chain words.
 __global__ __launch_bounds__(256) void k_sort_init(SortState st) {
@@ -138,7 +142,7 @@ __global__ __launch_bounds__(256) void k_sort_init(SortState st) {
     const int64_t words = (int64_t)st.blocks * RS_BINS * (st.wide ? 2 : 1);
     for (int64_t i = i0; i < words; i += step) st.status[i] = 0;
     if (i0 < 2) st.out[i0] = 0;
-    if (i0 == 0) *st.failed = 0;
+    if (i0 < 2) st.failed[i0] = 0;
 }
 
 // Digit totals of every place in one read, eight keys per thread at a time.
@@ -214,14 +218,21 @@ __global__ __launch_bounds__(RS_BINS) void k_plan(SortState st, int64_t n) {
 // Chain of the blocks of a place: one word per block and digit, the block's
 // count first (COUNT), then the digit's next output position where the block
 // starts (START), which a serving workgroup puts in its place.
-constexpr uint32_t kChainSpins = 1u << 22;
-// A bounded wait of `place` has run out.  What the place then writes lies in the
-// output, but is no permutation of the keys: the digit totals do not hold for
-// it, and later places that went by them would write past the arrays.
+//
+// No wait needs to end.  A place and a persistent kernel of another stream that
+// are each partly resident keep the other's missing workgroups off the GPU (XCDs
+// dispatch on their own, so even a block's predecessors may be missing).  A
+// serving workgroup gives up after kChainSpins polls without new counts (about 50
+// ms; a place of 2^26 keys takes 0.3, and the long blocks of 2^32 keys should publish
+// 15 apart at most); blocks without their starts then list themselves and leave
+// their keys where they are, later places move nothing, and the host finishes the
+// place (no block waits any more: all counts are there) and the places after it.
+constexpr uint32_t kChainSpins = 1u << 16;
 __device__ __forceinline__ void place_failed(const SortState& st, int place) {
-    st.out[1] = 1;
-    st.failed[0] = (uint32_t)place + 1;
+    st.out[1] = place + 1;
+    st_relaxed(st.failed, (uint32_t)place + 1);
 }
+__device__ __forceinline__ uint16_t* unfinished_blocks(const SortState& st) { return (uint16_t*)st.copies; }
 template <typename W>
 struct ChainWord {
     static constexpr W COUNT = (W)1 << (8 * sizeof(W) - 2);
@@ -243,9 +254,7 @@ __device__ __forceinline__ void chain_store(W* status, int block, int d, W w) {
 // one digit.  Workgroups are dispatched in order, so the servers run, and the
 // lowest block without counts runs, or will as soon as there is room for it beside
 // the workgroups dispatched before it that wait for it (none in plain order, up to
-// GROUPED_AHEAD in that of place_block).  Should other kernels leave less room, the
-// bounded wait records it (place_failed) and the remaining blocks go on with the
-// starts there are (which lie in the output).
+// GROUPED_AHEAD in that of place_block); other kernels may leave less room (above).
 constexpr int SERVE_DIGITS = 16;  // one 64-byte line of 32-bit words
 constexpr int SERVERS = RS_BINS / SERVE_DIGITS;
 constexpr int SERVE_SUBS = kWave / SERVE_DIGITS;
@@ -263,16 +272,19 @@ struct ServeShared {
     int lead[OS_WAVES];
 };
 
-template <typename W, int ROW>
+// RESUME: goes on where the serving workgroup of the place stopped.
+template <typename W, int ROW, bool RESUME>
 __device__ __forceinline__ void serve_place(W* status, const SortState& st, int place, ServeShared& s) {
     constexpr int WAVE_BLOCKS = SERVE_SUBS * ROW;
     const int tid = threadIdx.x, lane = lane_id(), wid = tid / kWave;
     const int col = lane % SERVE_DIGITS, sub = lane / SERVE_DIGITS;
     const int d = (int)blockIdx.x * SERVE_DIGITS + col;
     const int blocks = st.blocks;
-    W start = (W)st.base[place * RS_BINS + d];
+    W start = (W)(RESUME ? st.served[SERVERS + d] : st.base[place * RS_BINS + d]);
     uint32_t spins = 0;
-    for (int first = 0; first < blocks;) {
+    int first = RESUME ? (int)st.served[blockIdx.x] : 0;
+    if (RESUME && chain_load(status, blocks - 1, d) >= ChainWord<W>::START) return;  // served all
+    while (first < blocks) {
         const int mine = first + wid * WAVE_BLOCKS + sub * ROW;
         W w[ROW];
 #pragma unroll
@@ -327,12 +339,15 @@ __device__ __forceinline__ void serve_place(W* status, const SortState& st, int 
         __syncthreads();
         start = next;
         first += taken;
-        if (taken == 0) {
+        if (taken) {
+            spins = 0;
+        } else {
             if (++spins > kChainSpins) {
-                if (tid == 0) place_failed(st, place);
-                for (int b = first + tid / SERVE_DIGITS; b < blocks; b += OS_THREADS / SERVE_DIGITS)
-                    chain_store(status, b, (int)blockIdx.x * SERVE_DIGITS + tid % SERVE_DIGITS,
-                                (W)(ChainWord<W>::START | start));
+                if (tid < SERVE_DIGITS) st.served[SERVERS + d] = (uint32_t)start;
+                if (tid == 0) {
+                    st.served[blockIdx.x] = (uint32_t)first;
+                    place_failed(st, place);
+                }
                 return;
             }
             __builtin_amdgcn_s_sleep(1);
@@ -340,19 +355,29 @@ __device__ __forceinline__ void serve_place(W* status, const SortState& st, int 
     }
 }
 
-// Where digit d of a block goes: waits for its server.
+template <bool RESUME>
+__device__ __forceinline__ void serve_place(uint32_t* status, const SortState& st, int place, ServeShared& s) {
+    if (st.wide)
+        serve_place<unsigned long long, SERVE_ROW_MANY, RESUME>((unsigned long long*)status, st, place, s);
+    else if (st.blocks <= SERVE_FEW_BLOCKS)
+        serve_place<uint32_t, SERVE_ROW_FEW, RESUME>(status, st, place, s);
+    else
+        serve_place<uint32_t, SERVE_ROW_MANY, RESUME>(status, st, place, s);
+}
+
+// The word with the start of a block's digit d, from its server.  Zero: gave up.
 template <typename W>
-__device__ __forceinline__ uint32_t await_start(const W* status, int block, int d, const SortState& st, int place) {
+__device__ __forceinline__ W await_start(const W* status, int block, int d, const SortState& st, int place) {
     W w;
     uint32_t spins = 0;
     while ((w = chain_load(status, block, d)) < ChainWord<W>::START) {
-        if (++spins > kChainSpins) {
+        if (++spins % 16 == 0 && (ld_relaxed(st.failed) || spins > 4 * kChainSpins)) {
             place_failed(st, place);
             return 0;
         }
         __builtin_amdgcn_s_sleep(2);
     }
-    return (uint32_t)(w & ChainWord<W>::VALUE);
+    return w;
 }
 
 // Block of the i-th working workgroup.  Workgroups go to the XCDs in turn; of
@@ -377,7 +402,8 @@ __device__ __forceinline__ int place_block(int i, int blocks, bool grouped) {
 // starts: 2^26 64-bit keys take 320 us (1.07 GB of keys in and out, 3.4 TB/s; 295
 // us with the wait left out), where counting and scattering kernels took 590.
 // The order of the XCDs (place_block) gives 20 to 30 us of that.
-template <typename K, int CONV, bool VALS, int ITEMS>
+// REST: the listed blocks of a place, whose starts are all there.
+template <typename K, int CONV, bool VALS, int ITEMS, bool REST>
 __global__ __launch_bounds__(OS_THREADS) void k_place(K* k0, K* k1, uint32_t* v0, uint32_t* v1, int64_t n, int place,
                                                       int shift, uint32_t mask, int64_t block_keys, SortState st) {
     constexpr int TILE = OS_THREADS * ITEMS;
@@ -389,31 +415,36 @@ __global__ __launch_bounds__(OS_THREADS) void k_place(K* k0, K* k1, uint32_t* v0
     __shared__ uint32_t tile_excl[RS_BINS];
     __shared__ int s_wave[OS_WAVES];
     __shared__ ServeShared s_serve;
+    __shared__ uint32_t s_gave_up;
 
     const int tid = threadIdx.x, lane = lane_id(), wid = __builtin_amdgcn_readfirstlane(tid / kWave);
-    const int block = place_block((int)blockIdx.x - SERVERS, st.blocks, st.grouped != 0);
+    const int block = REST ? (int)unfinished_blocks(st)[blockIdx.x]
+                           : place_block((int)blockIdx.x - SERVERS, st.blocks, st.grouped != 0);
     const size_t words = (size_t)st.blocks * RS_BINS * (st.wide ? 2 : 1);
-    // The other parity's words of this block, for the next place (its last
-    // user, the place before this one, has finished).
     uint32_t* status = st.status + (place & 1) * words;
-    uint32_t* next_status = st.status + ((place + 1) & 1) * words;
-    if (block >= 0)
-        for (int i = tid; i < RS_BINS * (st.wide ? 2 : 1); i += OS_THREADS)
-            next_status[(size_t)block * RS_BINS * (st.wide ? 2 : 1) + i] = 0;
     int moved = 0;  // places before this one that moved the keys
     for (int p = 0; p < place; ++p) moved += st.trivial[p] ? 0 : 1;
-    const bool skip = st.trivial[place] != 0;
-    const uint32_t failed = st.failed[0];
-    if (place == st.places - 1 && block == 0 && tid == 0) st.out[0] = (moved + (skip ? 0 : 1)) & 1;
-    if (skip || (failed && failed <= (uint32_t)place)) return;  // (failed == place + 1: in this launch, go on)
-    if (block < 0) {
-        if (st.wide)
-            serve_place<unsigned long long, SERVE_ROW_MANY>((unsigned long long*)status, st, place, s_serve);
-        else if (st.blocks <= SERVE_FEW_BLOCKS)
-            serve_place<uint32_t, SERVE_ROW_FEW>(status, st, place, s_serve);
-        else
-            serve_place<uint32_t, SERVE_ROW_MANY>(status, st, place, s_serve);
-        return;
+    // The other parity's words of this block, for the next place (its last user, the
+    // place before this one, has finished); while the starts are on their way, where
+    // the keys' loads need not wait for it (2^25 64-bit keys: 709 us, 720 at the head).
+    auto clear_next = [&] {
+        uint32_t* next_status = st.status + ((place + 1) & 1) * words;
+        for (int i = tid; i < RS_BINS * (st.wide ? 2 : 1); i += OS_THREADS)
+            next_status[(size_t)block * RS_BINS * (st.wide ? 2 : 1) + i] = 0;
+    };
+    if (!REST) {
+        const bool skip = st.trivial[place] != 0;
+        const uint32_t failed = st.failed[0];
+        if (place == st.places - 1 && block == 0 && tid == 0) st.out[0] = (moved + (skip ? 0 : 1)) & 1;
+        if (failed && failed <= (uint32_t)place) return;  // (failed == place + 1: in this launch, go on)
+        if (skip) {
+            if (block >= 0) clear_next();
+            return;
+        }
+        if (block < 0) {
+            serve_place<false>(status, st, place, s_serve);
+            return;
+        }
     }
     const K* kin = (moved & 1) ? k1 : k0;
     K* kout = (moved & 1) ? k0 : k1;
@@ -429,7 +460,7 @@ __global__ __launch_bounds__(OS_THREADS) void k_place(K* k0, K* k1, uint32_t* v0
         else
             chain_store(status, block, tid, ChainWord<uint32_t>::COUNT | count);
     };
-    if (!one_tile) {
+    if (!REST && !one_tile) {
         for (int i = lane; i < RS_BINS; i += kWave) wave_hist[wid][i] = 0;
         __syncthreads();
         for (int64_t tb = begin; tb < end; tb += TILE) {
@@ -450,6 +481,7 @@ __global__ __launch_bounds__(OS_THREADS) void k_place(K* k0, K* k1, uint32_t* v0
             for (int w = 0; w < OS_WAVES; ++w) count += wave_hist[w][tid];
             announce(count);
         }
+        clear_next();
         __syncthreads();
     }
     for (int64_t tile_base = begin; tile_base < end; tile_base += TILE) {
@@ -469,6 +501,7 @@ __global__ __launch_bounds__(OS_THREADS) void k_place(K* k0, K* k1, uint32_t* v0
             if (VALS) val[j] = vt[idx];
         }
         for (int i = lane; i < RS_BINS; i += kWave) wave_hist[wid][i] = 0;
+        if (!REST && tid == 0) s_gave_up = 0;
         __syncthreads();
         rank_tile<K, CONV, ITEMS>(key, rank, wave_hist[wid], wid, tile_n, shift, mask);
         __syncthreads();
@@ -481,8 +514,9 @@ __global__ __launch_bounds__(OS_THREADS) void k_place(K* k0, K* k1, uint32_t* v0
                 wave_hist[w][tid] = cnt;
                 cnt += c;
             }
-            if (one_tile) announce(cnt);
+            if (!REST && one_tile) announce(cnt);
         }
+        if (!REST && one_tile) clear_next();
         int tot;
         const int excl = wg_exclusive_scan<OS_THREADS>((int)cnt, tot, s_wave);
         if (tid < RS_BINS) tile_excl[tid] = (uint32_t)excl;
@@ -498,16 +532,25 @@ __global__ __launch_bounds__(OS_THREADS) void k_place(K* k0, K* k1, uint32_t* v0
         }
         if (tid < RS_BINS) {
             uint32_t at;
-            if (tile_base != begin)
+            if (tile_base != begin) {
                 at = next_out[tid];
-            else if (st.wide)
-                at = await_start((const unsigned long long*)status, block, tid, st, place);
-            else
-                at = await_start((const uint32_t*)status, block, tid, st, place);
+            } else if (st.wide) {
+                const unsigned long long w = await_start((const unsigned long long*)status, block, tid, st, place);
+                if (w == 0) s_gave_up = 1;
+                at = (uint32_t)(w & ChainWord<unsigned long long>::VALUE);
+            } else {
+                const uint32_t w = await_start((const uint32_t*)status, block, tid, st, place);
+                if (w == 0) s_gave_up = 1;
+                at = w & ChainWord<uint32_t>::VALUE;
+            }
             out_shift[tid] = at - (uint32_t)excl;
             next_out[tid] = at + cnt;
         }
         __syncthreads();
+        if (!REST && s_gave_up) {
+            if (tid == 0) unfinished_blocks(st)[atomic_add_u32(&st.failed[1], 1u)] = (uint16_t)block;
+            return;
+        }
 #pragma unroll
         for (int j = 0; j < ITEMS; ++j) {
             const int k = j * OS_THREADS + tid;
@@ -520,6 +563,17 @@ __global__ __launch_bounds__(OS_THREADS) void k_place(K* k0, K* k1, uint32_t* v0
         }
         __syncthreads();
     }
+}
+
+// A place with unfinished blocks: serves all of them (their counts are there).
+__global__ __launch_bounds__(OS_THREADS) void k_place_resume(SortState st, int place) {
+    __shared__ ServeShared s_serve;
+    serve_place<true>(st.status + (place & 1) * (size_t)st.blocks * RS_BINS * (st.wide ? 2 : 1), st, place, s_serve);
+}
+// ... and it is finished.
+__global__ __launch_bounds__(kWave) void k_place_finished(SortState st) {
+    if (threadIdx.x < 2) st.failed[threadIdx.x] = 0;
+    if (threadIdx.x == 0) st.out[1] = 0;
 }
 
 // Every place of a small sort in one workgroup: the keys stay in registers
@@ -642,6 +696,7 @@ SortState sort_state(const SortScratch& sc, const SortPlan& plan, int places, in
     st.base = st.copies + (size_t)HIST_COPIES * MAX_PLACES * RS_BINS;
     st.trivial = st.base + (size_t)MAX_PLACES * RS_BINS;
     st.failed = st.trivial + MAX_PLACES;
+    st.served = st.failed + 2;
     st.status = sc.base + kStateWords;
     st.out = out;
     st.blocks = plan.blocks;
@@ -651,25 +706,41 @@ SortState sort_state(const SortScratch& sc, const SortPlan& plan, int places, in
     return st;
 }
 
+// Places of a sort that stopped at `place`, `blocks` of whose blocks are unfinished.
+struct SortRest {
+    int place = -1;
+    uint32_t blocks = 0;
+};
+
 template <typename K, int CONV, bool VALS, int ITEMS>
 void launch_places(K* k0, K* k1, uint32_t* v0, uint32_t* v1, int64_t n, int begin_bit, int end_bit,
-                   const SortPlan& plan, const SortState& st, hipStream_t stream) {
-    const int64_t clear = (int64_t)HIST_COPIES * MAX_PLACES * RS_BINS + (int64_t)look_words(plan.blocks, plan.wide) / 2;
-    hipLaunchKernelGGL(k_sort_init, dim3((unsigned)std::min<int64_t>((clear + 1023) / 1024, 512)), dim3(256), 0, stream,
-                       st);
-    hipLaunchKernelGGL((k_histogram<K, CONV>), dim3(plan.hist_wgs), dim3(OS_THREADS), 0, stream, (const K*)k0, n,
-                       begin_bit, end_bit, st);
-    hipLaunchKernelGGL(k_plan, dim3(st.places), dim3(RS_BINS), 0, stream, st, n);
-    for (int place = 0, shift = begin_bit; shift < end_bit; shift += 8, ++place) {
-        const uint32_t mask = (1u << std::min(8, end_bit - shift)) - 1u;
-        hipLaunchKernelGGL((k_place<K, CONV, VALS, ITEMS>), dim3(plan.blocks + SERVERS), dim3(OS_THREADS), 0, stream, k0, k1, v0,
-                           v1, n, place, shift, mask, plan.block_keys, st);
+                   const SortPlan& plan, const SortState& st, const SortRest& rest, hipStream_t stream) {
+    auto mask_of = [&](int shift) { return (1u << std::min(8, end_bit - shift)) - 1u; };
+    if (rest.place < 0) {
+        const int64_t clear = (int64_t)HIST_COPIES * MAX_PLACES * RS_BINS + (int64_t)look_words(plan.blocks, plan.wide) / 2;
+        hipLaunchKernelGGL(k_sort_init, dim3((unsigned)std::min<int64_t>((clear + 1023) / 1024, 512)), dim3(256), 0,
+                           stream, st);
+        hipLaunchKernelGGL((k_histogram<K, CONV>), dim3(plan.hist_wgs), dim3(OS_THREADS), 0, stream, (const K*)k0, n,
+                           begin_bit, end_bit, st);
+        hipLaunchKernelGGL(k_plan, dim3(st.places), dim3(RS_BINS), 0, stream, st, n);
+    } else {
+        const int shift = begin_bit + 8 * rest.place;
+        hipLaunchKernelGGL(k_place_resume, dim3(SERVERS), dim3(OS_THREADS), 0, stream, st, rest.place);
+        if (rest.blocks)
+            hipLaunchKernelGGL((k_place<K, CONV, VALS, ITEMS, true>), dim3(rest.blocks), dim3(OS_THREADS), 0, stream,
+                               k0, k1, v0, v1, n, rest.place, shift, mask_of(shift), plan.block_keys, st);
+        hipLaunchKernelGGL(k_place_finished, dim3(1), dim3(kWave), 0, stream, st);
+    }
+    for (int place = rest.place + 1; place < st.places; ++place) {
+        const int shift = begin_bit + 8 * place;
+        hipLaunchKernelGGL((k_place<K, CONV, VALS, ITEMS, false>), dim3(plan.blocks + SERVERS), dim3(OS_THREADS), 0,
+                           stream, k0, k1, v0, v1, n, place, shift, mask_of(shift), plan.block_keys, st);
     }
 }
 
 template <typename K, int CONV>
 void launch_typed(void* k0, void* k1, uint32_t* v0, uint32_t* v1, int64_t n, int begin_bit, int end_bit,
-                  const SortPlan& plan, const SortScratch& sc, int32_t* out, hipStream_t stream) {
+                  const SortPlan& plan, const SortScratch& sc, int32_t* out, const SortRest& rest, hipStream_t stream) {
     if (n <= SMALL_KEYS) {
         if (v0)
             hipLaunchKernelGGL((k_small_sort<K, CONV, true>), dim3(1), dim3(SMALL_THREADS), 0, stream, (K*)k0, (K*)k1,
@@ -680,19 +751,9 @@ void launch_typed(void* k0, void* k1, uint32_t* v0, uint32_t* v1, int64_t n, int
         return;
     }
     const SortState st = sort_state(sc, plan, (end_bit - begin_bit + 7) / 8, out);
-    if (v0) {
-        if (plan.items == 16)
-            launch_places<K, CONV, true, 16>((K*)k0, (K*)k1, v0, v1, n, begin_bit, end_bit, plan, st, stream);
-        else
-            launch_places<K, CONV, true, 8>((K*)k0, (K*)k1, v0, v1, n, begin_bit, end_bit, plan, st, stream);
-    } else {
-        if (plan.items == 16)
-            launch_places<K, CONV, false, 16>((K*)k0, (K*)k1, nullptr, nullptr, n, begin_bit, end_bit, plan, st,
-                                              stream);
-        else
-            launch_places<K, CONV, false, 8>((K*)k0, (K*)k1, nullptr, nullptr, n, begin_bit, end_bit, plan, st,
-                                             stream);
-    }
+    auto launch = v0 ? (plan.items == 16 ? launch_places<K, CONV, true, 16> : launch_places<K, CONV, true, 8>)
+                     : (plan.items == 16 ? launch_places<K, CONV, false, 16> : launch_places<K, CONV, false, 8>);
+    launch((K*)k0, (K*)k1, v0, v1, n, begin_bit, end_bit, plan, st, rest, stream);
 }
 
 int key_bits(int32_t key_type) {
@@ -761,7 +822,7 @@ b40c_status reserve_scratch(DeviceBuffer& mem, size_t words) {
     return mem.reserve(kNoAllocWords * sizeof(uint32_t));
 }
 
-// One sort's report words (selector, failure): a pinned slot, or, without one,
+// One sort's report words (selector, unfinished place + 1): a pinned slot, or, without one,
 // the first words of the scratch, copied back after the sort.
 struct SortReport {
     ReportSlot slot;
@@ -778,18 +839,19 @@ struct SortReport {
 };
 }  // namespace
 
-// Launches the sort (no allocation, no synchronization).
+// Launches the sort, or what is left of it (no allocation, no synchronization).
 static b40c_status radix_sort_launch(int32_t key_type, void* k0, void* k1, uint32_t* v0, uint32_t* v1, int64_t n,
                                      int begin_bit, int end_bit, int num_cus, const SortPolicy& pol,
-                                     const SortScratch& sc, int32_t* report, hipStream_t stream) {
+                                     const SortScratch& sc, int32_t* report, const SortRest& rest,
+                                     hipStream_t stream) {
     const SortPlan plan = sort_plan(n, num_cus, pol, sc.words);
     switch (key_type) {
-        case B40C_KEY_U32: launch_typed<uint32_t, KC_UNSIGNED>(k0, k1, v0, v1, n, begin_bit, end_bit, plan, sc, report, stream); break;
-        case B40C_KEY_I32: launch_typed<uint32_t, KC_SIGNED>(k0, k1, v0, v1, n, begin_bit, end_bit, plan, sc, report, stream); break;
-        case B40C_KEY_F32: launch_typed<uint32_t, KC_FLOAT>(k0, k1, v0, v1, n, begin_bit, end_bit, plan, sc, report, stream); break;
-        case B40C_KEY_U64: launch_typed<uint64_t, KC_UNSIGNED>(k0, k1, v0, v1, n, begin_bit, end_bit, plan, sc, report, stream); break;
-        case B40C_KEY_I64: launch_typed<uint64_t, KC_SIGNED>(k0, k1, v0, v1, n, begin_bit, end_bit, plan, sc, report, stream); break;
-        case B40C_KEY_F64: launch_typed<uint64_t, KC_FLOAT>(k0, k1, v0, v1, n, begin_bit, end_bit, plan, sc, report, stream); break;
+        case B40C_KEY_U32: launch_typed<uint32_t, KC_UNSIGNED>(k0, k1, v0, v1, n, begin_bit, end_bit, plan, sc, report, rest, stream); break;
+        case B40C_KEY_I32: launch_typed<uint32_t, KC_SIGNED>(k0, k1, v0, v1, n, begin_bit, end_bit, plan, sc, report, rest, stream); break;
+        case B40C_KEY_F32: launch_typed<uint32_t, KC_FLOAT>(k0, k1, v0, v1, n, begin_bit, end_bit, plan, sc, report, rest, stream); break;
+        case B40C_KEY_U64: launch_typed<uint64_t, KC_UNSIGNED>(k0, k1, v0, v1, n, begin_bit, end_bit, plan, sc, report, rest, stream); break;
+        case B40C_KEY_I64: launch_typed<uint64_t, KC_SIGNED>(k0, k1, v0, v1, n, begin_bit, end_bit, plan, sc, report, rest, stream); break;
+        case B40C_KEY_F64: launch_typed<uint64_t, KC_FLOAT>(k0, k1, v0, v1, n, begin_bit, end_bit, plan, sc, report, rest, stream); break;
         default: return fail(B40C_ERR_INVALID_ARG, "radix sort: unknown key type %d", key_type);
     }
     B40C_HIP(hipGetLastError());
@@ -804,16 +866,24 @@ static b40c_status radix_sort_sync(int32_t key_type, void* k0, void* k1, uint32_
                                    const SortScratch& sc, int32_t* selector, hipStream_t stream, bool pinned = true) {
     SortReport report;
     report.take(sc, pinned);
-    const b40c_status launched =
-        radix_sort_launch(key_type, k0, k1, v0, v1, n, begin_bit, end_bit, num_cus, pol, sc, report.dev, stream);
-    if (launched != B40C_OK) {
-        // Some kernels may be on their way: the report is theirs until they end.
-        (void)hipStreamSynchronize(stream);
-        return launched;
-    }
+    SortRest rest;
     int32_t words[2] = {0, 0};
-    B40C_TRY(report.wait(words, stream));
-    if (words[1]) return fail(B40C_ERR_HIP, "radix sort: a block waited too long for the blocks before it");
+    do {
+        const b40c_status launched = radix_sort_launch(key_type, k0, k1, v0, v1, n, begin_bit, end_bit, num_cus, pol,
+                                                       sc, report.dev, rest, stream);
+        if (launched != B40C_OK) {
+            // Some kernels may be on their way: the report is theirs until they end.
+            (void)hipStreamSynchronize(stream);
+            return launched;
+        }
+        B40C_TRY(report.wait(words, stream));
+        if (words[1]) {  // a place later each time
+            rest.place = words[1] - 1;
+            const uint32_t* unfinished = sort_state(sc, SortPlan{}, 0, nullptr).failed + 1;
+            B40C_HIP(hipMemcpyAsync(&rest.blocks, unfinished, sizeof(rest.blocks), hipMemcpyDeviceToHost, stream));
+            B40C_HIP(hipStreamSynchronize(stream));
+        }
+    } while (words[1]);
     *selector = words[0];
     return B40C_OK;
 }

@@ -427,33 +427,6 @@ void case_sorts() {
     for (size_t n : {1000, 9000, 30001}) sort_pairs(n, 20);
 }
 
-// A place whose second block starts after a server's bounded wait has run out: the
-// sort fails, and the places after it, whose digit totals no longer hold, write
-// nothing outside the arrays.
-void case_sort_wait_runs_out() {
-    emu::dev().chain_spins = 50;
-    std::atomic<int> places{0}, servers_ended{0};
-    emu::dev().on_start = [&](const std::string& k, unsigned id) {
-        if (k.find("k_place") == std::string::npos || id != 16 + 1) return;
-        if (places++ == 0)
-            while (servers_ended.load() == 0) sched_yield();
-    };
-    emu::dev().on_end = [&](const std::string& k, unsigned id) {
-        if (k.find("k_place") != std::string::npos && id < 16) ++servers_ended;
-    };
-    const size_t n = 20000;
-    const std::vector<uint64_t> k = random_keys(n, 64, 5);
-    DeviceArray<uint64_t> a(k), b(n);
-    int32_t sel = -1;
-    const b40c_status s = b40c_radix_sort_u64(a.ptr(), b.ptr(), (int64_t)n, 0, 64, &sel);
-    REQUIRE(places > 1, "the sort took no second place");
-    REQUIRE(s == B40C_ERR_HIP, "the sort returned %d", (int)s);
-    emu::dev().chain_spins = 1u << 22;
-    emu::dev().on_start = nullptr;
-    emu::dev().on_end = nullptr;
-    sort_u64(n, 64);
-}
-
 // A small device that runs 20 workgroups at a time: every block of a place whose
 // turn has come can start, whatever the others wait for.
 void case_sort_few_resident() {
@@ -560,25 +533,32 @@ void case_primitives() {
 }
 
 // Calls `f` while the workgroup `late` of every kernel whose name holds `kernel`
-// starts only when a workgroup below `servers` has ended, which it does only by
-// giving up waiting; returns how often that happened.
-int with_late_workgroup(const char* kernel, unsigned late, unsigned servers, const std::function<void()>& f) {
-    std::atomic<int> gave_up{0}, held{0};
+// (in the first launch only, or in every one) starts only when a workgroup that
+// depends on it has ended, which it does only by giving up waiting: one of the
+// serving ones (below `servers`) if `late` is a block, a block if it serves.
+// Returns how often that happened.
+int with_late_workgroup(const char* kernel, unsigned late, unsigned servers, bool every, const std::function<void()>& f) {
+    std::atomic<unsigned> ended{0}, highest{0};
+    std::atomic<int> launches{0};
     emu::dev().chain_spins = 50;
     emu::dev().on_start = [&](const std::string& k, unsigned id) {
         if (k.find(kernel) == std::string::npos || id != late) return;
-        const int before = gave_up.load();
-        if (held++ == 0)
-            while (gave_up.load() == before) sched_yield();
+        const unsigned before = (unsigned)launches++;
+        if (before && !every) return;
+        const unsigned each = late < servers ? highest.load() + 1 - servers : servers;
+        while (ended.load() <= before * each) sched_yield();
     };
     emu::dev().on_end = [&](const std::string& k, unsigned id) {
-        if (k.find(kernel) != std::string::npos && id < servers) ++gave_up;
+        if (k.find(kernel) == std::string::npos) return;
+        for (unsigned h = highest; h < id && !highest.compare_exchange_weak(h, id);) {
+        }
+        if ((id < servers) != (late < servers)) ++ended;
     };
     f();
     emu::dev().chain_spins = 1u << 14;
     emu::dev().on_start = nullptr;
     emu::dev().on_end = nullptr;
-    return held.load();
+    return launches.load();
 }
 
 // Chained calls one of whose blocks starts after the serving workgroup has given
@@ -599,19 +579,57 @@ void case_late_blocks() {
         std::printf("workgroup %u late\n", late);
         std::fflush(stdout);
         DeviceArray<uint32_t> in(x);
-        const int scans = with_late_workgroup("k_scan_chained", late, 1, [&] {
+        const int scans = with_late_workgroup("k_scan_chained", late, 1, false, [&] {
             uint64_t total = 0;
             OK(b40c_scan_u32(in.ptr(), in.ptr(), (int64_t)n, 1, &total));
             REQUIRE(total == sum, "the total");
         });
         REQUIRE(scans > 0 && in.get(n) == y, "the scan");
         DeviceArray<uint64_t> ka(k), kb(n);
-        const int trims = with_late_workgroup("k_trim_chained", late, 1, [&] {
+        const int trims = with_late_workgroup("k_trim_chained", late, 1, false, [&] {
             int64_t kept = 0;
             OK(b40c_consecutive_removal_u64(ka.ptr(), nullptr, kb.ptr(), nullptr, (int64_t)n, &kept));
             REQUIRE(kept == (int64_t)wk.size(), "%lld kept", (long long)kept);
         });
         REQUIRE(trims > 0 && kb.get(wk.size()) == wk, "the removal");
+        const HostGraph h = skewed_graph(12, 12, false, 3);
+        std::vector<int32_t> r, off((size_t)h.n + 1), cols((size_t)h.m());
+        for (int32_t v = 0; v < h.n; ++v) r.insert(r.end(), (size_t)(h.off[(size_t)v + 1] - h.off[(size_t)v]), v);
+        b40c_graph* g = nullptr;
+        const int builds = with_late_workgroup("k_csr_chained", late, 1, false, [&] {
+            OK(b40c_graph_from_coo_unique(h.n, h.m(), r.data(), h.cols.data(), 0, &g));
+        });
+        OK(b40c_graph_copy_to_host(g, off.data(), cols.data()));
+        REQUIRE(builds > 0 && off == h.off && cols == h.cols, "the CSR");
+        b40c_graph_destroy(g);
+    }
+}
+
+// Sorts one of whose workgroups starts in each place only after those that need it
+// have given up: a block or a serving workgroup, with blocks of one tile and of
+// several, with values, and in the fixed scratch.
+void case_late_sorts() {
+    const char* place = "k_place<K, CONV, VALS, ITEMS, false>";
+    for (unsigned late : {16u, 17u, 19u, 3u}) {
+        std::printf("workgroup %u late\n", late);
+        std::fflush(stdout);
+        const int places = with_late_workgroup(place, late, 16, true, [] { sort_u64(20000, 64); });
+        REQUIRE(places > 8, "%d launches of places", places);
+        REQUIRE(with_late_workgroup(place, late, 16, true, [] { sort_pairs(20000, 20); }) > 3, "no place was late");
+        b40c_sort_enactor* e = nullptr;
+        OK(b40c_sort_enactor_create(&e));
+        OK(b40c_sort_enactor_set_policy(e, 8, 1));
+        REQUIRE(with_late_workgroup(place, late, 16, true, [&] { sort_u64(70000, 40, e); }) > 5, "no place was late");
+        sort_u64(70000, 40, e);
+        b40c_sort_enactor_destroy(e);
+        const size_t n = 30011;
+        std::vector<uint64_t> k = random_keys(n, 12, 3);
+        DeviceArray<uint64_t> a(k), b(n);
+        int32_t sel = -1;
+        with_late_workgroup(place, late, 16, true,
+                            [&] { OK(b40c_radix_sort_u64_noalloc(a.ptr(), b.ptr(), (int64_t)n, 0, 12, &sel)); });
+        std::sort(k.begin(), k.end());
+        REQUIRE((sel ? b : a).get(n) == k, "the sort in the fixed scratch");
     }
 }
 
@@ -801,8 +819,6 @@ int main(int argc, char** argv) {
         case_shared_problem(arg(0));
     else if (name == "sorts")
         case_sorts();
-    else if (name == "sort_wait_runs_out")
-        case_sort_wait_runs_out();
     else if (name == "sort_few_resident")
         case_sort_few_resident();
     else if (name == "sort_grouped")
@@ -815,6 +831,8 @@ int main(int argc, char** argv) {
         case_primitives();
     else if (name == "late_blocks")
         case_late_blocks();
+    else if (name == "late_sorts")
+        case_late_sorts();
     else if (name == "scan_segments")
         case_scan_segments();
     else if (name == "builds")

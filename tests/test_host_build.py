@@ -77,12 +77,6 @@ def test_search_depth_with_a_late_first_workgroup(check):
     check("late_first_workgroup")
 
 
-def test_sort_whose_wait_runs_out(check):
-    """A sort that fails in its first place writes nothing outside its arrays in
-    the later ones, and the next sort is right."""
-    check("sort_wait_runs_out")
-
-
 @pytest.mark.parametrize("case", ["sort_few_resident", "sort_grouped"])
 def test_sort_progress(check, case):
     """A place ends whatever waits for whatever: 20 workgroups at a time on a
@@ -137,7 +131,13 @@ def test_average_duty(check):
 
 
 def test_late_blocks(check):
-    """Scans and removals where a block cannot start while the others wait for
+    """Scans, removals and CSR builds where a block cannot start while the others wait for
     it (as beside a persistent kernel that holds the GPU): the call finishes what
     gave up; it failed."""
     check("late_blocks")
+
+
+def test_late_sorts(check):
+    """The same of sorts, where such a place failed and the later ones moved
+    nothing; a serving workgroup may be the one that cannot start."""
+    check("late_sorts")
