@@ -25,9 +25,11 @@ constexpr int CHAIN_STRIDE = 8;
 // No wait needs to end.  A chained kernel and a persistent one that are each
 // partly resident keep the other's missing workgroups off the GPU (XCDs dispatch
 // on their own, so even a block's predecessors may be missing).  The serving
-// workgroup gives up after this many polls without a new sum (about 15 ms; a
-// poll is 0.7 us and a whole scan of 2^28 elements 0.5 ms); the blocks then list
-// themselves and leave, and the host finishes them when all sums are there.
+// workgroup gives up after kChainSpins polls without a new sum, a block after a
+// quarter of them without its prefix (about 11 and 3 ms; a poll is 0.7 us and a whole
+// scan of 2^28 elements 0.5 ms).  Such blocks list themselves and leave, and the
+// host finishes them when all sums are there.  (Blocks that also looked whether the
+// server had given up made a scan of 2^26 elements 1 to 2 us slower.)
 constexpr uint32_t kChainSpins = 1u << 14;
 
 // Report of a chained call.
@@ -38,9 +40,8 @@ struct ChainReport {
 
 // Device words of a chained call beside the blocks' words.
 struct ChainMeta {
-    uint64_t before;      // where the serving workgroup stopped: the sum,
+    uint64_t before;      // where the serving workgroup gave up: the sum,
     int32_t base;         // and the first block without its prefix
-    uint32_t gone;        // it gave up
     uint32_t unfinished;  // blocks in the list
 };
 
@@ -77,7 +78,7 @@ __device__ __forceinline__ void chain_store(const Chain& c, int b, unsigned long
 __global__ __launch_bounds__(CHAIN_THREADS) void k_chain_init(Chain c) {
     for (int i = blockIdx.x * CHAIN_THREADS + threadIdx.x; i < c.blocks; i += gridDim.x * CHAIN_THREADS)
         c.words[(size_t)i * CHAIN_STRIDE] = 0;
-    if (blockIdx.x == 0 && threadIdx.x == 0) *c.meta = ChainMeta{c.before, 0, 0u, 0u};
+    if (blockIdx.x == 0 && threadIdx.x == 0) *c.meta = ChainMeta{c.before, 0, 0u};
 }
 
 struct ChainServeShared {
@@ -133,12 +134,12 @@ __device__ __forceinline__ void chain_serve(const Chain& c, ChainServeShared& s,
         }
     }
     if (tid == 0) {
-        c.report->total = before;
-        c.meta->before = before;
-        c.meta->base = base;
         if (base < c.blocks) {
-            st_relaxed(&c.meta->gone, 1u);
+            c.meta->before = before;
+            c.meta->base = base;
             c.report->open = 1;
+        } else {
+            c.report->total = before;
         }
     }
 }
@@ -152,7 +153,7 @@ __device__ __forceinline__ unsigned long long chain_before(const Chain& c, int b
     unsigned long long w;
     uint32_t spins = 0;
     while ((w = chain_load(c, block)) < CHAIN_PREFIX) {
-        if ((++spins % 16 == 0 && ld_relaxed(&c.meta->gone)) || spins > 4 * kChainSpins) {
+        if (++spins > kChainSpins / 4) {
             c.report->open = 1;
             const uint32_t at = atomic_add_u32(&c.meta->unfinished, 1u);
             c.words[(size_t)at * CHAIN_STRIDE + 1] = (unsigned long long)block;
@@ -165,6 +166,7 @@ __device__ __forceinline__ unsigned long long chain_before(const Chain& c, int b
 
 __global__ __launch_bounds__(CHAIN_THREADS) void k_chain_resume(Chain c) {
     __shared__ ChainServeShared s;
+    if (chain_load(c, c.blocks - 1) >= CHAIN_PREFIX) return;  // only blocks gave up
     chain_serve(c, s, c.meta->before, c.meta->base);
 }
 

@@ -371,7 +371,7 @@ __device__ __forceinline__ W await_start(const W* status, int block, int d, cons
     W w;
     uint32_t spins = 0;
     while ((w = chain_load(status, block, d)) < ChainWord<W>::START) {
-        if (++spins % 16 == 0 && (ld_relaxed(st.failed) || spins > 4 * kChainSpins)) {
+        if (++spins % 256 == 0 && (ld_relaxed(st.failed) || spins > 4 * kChainSpins)) {
             place_failed(st, place);
             return 0;
         }
