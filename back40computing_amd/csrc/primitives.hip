@@ -172,11 +172,12 @@ constexpr int64_t kChainScanMax = 1ll << 30;  // sums of 32-bit values stay belo
 constexpr int SCAN_SUB = 8;
 constexpr int64_t SCAN_BLOCK = (int64_t)PT * VEC32 * SCAN_SUB;
 
-// Arrays are scanned in segments of at most kScanSegment elements, one after the
-// other: their chain words stay below 2 MB, which
-// the runtime serves from chunks it keeps (8 us after an upload).  More are mapped
-// anew on every call: 2^28 elements in place after an upload took 790 us, with
-// 550 to 610 in segments, as three passes 650 to 730.
+// Arrays are scanned in segments of at most kScanSegment elements, each after a wait
+// for the one before: their chain words stay below 2 MB, which the runtime serves
+// from chunks it keeps (8 us after an upload).  More are mapped anew on every call:
+// 2^28 elements in place after an upload took 750 to 870 us, in segments 560 to 730,
+// as three passes 650 to 730 (2^29 elements in a loop: 996 us in segments, 988 in one
+// launch).
 constexpr int64_t kScanSegment = (1ll << 28) - (1ll << 20);
 
 template <bool REST>
