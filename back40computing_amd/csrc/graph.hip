@@ -390,8 +390,9 @@ b40c_status csr_from_sorted_keys(const KeyArena& a, int64_t nkeys, int shift, ui
         ChainCall call;
         B40C_TRY(call.start(blocks, stream, a.scratch));
         B40C_TRY(call.run(blocks, 0, E, stream, [&](const Chain& chain, unsigned wgs, bool rest) {
-            hipLaunchKernelGGL(rest ? k_csr_chained<true> : k_csr_chained<false>, dim3(wgs), dim3(CHAIN_THREADS), 0, stream, a.k0, nkeys, shift, sentinel,
-                               n, reinterpret_cast<int32_t*>(a.k1), g->offsets.as<int32_t>(), chain);
+            hipLaunchKernelGGL(rest ? k_csr_chained<true> : k_csr_chained<false>, dim3(wgs), dim3(CHAIN_THREADS), 0,
+                               stream, a.k0, nkeys, shift, sentinel, n, reinterpret_cast<int32_t*>(a.k1),
+                               g->offsets.as<int32_t>(), chain);
         }));
     }
     if (E > 0x7FFFFFFFull)
